@@ -206,6 +206,69 @@ __global__ void k_sum_groups(const T *h, long per, int stride, unsigned long lon
     }
 }
 
+// Histograms on their way to the host.  The host's arrays are one per field
+// while a bin holds its fields side by side: n bins from b0 on leave as six
+// columns of n words (count as an integer, den, and the four sums) straight
+// into pinned host memory, so the link carries 48 of the bin's 64 bytes in
+// 512-byte runs per wave and no host pass takes the bins apart.  The PCIe
+// link bounds it: 413 526 bins (41^3 x 6) take 0.4 ms, 4.5 ms as a pageable
+// copy of the bins and a host loop over them.
+// cnt, den: per (K_T, K_phi) group of `per` bins, the sums of the counts and
+// of the denominators (the reference's pair counters), one atomic per wave
+// and group.  out null: the sums only.
+__global__ __launch_bounds__(256) void k_read_bins(const double *bins, long b0, int n, long per,
+                                                   unsigned long long *out,
+                                                   unsigned long long *cnt,
+                                                   unsigned long long *den) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const bool on = i < n;
+    const long k = b0 + min(i, n - 1);
+    const double *b = bins + k * BIN_STRIDE;
+    const unsigned long long c = (unsigned long long)b[BIN_COUNT];
+    const unsigned long long d = ((const unsigned long long *)b)[BIN_DEN];
+    if (out && on) {
+        const unsigned long long *w = (const unsigned long long *)b;
+        out[i] = c;
+        out[(long)n + i] = d;
+        out[2l * n + i] = w[BIN_QO];
+        out[3l * n + i] = w[BIN_QS];
+        out[4l * n + i] = w[BIN_QL];
+        out[5l * n + i] = w[BIN_NUM];
+    }
+    const int g = (int)(k / per);
+    unsigned long long sc = on ? c : 0ull, sd = on ? d : 0ull;
+    if (__builtin_amdgcn_readfirstlane(g) == __builtin_amdgcn_readlane(g, 63)) {
+        for (int off = 32; off > 0; off >>= 1) {
+            sc += __shfl_down(sc, off);
+            sd += __shfl_down(sd, off);
+        }
+        if (__lane_id() != 0) return;
+    }
+    if (sc) atomic_add_u64(&cnt[g], sc);
+    if (sd) atomic_add_u64(&den[g], sd);
+}
+
+// The rest of a result, into pinned host memory: the groups' pair counters,
+// the q_inv arrays, and the q_inv counters per K_T bin (one wave each).
+__global__ __launch_bounds__(256) void k_read_tail(const unsigned long long *sums, int nsums,
+                                                   DevHist H, int nq, int n_KT, int q,
+                                                   unsigned long long *out) {
+    unsigned long long *oq = out + nsums;
+    const unsigned long long *src[4] = {H.qinv_count, H.qinv_den,
+                                        (const unsigned long long *)H.qinv_sum,
+                                        (const unsigned long long *)H.qinv_num};
+    for (int i = threadIdx.x; i < nsums; i += 256) out[i] = sums[i];
+    for (int f = 0; f < 4; f++)
+        for (int i = threadIdx.x; i < nq; i += 256) oq[(long)f * nq + i] = src[f][i];
+    unsigned long long *oc = oq + 4l * nq;
+    for (int k = threadIdx.x >> 6; k < 2 * n_KT; k += 4) {
+        unsigned long long s = 0;
+        for (int i = __lane_id(); i < q; i += 64) s += src[k / n_KT][(long)(k % n_KT) * q + i];
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
+        if (__lane_id() == 0) oc[k] = s;
+    }
+}
+
 // ------------------------------------------------------------------ host
 
 // Fast-kernel records of one ordering of a slot (RecordSet on the device).
@@ -252,6 +315,9 @@ struct hbt_ctx {
     size_t stage_cap = 0;
     char *h_stage2 = nullptr;  // and fast-kernel records
     size_t stage2_cap = 0;
+    char *h_read = nullptr;    // pinned staging of results: kReadSlots chunks, then the tail
+    size_t read_cap = 0;
+    hipEvent_t read_ev[4] = {};
     int cu_count = 0;
     long nbins = 0, nq = 0;
     double *d_bins = nullptr;  // [nbins][BIN_STRIDE]
@@ -1517,7 +1583,7 @@ int hbt_create(const hbt_config *cfg, hbt_ctx **out) {
     if (!rc) rc = dev_alloc(cp, &c->d_qinv_num, c->nq);
     if (!rc) rc = dev_alloc(cp, &c->d_stage, 10);
     if (!rc) rc = dev_alloc(cp, &c->d_binned, 2);
-    if (!rc) rc = dev_alloc(cp, &c->d_sums, (size_t)k.n_KT * std::max(1, D.P.nphi));
+    if (!rc) rc = dev_alloc(cp, &c->d_sums, 2 * (size_t)k.n_KT * std::max(1, D.P.nphi));
     if (!rc) rc = dev_alloc(cp, &c->d_counter, (size_t)kQueueStride * kMaxQueues);
     if (!rc) rc = dev_alloc(cp, &c->d_view, 1);
     if (!rc) rc = dev_alloc(cp, &c->d_defer, kDeferCap);
@@ -1554,6 +1620,9 @@ int hbt_destroy(hbt_ctx *c) {
     if (c->stream) hipStreamDestroy(c->stream);
     if (c->h_stage) hipHostFree(c->h_stage);
     if (c->h_stage2) hipHostFree(c->h_stage2);
+    if (c->h_read) hipHostFree(c->h_read);
+    for (auto &ev : c->read_ev)
+        if (ev) hipEventDestroy(ev);
     delete c;
     return HBT_OK;
 }
@@ -1902,45 +1971,70 @@ int hbt_last_kernel_ms(hbt_ctx *c, double *same_ms, double *mixed_ms) {
     return HBT_OK;
 }
 
+// Results leave in chunks of bins through kReadSlots pinned slots: while the
+// link fills one, the host pool copies another into the caller's arrays
+// (first touched there, so their page faults are spread over its threads).
+// A chunk is a quarter of the bins, at least 8192 and at most 65536 (3 MB):
+// larger ones only add to the first chunk's latency, smaller ones to the
+// launches.
 int hbt_read(hbt_ctx *c, hbt_result *o) {
     if (!c || !o) return HBT_ERR_ARG;
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    {
-        const int rc = resolve_deferred(c);
-        if (rc) return rc;
-    }
-    const size_t q8 = (size_t)c->nq * 8;
-    if (o->num_count || o->den || o->q_out_sum || o->q_side_sum || o->q_long_sum || o->num) {
-        std::vector<double> aos((size_t)c->nbins * BIN_STRIDE);
-        HIPCHECK(c, hipMemcpy(aos.data(), c->d_bins, aos.size() * 8, hipMemcpyDeviceToHost));
-        for (long k = 0; k < c->nbins; k++) {
-            const double *b = aos.data() + k * BIN_STRIDE;
-            if (o->num_count) o->num_count[k] = (uint64_t)b[BIN_COUNT];
-            if (o->den) std::memcpy(&o->den[k], b + BIN_DEN, 8);
-            if (o->q_out_sum) o->q_out_sum[k] = b[BIN_QO];
-            if (o->q_side_sum) o->q_side_sum[k] = b[BIN_QS];
-            if (o->q_long_sum) o->q_long_sum[k] = b[BIN_QL];
-            if (o->num) o->num[k] = b[BIN_NUM];
-        }
-    }
-    struct {
-        void *dst;
-        const void *src;
-    } cp[] = {{o->qinv_count, c->d_qinv_count}, {o->qinv_den, c->d_qinv_den},
-              {o->qinv_sum, c->d_qinv_sum},     {o->qinv_num, c->d_qinv_num}};
-    for (auto &x : cp)
-        if (x.dst) HIPCHECK(c, hipMemcpy(x.dst, x.src, q8, hipMemcpyDeviceToHost));
-    const int nKT = c->cfg.n_KT, nphi = c->P.nphi;
+    if (int rc = resolve_deferred(c)) return rc;
+    constexpr int kReadSlots = sizeof(c->read_ev) / sizeof(c->read_ev[0]);
+    const int nKT = c->cfg.n_KT, nphi = c->P.nphi, groups = nKT * nphi;
     const long per = (long)c->P.qnpts * c->P.qnpts * c->P.qnpts;
-    std::vector<unsigned long long> sn, sd, qn, qd;
-    int rc = group_sums(c, (const double *)(c->d_bins + BIN_COUNT), per, nKT * nphi,
-                        BIN_STRIDE, sn);
-    if (!rc)
-        rc = group_sums(c, (const unsigned long long *)(c->d_bins + BIN_DEN), per, nKT * nphi,
-                        BIN_STRIDE, sd);
-    if (!rc) rc = group_sums(c, c->d_qinv_count, c->P.qnpts, nKT, 1, qn);
-    if (!rc) rc = group_sums(c, c->d_qinv_den, c->P.qnpts, nKT, 1, qd);
-    if (rc) return rc;
+    void *dst[6] = {o->num_count, o->den,        o->q_out_sum,
+                    o->q_side_sum, o->q_long_sum, o->num};
+    bool want = false;
+    for (void *p : dst) want = want || p;
+    const int chunk =
+        (int)std::min(c->nbins, std::min(65536l, std::max(8192l, (c->nbins / 4 + 255) / 256 * 256)));
+    const int nchunks = (int)((c->nbins + chunk - 1) / chunk);
+    const size_t slot_bytes = want ? (size_t)chunk * 48 : 0;
+    const size_t tail_words = 2 * (size_t)groups + 4 * (size_t)c->nq + 2 * (size_t)nKT;
+    HIPCHECK(c, ensure_pinned(&c->h_read, &c->read_cap, kReadSlots * slot_bytes + tail_words * 8));
+    for (auto &e : c->read_ev)
+        if (!e) HIPCHECK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    unsigned long long *tail = (unsigned long long *)(c->h_read + kReadSlots * slot_bytes);
+    HIPCHECK(c, launch_zero_words(c->d_sums, 2 * (size_t)groups, c->stream));
+    auto launch = [&](int k) -> hipError_t {
+        const long b0 = (long)k * chunk;
+        const int n = (int)std::min<long>(chunk, c->nbins - b0);
+        char *slot = c->h_read + (size_t)(k % kReadSlots) * slot_bytes;
+        hipLaunchKernelGGL(k_read_bins, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_bins,
+                           b0, n, per, want ? (unsigned long long *)slot : nullptr, c->d_sums,
+                           c->d_sums + groups);
+        if (k == nchunks - 1)
+            hipLaunchKernelGGL(k_read_tail, dim3(1), dim3(256), 0, c->stream, c->d_sums,
+                               2 * groups, hist_view(c), (int)c->nq, nKT, c->P.qnpts, tail);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : hipEventRecord(c->read_ev[k % kReadSlots], c->stream);
+    };
+    for (int k = 0; k < nchunks && (k < kReadSlots || !want); k++) HIPCHECK(c, launch(k));
+    for (int k = 0; k < nchunks && want; k++) {
+        HIPCHECK(c, hipEventSynchronize(c->read_ev[k % kReadSlots]));
+        const long b0 = (long)k * chunk;
+        const long n = std::min<long>(chunk, c->nbins - b0);
+        const unsigned long long *src =
+            (const unsigned long long *)(c->h_read + (size_t)(k % kReadSlots) * slot_bytes);
+        // words [w0, w1) of the slot's six columns, 32 KB a thread at least
+        parallel_ranges(6 * n, 4096, [&](long long w0, long long w1) {
+            while (w0 < w1) {
+                const long f = (long)(w0 / n), i = (long)(w0 - f * n);
+                const long m = std::min<long>(n - i, (long)(w1 - w0));
+                if (dst[f])
+                    std::memcpy((char *)dst[f] + (b0 + i) * 8, src + f * n + i, (size_t)m * 8);
+                w0 += m;
+            }
+        });
+        if (k + kReadSlots < nchunks) HIPCHECK(c, launch(k + kReadSlots));
+    }
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    const unsigned long long *sn = tail, *sd = tail + groups, *qi = tail + 2 * (size_t)groups;
+    const unsigned long long *qn = qi + 4 * c->nq, *qd = qn + nKT;
+    void *qdst[4] = {o->qinv_count, o->qinv_den, o->qinv_sum, o->qinv_num};
+    for (int f = 0; f < 4; f++)
+        if (qdst[f]) std::memcpy(qdst[f], qi + (size_t)f * c->nq, (size_t)c->nq * 8);
     for (int k = 0; k < nKT; k++) {
         uint64_t a = 0, b = 0;
         for (int p = 0; p < nphi; p++) {
@@ -1954,7 +2048,7 @@ int hbt_read(hbt_ctx *c, hbt_result *o) {
         if (o->cnt_den_qinv) o->cnt_den_qinv[k] = qd[k];
     }
     if (c->P.azimuthal) {
-        for (int k = 0; k < nKT * nphi; k++) {
+        for (int k = 0; k < groups; k++) {
             if (o->cnt_num_ktphi) o->cnt_num_ktphi[k] = sn[k];
             if (o->cnt_den_ktphi) o->cnt_den_ktphi[k] = sd[k];
         }

@@ -12,6 +12,7 @@
 #include <cstring>
 #include <functional>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <type_traits>
@@ -579,20 +580,33 @@ inline void result_from_host(const Derived &d, const hbt_config &k, const double
     const long per = (long)P.qnpts * P.qnpts * P.qnpts;
     const int nKT = k.n_KT, nphi = P.nphi;
     std::vector<unsigned long long> sn((size_t)nKT * nphi, 0), sd((size_t)nKT * nphi, 0);
-    for (long b = 0; b < d.nbins; b++) {
-        const double *x = aos + b * BIN_STRIDE;
-        unsigned long long den;
-        const unsigned long long cnt = (unsigned long long)x[BIN_COUNT];
-        std::memcpy(&den, x + BIN_DEN, 8);
-        sn[b / per] += cnt;
-        sd[b / per] += den;
-        if (o->num_count) o->num_count[b] = cnt;
-        if (o->den) o->den[b] = den;
-        if (o->q_out_sum) o->q_out_sum[b] = x[BIN_QO];
-        if (o->q_side_sum) o->q_side_sum[b] = x[BIN_QS];
-        if (o->q_long_sum) o->q_long_sum[b] = x[BIN_QL];
-        if (o->num) o->num[b] = x[BIN_NUM];
-    }
+    // bin ranges on the host pool (16 threads: 26 MB of bins and the first
+    // touch of the caller's arrays take 0.9 ms, 3.9 ms on one)
+    std::mutex mu;
+    parallel_ranges(d.nbins, 1 << 13, [&](long long b0, long long b1) {
+        while (b0 < b1) {
+            const long long g = b0 / per, end = std::min(b1, (g + 1) * per);
+            unsigned long long tn = 0, td = 0;
+            for (long long b = b0; b < end; b++) {
+                const double *x = aos + b * BIN_STRIDE;
+                unsigned long long den;
+                const unsigned long long cnt = (unsigned long long)x[BIN_COUNT];
+                std::memcpy(&den, x + BIN_DEN, 8);
+                tn += cnt;
+                td += den;
+                if (o->num_count) o->num_count[b] = cnt;
+                if (o->den) o->den[b] = den;
+                if (o->q_out_sum) o->q_out_sum[b] = x[BIN_QO];
+                if (o->q_side_sum) o->q_side_sum[b] = x[BIN_QS];
+                if (o->q_long_sum) o->q_long_sum[b] = x[BIN_QL];
+                if (o->num) o->num[b] = x[BIN_NUM];
+            }
+            std::lock_guard<std::mutex> lk(mu);
+            sn[(size_t)g] += tn;
+            sd[(size_t)g] += td;
+            b0 = end;
+        }
+    });
     const size_t q8 = (size_t)d.nq * 8;
     if (o->qinv_count) std::memcpy(o->qinv_count, qc, q8);
     if (o->qinv_den) std::memcpy(o->qinv_den, qd, q8);

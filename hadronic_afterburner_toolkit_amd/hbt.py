@@ -439,11 +439,13 @@ def _alloc_results(p, nphi):
     nkt = int(p["n_KT"])
     nb = nkt * nphi * q ** 3
     nq = nkt * q
+    # the histograms are written in full by the library; the counters of the
+    # analyses that are off stay 0
     r = Results(
-        num_count=np.zeros(nb, np.uint64), den=np.zeros(nb, np.uint64),
-        q_out_sum=np.zeros(nb), q_side_sum=np.zeros(nb), q_long_sum=np.zeros(nb),
-        num=np.zeros(nb), qinv_count=np.zeros(nq, np.uint64),
-        qinv_den=np.zeros(nq, np.uint64), qinv_sum=np.zeros(nq), qinv_num=np.zeros(nq),
+        num_count=np.empty(nb, np.uint64), den=np.empty(nb, np.uint64),
+        q_out_sum=np.empty(nb), q_side_sum=np.empty(nb), q_long_sum=np.empty(nb),
+        num=np.empty(nb), qinv_count=np.empty(nq, np.uint64),
+        qinv_den=np.empty(nq, np.uint64), qinv_sum=np.empty(nq), qinv_num=np.empty(nq),
         cnt_num_kt=np.zeros(nkt, np.uint64), cnt_den_kt=np.zeros(nkt, np.uint64),
         cnt_num_qinv=np.zeros(nkt, np.uint64), cnt_den_qinv=np.zeros(nkt, np.uint64),
         cnt_num_ktphi=np.zeros(nkt * nphi, np.uint64),
