@@ -125,7 +125,7 @@ __device__ __forceinline__ int cap_same_pair(const DevParams &P, const DevHist &
     r.qs = b.q_side;
     r.ql = b.q_long;
     r.c = cos_qx;
-    add_same_direct(H, r);
+    add_same_direct(H.bins, r);
     return st;
 }
 
@@ -154,7 +154,7 @@ __device__ __forceinline__ int cap_mixed_pair(const DevParams &P, const DevHist 
     if (qinv_ok && admitted(C.cutq[b.kt], gi, pos))
         atomic_add_u64(&H.qinv_den[(long)b.kt * P.qnpts + (qinv_ok - 1)], 1ull);
     if (!bin || !admitted(C.cut3[key3_of(P, b)], gi, pos)) return st & ~ST_BIN;
-    add_mixed_direct(H, bin_index(P, b.kt, b.kphi, b.io, b.is, b.il));
+    add_mixed_direct(H.bins, bin_index(P, b.kt, b.kphi, b.io, b.is, b.il));
     return st;
 }
 

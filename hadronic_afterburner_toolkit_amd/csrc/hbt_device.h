@@ -32,7 +32,11 @@ struct DevParams {
     double pf_mid;
     float f_half, f_h2, f_midh2, f_negc, f_mid, f_pad;
     // precision-form exact-stage constants
-    double inv_dKT, inv_dq, inv_two_pi, two_pi_hi, two_pi_lo, inv_dKphi;
+    // (bin coordinates raised by one: kt_scale * 2 K_perp + kt_off, inv_dq * q
+    // + q_off; a pair with one within `guard` of an integer takes the literal
+    // cascade)
+    double kt_scale, kt_off, inv_dq, q_off, guard;
+    double inv_two_pi, two_pi_hi, two_pi_lo, inv_dKphi;
     // K_phi angles closer than this (rad) to a bin edge, 0 or 2 pi are
     // decided on the host with glibc's atan2 (the device's may differ from it
     // in the last bits)
@@ -102,7 +106,8 @@ __device__ __forceinline__ void atomic_add_f64(double *p, double v) {
     unsafeAtomicAdd(p, v);
 }
 
-__host__ __device__ __forceinline__ long bin_index(const DevParams &P, int kt, int kphi, int io,
+template <typename Params>
+__host__ __device__ __forceinline__ long bin_index(const Params &P, int kt, int kphi, int io,
                                                    int is, int il) {
     const long q = P.qnpts;
     return ((((long)kt * P.nphi + kphi) * q + io) * q + is) * q + il;
@@ -251,6 +256,7 @@ struct SameRec {
     long k;
     double qo, qs, ql, c;
     int s, is, il;  // slab (K_T, K_phi, q_out plane) and q_side, q_long bins of k
+    bool sure;      // every coordinate at least DevParams::guard from a bin edge
 };
 
 // Same-event pair: cascade and cos (HBT_correlation.cpp:339-356, :431-446).
@@ -265,6 +271,7 @@ __device__ __forceinline__ int eval_same_f64(const DevParams &P, const DevHist &
     PairBins b;
     double q_inv;
     int qinv_ok;
+    rec.sure = false;
     int st = cascade_f64<false, EXT>(P, p1x, p1y, p1z, p1E, p2x, p2y, p2z, p2E, psi_ref, b,
                                      q_inv, qinv_ok);
     if (!(st & (ST_BIN | ST_DEFER)) && !qinv_ok) return st;
@@ -321,8 +328,8 @@ __device__ __forceinline__ int eval_mixed_f64(const DevParams &P, const DevHist 
 }
 
 // Direct accumulation of one pair (HBT_correlation.cpp:437-446, :681-683).
-__device__ __forceinline__ void add_same_direct(const DevHist &H, const SameRec &r) {
-    double *b = H.bins + r.k * BIN_STRIDE;
+__device__ __forceinline__ void add_same_direct(double *bins, const SameRec &r) {
+    double *b = bins + r.k * BIN_STRIDE;
     atomic_add_f64(b + BIN_COUNT, 1.0);
     atomic_add_f64(b + BIN_QO, r.qo);
     atomic_add_f64(b + BIN_QS, r.qs);
@@ -333,8 +340,8 @@ __device__ __forceinline__ void add_same_direct(const DevHist &H, const SameRec 
 // word, with the carry added to the high word by the add that wraps: the
 // value stays exact, and 32-bit adds cost ~14 % less at the memory side,
 // where histogram atomics are executed.
-__device__ __forceinline__ void add_mixed_direct(const DevHist &H, long k) {
-    unsigned *lo = (unsigned *)(H.bins + k * BIN_STRIDE + BIN_DEN);  // little-endian low word
+__device__ __forceinline__ void add_mixed_direct(double *bins, long k) {
+    unsigned *lo = (unsigned *)(bins + k * BIN_STRIDE + BIN_DEN);  // little-endian low word
     if (__hip_atomic_fetch_add(lo, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0xffffffffu)
         __hip_atomic_fetch_add(lo + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -348,7 +355,7 @@ __device__ __forceinline__ int bin_same_f64(const DevParams &P, const DevHist &H
     SameRec r;
     const int st = eval_same_f64<EXT>(P, H, psi_ref, p1x, p1y, p1z, p1E, x1, y1, z1, t1, p2x,
                                       p2y, p2z, p2E, x2, y2, z2, t2, r);
-    if (st & ST_BIN) add_same_direct(H, r);
+    if (st & ST_BIN) add_same_direct(H.bins, r);
     return st;
 }
 
@@ -359,7 +366,7 @@ __device__ __forceinline__ int bin_mixed_f64(const DevParams &P, const DevHist &
     long k = 0;
     const int st =
         eval_mixed_f64<EXT>(P, H, psi_ref, p1x, p1y, p1z, p1E, p2x, p2y, p2z, p2E, k);
-    if (st & ST_BIN) add_mixed_direct(H, k);
+    if (st & ST_BIN) add_mixed_direct(H.bins, k);
     return st;
 }
 

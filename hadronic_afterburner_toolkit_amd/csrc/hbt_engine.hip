@@ -7,8 +7,8 @@
 //   once.  Per slot: the particles kept by the rapidity cut in the
 //   reference's gather order, as eight FP64 arrays px,py,pz,E,x,y,z,t
 //   (64 B/particle); event offsets (int64, nev+1); group -> first event
-//   (int32, G+1); the fast kernel's prefilter records (PfRec64 32 B + cw
-//   8 B, PfRec32 16 B + cw 4 B per particle).
+//   (int32, G+1); the fast kernel's prefilter operands (PfOp 16 B, PfBeta
+//   8 B per particle).
 //   Mixing plan: per event e, rows [rowoff[e], rowoff[e+1]) each holding the
 //   partner event (global index in the mixed list) and cos, sin of its
 //   rotation.  Histograms: flat [kt][kphi][iqout][iqside][iqlong] (iqlong
@@ -17,7 +17,7 @@
 //
 // Kernels:
 //   k_same_plain / k_mixed_plain  LDS-tiled direct cascade (plain mode)
-//   k_fast<double|float, R>       persistent work-queue kernel: prefilter +
+//   k_fast<double|float>          persistent work-queue kernel: prefilter +
 //                                 compaction + exact cascade (hbt_fast.h);
 //                                 one launch covers every same-event and
 //                                 mixed pair of all resident groups
@@ -173,9 +173,9 @@ __global__ void k_apply_defer(const DeferAdd *a, int n) {
     H.bins = d.bins;
     if (d.kind == 0) {
         const SameRec r{d.k, d.v[1], d.v[2], d.v[3], d.v[4]};
-        add_same_direct(H, r);
+        add_same_direct(H.bins, r);
     } else {
-        add_mixed_direct(H, d.k);
+        add_mixed_direct(H.bins, d.k);
     }
 }
 
@@ -271,13 +271,11 @@ __global__ __launch_bounds__(256) void k_read_tail(const unsigned long long *sum
 
 // ------------------------------------------------------------------ host
 
-// Fast-kernel records of one ordering of a slot (RecordSet on the device).
+// One ordering of a slot's fast list on the device.
 struct DevRecords {
     PartRec *rec = nullptr;
-    PfRec64 *pf64 = nullptr;
-    PfRec32 *pf32 = nullptr;
-    double *cw64 = nullptr;
-    float *cw32 = nullptr;
+    PfOp *pf = nullptr;
+    PfBeta *bw = nullptr;
 };
 
 struct Slot {
@@ -460,7 +458,7 @@ void free_slot(Slot &s) {
     }
     if (s.d_off) hipFree(s.d_off);
     for (DevRecords *r : {&s.ev, &s.srt}) {
-        void *ptrs[] = {r->rec, r->pf64, r->pf32, r->cw64, r->cw32};
+        void *ptrs[] = {r->rec, r->pf, r->bw};
         for (void *q : ptrs)
             if (q) hipFree(q);
     }
@@ -635,19 +633,12 @@ View make_view(hbt_ctx *c) {
     const Slot &s1 = mixed_slot(c);
     v.A = s0.ev.rec;
     v.B = s1.ev.rec;
-    const bool f32 = c->cfg.precision == HBT_PREC_FP32C;
-    auto pf = [&](const DevRecords &r) {
-        return f32 ? (const void *)r.pf32 : (const void *)r.pf64;
-    };
-    auto cw = [&](const DevRecords &r) {
-        return f32 ? (const void *)r.cw32 : (const void *)r.cw64;
-    };
-    v.pfA = pf(s0.ev);
-    v.pfB = pf(s1.ev);
-    v.pfS = pf(s0.srt);
-    v.cwA = cw(s0.ev);
-    v.cwB = cw(s1.ev);
-    v.cwS = cw(s0.srt);
+    v.pfA = s0.ev.pf;
+    v.pfB = s1.ev.pf;
+    v.pfS = s0.srt.pf;
+    v.bwA = s0.ev.bw;
+    v.bwB = s1.ev.bw;
+    v.bwS = s0.srt.bw;
     v.origS = s0.d_orig;
     v.AS = s0.srt.rec;
     v.mwin = c->d_wins;
@@ -837,7 +828,7 @@ int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st) {
             return fail(c, HBT_ERR_STATE, "slab regions sized for another launch shape");
         HIPCHECK(c, launch_zero_words(a.slab.stats, (size_t)2 * a.slab.S + 1, st));
     }
-    HIPCHECK(c, launch_fast_kernel(a, f32, c->tune.R, c->P.qinv || c->P.azimuthal, blocks, st));
+    HIPCHECK(c, launch_fast_kernel(a, f32, c->P.qinv || c->P.azimuthal, blocks, st));
     if (slab) {
         const int nu = c->slab.nunits;
         if (f32)
@@ -943,8 +934,12 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
     // which keeps a group's items together): the persistent waves pull items
     // in queue order, so the launch ends on small items instead of one wave
     // finishing a large one (uneven multiplicities make items differ by 10x
-    // and more)
-    // (a counting sort over the 33 classes of a 64-bit count)
+    // and more).  Inside a class same-event and mixed items take turns in
+    // proportion to their numbers: the mixed items' denominator adds are bound
+    // by the memory-side atomic rate, the same-event items by arithmetic, and
+    // side by side they overlap.
+    // (a counting sort over the 33 classes of a 64-bit count, then a merge of
+    // the two kinds of each class)
     auto size_class = [&](size_t k) {
         int c = 0;
         for (uint64_t v = pairs[k]; v >= 4; v >>= 2) c++;
@@ -965,7 +960,19 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
         sorted[at] = L.items[k];
         spairs[at] = pairs[k];
     }
-    L.items.swap(sorted);
+    // (start[c] is now the end of class c's run: same-event items, then mixed)
+    for (size_t c = 0, b = 0; c < 33; b = start[c++]) {
+        const size_t e = start[c];
+        size_t i = b, m = b;
+        while (m < e && sorted[m].kind == 0) m++;
+        const size_t ns = m - b, nm = e - m;
+        for (size_t at = b, j = m; at < e; at++) {
+            const bool take_same = j == e || (i < m && (i - b) * nm <= (j - m) * ns);
+            const size_t k = take_same ? i++ : j++;
+            L.items[at] = sorted[k];
+            pairs[at] = spairs[k];
+        }
+    }
     // per-XCD queues where a group's records take at most 3/4 of one XCD's
     // L2, which also holds the mixed lists and the histogram lines (on the
     // bench workloads: 1 % on the headline's precision form, 3 % on the
@@ -976,9 +983,8 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
     long long maxg = 0;
     for (int g = 0; g < s.ngroups; g++)
         maxg = std::max(maxg, s.foff[(size_t)s.grp_ev[g + 1]] - s.foff[(size_t)s.grp_ev[g]]);
-    const bool f32 = c->cfg.precision == HBT_PREC_FP32C;
-    const size_t rec = sizeof(PartRec) + (f32 ? sizeof(PfRec32) + 4 : sizeof(PfRec64) + 8);
-    assign_queues(L, spairs, s.ngroups,
+    const size_t rec = sizeof(PartRec) + sizeof(PfOp) + sizeof(PfBeta);
+    assign_queues(L, pairs, s.ngroups,
                   (size_t)maxg * rec * 4 <= kL2BytesPerXcd * 3 ? kMaxQueues : 1);
 }
 
@@ -1360,7 +1366,7 @@ int prepare_and_capture(hbt_ctx *c) {
 // buffers, gathers the kept columns into the pinned staging buffer on
 // several threads and queues their copies (and the event offsets') on the
 // context's stream.
-int upload_columns(hbt_ctx *c, Slot &s, bool f32, int32_t nev, const HostParticles &h,
+int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
                    const double *const soa[8]) {
     int rc = quiesce(c);
     if (rc) return rc;
@@ -1377,13 +1383,11 @@ int upload_columns(hbt_ctx *c, Slot &s, bool f32, int32_t nev, const HostParticl
     }
     if ((size_t)nf > s.cap_f || !s.d_orig) {
         for (DevRecords *r : {&s.ev, &s.srt}) {
-            if (!rc) rc = dev_alloc(c, &r->rec, (size_t)nf);
-            if (!rc && !f32) rc = dev_alloc(c, &r->pf64, (size_t)nf);
-            if (!rc && f32) rc = dev_alloc(c, &r->pf32, (size_t)nf);
-            if (!rc && !f32) rc = dev_alloc(c, &r->cw64, (size_t)nf);
-            if (!rc && f32) rc = dev_alloc(c, &r->cw32, (size_t)nf);
+            if (!rc) rc = dev_alloc(c, &r->rec, (size_t)nf + kPfPad);
+            if (!rc) rc = dev_alloc(c, &r->pf, (size_t)nf + kPfPad);
+            if (!rc) rc = dev_alloc(c, &r->bw, (size_t)nf + kPfPad);
         }
-        if (!rc) rc = dev_alloc(c, &s.d_orig, (size_t)nf);
+        if (!rc) rc = dev_alloc(c, &s.d_orig, (size_t)nf + kPfPad);
         if (rc) return rc;
         s.cap_f = (size_t)nf;
     }
@@ -1419,14 +1423,13 @@ int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev
     HostParticles h;
     std::string err;
     Slot &s = c->slot[slot];
-    const bool f32 = c->cfg.precision == HBT_PREC_FP32C;  // prefilter records of one precision
     // Once the kept particles are known: wait for work queued on the stream
     // (a batch launched without hbt_sync may still read the slot and the
     // staging), size the device buffers, and queue the columns' copies, which
     // then run while the host sorts the fast lists by px.
     int hook_rc = HBT_OK;
     const std::function<int()> after_keep = [&]() -> int {
-        hook_rc = upload_columns(c, s, f32, nev, h, soa);
+        hook_rc = upload_columns(c, s, nev, h, soa);
         return hook_rc;
     };
     int rc = gather_particles(c->D, c->cfg, ngroups, grp_ev, nev, ev_off, soa, h, err, &after_keep);
@@ -1438,29 +1441,13 @@ int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev
     auto add = [&](void *dst, const void *src, size_t bytes) {
         if (dst && bytes) pieces.push_back(StagePiece{dst, src, bytes});
     };
-    if (nf > 0) {
-        const std::pair<DevRecords *, const RecordSet *> sets[] = {{&s.ev, &h.fast},
-                                                                   {&s.srt, &h.srt}};
-        for (const auto &x : sets) {
-            DevRecords &d = *x.first;
-            const RecordSet &r = *x.second;
-            // the srt set holds prefilter records only: its full records are
-            // gathered on the device below
-            if (x.first == &s.ev) add(d.rec, r.rec.data(), (size_t)nf * sizeof(PartRec));
-            if (f32) {
-                add(d.pf32, r.pf32.data(), (size_t)nf * sizeof(PfRec32));
-                add(d.cw32, r.cw32.data(), (size_t)nf * 4);
-            } else {
-                add(d.pf64, r.pf64.data(), (size_t)nf * sizeof(PfRec64));
-                add(d.cw64, r.cw64.data(), (size_t)nf * 8);
-            }
-        }
-        add(s.d_orig, h.orr.data(), (size_t)nf * sizeof(OrigRank));
-    }
+    add(s.ev.rec, h.fast.data(), (size_t)nf * sizeof(PartRec));
+    add(s.d_orig, h.orr.data(), (size_t)nf * sizeof(OrigRank));
     HIPCHECK(c, ensure_pinned(&c->h_stage2, &c->stage2_cap, stage_bytes(pieces)));
     HIPCHECK(c, stage_pieces(c->h_stage2, pieces, c->stream));
-    // the records in the cell-sorted order, for the exact stage of same-event pairs
-    HIPCHECK(c, gather_srt(s.ev.rec, s.d_orig, s.srt.rec, nf, c->stream));
+    // the prefilter's operands, and the records in the cell-sorted order
+    HIPCHECK(c, build_lists(pf_maker(c->D, h.bm), s.ev.rec, s.d_orig, s.srt.rec, s.ev.pf, s.ev.bw,
+                            s.srt.pf, s.srt.bw, nf, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     s.nf = nf;
     s.foff = std::move(h.foff);
@@ -1491,28 +1478,21 @@ int check_slots(hbt_ctx *c) {
 
 namespace hbt {
 
-hipError_t launch_fast_kernel(const FastArgs &a, bool f32, int R, bool ext, long blocks,
+hipError_t launch_fast_kernel(const FastArgs &a, bool f32, bool ext, long blocks,
                               hipStream_t st) {
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, a.counter, a.nqueues);
-    // the K_phi instance's slab fill counters live in dynamic LDS
-    const size_t dyn = ext && a.slab.vals ? (size_t)a.slab.S * sizeof(unsigned) : 0;
-    if (dyn > (size_t)kMaxSlabsKphi * sizeof(unsigned)) return hipErrorInvalidValue;
-#define HBT_LAUNCH(T, RR, X) \
-    hipLaunchKernelGGL((k_fast<T, RR, X>), dim3(blocks), dim3(256), dyn, st, a)
-#define HBT_LAUNCH_R(T, X)                    \
-    do {                                      \
-        if (R == 1) HBT_LAUNCH(T, 1, X);      \
-        else if (R == 4) HBT_LAUNCH(T, 4, X); \
-        else HBT_LAUNCH(T, 2, X);             \
-    } while (0)
-    if (f32) {
-        if (ext) HBT_LAUNCH_R(float, true);
-        else HBT_LAUNCH_R(float, false);
+    if (a.slab.vals && a.slab.S > (ext ? kMaxSlabsKphi : kMaxSlabs)) return hipErrorInvalidValue;
+    const size_t dyn = fast_dynamic_lds(a.slab, ext);
+#define HBT_LAUNCH(T, X) \
+    hipLaunchKernelGGL((k_fast<T, X>), dim3(blocks), dim3(256), dyn, st, a)
+    // (with the q_inv branch on every pair takes the literal cascade)
+    if (f32 && !a.P.qinv) {
+        if (ext) HBT_LAUNCH(float, true);
+        else HBT_LAUNCH(float, false);
     } else {
-        if (ext) HBT_LAUNCH_R(double, true);
-        else HBT_LAUNCH_R(double, false);
+        if (ext) HBT_LAUNCH(double, true);
+        else HBT_LAUNCH(double, false);
     }
-#undef HBT_LAUNCH_R
 #undef HBT_LAUNCH
     return hipGetLastError();
 }
@@ -1891,7 +1871,6 @@ int hbt_autotune(hbt_ctx *c, hbt_tuning *best_out) {
     if (c->cfg.binning == 2) c->slab_binning = false;
     // small j chunks and one window per mixed item give small batches
     // enough items to fill the chip; large ones amortize the per-item setup
-    const int Rs[] = {1, 2, 4};
     const int JCs[] = {256, 1024, 4096};
     const int KCs[] = {1, 4, 16};
     const int BPCs[] = {4, 8, 16};
@@ -1913,24 +1892,23 @@ int hbt_autotune(hbt_ctx *c, hbt_tuning *best_out) {
         c->slab_binning = slab;
         return upload_items(c, items);
     };
-    for (int R : Rs)
-        for (int jc : JCs)
-            for (int kc : KCs)
-                for (int bpc : BPCs) {
-                    const hbt_tuning t{R, jc, kc, bpc, 0.0};
-                    int rc = use(t, c->slab_binning);
+    for (int jc : JCs)
+        for (int kc : KCs)
+            for (int bpc : BPCs) {
+                const hbt_tuning t{1, jc, kc, bpc, 0.0};
+                int rc = use(t, c->slab_binning);
+                if (rc) return rc;
+                for (int m = 0; m < (both ? 2 : 1); m++) {
+                    if (both) c->slab_binning = m == 1;
+                    float ms = 0.f;
+                    rc = timed_fast(c, &ms);
+                    if (!rc) rc = timed_fast(c, &ms);
                     if (rc) return rc;
-                    for (int m = 0; m < (both ? 2 : 1); m++) {
-                        if (both) c->slab_binning = m == 1;
-                        float ms = 0.f;
-                        rc = timed_fast(c, &ms);
-                        if (!rc) rc = timed_fast(c, &ms);
-                        if (rc) return rc;
-                        hbt_tuning tm = t;
-                        tm.ms = ms;
-                        cands.push_back(Cand{tm, c->slab_binning});
-                    }
+                    hbt_tuning tm = t;
+                    tm.ms = ms;
+                    cands.push_back(Cand{tm, c->slab_binning});
                 }
+            }
     std::sort(cands.begin(), cands.end(),
               [](const Cand &x, const Cand &y) { return x.t.ms < y.t.ms; });
     constexpr int kFinalists = 4, kRetime = 5;

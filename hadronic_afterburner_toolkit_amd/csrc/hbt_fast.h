@@ -7,23 +7,24 @@
 // idle while any lane continues, so a direct port pays the whole cascade
 // (sqrt, three to five divisions, cos) for almost every pair.  Here the
 // work items' windows leave out most pairs unevaluated, every evaluated pair
-// costs 16 VALU operations, and only its survivors (~1.4% of the enumerated
-// pairs on the bench workload) reach the exact cascade, 64 at a time with
-// all lanes busy.
+// costs three matrix-core products and 7 VALU operations, and only its
+// survivors (~1.4% of the enumerated pairs on the bench workload) reach the
+// exact cascade, 64 at a time with all lanes busy.
 //
 // Prefilter (all conservative: a pair the exact cascade accepts always
 // passes; the margins exceed the rounding error of both computations):
 //   T = |p1T + p2T|^2 = 4 K_perp^2           in [4 KT_min^2, 4 KT_max^2]
 //   q_out^2 = dn^2 / T <= H^2                (q_out = (p1T - p2T).(p1T + p2T)
-//        / |p1T + p2T| = dn / sqrt(T), dn = n1 - n2)
-//   q_side^2 = Q - q_out^2 <= H^2            (Q = |p1T - p2T|^2)
+//        / |p1T + p2T| = dn / sqrt(T), dn = n1 - n2, n = |pT|^2)
+//   q_side^2 = C^2 / T <= H^2                (q_side = (p1T - p2T)x(p1T + p2T)
+//        / |p1T + p2T|, whose numerator is C = 2 (p1x p2y - p1y p2x))
 //   |beta1 - beta2| <= (H/2) (1/E1 + 1/E2)   (from |q_long| <= H, M_t <= K_E,
 //        q_long M_t = E2 pz1 - E1 pz2; beta = pz/E)
-// with H = max(|q_lo_cut|, |q_hi_cut|), the q windows tested without a
-// division as dn^2 <= H^2 T and (Q - H^2) T <= dn^2.  T and Q come from one
-// dot product: T = n1 + n2 + 2 p1.p2, Q = n1 + n2 - 2 p1.p2 (n = |pT|^2).
+// with H = max(|q_lo_cut|, |q_hi_cut|).  The two q windows are one test,
+// max(|dn|, |C|)^2 <= H^2 T.  T, dn and C are bilinear in the two particles'
+// (px, py, n, 1), so the matrix cores form them.
 // For mixed pairs the i particle is rotated by -theta instead of rotating
-// every j by +theta (T, Q, dn and beta are rotation invariant); the exact
+// every j by +theta (T, dn, C and beta are rotation invariant); the exact
 // cascade then uses the reference's rotated j (HBT_correlation.cpp:522-523).
 #pragma once
 #include "hbt_device.h"
@@ -36,7 +37,9 @@ namespace hbt {
 // Per-particle prefilter record: nrm = px^2+py^2 - mid/2 (so that
 // n1 + n2 + 2 p1.p2 = T - mid), and blo, the lower end of the particle's
 // beta interval [beta - cw, beta + cw] (beta = pz/E, or pz without the LCMS
-// boost); the upper end bhi is kept in a separate array beside the records.
+// boost); the upper end bhi is kept beside the records.  The kernel reads the
+// FP32 records, which pass every pair the exact cascade of either precision
+// accepts; the FP64 ones state the same tests without FP32's rounding.
 struct PfRec64 {
     double px, py, nrm, blo;
 };
@@ -44,36 +47,49 @@ struct PfRec32 {
     float px, py, nrm, blo;
 };
 
-// Prefilter constants in the records' precision (FP64 or FP32 set of
-// DevParams): the T window's centre and half-width, H^2, mid - H^2, and the
-// q windows' margin c as -c and -2c.
+// Prefilter constants in the records' precision: X = s (T - mid) is formed
+// with the scale s = H^2 (1 with the q_inv branch on, whose q test passes
+// every pair); sh bounds |X| (the T window's half-width, scaled and rounded
+// up; nsh2 = -sh^2), c0 = H^2 mid + c bounds max(|dn|, |C|)^2 - X, with the q
+// margin c (infinite with the q_inv branch on).
 template <typename Prec>
 struct PfConst {
-    Prec half, mid, h2, midh2, negc, neg2c;
+    Prec s, nsh2, c0;
 };
 
 template <typename Prec>
 __host__ __device__ __forceinline__ PfConst<Prec> pf_const(const DevParams &P) {
     constexpr bool f64 = std::is_same<Prec, double>::value;
+    constexpr double eps = f64 ? 1.1102230246251565e-16 : 5.9604644775390625e-8;
     PfConst<Prec> k;
-    k.half = (Prec)(f64 ? P.pf_half : P.f_half);
-    k.mid = (Prec)(f64 ? P.pf_mid : P.f_mid);
-    k.h2 = (Prec)(f64 ? P.pf_h2 : P.f_h2);
-    k.midh2 = (Prec)(f64 ? P.pf_midh2 : P.f_midh2);
-    k.negc = (Prec)(f64 ? P.pf_negc : P.f_negc);
-    k.neg2c = k.negc * (Prec)2;
+    k.s = (Prec)(P.qinv ? 1.0 : P.pf_h2);
+    const double sh = (double)k.s * (f64 ? P.pf_half : (double)P.f_half);
+    k.nsh2 = (Prec)(-sh * sh * (1.0 + 16.0 * eps));
+    k.c0 = (Prec)(((double)k.s * P.pf_mid) * (1.0 + 4.0 * eps) -
+                  (f64 ? P.pf_negc : (double)P.f_negc));
     return k;
 }
 
 // The prefilter's tests of one pair (for a mixed pair, i rotated by
-// -theta), as five comparisons lhs[k] <= rhs[k]: the K_T window |T - mid|
-// <= half; q_out: dn^2 - c <= H^2 T; q_side: (Q - H^2) T - 2c <= dn^2 - c;
-// beta: |beta_i - beta_j| <= cw_i + cw_j as the overlap of the two beta
-// intervals, blo_i <= bhi_j and blo_j <= bhi_i (no arithmetic).  The kernel
-// and the host's check of the margins evaluate this same function.
+// -theta): it passes where all four values are negative.  K_T window: X^2 -
+// (s half)^2; q_out and q_side: max(|dn|, |C|)^2 - X - (H^2 mid + c); beta:
+// |beta_i - beta_j| <= cw_i + cw_j as the overlap of the two beta intervals,
+// blo_i - bhi_j and blo_j - bhi_i.  The margins leave every pair the exact
+// cascade accepts strictly inside.  The host's check of the margins evaluates
+// this function; the kernel forms X, dn and C on the matrix cores, whose order
+// of the four products the margins cover too.
+__host__ __device__ __forceinline__ float pf_fma(float a, float b, float c) {
+    return __builtin_fmaf(a, b, c);
+}
+__host__ __device__ __forceinline__ double pf_fma(double a, double b, double c) {
+    return __builtin_fma(a, b, c);
+}
+__host__ __device__ __forceinline__ float pf_abs(float a) { return __builtin_fabsf(a); }
+__host__ __device__ __forceinline__ double pf_abs(double a) { return __builtin_fabs(a); }
+
 template <typename Prec>
 struct PfTerms {
-    Prec lhs[5], rhs[5];
+    Prec v[4];
 };
 
 template <typename Prec>
@@ -81,32 +97,59 @@ __host__ __device__ __forceinline__ PfTerms<Prec> pf_terms(Prec ix, Prec iy, Pre
                                                            Prec ihi, Prec jx, Prec jy, Prec jn,
                                                            Prec jlo, Prec jhi,
                                                            const PfConst<Prec> &k) {
-    PfTerms<Prec> t;
-    const Prec d = fma(ix, jx, iy * jy);
-    const Prec sn = in + jn;
-    const Prec u = fma((Prec)2, d, sn);   // T - mid
-    const Prec v = fma((Prec)-2, d, sn);  // Q - mid
-    const Prec dn = in - jn;
-    const Prec T = u + k.mid;
-    const Prec ddc = fma(dn, dn, k.negc);
-    t.lhs[0] = fabs(u);
-    t.rhs[0] = k.half;
-    t.lhs[1] = ddc;
-    t.rhs[1] = T * k.h2;
-    t.lhs[2] = fma(v + k.midh2, T, k.neg2c);
-    t.rhs[2] = ddc;
-    t.lhs[3] = ilo;
-    t.rhs[3] = jhi;
-    t.lhs[4] = jlo;
-    t.rhs[4] = ihi;
-    return t;
+    const Prec s2 = (Prec)2 * k.s;
+    const Prec X = pf_fma(jx, s2 * ix, pf_fma(jy, s2 * iy, pf_fma(jn, k.s, k.s * in)));
+    const Prec dn = pf_fma(jn, (Prec)-0.5, (Prec)0.5 * in);
+    const Prec m = pf_abs(pf_fma(jx, -iy, pf_fma(jy, ix, dn))) + pf_abs(pf_fma(jx, iy, pf_fma(jy, -ix, dn)));
+    return PfTerms<Prec>{{pf_fma(X, X, k.nsh2), pf_fma(m, m, -X) - k.c0, ilo - jhi, jlo - ihi}};
 }
 
 template <typename Prec>
 __host__ __device__ __forceinline__ bool pf_pass(const PfTerms<Prec> &t) {
-    return t.lhs[0] <= t.rhs[0] && t.lhs[1] <= t.rhs[1] && t.lhs[2] <= t.rhs[2] &&
-           t.lhs[3] <= t.rhs[3] && t.lhs[4] <= t.rhs[4];
+    return t.v[0] < 0 && t.v[1] < 0 && t.v[2] < 0 && t.v[3] < 0;
 }
+
+// What a particle's prefilter record needs beside its momentum: the window
+// centre, the beta half-width's numerator H/2, the largest |beta| of the list
+// (FP32 margins), and the analysis' boost and q_inv switches.
+struct PfMake {
+    double mid, c_beta, bm;
+    int boost, qinv;
+};
+
+// The neighbouring float below (up = false) or above; infinities and NaN stay.
+__host__ __device__ __forceinline__ float next_float(float x, bool up) {
+    if (!(fabsf(x) < INFINITY)) return x;
+    if (x == 0.0f) return up ? 1.401298464e-45f : -1.401298464e-45f;
+    const int b = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, b + ((x > 0.0f) == up ? 1 : -1));
+}
+
+// FP32 record of one particle: cw also covers the rounding of beta (|beta|
+// <= bm over the list) and of cw itself; the interval's ends are rounded to
+// nearest, then one FP32 ulp outward.
+__host__ __device__ __forceinline__ void pf_make(const PfMake &m, double px, double py, double pz,
+                                                 double E, PfRec32 &r, float &bhi) {
+    const double eps32 = 5.9604644775390625e-8;
+    const double beta = m.boost ? pz / E : pz;
+    const double cw = m.qinv ? INFINITY
+                             : (m.boost ? m.c_beta / E : m.c_beta) * (1.0 + 8 * eps32) +
+                                   4 * eps32 * fmax(1.0, m.bm);
+    r = PfRec32{(float)px, (float)py, (float)(px * px + py * py - 0.5 * m.mid),
+                next_float((float)(beta - cw), false)};
+    bhi = next_float((float)(beta + cw), true);
+}
+
+// A particle as the kernel's matrix-core operand, and its beta interval.
+struct __align__(16) PfOp {
+    float px, py, nrm, one;
+};
+struct __align__(8) PfBeta {
+    float lo, hi;
+};
+// Entries past a list's end that the kernel may read (and ignore): its j
+// tiles come in pairs of 16.
+constexpr int kPfPad = 32;
 
 // Same-event pair orientation: for a position in the cell-sorted list, the
 // particle's index in the fast list and its rank in gather order (the
@@ -125,12 +168,12 @@ struct View {
     DevHist H;
     const PartRec *A;    // same-event fast list, 64 B per particle
     const PartRec *B;    // mixed fast list (separate, or an alias of A)
-    const void *pfA;     // PfRec64 (FP64 kernel) or PfRec32 (precision form) of A
-    const void *pfB;     // of B
-    const void *pfS;     // of the same-event fast list sorted by (px cell, py) per group
-    const void *cwA;     // per-particle upper end bhi of the beta interval of A, like pfA
-    const void *cwB;
-    const void *cwS;
+    const PfOp *pfA;     // prefilter operands of A, of B,
+    const PfOp *pfB;
+    const PfOp *pfS;     // and of the same-event fast list sorted by (px cell, py) per group
+    const PfBeta *bwA;   // their beta intervals
+    const PfBeta *bwB;
+    const PfBeta *bwS;
     const OrigRank *origS;     // cell-sorted position -> fast-list index and gather rank
     const PartRec *AS;         // records of the same-event fast list in the cell-sorted order
     const JWin *mwin;          // partner windows of the mixed items
@@ -143,21 +186,39 @@ struct View {
     DevParams P;
 };
 
-// The cell-sorted copy of the same-event records, AS[q] = A[origS[q].idx],
-// built on the device once the lists are resident.
-static __global__ __launch_bounds__(256) void k_gather_srt(const PartRec *__restrict__ A,
-                                                           const OrigRank *__restrict__ orr,
-                                                           PartRec *__restrict__ AS,
-                                                           long long nf) {
+// The fast lists on the device, from the uploaded records A (per event,
+// |pT|-sorted) and the cell-sorted order: the prefilter operands and beta
+// intervals of both orders, and the cell-sorted copy of the records, AS[q] =
+// A[orr[q].idx].
+static __global__ __launch_bounds__(256) void k_build_lists(PfMake m, const PartRec *__restrict__ A,
+                                                            const OrigRank *__restrict__ orr,
+                                                            PartRec *__restrict__ AS,
+                                                            PfOp *__restrict__ pfA,
+                                                            PfBeta *__restrict__ bwA,
+                                                            PfOp *__restrict__ pfS,
+                                                            PfBeta *__restrict__ bwS,
+                                                            long long nf) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < nf) AS[q] = A[orr[q].idx];
+    if (q >= nf) return;
+    PfRec32 r;
+    float hi;
+    const PartRec a = A[q];
+    pf_make(m, a.px, a.py, a.pz, a.E, r, hi);
+    pfA[q] = PfOp{r.px, r.py, r.nrm, 1.0f};
+    bwA[q] = PfBeta{r.blo, hi};
+    const PartRec s = A[orr[q].idx];
+    AS[q] = s;
+    pf_make(m, s.px, s.py, s.pz, s.E, r, hi);
+    pfS[q] = PfOp{r.px, r.py, r.nrm, 1.0f};
+    bwS[q] = PfBeta{r.blo, hi};
 }
 
-static inline hipError_t gather_srt(const PartRec *A, const OrigRank *orr, PartRec *AS,
-                                    long long nf, hipStream_t st) {
+static inline hipError_t build_lists(const PfMake &m, const PartRec *A, const OrigRank *orr,
+                                     PartRec *AS, PfOp *pfA, PfBeta *bwA, PfOp *pfS, PfBeta *bwS,
+                                     long long nf, hipStream_t st) {
     if (nf <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_gather_srt, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, st, A,
-                       orr, AS, nf);
+    hipLaunchKernelGGL(k_build_lists, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, st, m, A,
+                       orr, AS, pfA, bwA, pfS, bwS, nf);
     return hipGetLastError();
 }
 
@@ -180,131 +241,174 @@ struct FastArgs {
     SlabArgs slab;
 };
 
-// The view table does not change during a launch.  Reading it through the
-// constant address space marks its pointers as invariant scalar loads, which
-// the compiler re-issues where they are used instead of holding ~40 SGPRs
-// for the whole work item.
+// Read-only, wave-uniform data (the view table, the kernel's arguments, work
+// items, partner windows, rotations) is read through the constant address
+// space: scalar loads into scalar registers.
 #if defined(__HIP_DEVICE_COMPILE__)
-#define HBT_LOAD_VIEW(tab, k) (((const __attribute__((address_space(4))) View *)(tab))[k])
+#define HBT_AS4 __attribute__((address_space(4)))
 #else
-#define HBT_LOAD_VIEW(tab, k) ((tab)[k])
+#define HBT_AS4
 #endif
+#define HBT_CONST(T, p) ((const HBT_AS4 T *)(p))
+using CView = const HBT_AS4 View;
+using CParams = const HBT_AS4 DevParams;
+using CArgs = const HBT_AS4 FastArgs;
 
-// The view table entry k, read anew where this is called: the empty asm
-// hides the table's address from the optimiser, so the loads that follow
-// cannot be hoisted out of the caller's loop.  For the exact stage, whose
-// grid constants and pointers would otherwise be loaded once per work item
-// and held in (spilled) scalar registers across the whole j loop.
-__device__ __forceinline__ View view_fresh(const View *views, int k) {
+// p, hidden from the optimiser: loads through it stay where they are written
+// instead of being hoisted out of the caller's loops and held (spilled) in
+// scalar registers.  For the exact stage, which reads its grid constants and
+// pointers where it uses them.
+template <typename T>
+__device__ __forceinline__ T *fresh(T *p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const __attribute__((address_space(4))) View *t =
-        (const __attribute__((address_space(4))) View *)views + k;
-    __asm__ volatile("" : "+s"(t));
-    return *t;
+    __asm__ volatile("" : "+s"(p));
+#endif
+    return p;
+}
+// The view table entry k, and the kernel's arguments.
+__device__ __forceinline__ CView *view_at(const View *views, int k) {
+    return fresh(HBT_CONST(View, views) + __builtin_amdgcn_readfirstlane(k));
+}
+__device__ __forceinline__ CArgs *kernel_args() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return fresh((CArgs *)__builtin_amdgcn_kernarg_segment_ptr());
 #else
-    return views[k];
+    return nullptr;
 #endif
 }
 
 // ------------------------------------------------------- wave helpers
 
-// Mask of lanes where a <= b (ordered: NaN compares false), as one SGPR pair.
-__device__ __forceinline__ unsigned long long le_mask(float a, float b) {
-    return __builtin_amdgcn_fcmpf(a, b, 5 /* FCMP_OLE */);
-}
-__device__ __forceinline__ unsigned long long le_mask(double a, double b) {
-    return __builtin_amdgcn_fcmp(a, b, 5 /* FCMP_OLE */);
-}
-__host__ __device__ __forceinline__ float absv(float x) { return __builtin_fabsf(x); }
-__host__ __device__ __forceinline__ double absv(double x) { return __builtin_fabs(x); }
-
-// Value of lane t (t uniform) in every lane.
-__device__ __forceinline__ float bcast(float v, int t) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), t));
-}
-__device__ __forceinline__ double bcast(double v, int t) {
-    const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, t);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), t);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-// Lanes 0..n-1 (n clamped to [0, 64]); 32-bit count.
-__device__ __forceinline__ unsigned long long low_lanes32(int n) {
-    return n <= 0 ? 0ull : (n >= 64 ? ~0ull : ((1ull << n) - 1ull));
-}
-// Lanes 0..n-1 (n clamped to [0, 64]).
-__device__ __forceinline__ unsigned long long low_lanes(long long n) {
-    return n <= 0 ? 0ull : (n >= 64 ? ~0ull : ((1ull << n) - 1ull));
-}
-
 // ---------------------------------------------------------------- drain
 // Each lane takes one queued survivor (lane < cnt), runs the exact cascade.
+// A wave's LDS.  The exact stage takes 64 scattered survivors at a time; read
+// from memory, each of their 128-byte pairs of records would cost the vector
+// cache eight accesses per lane (measured: its address and data units 88 and
+// 96 % busy, k_fast 8.0 ms on the headline workload).  So the tile's 64 i
+// records are staged here once per item, and the 32 j records of a pair of
+// tiles while its prefilter runs, by loads that cover whole lines; two j
+// buffers let the survivors of a pair that do not fill a wave wait for the
+// next pair's.  Chunk c (16 bytes) of row r sits at chunk c ^ (r / 4) of its
+// row, which spreads 64 random rows over all banks.
+struct __align__(16) WaveLds {
+    char irec[64 * sizeof(PartRec)];
+    char jrec[2][32 * sizeof(PartRec)];
+    double2 rot[2];            // (cos, sin) of the j buffers' rotations
+    int irank[64], jrank[2][32];
+    unsigned short ring[128];  // queued survivors: i slot | j row << 6 | j buffer << 11
+};
+
+// Staged record `row`: chunks 0 and 1 (momentum), 2 and 3 (space-time).
+struct PartMom {
+    double px, py, pz, E;
+};
+__device__ __forceinline__ unsigned lds_row(unsigned row) {
+    return row * (unsigned)sizeof(PartRec) + ((row & 12u) << 2);
+}
+__device__ __forceinline__ PartMom lds_mom(const char *rec, unsigned at) {
+    const double2 u = *(const double2 *)(rec + at), v = *(const double2 *)(rec + (at ^ 16u));
+    return PartMom{u.x, u.y, v.x, v.y};
+}
+__device__ __forceinline__ PartRec lds_rec(const char *rec, unsigned at) {
+    const PartMom m = lds_mom(rec, at), p = lds_mom(rec, at ^ 32u);
+    return PartRec{m.px, m.py, m.pz, m.E, p.px, p.py, p.pz, p.E};
+}
+// The exact stage of one pair whose staged records lie at a and b of rec, in
+// the reference's orientation (same-event: particle 1 is the earlier in gather
+// order); mixed: c, s rotate the partner.
 template <typename Prec, bool EXT>
 struct Exact;
 
 template <bool EXT>
 struct Exact<double, EXT> {
-    // i, j are positions in the cell-sorted list; origS maps them to the
-    // fast list, and the pair is evaluated in the reference's orientation
-    // (particle 1 = the earlier in gather order).
-    static __device__ __forceinline__ int same(const DevParams &P, const View &v, double psi,
-                                               long long i, long long j, SameRec &rec) {
-        const OrigRank oi = v.origS[i], oj = v.origS[j];
-        const bool fwd = oi.rank < oj.rank;
-        const PartRec p = v.A[fwd ? oi.idx : oj.idx], r = v.A[fwd ? oj.idx : oi.idx];
-        return eval_same_f64<EXT>(P, v.H, psi, p.px, p.py, p.pz, p.E, p.x, p.y, p.z, p.t, r.px,
-                                  r.py, r.pz, r.E, r.x, r.y, r.z, r.t, rec);
+    static __device__ __forceinline__ int same(CView *vp, double psi, const char *rec, unsigned a,
+                                               unsigned b, SameRec &out) {
+        const DevParams P = vp->P;
+        const DevHist H = vp->H;
+        const PartRec p = lds_rec(rec, a), r = lds_rec(rec, b);
+        return eval_same_f64<EXT>(P, H, psi, p.px, p.py, p.pz, p.E, p.x, p.y, p.z, p.t, r.px,
+                                  r.py, r.pz, r.E, r.x, r.y, r.z, r.t, out);
     }
-    static __device__ __forceinline__ int mixed(const DevParams &P, const View &v, double psi,
-                                                long long i, long long j, double c, double s,
-                                                long &k) {
-        const PartRec &p = v.A[i];
-        const PartRec &r = v.B[j];
-        const double px = r.px, py = r.py;
-        return eval_mixed_f64<EXT>(P, v.H, psi, p.px, p.py, p.pz, p.E, px * c - py * s,
-                                   px * s + py * c, r.pz, r.E, k);
+    static __device__ __forceinline__ int mixed(CView *vp, double psi, const char *rec, unsigned a,
+                                                unsigned b, double2 cs, long &k) {
+        const DevParams P = vp->P;
+        const DevHist H = vp->H;
+        const PartMom p = lds_mom(rec, a), r = lds_mom(rec, b);
+        return eval_mixed_f64<EXT>(P, H, psi, p.px, p.py, p.pz, p.E, r.px * cs.x - r.py * cs.y,
+                                   r.px * cs.y + r.py * cs.x, r.pz, r.E, k);
     }
 };
 
+// The precision form: negative where a decision is ambiguous.
 template <bool EXT>
 struct Exact<float, EXT> {
-    // The records come from the cell-sorted copy, so their loads do not
-    // wait for the gather ranks; the ranks only orient the pair.
-    static __device__ __forceinline__ int same(const DevParams &P, const View &v, double psi,
-                                               long long i, long long j, SameRec &rec) {
-        const int ri = v.origS[i].rank, rj = v.origS[j].rank;
-        return eval_same_fast<EXT>(P, v.H, psi, v.AS[i], v.AS[j], rj < ri, rec);
+    static __device__ __forceinline__ int same(CView *vp, double psi, const char *rec, unsigned a,
+                                               unsigned b, SameRec &out) {
+        const PartRec p = lds_rec(rec, a), r = lds_rec(rec, b);
+        out.sure = true;
+        return eval_same_fast<EXT>(vp->P, psi, p, r, out);
     }
-    static __device__ __forceinline__ int mixed(const DevParams &P, const View &v, double psi,
-                                                long long i, long long j, double c, double s,
-                                                long &k) {
-        const PartRec &p = v.A[i];
-        const PartRec &r = v.B[j];
-        const double px = r.px, py = r.py;
-        return eval_mixed_fast<EXT>(P, v.H, psi, p.px, p.py, p.pz, p.E, px * c - py * s,
-                                    px * s + py * c, r.pz, r.E, k);
+    static __device__ __forceinline__ int mixed(CView *vp, double psi, const char *rec, unsigned a,
+                                                unsigned b, double2 cs, long &k) {
+        const PartMom p = lds_mom(rec, a), r = lds_mom(rec, b);
+        return eval_mixed_fast<EXT>(vp->P, psi, p.px, p.py, p.pz, p.E, r.px * cs.x - r.py * cs.y,
+                                    r.px * cs.y + r.py * cs.x, r.pz, r.E, k);
     }
 };
 
-// A binned pair's value as the form accumulates it: FP64 as computed, or,
-// in the precision form with slab binning (whose records hold FP32 values),
-// rounded to FP32 on the direct path too.
+// Records of one queued survivor: offsets in the wave's LDS, same-event pairs
+// in the reference's orientation.
+struct PairAt {
+    unsigned a, b, buf;
+};
+__device__ __forceinline__ PairAt pair_at(const WaveLds &wl, unsigned ent, bool mixed) {
+    const unsigned i = ent & 63u, j = ent >> 6 & 31u, buf = ent >> 11;
+    const unsigned ai = lds_row(i);
+    const unsigned aj = (unsigned)offsetof(WaveLds, jrec) + buf * 2048u + lds_row(j);
+    const bool swap = !mixed && wl.irank[i] > wl.jrank[buf][j];
+    return PairAt{swap ? aj : ai, swap ? ai : aj, buf};
+}
+
+// One same-event pair added directly.  With slab binning the precision
+// form's per-pair values are FP32 on either path (its records hold FP32
+// values), so the path a pair takes does not change what it adds; without it
+// they stay FP64.
 template <typename Prec>
-__device__ __forceinline__ double fp_pair(double v, bool slab) {
-    return std::is_same<Prec, float>::value && slab ? (double)(float)v : v;
+__device__ __forceinline__ void add_same_slabwise(double *bins, SameRec rec, bool slab) {
+    if (std::is_same<Prec, float>::value && slab) {
+        rec.qo = (double)(float)rec.qo;
+        rec.qs = (double)(float)rec.qs;
+        rec.ql = (double)(float)rec.ql;
+        rec.c = (double)(float)rec.c;
+    }
+    add_same_direct(bins, rec);
+}
+
+// Lane l's part of staging 64 / n rows from src (rows past `last` repeat it):
+// chunk l % n of row r0 + l / n, n = 4 chunks, or 2 where only the momentum is
+// wanted.
+template <int N>
+__device__ __forceinline__ double2 stage_load(const PartRec *src, int lane, int r0, int last) {
+    const int row = min(r0 + lane / N, last);
+    return *(const double2 *)((const char *)src + (unsigned)(row * 64 + (lane & (N - 1)) * 16));
+}
+template <int N>
+__device__ __forceinline__ void stage_store(char *rec, int lane, int r0, double2 v) {
+    const unsigned row = (unsigned)(r0 + lane / N), c = (unsigned)lane & (N - 1);
+    *(double2 *)(rec + (lds_row(row) ^ (c << 4))) = v;
 }
 
 // Per-wave LDS staging of binned same-event pairs for the cooperative
-// scatter: bin index and the four sums of up to 64 pairs.
+// scatter: bin index and the four sums of up to 24 pairs (two instructions'
+// worth; more would cost the fourth block per CU its LDS).
+constexpr int kStage = 24;
 struct Stage {
-    long k[64];
-    double v[64][4];
+    long k[kStage];
+    double v[kStage][4];
 };
 
 // Each lane with lane < cnt takes one queued survivor and runs the exact
-// cascade.  Same-event entries: (j - j0) << 8 | slot; mixed entries:
-// (window - j0) << 26 | (j - window start) << 8 | slot, slot = r*64 + lane
-// of the i particle in the tile.
+// cascade.
 // Binned same-event pairs are added cooperatively: they are staged in LDS,
 // then groups of 5 lanes add one pair's count and four sums, so one atomic
 // instruction touches 12 bins (12 cache lines) instead of 64.  Atomic
@@ -312,74 +416,111 @@ struct Stage {
 // about 2.4e10 per second whatever the histogram's size or placement, so
 // the count is an FP64 add in the same instruction as the sums: one access
 // per binned pair.
-template <typename Prec, bool EXT, int QCAP>
-__device__ __forceinline__ int drain(const DevParams &P, const View &v, const unsigned *q,
-                                     Stage &stg,
-                                     unsigned head, int cnt, const WorkItem &w, double psi,
-                                     const SlabArgs &sl, unsigned *fill, const int *scap,
-                                     const long long *sbase, unsigned &direct_n) {
+// unsure: the lanes whose pair the precision form could not decide, unsure_phi
+// those of them that miss only their K_phi bin.
+template <typename Prec, bool EXT>
+__device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, Stage &stg,
+                                     unsigned head, int cnt, bool mixed, double psi,
+                                     unsigned *next, const unsigned *lim,
+                                     unsigned long long &direct_n, unsigned long long &unsure,
+                                     unsigned long long &unsure_phi) {
     const int lane = __lane_id();
     int st = 0;
     SameRec rec;
     long kmix = 0;
     if (lane < cnt) {
-        const unsigned ent = q[(head + lane) & (QCAP - 1)];
-        const int slot = (int)(ent & 255u);
-        if (slot < w.ni) {  // always true: only lanes inside the tile enqueue
-            const long long i = w.i0 + slot;
-            if (w.kind == 0) {
-                st = Exact<Prec, EXT>::same(P, v, psi, i, w.j0 + (ent >> 8), rec);
-            } else {
-                const JWin jw = v.mwin[w.j0 + (ent >> 26)];
-                const long long j = jw.b + ((ent >> 8) & 0x3ffffu);
-                st = Exact<Prec, EXT>::mixed(P, v, psi, i, j, v.plan_cs[2 * jw.row],
-                                             v.plan_cs[2 * jw.row + 1], kmix);
-            }
-        }
+        const PairAt pr = pair_at(wl, wl.ring[(head + lane) & 127u], mixed);
+        const char *base = (const char *)&wl;
+        if (mixed)
+            st = Exact<Prec, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], kmix);
+        else
+            st = Exact<Prec, EXT>::same(vp, psi, base, pr.a, pr.b, rec);
     }
-    const bool binned = (st & ST_BIN) != 0;
+    if (std::is_same<Prec, float>::value) {
+        unsure = __ballot(st < 0);
+        if (EXT) unsure_phi = __ballot(st == -2);
+    }
+    const bool binned = st > 0 && (st & ST_BIN) != 0;
+    const int nbinned = __popcll(__ballot(binned));
     // slab binning: a same-event pair becomes a record of its (block, slab)
     // region; a full region, or stored values that would land in another
     // bin, send it down the direct path.  Mixed pairs are always direct.
     // (The host turns slab binning off for q_inv analyses.)
-    const bool slab = sl.vals != nullptr;
-    if (w.kind != 0) {
-        if (binned) add_mixed_direct(v.H, kmix);
-        return binned ? 1 : 0;
+    const bool slab = ka->slab.vals != nullptr;
+    if (mixed) {
+        if (binned) add_mixed_direct(vp->H.bins, kmix);
+        return nbinned;
     }
     bool direct = binned;
-    if (slab && binned) {
-        direct = !slab_put_same<Prec>(sl, fill, scap, sbase, rec);
-        direct_n += direct ? 1u : 0u;
-    }
+    if (slab && binned) direct = !slab_put_same<Prec>(ka->slab, next, lim, rec);
     const unsigned long long m = __ballot(direct);
     const int nb = __popcll(m);
-    if (nb == 0) return binned ? 1 : 0;
-    if (direct) {
-        const unsigned idx = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        stg.k[idx] = rec.k;
-        // with slab binning the precision form's per-pair values are FP32 on
-        // either path (its records hold them as FP32), so the path a pair
-        // takes does not change what it adds; without it they stay FP64
-        stg.v[idx][0] = fp_pair<Prec>(rec.qo, slab);
-        stg.v[idx][1] = fp_pair<Prec>(rec.qs, slab);
-        stg.v[idx][2] = fp_pair<Prec>(rec.ql, slab);
-        stg.v[idx][3] = fp_pair<Prec>(rec.c, slab);
+    if (nb == 0) return nbinned;
+    double *bins = vp->H.bins;
+    if (slab) {  // few
+        direct_n += nb;
+        if (direct) add_same_slabwise<Prec>(bins, rec, true);
+        return nbinned;
     }
-    __builtin_amdgcn_wave_barrier();
+    const unsigned idx = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
     // lane sub of a group adds field sub of its pair's bin: the count (an
     // exact FP64 integer) and the four sums go out as one FP64 atomic
     // instruction, one cache line per pair
     const int grp = lane / 5, sub = lane - 5 * grp;
-    for (int base = 0; base < nb; base += 12) {
-        const int p = base + grp;
-        if (lane < 60 && p < nb)
-            atomic_add_f64(v.H.bins + stg.k[p] * BIN_STRIDE + sub,
-                           sub == 0 ? 1.0 : stg.v[p][max(sub - 1, 0)]);
+    for (int b0 = 0; b0 < nb; b0 += kStage) {
+        __builtin_amdgcn_wave_barrier();
+        if (direct && idx - b0 < (unsigned)kStage) {
+            stg.k[idx - b0] = rec.k;
+            stg.v[idx - b0][0] = rec.qo;
+            stg.v[idx - b0][1] = rec.qs;
+            stg.v[idx - b0][2] = rec.ql;
+            stg.v[idx - b0][3] = rec.c;
+        }
+        __builtin_amdgcn_wave_barrier();
+        const int n = min(kStage, nb - b0);
+        for (int base = 0; base < n; base += 12) {
+            const int p = base + grp;
+            if (lane < 60 && p < n)
+                atomic_add_f64(bins + stg.k[p] * BIN_STRIDE + sub,
+                               sub == 0 ? 1.0 : stg.v[p][max(sub - 1, 0)]);
+        }
     }
     __builtin_amdgcn_wave_barrier();
-    return binned ? 1 : 0;
+    return nbinned;
+}
+
+// The pairs the precision form could not decide, by the literal cascade of
+// the FP64 form, each added directly.  After the exact stage of its batch
+// rather than inside it: the literal cascade's registers then do not add to
+// the exact stage's.  cos stays the form's own (FP32), except for the lanes
+// cos64.
+template <bool EXT>
+__device__ __forceinline__ int drain_literal(CView *vp, CArgs *ka, const WaveLds &wl, unsigned head,
+                                             unsigned long long lanes, unsigned long long cos64,
+                                             bool mixed, double psi,
+                                             unsigned long long &direct_n) {
+    const int lane = __lane_id();
+    bool binned = false;
+    if (lanes >> lane & 1ull) {
+        const PairAt pr = pair_at(wl, wl.ring[(head + lane) & 127u], mixed);
+        const char *base = (const char *)&wl;
+        if (mixed) {
+            long k = 0;
+            binned = (Exact<double, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], k) &
+                      ST_BIN) != 0;
+            if (binned) add_mixed_direct(vp->H.bins, k);
+        } else {
+            SameRec rec;
+            binned = (Exact<double, EXT>::same(vp, psi, base, pr.a, pr.b, rec) & ST_BIN) != 0;
+            if (!(cos64 >> lane & 1ull))
+                rec.c = pair_cos_f32(vp->P, lds_rec(base, pr.a), lds_rec(base, pr.b));
+            if (binned) add_same_slabwise<float>(vp->H.bins, rec, ka->slab.vals != nullptr);
+        }
+    }
+    const int n = __popcll(__ballot(binned));
+    if (!mixed && ka->slab.vals) direct_n += n;
+    return n;
 }
 
 // XCD of the executing wave (hardware register XCC_ID, bits 3:0).
@@ -387,88 +528,86 @@ __device__ __forceinline__ int xcc_id() {
     return (int)(__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 7u);
 }
 
-// j records are read with scalar loads (uniform address, read-only data
-// seen through the constant address space), so the j values arrive in SGPRs
-// and cost no vector instructions to broadcast.
-#if defined(__HIP_DEVICE_COMPILE__)
-#define HBT_CONST(T, p) ((const __attribute__((address_space(4))) T *)(p))
-#else
-#define HBT_CONST(T, p) ((const T *)(p))
-#endif
+typedef float v4f __attribute__((ext_vector_type(4)));
 
-// Survivors queued between drains: fewer than 64 plus one unrolled step of
-// JU j's times 64R lanes.
-constexpr int JU = 4;
-template <int R>
-struct Ring {
-    static constexpr int NEED = 64 + JU * 64 * R;
-    static constexpr int CAP = NEED <= 256 ? 256 : (NEED <= 512 ? 512 : 1024);
+// Matrix-core operands of the 16 i particles of a block, one value per lane:
+// lane l holds component l / 16 of particle l % 16.  Against a j tile's rows
+// (px, py, n, 1): X = s (T - mid), and P = (dn + C) / 2, M = (dn - C) / 2
+// with dn = in - jn and C = 2 (ix jy - iy jx), so that max(|dn|, |C|) =
+// |P| + |M| is one addition (a maximum would first quiet both operands).
+struct PfBlock {
+    float X, P, M;
 };
+__device__ __forceinline__ PfBlock pf_block(const PfConst<float> &k, int comp, float x, float y,
+                                            float n) {
+    PfBlock o;
+    const float s2 = 2.0f * k.s;
+    o.X = comp == 0 ? s2 * x : comp == 1 ? s2 * y : comp == 2 ? k.s : k.s * n;
+    const float c = comp == 0 ? -y : comp == 1 ? x : 0.0f;
+    const float d = comp == 2 ? -0.5f : comp == 3 ? 0.5f * n : 0.0f;
+    o.P = d + c;
+    o.M = d - c;
+    return o;
+}
+
+// Bits (from the top: block b, row r at bit 15 - (4 b + r)) of the rows of a
+// tile that are in range: the first n of this lane's four rows.
+__device__ __forceinline__ unsigned rows_first(int n) {
+    const int k = min(max(n, 0), 4);
+    return ((0xfu << (4 - k)) & 0xfu) * 0x1111u;
+}
 
 // ---------------------------------------------------------------- kernel
 // Persistent: each wave pulls work items from the queue of its XCD (the host
 // puts all items of a group in one queue, so a group's particles stay in one
-// XCD's L2), then from the next queues in turn, until all are empty.  Per item the wave holds 64R i particles (R per lane) and walks
-// its j segments (same-event: one range with j > i in the cell-sorted list;
-// mixed: one partner window per segment with the i particles rotated by
-// -theta),
-// JU j's per step.  Survivors of the prefilter go to the wave's LDS ring;
-// whenever 64 are queued they are binned, one per lane, and the last
-// survivors of the item are flushed at its final step (the exact cascade
-// has a single call site).
-// Occupancy: the exact stage is latency-bound (the particle records' loads
-// and its FP64 chain), so the kernels trade a few spilled registers for
-// more waves per SIMD: common case 6 at R=1 (80 VGPRs; the LDS of six
-// blocks fills the CU's 160 KB) and 4 at R=2 (128 VGPRs).  At R=1, 6 waves
-// ran the precision form's bench step 3 % faster than 5, and 5 ran it 5 %
-// faster than 4.  The K_phi / q_inv
-// instances carry the literal cascade with atan2 and the host-defer path
-// inline (168 VGPRs unconstrained): the precision form's, which reaches it
-// only for guard-band pairs, runs at 4 (128 VGPRs, spills in that rare
-// path), 10 % faster than at 3 on the batched K_phi workload; the FP64
-// form's, where it is the main path, at 3.  R=4 keeps the compiler's choice.
-template <typename Prec, int R, bool EXT>
+// XCD's L2), then from the next queues in turn, until all are empty.  Per
+// item the wave holds 64 i particles as four blocks of 16 matrix columns and
+// walks its j segments (same-event: one range with j > i in the cell-sorted
+// list; mixed: one partner window per segment with the i particles rotated
+// by -theta) in pairs of tiles of 16 j rows.  Three 16x16x4 FP32 products
+// per block and tile give X, P and M of 256 pairs, four per lane; 6 VALU
+// operations test a pair and a seventh shifts the outcome into the lane's bit
+// word (the scalar form took 16, and 7 more to queue the survivors of each
+// j).  Then each lane with bits left queues one survivor per round, and
+// whenever 64 are queued they are binned, one per lane; the last survivors of
+// a pair of tiles wait for at most the next pair's (the exact cascade has a
+// single call site).
+// Occupancy: four blocks' LDS fill the CU's 160 KB, so four waves per SIMD
+// (128 VGPRs, no spills in the common case); the K_phi / q_inv instance of
+// the FP64 form, whose main path is the literal cascade with atan2 and the
+// host-defer path, runs at three.
+template <typename Prec, bool EXT>
 constexpr int fast_waves_per_eu() {
-    return R == 4 ? 1
-                  : (EXT ? (std::is_same<Prec, float>::value ? 4 : 3) : (R == 1 ? 6 : 4));
+    return EXT && std::is_same<Prec, double>::value ? 3 : 4;
 }
 
-template <typename Prec, int R, bool EXT>
+// Dynamic LDS: with slab binning each slab's next record in this block's
+// region and (common case) the regions' ends; without it the waves' Stages.
+inline size_t fast_dynamic_lds(const SlabArgs &s, bool ext) {
+    return s.vals ? (size_t)s.S * sizeof(unsigned) * (ext ? 1 : 2) : 4 * sizeof(Stage);
+}
+
+template <typename Prec, bool EXT>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, R, EXT>()))) void k_fast(FastArgs a) {
-    using Rec = typename std::conditional<std::is_same<Prec, double>::value, PfRec64,
-                                          PfRec32>::type;
-    constexpr int QCAP = Ring<R>::CAP;
-    __shared__ unsigned ring[4][QCAP];
-    __shared__ Stage stage[4];
-    // slab binning: records per slab of this block, and (common-case
-    // instances) the regions' capacity and first record per slab; the K_phi
-    // instance keeps its up to kMaxSlabsKphi fill counters in the launch's
-    // dynamic LDS (none when it bins with atomics) and reads capacity and
-    // first record from SlabArgs
-    extern __shared__ unsigned slab_fill_dyn[];
-    __shared__ unsigned slab_fill_st[EXT ? 1 : kMaxSlabs];
-    unsigned *const slab_fill = EXT ? slab_fill_dyn : slab_fill_st;
-    __shared__ int slab_cap[EXT ? 1 : kMaxSlabs];
-    __shared__ long long slab_base[EXT ? 1 : kMaxSlabs];
+__attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_fast(FastArgs a) {
+    __shared__ WaveLds wave_lds[4];
+    extern __shared__ __align__(16) char dyn_lds[];
+    unsigned *const slab_next = (unsigned *)dyn_lds;
+    unsigned *const slab_lim = EXT ? nullptr : slab_next + a.slab.S;
     const bool slab = a.slab.vals != nullptr;
     if (slab) {
         for (int k = threadIdx.x; k < a.slab.S; k += blockDim.x) {
-            slab_fill[k] = 0u;
-            if (!EXT) {
-                slab_cap[k] = a.slab.scap[k];
-                slab_base[k] = a.slab.sbase[k];
-            }
+            slab_next[k] = slab_first(a.slab, k, blockIdx.x);
+            if (!EXT) slab_lim[k] = slab_first(a.slab, k, blockIdx.x + 1);
         }
         __syncthreads();
     }
-    const int *scap = EXT ? a.slab.scap : slab_cap;
-    const long long *sbase = EXT ? a.slab.sbase : slab_base;
-    unsigned direct_n = 0;
+    unsigned long long direct_n = 0;  // wave totals, uniform
     const int lane = __lane_id();
-    unsigned *q = ring[threadIdx.x >> 6];
-    Stage &stg = stage[threadIdx.x >> 6];
-    const PfConst<Prec> pk = pf_const<Prec>(a.P);
+    const int col = lane & 15, comp = lane >> 4, row0 = 4 * comp;
+    WaveLds &wl = wave_lds[threadIdx.x >> 6];
+    Stage &stg = ((Stage *)dyn_lds)[threadIdx.x >> 6];
+    const PfConst<float> pk = pf_const<float>(a.P);
     unsigned long long nb_same = 0, nb_mixed = 0;
 
     const int nq = a.nqueues;
@@ -476,156 +615,214 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, R, EXT>()))) void k_f
     int queues_left = nq;
     for (;;) {
         int it = 0;
-        if (lane == 0) it = atomicAdd(a.counter + kQueueStride * wq, 1);
+        CArgs *ka = kernel_args();
+        if (lane == 0) it = atomicAdd(ka->counter + kQueueStride * wq, 1);
         it = __builtin_amdgcn_readfirstlane(__shfl(it, 0));
-        if (it >= a.qoff[wq + 1] - a.qoff[wq]) {  // this queue is empty: the next one
+        const int q0 = ka->qoff[wq];
+        if (it >= ka->qoff[wq + 1] - q0) {  // this queue is empty: the next one
             if (--queues_left == 0) break;
             wq = (wq + 1) & (nq - 1);
             continue;
         }
-        const WorkItem w = a.items[a.qoff[wq] + it];
-        const View v = HBT_LOAD_VIEW(a.views, w.view);
-        const double psi = v.psi[w.grp];
+        const WorkItem w = HBT_CONST(WorkItem, ka->items)[q0 + it];
+        CView *vp = view_at(ka->views, w.view);
+        const double psi = HBT_CONST(double, vp->psi)[w.grp];
         const bool mixed = w.kind != 0;
         // same-event tiles run over the cell-sorted list, mixed ones over the
         // |pT|-sorted fast lists
-        const Rec *__restrict__ pfi = (const Rec *)(mixed ? v.pfA : v.pfS);
-        const Prec *__restrict__ hii = (const Prec *)(mixed ? v.cwA : v.cwS);
-        const Rec *pfj = (const Rec *)(mixed ? v.pfB : v.pfS);
-        const Prec *hij = (const Prec *)(mixed ? v.cwB : v.cwS);
-        // i particles, R per lane
-        Prec ix[R], iy[R], in[R], ilo[R], ihi[R], rx[R], ry[R];
-        unsigned long long vmask[R];
-        unsigned slot[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            slot[r] = (unsigned)(r * 64 + lane);
-            vmask[r] = low_lanes((long long)w.ni - r * 64);
-            const long long i = w.i0 + min((int)slot[r], w.ni - 1);
-            const Rec p = pfi[i];
-            ix[r] = rx[r] = p.px;
-            iy[r] = ry[r] = p.py;
-            in[r] = p.nrm;
-            ilo[r] = p.blo;
-            ihi[r] = hii[i];
+        const PfOp *pfi = (mixed ? vp->pfA : vp->pfS) + w.i0;
+        const PfBeta *bwi = (mixed ? vp->bwA : vp->bwS) + w.i0;
+        const PfOp *pfj = mixed ? vp->pfB : vp->pfS;
+        const PfBeta *bwj = mixed ? vp->bwB : vp->bwS;
+        const PartRec *recj = mixed ? vp->B : vp->AS;
+        {
+            const PartRec *reci = (mixed ? vp->A : vp->AS) + w.i0;
+            const int last = w.ni - 1;
+            const double2 v0 = stage_load<4>(reci, lane, 0, last);
+            const double2 v1 = stage_load<4>(reci, lane, 16, last);
+            const double2 v2 = stage_load<4>(reci, lane, 32, last);
+            const double2 v3 = stage_load<4>(reci, lane, 48, last);
+            __builtin_amdgcn_wave_barrier();
+            stage_store<4>(wl.irec, lane, 0, v0);
+            stage_store<4>(wl.irec, lane, 16, v1);
+            stage_store<4>(wl.irec, lane, 32, v2);
+            stage_store<4>(wl.irec, lane, 48, v3);
+            if (!mixed) wl.irank[lane] = vp->origS[w.i0 + min(lane, last)].rank;
         }
-        const bool partial = w.ni < 64 * R;
-        const int nseg = mixed ? w.nj : 1;
-        unsigned head = 0, tail = 0;
-        for (int seg = 0; seg < nseg; seg++) {
-            long long pbase, jb, je;
-            unsigned segbits;
-            if (mixed) {
-                const JWin jw = v.mwin[w.j0 + seg];
-                pbase = jb = jw.b;
-                je = jw.e;
-                segbits = (unsigned)seg << 26;
-                const double c = v.plan_cs[2 * jw.row], s = v.plan_cs[2 * jw.row + 1];
+        float ilo[4], ihi[4];
+        PfBlock blk[4];
+        // The i blocks, rotated by -theta for a mixed segment; columns past
+        // the tile's end get n = inf, which fails the K_T window.
+        auto load_blocks = [&](double c, double s) {
 #pragma unroll
-                for (int r = 0; r < R; r++) {  // rotate i by -theta
-                    rx[r] = (Prec)((double)ix[r] * c + (double)iy[r] * s);
-                    ry[r] = (Prec)((double)iy[r] * c - (double)ix[r] * s);
+            for (int b = 0; b < 4; b++) {
+                const int slot = 16 * b + col, i = min(slot, w.ni - 1);
+                const PfOp p = pfi[i];
+                float x = p.px, y = p.py;
+                if (mixed) {
+                    x = (float)((double)p.px * c + (double)p.py * s);
+                    y = (float)((double)p.py * c - (double)p.px * s);
                 }
-            } else {
-                pbase = jb = w.j0;
-                je = w.j0 + w.nj;
-                segbits = 0;
+                blk[b] = pf_block(pk, comp, x, y, slot < w.ni ? p.nrm : INFINITY);
             }
-            const bool last_seg = seg == nseg - 1;
-            long long jc = jb;
-            do {  // chunks of 64 j's (at least one pass, for the final flush)
-                const int cnt = (int)max(0ll, min(64ll, je - jc));
-                const bool last = last_seg && jc + 64 >= je;
-                // same-event: lanes with i < j matter only where the chunk
-                // reaches into the tile itself
-                const bool diag = !mixed && jc < w.i0 + 64 * R;
-                int tri = (int)min(jc - w.i0, 1ll << 20);
-                unsigned ebase = segbits | ((unsigned)(jc - pbase) << 8);
-                const auto *cpf = HBT_CONST(Rec, pfj + jc);
-                const auto *chi = HBT_CONST(Prec, hij + jc);
-                int t = 0;
-                for (;;) {
-                    if (tail - head >= 64 || (last && t >= cnt && tail != head)) {
-                        const int n = (int)min(64u, tail - head);
-                        __builtin_amdgcn_wave_barrier();
-                        const View vd = view_fresh(a.views, w.view);
-                        const int nb = drain<Prec, EXT, QCAP>(vd.P, vd, q, stg, head, n, w, psi,
-                                                              a.slab, slab_fill, scap, sbase,
-                                                              direct_n);
-                        if (mixed)
-                            nb_mixed += nb;
-                        else
-                            nb_same += nb;
-                        head += n;
+        };
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const PfBeta r = bwi[min(16 * b + col, w.ni - 1)];
+            ilo[b] = r.lo;
+            ihi[b] = r.hi;
+        }
+        const int nseg = mixed ? w.nj : 1;
+        int seg = -1, jc = 0, je = 0;  // the segment, its next j and its end
+        unsigned head = 0, tail = 0, buf = 0;
+        double2 rot = {1.0, 0.0};
+        for (;;) {
+            while (jc >= je && ++seg < nseg) {  // the next segment
+                if (mixed) {
+                    const JWin jw = HBT_CONST(JWin, vp->mwin)[w.j0 + seg];
+                    jc = jw.b;
+                    je = jw.e;
+                    rot.x = HBT_CONST(double, vp->plan_cs)[2 * jw.row];
+                    rot.y = HBT_CONST(double, vp->plan_cs)[2 * jw.row + 1];
+                } else {
+                    jc = (int)w.j0;
+                    je = (int)w.j0 + w.nj;
+                }
+                load_blocks(rot.x, rot.y);
+            }
+            const bool end = jc >= je;
+            const unsigned mark = tail;  // survivors of earlier pairs
+            unsigned bits = 0, ent = 0;
+            if (!end) {
+                // 32 j's, two tiles (the lane's share as a 32-bit offset from
+                // a uniform base)
+                const int cnt = min(32, je - jc);
+                const char *pa = (const char *)(pfj + jc), *pb = (const char *)(bwj + jc);
+                float A[2];
+                PfBeta jw[2][4];
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    A[t] = *(const float *)(pa + (unsigned)(256 * t + 16 * col + 4 * comp));
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        jw[t][r] = *(const PfBeta *)(pb + (unsigned)(128 * t + 8 * (row0 + r)));
+                }
+                double2 s0, s1 = {0.0, 0.0};
+                int rank = 0;
+                if (mixed) {
+                    s0 = stage_load<2>(recj + jc, lane, 0, 31);
+                } else {
+                    s0 = stage_load<4>(recj + jc, lane, 0, 31);
+                    s1 = stage_load<4>(recj + jc, lane, 16, 31);
+                    rank = vp->origS[jc + (lane & 31)].rank;
+                }
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    if (16 * t >= cnt) {
+                        bits <<= 16;
                         continue;
                     }
-                    if (t >= cnt) break;
-                    // one j against the wave's 64R i particles
-                    auto pair_step = [&](int u, const Rec &jr, Prec jhi) {
 #pragma unroll
-                        for (int r = 0; r < R; r++) {
-                            const PfTerms<Prec> pt =
-                                pf_terms(rx[r], ry[r], in[r], ilo[r], ihi[r], jr.px, jr.py,
-                                         jr.nrm, jr.blo, jhi, pk);
-                            unsigned long long m = le_mask(pt.lhs[0], pt.rhs[0]) &
-                                                   le_mask(pt.lhs[1], pt.rhs[1]) &
-                                                   le_mask(pt.lhs[2], pt.rhs[2]) &
-                                                   le_mask(pt.lhs[3], pt.rhs[3]) &
-                                                   le_mask(pt.lhs[4], pt.rhs[4]);
-                            if (partial) m &= vmask[r];
-                            if (diag) m &= low_lanes32(tri + u - r * 64);
-                            if (m) {
-                                const unsigned pos = __builtin_amdgcn_mbcnt_hi(
-                                    (unsigned)(m >> 32),
-                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, tail));
-                                if (__builtin_amdgcn_inverse_ballot_w64(m))
-                                    q[pos & (QCAP - 1)] = (ebase + ((unsigned)u << 8)) | slot[r];
-                                tail += (unsigned)__popcll(m);
-                            }
+                    for (int b = 0; b < 4; b++) {
+                        const v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
+                        const v4f X =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].X, o, 0, 0, 0);
+                        const v4f U =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].P, o, 0, 0, 0);
+                        const v4f V =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].M, o, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const float e = fabsf(U[r]) + fabsf(V[r]);
+                            const float m = fmaxf(
+                                fmaxf(fmaf(e, e, -X[r]) - pk.c0, fmaf(X[r], X[r], pk.nsh2)),
+                                fmaxf(ilo[b] - jw[t][r].hi, jw[t][r].lo - ihi[b]));
+                            // bits << 1 | sign of m
+                            bits = __builtin_amdgcn_alignbit(bits, __builtin_bit_cast(unsigned, m),
+                                                             31);
                         }
-                    };
-                    if (t + JU <= cnt) {  // whole step: the JU records load together
-                        Rec jr[JU];
-                        Prec jw[JU];
-#pragma unroll
-                        for (int u = 0; u < JU; u++) {
-                            jr[u] = cpf[t + u];
-                            jw[u] = chi[t + u];
-                        }
-#pragma unroll
-                        for (int u = 0; u < JU; u++) pair_step(u, jr[u], jw[u]);
-                    } else {
-#pragma unroll
-                        for (int u = 0; u < JU; u++)
-                            if (t + u < cnt) pair_step(u, cpf[t + u], chi[t + u]);
                     }
-                    t += JU;
-                    tri += JU;
-                    ebase += (unsigned)JU << 8;
                 }
-                jc += 64;
-            } while (jc < je);
+                if (cnt < 32)  // rows past the segment's end
+                    bits &= rows_first(cnt - row0) << 16 | rows_first(cnt - 16 - row0);
+                if (!mixed && jc < (int)w.i0 + 64) {
+                    // the tile's own particles: only j > i
+                    const int d0 = (int)w.i0 - jc + col - row0 + 1;
+                    unsigned keep = 0;
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int b = 0; b < 4; b++)
+                            keep = keep << 4 | 0xfu >> min(max(d0 + 16 * b - 16 * t, 0), 4);
+                    bits &= keep;
+                }
+                buf ^= 1u;
+                ent = buf << 11 | (unsigned)row0 << 6 | (unsigned)col;
+                __builtin_amdgcn_wave_barrier();
+                if (mixed) {
+                    stage_store<2>(wl.jrec[buf], lane, 0, s0);
+                    if (lane == 0) wl.rot[buf] = rot;
+                } else {
+                    stage_store<4>(wl.jrec[buf], lane, 0, s0);
+                    stage_store<4>(wl.jrec[buf], lane, 16, s1);
+                    if (lane < 32) wl.jrank[buf][lane] = rank;
+                }
+                jc += 32;
+            }
+            for (;;) {
+                // queue one survivor of each lane that has any
+                unsigned long long m;
+                while ((m = __ballot(bits != 0u)) != 0ull && tail - head < 64u) {
+                    const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+                        (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, tail));
+                    if (bits != 0u) {
+                        const unsigned p = (unsigned)__builtin_clz(bits);  // 16 t + 4 b + r
+                        bits &= ~(0x80000000u >> p);
+                        wl.ring[pos & 127u] = (unsigned short)(ent + (((p & 16u) | (p & 3u)) << 6) +
+                                                               ((p & 12u) << 2));
+                    }
+                    tail += (unsigned)__popcll(m);
+                }
+                // a full wave; or, with nothing left to queue, the survivors
+                // whose j buffer the next pair takes (at the end: all)
+                const unsigned n = tail - head;
+                if (n < 64u && (m != 0ull || (end ? n == 0u : (int)(mark - head) <= 0))) break;
+                const int take = (int)min(64u, n);
+                __builtin_amdgcn_wave_barrier();
+                CArgs *kd = kernel_args();
+                unsigned long long unsure = 0, unsure_phi = 0;
+                int nb = drain<Prec, EXT>(view_at(kd->views, w.view), kd, wl, stg, head, take,
+                                          mixed, psi, slab_next, slab_lim, direct_n, unsure,
+                                          unsure_phi);
+                if (std::is_same<Prec, float>::value && __builtin_expect(unsure != 0ull, 0)) {
+                    kd = kernel_args();
+                    nb += drain_literal<EXT>(view_at(kd->views, w.view), kd, wl, head, unsure,
+                                             unsure_phi, mixed, psi, direct_n);
+                }
+                if (mixed)
+                    nb_mixed += nb;
+                else
+                    nb_same += nb;
+                head += take;
+            }
+            if (end) break;
         }
         __builtin_amdgcn_wave_barrier();
     }
     // per-wave totals of binned pairs
-    for (int off = 32; off > 0; off >>= 1) {
-        nb_same += __shfl_down(nb_same, off);
-        nb_mixed += __shfl_down(nb_mixed, off);
-    }
+    CArgs *ka = kernel_args();
     if (lane == 0) {
-        if (nb_same) atomic_add_u64(&a.binned[0], nb_same);
-        if (nb_mixed) atomic_add_u64(&a.binned[1], nb_mixed);
+        if (nb_same) atomic_add_u64(&ka->binned[0], nb_same);
+        if (nb_mixed) atomic_add_u64(&ka->binned[1], nb_mixed);
     }
     if (slab) {
         // the block's demand per slab, for k_slab_bin (which clamps it to the
         // regions' capacity) and for sizing later launches
-        unsigned long long dn = direct_n;
-        for (int off = 32; off > 0; off >>= 1) dn += __shfl_down(dn, off);
-        if (lane == 0 && dn) atomic_add_u64(&a.slab.stats[a.slab.S], dn);
+        if (lane == 0 && direct_n) atomic_add_u64(&ka->slab.stats[ka->slab.S], direct_n);
         __syncthreads();
-        for (int k = threadIdx.x; k < a.slab.S; k += blockDim.x)
-            a.slab.sfill[(long long)blockIdx.x * a.slab.S + k] = slab_fill[k];
+        for (int k = threadIdx.x; k < ka->slab.S; k += blockDim.x)
+            ka->slab.sfill[(long long)blockIdx.x * ka->slab.S + k] =
+                slab_next[k] - slab_first(ka->slab, k, blockIdx.x);
     }
 }
 

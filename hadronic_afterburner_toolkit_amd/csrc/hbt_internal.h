@@ -77,8 +77,15 @@ inline int derive(const hbt_config &k, Derived &d, std::string &err) {
     P.KT_max_sq = k.KT_max * k.KT_max;
     P.hbarC_inv = 1. / kHbarC;
     P.two_pi = 2. * M_PI;
-    P.inv_dKT = 1.0 / P.dKT;
     P.inv_dq = 1.0 / P.delta_q;
+    P.kt_scale = 0.5 / P.dKT;
+    P.kt_off = 1.0 - P.KT_min / P.dKT;
+    P.q_off = 1.0 - P.q_base * P.inv_dq;
+    // 1e-9 bins for the coordinates' rounding; the windows' cuts lie 1e-8 GeV
+    // inside the outer bin edges, and a record's q is rounded to FP32 (half
+    // an ulp, 2^-25 of at most H)
+    P.guard = 1e-9 + P.inv_dq * std::max(2e-8, 0x1p-24 * std::max(std::fabs(P.q_lo_cut),
+                                                                  std::fabs(P.q_hi_cut)));
     P.inv_two_pi = 1.0 / (2.0 * M_PI);
     P.inv_dKphi = 1.0 / P.dKphi;
     P.kphi_guard = (k.kphi_guard_prad > 0 ? k.kphi_guard_prad : 1) * 1e-12;
@@ -113,14 +120,17 @@ inline int derive(const hbt_config &k, Derived &d, std::string &err) {
     return HBT_OK;
 }
 
+inline PfMake pf_maker(const Derived &d, double bm) {
+    return PfMake{d.mid, d.c_beta, bm, d.P.boost, d.P.qinv};
+}
+
 // Prefilter record of one particle: px, py, nrm = |pT|^2 - mid/2, and its
 // beta interval [blo, bhi] = beta -/+ cw with cw = (H/2) / E (or H/2
 // without the LCMS boost; infinite with the q_inv branch on): the beta test
 // |beta1 - beta2| <= cw1 + cw2 holds exactly when blo1 <= bhi2 and
 // blo2 <= bhi1.  The ends are rounded outward (blo down, bhi up), so the
-// two comparisons pass every pair the real-valued test passes.  FP32
-// records: cw also covers the rounding of beta (|beta| <= bm over the list)
-// and of cw itself.
+// two comparisons pass every pair the real-valued test passes.  The kernel
+// uses the FP32 records (pf_make, on the device).
 inline void pf_record(const Derived &d, double px, double py, double pz, double E, double bm,
                       PfRec64 &r, double &bhi) {
     const DevParams &P = d.P;
@@ -132,25 +142,16 @@ inline void pf_record(const Derived &d, double px, double py, double pz, double 
 
 inline void pf_record(const Derived &d, double px, double py, double pz, double E, double bm,
                       PfRec32 &r, float &bhi) {
-    const double eps32 = 5.9604644775390625e-8;
-    const DevParams &P = d.P;
-    const double beta = P.boost ? pz / E : pz;
-    const double cw = P.qinv ? INFINITY
-                             : (P.boost ? d.c_beta / E : d.c_beta) * (1.0 + 8 * eps32) +
-                                   4 * eps32 * std::max(1.0, bm);
-    // to FP32 rounded to nearest, then one FP32 ulp outward
-    r = PfRec32{(float)px, (float)py, (float)(px * px + py * py - 0.5 * d.mid),
-                std::nextafter((float)(beta - cw), -INFINITY)};
-    bhi = std::nextafter((float)(beta + cw), INFINITY);
+    pf_make(pf_maker(d, bm), px, py, pz, E, r, bhi);
 }
 
 // Prefilter margins that depend on the data's momentum scale (|pT|^2 up to
 // pmax2), for the records' precision (FP32 in the precision form).  With
 // S = max(1, pmax2) + |mid|: the rounding of the records (px, py, nrm) and
-// of u, v, dn, T, Q - H^2 stays below 8 ulp of S, so that of the products
-// dn^2, (Q - H^2) T and H^2 T below 150 ulp of max(1, H^2) S^2 (|dn|, T,
-// Q <= 4 S); the T window allows 64 ulp of 2 S, each q window a margin c
-// of 256 ulp of max(1, H^2) S^2.
+// of their products and sums, in any order, stays below 12 ulp of S for T,
+// dn and C (|dn|, |C| <= 2 S, T <= 4 S), so that of m^2 - X below 100 ulp of
+// max(1, H^2) S^2; the T window allows 64 ulp of 2 S, the q window a margin
+// c of 256 ulp of max(1, H^2) S^2.
 inline void prefilter_margins(const Derived &d, double pmax2, DevParams &P) {
     const double pm = std::max(1.0, pmax2);
     const double eps32 = 5.9604644775390625e-8, eps64 = 1.1102230246251565e-16;
@@ -190,36 +191,6 @@ struct default_init_allocator : A {
 template <typename T>
 using hvec = std::vector<T, default_init_allocator<T>>;
 
-// Fast-kernel records of one ordering of a particle list: the 64-byte
-// particle records and the prefilter records of one precision (FP32 for
-// the precision form, FP64 otherwise; the other pair stays empty).
-struct RecordSet {
-    hvec<PartRec> rec;
-    hvec<PfRec64> pf64;
-    hvec<PfRec32> pf32;
-    hvec<double> cw64;
-    hvec<float> cw32;
-    void resize_prefilter(size_t n, bool f32) {
-        pf64.resize(f32 ? 0 : n);
-        cw64.resize(f32 ? 0 : n);
-        pf32.resize(f32 ? n : 0);
-        cw32.resize(f32 ? n : 0);
-    }
-    void resize(size_t n, bool f32) {
-        rec.resize(n);
-        resize_prefilter(n, f32);
-    }
-    void copy_from(const RecordSet &o, size_t dst, size_t src, bool f32) {  // prefilter records
-        if (f32) {
-            pf32[dst] = o.pf32[src];
-            cw32[dst] = o.cw32[src];
-        } else {
-            pf64[dst] = o.pf64[src];
-            cw64[dst] = o.cw64[src];
-        }
-    }
-};
-
 // Particles of one list after the rapidity cut, in the reference's gather
 // order (keep, off: the plain kernels and the order of the pair cap), and
 // the fast kernel's lists:
@@ -240,20 +211,20 @@ struct HostParticles {
     std::vector<double> psi2;     // psi_ref (n=2) per group, over all input particles
     long long nf = 0;             // fast-list particles
     std::vector<long long> foff;  // nev+1 fast-list offsets
-    RecordSet fast;               // fast list: records
+    hvec<PartRec> fast;           // fast list: records (the prefilter's follow on the device)
     hvec<double> f_pt;            // |pT| of the fast list (mixed windows)
-    RecordSet srt;                // (px cell, py)-sorted per group (prefilter records only)
     hvec<OrigRank> orr;           // srt position -> fast-list index, gather rank
     hvec<int> srt_cell;           // px cell in srt order (same-event windows)
     hvec<double> srt_py;          // py in srt order
     double pmax2 = 0.0;  // max px^2+py^2 over the fast list (FP32 prefilter margins)
+    double bm = 0.0;     // max |beta| over it
     // Empties the lists for the next gather and keeps their storage, so a
     // caller that reuses one (the request server's pool) writes into pages
     // already faulted in: fresh buffers cost a third of a gather in page
     // faults.
     void reset() {
         n = n_in = nf = 0;
-        pmax2 = 0.0;
+        pmax2 = bm = 0.0;
     }
 };
 
@@ -347,7 +318,7 @@ inline bool rapidity_kept(double pz, double E, double cut_min, double cut_max) {
 
 // Rapidity cut of the gathers (HBT_correlation.cpp:255-266, :468-476),
 // psi_ref per group (:181-183, :233-249; over all particles passed in), and
-// the prefilter records.  Events keep < 2^18 particles (the fast kernel's
+// the fast lists.  Events keep < 2^18 particles (the fast kernel's
 // survivor encoding).
 inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
                             const int32_t *grp_ev, int nev, const int64_t *ev_off,
@@ -364,7 +335,6 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
     for (int g = 0; g < ngroups; g++)
         if (grp_ev[g + 1] < grp_ev[g]) return err = "group offsets decrease", HBT_ERR_ARG;
     const DevParams &P = d.P;
-    const bool f32 = k.precision == HBT_PREC_FP32C;
     h.reset();  // every list below is sized and written in full
     h.n_in = nev > 0 ? ev_off[nev] - ev_off[0] : 0;
     const double cut_max = tanh(k.HBTrap_max);
@@ -401,22 +371,21 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
             h.foff[e + 1] = cf;
         }
     });
-    double bm = 0.0;
     for (int e = 0; e < nev; e++) {
         if (h.off[e + 1] >= (1 << 18))
             return err = "an event keeps more than 262143 particles", HBT_ERR_CAPACITY;
         h.off[e + 1] += h.off[e];
         h.foff[e + 1] += h.foff[e];
         h.pmax2 = std::max(h.pmax2, pmax[e]);
-        bm = std::max(bm, bmax[e]);
+        h.bm = std::max(h.bm, bmax[e]);
     }
     const long long n = h.off[nev], nf = h.foff[nev];
     if (n >= (1ll << 31)) return err = "buffer too large", HBT_ERR_CAPACITY;
     h.n = n;
     h.nf = nf;
     h.keep.resize((size_t)n);
-    RecordSet &F = h.fast;
-    F.resize((size_t)nf, f32);
+    hvec<PartRec> &F = h.fast;
+    F.resize((size_t)nf);
     h.f_pt.resize((size_t)nf);
     hvec<int> frank((size_t)nf);
     // pass 2, per event: gather order, then the fast list sorted by |pT|
@@ -440,11 +409,7 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
             for (const auto &x : ev) {
                 const int64_t i = h.keep[x.second];
                 const double px = soa[0][i], py = soa[1][i], pz = soa[2][i], E = soa[3][i];
-                F.rec[f] = PartRec{px, py, pz, E, soa[4][i], soa[5][i], soa[6][i], soa[7][i]};
-                if (f32)
-                    pf_record(d, px, py, pz, E, bm, F.pf32[f], F.cw32[f]);
-                else
-                    pf_record(d, px, py, pz, E, bm, F.pf64[f], F.cw64[f]);
+                F[f] = PartRec{px, py, pz, E, soa[4][i], soa[5][i], soa[6][i], soa[7][i]};
                 h.f_pt[f] = x.first;
                 frank[f] = (int)x.second;
                 f++;
@@ -472,8 +437,7 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
             }
         });
     }
-    // prefilter records per group sorted by px cell, then py (stable)
-    h.srt.resize_prefilter((size_t)nf, f32);
+    // each group's order by px cell, then py (stable)
     h.orr.resize((size_t)nf);
     h.srt_cell.resize((size_t)nf);
     h.srt_py.resize((size_t)nf);
@@ -483,15 +447,14 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
     auto sort_group = [&](long long g, CellOrderScratch &sc, std::vector<int> &order) {
         const long long g0 = h.foff[grp_ev[g]], g1 = h.foff[grp_ev[g + 1]];
         order.resize((size_t)(g1 - g0));
-        cell_order((int)(g1 - g0), [&](int k) { return F.rec[g0 + k].px; },
-                   [&](int k) { return F.rec[g0 + k].py; }, D, sc, order.data(),
+        cell_order((int)(g1 - g0), [&](int k) { return F[g0 + k].px; },
+                   [&](int k) { return F[g0 + k].py; }, D, sc, order.data(),
                    h.srt_cell.data() + g0, lone);
         auto copy = [&](long long q0, long long q1) {
             for (long long q = g0 + q0; q < g0 + q1; q++) {
                 const int src = (int)g0 + order[(size_t)(q - g0)];
-                h.srt.copy_from(F, (size_t)q, (size_t)src, f32);
                 h.orr[q] = OrigRank{src, frank[src]};
-                h.srt_py[q] = F.rec[src].py;
+                h.srt_py[q] = F[src].py;
             }
         };
         if (lone)
@@ -518,8 +481,11 @@ constexpr size_t kItemsPerWave = 4;
 // L2 of one XCD (MI355X: 4 MB).
 constexpr size_t kL2BytesPerXcd = (size_t)4 << 20;
 
+// A tile is the 64 particles of a wave's four matrix blocks, whatever
+// t.R (its range of 1, 2 and 4 stays accepted): larger tiles would widen
+// every window and hold no more particles at once.
 inline ItemShape item_shape(const hbt_tuning &t) {
-    return ItemShape{64 * t.R, std::max(64, t.jchunk), std::max(1, std::min(t.kchunk, 64))};
+    return ItemShape{64, std::max(64, t.jchunk), std::max(1, std::min(t.kchunk, 64))};
 }
 
 // Pairs left to the host by the device (DeferRec): room per context or
@@ -637,8 +603,8 @@ inline void result_from_host(const Derived &d, const hbt_config &k, const double
 }
 
 // Defined in hbt_engine.hip.  Zeroes the work counter and launches
-// k_fast<Prec, R, EXT> with `blocks` workgroups of 256 on stream st.
-hipError_t launch_fast_kernel(const FastArgs &a, bool f32, int R, bool ext, long blocks,
+// k_fast<Prec, EXT> with `blocks` workgroups of 256 on stream st.
+hipError_t launch_fast_kernel(const FastArgs &a, bool f32, bool ext, long blocks,
                               hipStream_t st);
 // Zeroes n 8-byte words with a fill kernel (safe inside graph capture).
 hipError_t launch_zero_words(void *p, size_t n, hipStream_t st);

@@ -32,7 +32,7 @@
 // q_inv arrays (count, den, sum, num) of nq words each, the deferred-pair
 // count -- copied back in one piece -- and the deferred-pair records), and
 // per part (256-byte aligned parts): particle records (64 B), prefilter
-// records (32 or 16 B), c/E bounds, plan windows, (cos, sin) per row, and
+// operands (16 B), beta intervals (8 B), plan windows, (cos, sin) per row, and
 // psi_ref per group.  A part's same-event list also serves as its mixed list
 // (partners are events of the same group).
 #include <hip/hip_runtime.h>
@@ -128,7 +128,7 @@ struct Part {
     double pmax2 = 0.0;
     // device residency
     size_t foot = 0, arena_off = 0;
-    size_t o_rec = 0, o_srec = 0, o_pf = 0, o_cw = 0, o_spf = 0, o_scw = 0, o_orig = 0, o_win = 0,
+    size_t o_rec = 0, o_srec = 0, o_pf = 0, o_bw = 0, o_spf = 0, o_sbw = 0, o_orig = 0, o_win = 0,
            o_cs = 0, o_psi = 0;
     int view = -1;
     View v{};
@@ -234,21 +234,21 @@ size_t part_layout(const hbt_server *s, Part *p, long long nf, long long rows, s
     Part tmp;
     Part &r = p ? *p : tmp;
     size_t o = 0;
-    // fast-list records and their cell-sorted copy, the prefilter records of both
+    // fast-list records and their cell-sorted copy, the prefilter's operands of both
     for (size_t *po : {&r.o_rec, &r.o_srec}) {
         *po = o;
-        o = align256(o + (size_t)nf * sizeof(PartRec));
+        o = align256(o + (size_t)(nf + kPfPad) * sizeof(PartRec));
     }
     for (size_t *po : {&r.o_pf, &r.o_spf}) {
         *po = o;
-        o = align256(o + (size_t)nf * (s->f32 ? sizeof(PfRec32) : sizeof(PfRec64)));
+        o = align256(o + (size_t)(nf + kPfPad) * sizeof(PfOp));
     }
-    for (size_t *po : {&r.o_cw, &r.o_scw}) {
+    for (size_t *po : {&r.o_bw, &r.o_sbw}) {
         *po = o;
-        o = align256(o + (size_t)nf * (s->f32 ? 4 : 8));
+        o = align256(o + (size_t)(nf + kPfPad) * sizeof(PfBeta));
     }
     r.o_orig = o;
-    o = align256(o + (size_t)nf * sizeof(OrigRank));
+    o = align256(o + (size_t)(nf + kPfPad) * sizeof(OrigRank));
     r.o_win = o;
     o = align256(o + std::max<size_t>(nwins, 1) * sizeof(JWin));
     r.o_cs = o;
@@ -276,10 +276,10 @@ void make_part_view(hbt_server *s, Part &p) {
     v.H.ndefer = (unsigned *)(h + s->defer_count_off);
     v.H.defer_cap = kReqDeferCap;
     v.A = v.B = (const PartRec *)(b + p.o_rec);
-    v.pfA = v.pfB = (const void *)(b + p.o_pf);
-    v.cwA = v.cwB = (const void *)(b + p.o_cw);
-    v.pfS = (const void *)(b + p.o_spf);
-    v.cwS = (const void *)(b + p.o_scw);
+    v.pfA = v.pfB = (const PfOp *)(b + p.o_pf);
+    v.bwA = v.bwB = (const PfBeta *)(b + p.o_bw);
+    v.pfS = (const PfOp *)(b + p.o_spf);
+    v.bwS = (const PfBeta *)(b + p.o_sbw);
     v.origS = (const OrigRank *)(b + p.o_orig);
     v.AS = (const PartRec *)(b + p.o_srec);
     v.mwin = (const JWin *)(b + p.o_win);
@@ -301,19 +301,7 @@ hipError_t upload_part(hbt_server *s, Part &p) {
     auto cp = [&](size_t off, const void *src, size_t bytes) {
         if (bytes) pieces.push_back(StagePiece{b + off, src, bytes});
     };
-    const std::pair<const RecordSet *, size_t> sets[] = {{&p.hp.fast, 0}, {&p.hp.srt, 1}};
-    for (const auto &x : sets) {
-        const RecordSet &R = *x.first;
-        const bool srt = x.second == 1;
-        if (!srt) cp(p.o_rec, R.rec.data(), (size_t)nf * sizeof(PartRec));
-        if (s->f32) {
-            cp(srt ? p.o_spf : p.o_pf, R.pf32.data(), (size_t)nf * sizeof(PfRec32));
-            cp(srt ? p.o_scw : p.o_cw, R.cw32.data(), (size_t)nf * 4);
-        } else {
-            cp(srt ? p.o_spf : p.o_pf, R.pf64.data(), (size_t)nf * sizeof(PfRec64));
-            cp(srt ? p.o_scw : p.o_cw, R.cw64.data(), (size_t)nf * 8);
-        }
-    }
+    cp(p.o_rec, p.hp.fast.data(), (size_t)nf * sizeof(PartRec));
     cp(p.o_orig, p.hp.orr.data(), p.hp.orr.size() * sizeof(OrigRank));
     cp(p.o_win, p.wins.data(), p.wins.size() * sizeof(JWin));
     cp(p.o_cs, p.plan_cs.data(), p.plan_cs.size() * 8);
@@ -323,8 +311,10 @@ hipError_t upload_part(hbt_server *s, Part &p) {
     if (e == hipSuccess) e = ensure_pinned(&s->h_stage, &s->stage_cap, stage_bytes(pieces));
     if (e == hipSuccess) e = stage_pieces(s->h_stage, pieces, s->s_upload);
     if (e == hipSuccess)
-        e = gather_srt((const PartRec *)(b + p.o_rec), (const OrigRank *)(b + p.o_orig),
-                       (PartRec *)(b + p.o_srec), nf, s->s_upload);
+        e = build_lists(pf_maker(s->D, p.hp.bm), (const PartRec *)(b + p.o_rec),
+                        (const OrigRank *)(b + p.o_orig), (PartRec *)(b + p.o_srec),
+                        (PfOp *)(b + p.o_pf), (PfBeta *)(b + p.o_bw), (PfOp *)(b + p.o_spf),
+                        (PfBeta *)(b + p.o_sbw), nf, s->s_upload);
     if (e == hipSuccess)
         e = hipMemcpyAsync(s->d_views + p.view, &p.v, sizeof(View), hipMemcpyHostToDevice,
                            s->s_upload);
@@ -525,7 +515,7 @@ void launcher_loop(hbt_server *s) {
                 1l, std::min<long>((long)s->cu_count * s->sc.tune.blocks_per_cu,
                                    ((long)items.size() + 3) / 4));
             if (e == hipSuccess)
-                e = launch_fast_kernel(a, s->f32, s->sc.tune.R, s->ext, blocks, s->s_compute);
+                e = launch_fast_kernel(a, s->f32, s->ext, blocks, s->s_compute);
             if (e == hipSuccess) e = hipEventRecord(s->step_t1[buf], s->s_compute);
             if (e == hipSuccess) e = hipEventRecord(s->step_ev[buf], s->s_compute);
             if (e == hipSuccess) {

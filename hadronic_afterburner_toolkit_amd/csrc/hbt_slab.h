@@ -64,6 +64,13 @@ struct SlabArgs {
     double q_base, inv_dq;     // q_side / q_long bin of a stored value
 };
 
+// First record of block b's region of slab s (the regions hold fewer than
+// 2^32 records).
+template <typename Args>
+__device__ __forceinline__ unsigned slab_first(const Args &a, int s, unsigned b) {
+    return (unsigned)a.sbase[s] + b * (unsigned)a.scap[s];
+}
+
 // Totals of one unit, per bin of its slab.
 struct SlabPart {
     double cnt, qo, qs, ql, c;
@@ -73,40 +80,41 @@ struct SlabPart {
 // k_slab_bin evaluate it on the same stored value with the same two
 // rounded operations (the build contracts nothing), so they agree bit for
 // bit; k_fast writes a record only where it equals the pair's bin.
-__device__ __forceinline__ int slab_coord(const SlabArgs &a, double v) {
+template <typename Args>
+__device__ __forceinline__ int slab_coord(const Args &a, double v) {
     return (int)((v - a.q_base) * a.inv_dq);
 }
 
-// An FP32 record value k_slab_bin sums exactly in its fixed point: 0, or
-// 2^-17 <= |v| <= 1 (then v is a multiple of 2^-40 and |v| 2^40 <= 2^40).
-__device__ __forceinline__ bool fix_exact(float v) {
-    const float m = fabsf(v);
-    return m == 0.0f || (m >= 0x1p-17f && m <= 1.0f);
+// FP32 record values k_slab_bin sums exactly in its fixed point: 2^-17 <=
+// |v| <= 1 (then v is a multiple of 2^-40 and |v| 2^40 <= 2^40).  (0 would be
+// exact too; such a pair takes the direct path, which adds the same.)
+__device__ __forceinline__ bool fix_exact(float a, float b, float c, float d) {
+    const float lo = fminf(fminf(fabsf(a), fabsf(b)), fminf(fabsf(c), fabsf(d)));
+    const float hi = fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d)));
+    return lo >= 0x1p-17f && hi <= 1.0f;
 }
 
 // A binned same-event pair r as a record of this block's region of slab
 // r.s; false: the pair takes the direct path (also for a precision-form
-// value the fixed point would not hold exactly).  fill: the block's LDS fill
-// counters; cap and base: the regions' capacity and first record (as in
-// SlabArgs), LDS copies or SlabArgs' own arrays.
-template <typename Prec>
-__device__ __forceinline__ bool slab_put_same(const SlabArgs &a, unsigned *fill, const int *cap,
-                                              const long long *base, const SameRec &r) {
+// value the fixed point would not hold exactly, and for stored values that
+// would land in another bin, which only a pair near an edge can have).
+// next: the block's LDS array of each slab's next record; a region ends at
+// lim[s], the block's LDS copy, or (lim null) where SlabArgs says.
+template <typename Prec, typename Args>
+__device__ __forceinline__ bool slab_put_same(const Args &a, unsigned *next,
+                                              const unsigned *lim, const SameRec &r) {
     constexpr bool f32 = std::is_same<Prec, float>::value;
-    if (slab_coord(a, f32 ? (double)(float)r.qs : r.qs) != r.is ||
-        slab_coord(a, f32 ? (double)(float)r.ql : r.ql) != r.il)
+    if (!r.sure && (slab_coord(a, f32 ? (double)(float)r.qs : r.qs) != r.is ||
+                    slab_coord(a, f32 ? (double)(float)r.ql : r.ql) != r.il))
         return false;
-    if (f32 && !(fix_exact((float)r.qo) && fix_exact((float)r.qs) && fix_exact((float)r.ql) &&
-                 fix_exact((float)r.c)))
-        return false;
-    const unsigned pos = atomicAdd(&fill[r.s], 1u);
-    const int c = cap[r.s];
-    if (pos >= (unsigned)c) return false;
-    const long long e = base[r.s] + (long long)blockIdx.x * c + pos;
+    const float4 v = make_float4((float)r.qo, (float)r.qs, (float)r.ql, (float)r.c);
+    if (f32 && !fix_exact(v.x, v.y, v.z, v.w)) return false;
+    const unsigned e = atomicAdd(&next[r.s], 1u);
+    if (e >= (lim ? lim[r.s] : slab_first(a, r.s, blockIdx.x + 1))) return false;
     if (f32) {
-        ((float4 *)a.vals)[e] = make_float4((float)r.qo, (float)r.qs, (float)r.ql, (float)r.c);
+        ((float4 *)a.vals)[e] = v;
     } else {
-        double2 *d = (double2 *)a.vals + 2 * e;
+        double2 *d = (double2 *)a.vals + 2ull * e;
         d[0] = make_double2(r.qo, r.qs);
         d[1] = make_double2(r.ql, r.c);
     }
