@@ -361,11 +361,12 @@ struct Exact<float, EXT> {
 struct PairAt {
     unsigned a, b, buf;
 };
+template <bool RANKED>
 __device__ __forceinline__ PairAt pair_at(const WaveLds &wl, unsigned ent, bool mixed) {
     const unsigned i = ent & 63u, j = ent >> 6 & 31u, buf = ent >> 11;
     const unsigned ai = lds_row(i);
     const unsigned aj = (unsigned)offsetof(WaveLds, jrec) + buf * 2048u + lds_row(j);
-    const bool swap = !mixed && wl.irank[i] > wl.jrank[buf][j];
+    const bool swap = RANKED && !mixed && wl.irank[i] > wl.jrank[buf][j];
     return PairAt{swap ? aj : ai, swap ? ai : aj, buf};
 }
 
@@ -418,7 +419,7 @@ struct Stage {
 // per binned pair.
 // unsure: the lanes whose pair the precision form could not decide, unsure_phi
 // those of them that miss only their K_phi bin.
-template <typename Prec, bool EXT>
+template <typename Prec, bool EXT, bool RANKED>
 __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, Stage &stg,
                                      unsigned head, int cnt, bool mixed, double psi,
                                      unsigned *next, const unsigned *lim,
@@ -429,7 +430,7 @@ __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, St
     SameRec rec;
     long kmix = 0;
     if (lane < cnt) {
-        const PairAt pr = pair_at(wl, wl.ring[(head + lane) & 127u], mixed);
+        const PairAt pr = pair_at<RANKED>(wl, wl.ring[(head + lane) & 127u], mixed);
         const char *base = (const char *)&wl;
         if (mixed)
             st = Exact<Prec, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], kmix);
@@ -495,7 +496,7 @@ __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, St
 // rather than inside it: the literal cascade's registers then do not add to
 // the exact stage's.  cos stays the form's own (FP32), except for the lanes
 // cos64.
-template <bool EXT>
+template <bool EXT, bool RANKED>
 __device__ __forceinline__ int drain_literal(CView *vp, CArgs *ka, const WaveLds &wl, unsigned head,
                                              unsigned long long lanes, unsigned long long cos64,
                                              bool mixed, double psi,
@@ -503,7 +504,7 @@ __device__ __forceinline__ int drain_literal(CView *vp, CArgs *ka, const WaveLds
     const int lane = __lane_id();
     bool binned = false;
     if (lanes >> lane & 1ull) {
-        const PairAt pr = pair_at(wl, wl.ring[(head + lane) & 127u], mixed);
+        const PairAt pr = pair_at<RANKED>(wl, wl.ring[(head + lane) & 127u], mixed);
         const char *base = (const char *)&wl;
         if (mixed) {
             long k = 0;
@@ -557,25 +558,234 @@ __device__ __forceinline__ unsigned rows_first(int n) {
     return ((0xfu << (4 - k)) & 0xfu) * 0x1111u;
 }
 
+// What a wave carries from item to item: totals of binned pairs (uniform), and
+// the block's slab regions.
+struct WaveTotals {
+    unsigned long long same = 0, mixed = 0, direct = 0;
+    unsigned *slab_next;
+    const unsigned *slab_lim;
+};
+
+// ------------------------------------------------------------------ an item
+// The wave holds the item's 64 i particles as four blocks of 16 matrix
+// columns and walks its j segments (same-event: one range with j > i;
+// mixed: one partner window, window(seg), per segment with the i particles
+// rotated by -theta) in pairs of tiles of 16 j rows.  Three 16x16x4 FP32
+// products per block and tile give X, P and M of 256 pairs, four per lane; 8
+// VALU operations test a pair and a ninth shifts the outcome into the lane's
+// bit word.  (The scalar form took 16, and 7 more to queue the survivors of
+// each j; comparisons whose masks are combined in scalar registers take 7,
+// but the hops between the two units leave the VALU idle: 8000 cycles per
+// pair of tiles and wave against 6200.)  Then each lane with bits left queues
+// one survivor per round, and whenever 64 are queued they are binned, one per
+// lane; the last survivors of a pair of tiles wait for at most the next
+// pair's (the exact cascade has a single call site).
+// RANKED: a same-event pair is oriented by the gather ranks of its particles;
+// otherwise by their places in the list.
+template <typename Prec, bool EXT, bool RANKED, typename Window>
+__device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double psi,
+                                          const PfConst<float> &pk, WaveLds &wl, Stage &stg,
+                                          WaveTotals &tot, Window window) {
+    const bool mixed = w.kind != 0;
+    const int lane = __lane_id();
+    const int col = lane & 15, comp = lane >> 4, row0 = 4 * comp;
+    // same-event tiles run over the cell-sorted list, mixed ones over the
+    // |pT|-sorted fast lists
+    const PfOp *pfi = (mixed ? vp->pfA : vp->pfS) + w.i0;
+    const PfBeta *bwi = (mixed ? vp->bwA : vp->bwS) + w.i0;
+    const PfOp *pfj = mixed ? vp->pfB : vp->pfS;
+    const PfBeta *bwj = mixed ? vp->bwB : vp->bwS;
+    const PartRec *recj = mixed ? vp->B : vp->AS;
+    {
+        const PartRec *reci = (mixed ? vp->A : vp->AS) + w.i0;
+        const int last = w.ni - 1;
+        const double2 v0 = stage_load<4>(reci, lane, 0, last);
+        const double2 v1 = stage_load<4>(reci, lane, 16, last);
+        const double2 v2 = stage_load<4>(reci, lane, 32, last);
+        const double2 v3 = stage_load<4>(reci, lane, 48, last);
+        __builtin_amdgcn_wave_barrier();
+        stage_store<4>(wl.irec, lane, 0, v0);
+        stage_store<4>(wl.irec, lane, 16, v1);
+        stage_store<4>(wl.irec, lane, 32, v2);
+        stage_store<4>(wl.irec, lane, 48, v3);
+        if (RANKED && !mixed) wl.irank[lane] = vp->origS[w.i0 + min(lane, last)].rank;
+    }
+    float ilo[4], ihi[4];
+    PfBlock blk[4];
+    // The i blocks, rotated by -theta for a mixed segment (columns past the
+    // tile's end repeat its last particle; `cols` masks them).
+    auto load_blocks = [&](double c, double s) {
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const PfOp p = pfi[min(16 * b + col, w.ni - 1)];
+            float x = p.px, y = p.py;
+            if (mixed) {
+                x = (float)((double)p.px * c + (double)p.py * s);
+                y = (float)((double)p.py * c - (double)p.px * s);
+            }
+            blk[b] = pf_block(pk, comp, x, y, p.nrm);
+        }
+    };
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        const PfBeta r = bwi[min(16 * b + col, w.ni - 1)];
+        ilo[b] = r.lo;
+        ihi[b] = r.hi;
+    }
+    unsigned cols = 0;  // the bits of the blocks' columns inside the tile
+#pragma unroll
+    for (int b = 0; b < 4; b++) cols = cols << 4 | (16 * b + col < w.ni ? 0xfu : 0u);
+    cols |= cols << 16;
+    const int nseg = mixed ? w.nj : 1;
+    int seg = -1, jc = 0, je = 0;  // the segment, its next j and its end
+    unsigned head = 0, tail = 0, buf = 0;
+    double2 rot = {1.0, 0.0};
+    for (;;) {
+        while (jc >= je && ++seg < nseg) {  // the next segment
+            if (mixed) {
+                const JWin jw = window(seg);
+                jc = jw.b;
+                je = jw.e;
+                rot.x = HBT_CONST(double, vp->plan_cs)[2 * jw.row];
+                rot.y = HBT_CONST(double, vp->plan_cs)[2 * jw.row + 1];
+            } else {
+                jc = (int)w.j0;
+                je = (int)w.j0 + w.nj;
+            }
+            load_blocks(rot.x, rot.y);
+        }
+        const bool end = jc >= je;
+        const unsigned mark = tail;  // survivors of earlier pairs
+        unsigned bits = 0, ent = 0;
+        if (!end) {
+            // 32 j's, two tiles (the lane's share as a 32-bit offset from
+            // a uniform base)
+            const int cnt = min(32, je - jc);
+            const char *pa = (const char *)(pfj + jc), *pb = (const char *)(bwj + jc);
+            float A[2];
+            PfBeta jw[2][4];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                A[t] = *(const float *)(pa + (unsigned)(256 * t + 16 * col + 4 * comp));
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    jw[t][r] = *(const PfBeta *)(pb + (unsigned)(128 * t + 8 * (row0 + r)));
+            }
+            double2 s0, s1 = {0.0, 0.0};
+            int rank = 0;
+            if (mixed) {
+                s0 = stage_load<2>(recj + jc, lane, 0, 31);
+            } else {
+                s0 = stage_load<4>(recj + jc, lane, 0, 31);
+                s1 = stage_load<4>(recj + jc, lane, 16, 31);
+                if (RANKED) rank = vp->origS[jc + (lane & 31)].rank;
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                if (16 * t >= cnt) {
+                    bits <<= 16;
+                    continue;
+                }
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
+                    const v4f X =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].X, o, 0, 0, 0);
+                    const v4f U =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].P, o, 0, 0, 0);
+                    const v4f V =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].M, o, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float e = fabsf(U[r]) + fabsf(V[r]);
+                        const float m = fmaxf(
+                            fmaxf(fmaf(e, e, -X[r]) - pk.c0, fmaf(X[r], X[r], pk.nsh2)),
+                            fmaxf(ilo[b] - jw[t][r].hi, jw[t][r].lo - ihi[b]));
+                        // bits << 1 | sign of m
+                        bits = __builtin_amdgcn_alignbit(bits, __builtin_bit_cast(unsigned, m),
+                                                         31);
+                    }
+                }
+            }
+            bits &= cols;
+            if (cnt < 32)  // rows past the segment's end
+                bits &= rows_first(cnt - row0) << 16 | rows_first(cnt - 16 - row0);
+            if (!mixed && jc < (int)w.i0 + 64) {
+                // the tile's own particles: only j > i
+                const int d0 = (int)w.i0 - jc + col - row0 + 1;
+                unsigned keep = 0;
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int b = 0; b < 4; b++)
+                        keep = keep << 4 | 0xfu >> min(max(d0 + 16 * b - 16 * t, 0), 4);
+                bits &= keep;
+            }
+            buf ^= 1u;
+            ent = buf << 11 | (unsigned)row0 << 6 | (unsigned)col;
+            __builtin_amdgcn_wave_barrier();
+            if (mixed) {
+                stage_store<2>(wl.jrec[buf], lane, 0, s0);
+                if (lane == 0) wl.rot[buf] = rot;
+            } else {
+                stage_store<4>(wl.jrec[buf], lane, 0, s0);
+                stage_store<4>(wl.jrec[buf], lane, 16, s1);
+                if (RANKED && lane < 32) wl.jrank[buf][lane] = rank;
+            }
+            jc += 32;
+        }
+        for (;;) {
+            // queue one survivor of each lane that has any
+            unsigned long long m;
+            while ((m = __ballot(bits != 0u)) != 0ull && tail - head < 64u) {
+                const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, tail));
+                if (bits != 0u) {
+                    const unsigned p = (unsigned)__builtin_clz(bits);  // 16 t + 4 b + r
+                    bits &= ~(0x80000000u >> p);
+                    wl.ring[pos & 127u] = (unsigned short)(ent + (((p & 16u) | (p & 3u)) << 6) +
+                                                           ((p & 12u) << 2));
+                }
+                tail += (unsigned)__popcll(m);
+            }
+            // a full wave; or, with nothing left to queue, the survivors
+            // whose j buffer the next pair takes (at the end: all)
+            const unsigned n = tail - head;
+            if (n < 64u && (m != 0ull || (end ? n == 0u : (int)(mark - head) <= 0))) break;
+            const int take = (int)min(64u, n);
+            __builtin_amdgcn_wave_barrier();
+            CArgs *kd = kernel_args();
+            unsigned long long unsure = 0, unsure_phi = 0;
+            int nb = drain<Prec, EXT, RANKED>(view_at(kd->views, w.view), kd, wl, stg, head, take,
+                                      mixed, psi, tot.slab_next, tot.slab_lim, tot.direct, unsure,
+                                      unsure_phi);
+            if (std::is_same<Prec, float>::value && __builtin_expect(unsure != 0ull, 0)) {
+                kd = kernel_args();
+                nb += drain_literal<EXT, RANKED>(view_at(kd->views, w.view), kd, wl, head, unsure,
+                                         unsure_phi, mixed, psi, tot.direct);
+            }
+            if (mixed)
+                tot.mixed += nb;
+            else
+                tot.same += nb;
+            head += take;
+        }
+        if (end) break;
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
 // ---------------------------------------------------------------- kernel
 // Persistent: each wave pulls work items from the queue of its XCD (the host
 // puts all items of a group in one queue, so a group's particles stay in one
-// XCD's L2), then from the next queues in turn, until all are empty.  Per
-// item the wave holds 64 i particles as four blocks of 16 matrix columns and
-// walks its j segments (same-event: one range with j > i in the cell-sorted
-// list; mixed: one partner window per segment with the i particles rotated
-// by -theta) in pairs of tiles of 16 j rows.  Three 16x16x4 FP32 products
-// per block and tile give X, P and M of 256 pairs, four per lane; 6 VALU
-// operations test a pair and a seventh shifts the outcome into the lane's bit
-// word (the scalar form took 16, and 7 more to queue the survivors of each
-// j).  Then each lane with bits left queues one survivor per round, and
-// whenever 64 are queued they are binned, one per lane; the last survivors of
-// a pair of tiles wait for at most the next pair's (the exact cascade has a
-// single call site).
+// XCD's L2), then from the next queues in turn, until all are empty.
 // Occupancy: four blocks' LDS fill the CU's 160 KB, so four waves per SIMD
-// (128 VGPRs, no spills in the common case); the K_phi / q_inv instance of
-// the FP64 form, whose main path is the literal cascade with atan2 and the
+// (128 VGPRs, no spills in the hot path); the K_phi / q_inv instance of the
+// FP64 form, whose main path is the literal cascade with atan2 and the
 // host-defer path, runs at three.
+// Headline workload (2.5e10 pairs, 4.8e9 evaluated): 5.6 ms in the precision
+// form, of which the prefilter alone 2.6 and the mixed adds' atomic floor 3.3;
+// 8.0 ms with scalar tests and records fetched by scattered loads.
 template <typename Prec, bool EXT>
 constexpr int fast_waves_per_eu() {
     return EXT && std::is_same<Prec, double>::value ? 3 : 4;
@@ -602,13 +812,13 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_fast
         }
         __syncthreads();
     }
-    unsigned long long direct_n = 0;  // wave totals, uniform
+    WaveTotals tot;
+    tot.slab_next = slab_next;
+    tot.slab_lim = slab_lim;
     const int lane = __lane_id();
-    const int col = lane & 15, comp = lane >> 4, row0 = 4 * comp;
     WaveLds &wl = wave_lds[threadIdx.x >> 6];
     Stage &stg = ((Stage *)dyn_lds)[threadIdx.x >> 6];
     const PfConst<float> pk = pf_const<float>(a.P);
-    unsigned long long nb_same = 0, nb_mixed = 0;
 
     const int nq = a.nqueues;
     int wq = xcc_id() & (nq - 1);  // nq is a power of two
@@ -627,198 +837,20 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_fast
         const WorkItem w = HBT_CONST(WorkItem, ka->items)[q0 + it];
         CView *vp = view_at(ka->views, w.view);
         const double psi = HBT_CONST(double, vp->psi)[w.grp];
-        const bool mixed = w.kind != 0;
-        // same-event tiles run over the cell-sorted list, mixed ones over the
-        // |pT|-sorted fast lists
-        const PfOp *pfi = (mixed ? vp->pfA : vp->pfS) + w.i0;
-        const PfBeta *bwi = (mixed ? vp->bwA : vp->bwS) + w.i0;
-        const PfOp *pfj = mixed ? vp->pfB : vp->pfS;
-        const PfBeta *bwj = mixed ? vp->bwB : vp->bwS;
-        const PartRec *recj = mixed ? vp->B : vp->AS;
-        {
-            const PartRec *reci = (mixed ? vp->A : vp->AS) + w.i0;
-            const int last = w.ni - 1;
-            const double2 v0 = stage_load<4>(reci, lane, 0, last);
-            const double2 v1 = stage_load<4>(reci, lane, 16, last);
-            const double2 v2 = stage_load<4>(reci, lane, 32, last);
-            const double2 v3 = stage_load<4>(reci, lane, 48, last);
-            __builtin_amdgcn_wave_barrier();
-            stage_store<4>(wl.irec, lane, 0, v0);
-            stage_store<4>(wl.irec, lane, 16, v1);
-            stage_store<4>(wl.irec, lane, 32, v2);
-            stage_store<4>(wl.irec, lane, 48, v3);
-            if (!mixed) wl.irank[lane] = vp->origS[w.i0 + min(lane, last)].rank;
-        }
-        float ilo[4], ihi[4];
-        PfBlock blk[4];
-        // The i blocks, rotated by -theta for a mixed segment; columns past
-        // the tile's end get n = inf, which fails the K_T window.
-        auto load_blocks = [&](double c, double s) {
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int slot = 16 * b + col, i = min(slot, w.ni - 1);
-                const PfOp p = pfi[i];
-                float x = p.px, y = p.py;
-                if (mixed) {
-                    x = (float)((double)p.px * c + (double)p.py * s);
-                    y = (float)((double)p.py * c - (double)p.px * s);
-                }
-                blk[b] = pf_block(pk, comp, x, y, slot < w.ni ? p.nrm : INFINITY);
-            }
-        };
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const PfBeta r = bwi[min(16 * b + col, w.ni - 1)];
-            ilo[b] = r.lo;
-            ihi[b] = r.hi;
-        }
-        const int nseg = mixed ? w.nj : 1;
-        int seg = -1, jc = 0, je = 0;  // the segment, its next j and its end
-        unsigned head = 0, tail = 0, buf = 0;
-        double2 rot = {1.0, 0.0};
-        for (;;) {
-            while (jc >= je && ++seg < nseg) {  // the next segment
-                if (mixed) {
-                    const JWin jw = HBT_CONST(JWin, vp->mwin)[w.j0 + seg];
-                    jc = jw.b;
-                    je = jw.e;
-                    rot.x = HBT_CONST(double, vp->plan_cs)[2 * jw.row];
-                    rot.y = HBT_CONST(double, vp->plan_cs)[2 * jw.row + 1];
-                } else {
-                    jc = (int)w.j0;
-                    je = (int)w.j0 + w.nj;
-                }
-                load_blocks(rot.x, rot.y);
-            }
-            const bool end = jc >= je;
-            const unsigned mark = tail;  // survivors of earlier pairs
-            unsigned bits = 0, ent = 0;
-            if (!end) {
-                // 32 j's, two tiles (the lane's share as a 32-bit offset from
-                // a uniform base)
-                const int cnt = min(32, je - jc);
-                const char *pa = (const char *)(pfj + jc), *pb = (const char *)(bwj + jc);
-                float A[2];
-                PfBeta jw[2][4];
-#pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    A[t] = *(const float *)(pa + (unsigned)(256 * t + 16 * col + 4 * comp));
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        jw[t][r] = *(const PfBeta *)(pb + (unsigned)(128 * t + 8 * (row0 + r)));
-                }
-                double2 s0, s1 = {0.0, 0.0};
-                int rank = 0;
-                if (mixed) {
-                    s0 = stage_load<2>(recj + jc, lane, 0, 31);
-                } else {
-                    s0 = stage_load<4>(recj + jc, lane, 0, 31);
-                    s1 = stage_load<4>(recj + jc, lane, 16, 31);
-                    rank = vp->origS[jc + (lane & 31)].rank;
-                }
-#pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    if (16 * t >= cnt) {
-                        bits <<= 16;
-                        continue;
-                    }
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
-                        const v4f X =
-                            __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].X, o, 0, 0, 0);
-                        const v4f U =
-                            __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].P, o, 0, 0, 0);
-                        const v4f V =
-                            __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].M, o, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const float e = fabsf(U[r]) + fabsf(V[r]);
-                            const float m = fmaxf(
-                                fmaxf(fmaf(e, e, -X[r]) - pk.c0, fmaf(X[r], X[r], pk.nsh2)),
-                                fmaxf(ilo[b] - jw[t][r].hi, jw[t][r].lo - ihi[b]));
-                            // bits << 1 | sign of m
-                            bits = __builtin_amdgcn_alignbit(bits, __builtin_bit_cast(unsigned, m),
-                                                             31);
-                        }
-                    }
-                }
-                if (cnt < 32)  // rows past the segment's end
-                    bits &= rows_first(cnt - row0) << 16 | rows_first(cnt - 16 - row0);
-                if (!mixed && jc < (int)w.i0 + 64) {
-                    // the tile's own particles: only j > i
-                    const int d0 = (int)w.i0 - jc + col - row0 + 1;
-                    unsigned keep = 0;
-#pragma unroll
-                    for (int t = 0; t < 2; t++)
-#pragma unroll
-                        for (int b = 0; b < 4; b++)
-                            keep = keep << 4 | 0xfu >> min(max(d0 + 16 * b - 16 * t, 0), 4);
-                    bits &= keep;
-                }
-                buf ^= 1u;
-                ent = buf << 11 | (unsigned)row0 << 6 | (unsigned)col;
-                __builtin_amdgcn_wave_barrier();
-                if (mixed) {
-                    stage_store<2>(wl.jrec[buf], lane, 0, s0);
-                    if (lane == 0) wl.rot[buf] = rot;
-                } else {
-                    stage_store<4>(wl.jrec[buf], lane, 0, s0);
-                    stage_store<4>(wl.jrec[buf], lane, 16, s1);
-                    if (lane < 32) wl.jrank[buf][lane] = rank;
-                }
-                jc += 32;
-            }
-            for (;;) {
-                // queue one survivor of each lane that has any
-                unsigned long long m;
-                while ((m = __ballot(bits != 0u)) != 0ull && tail - head < 64u) {
-                    const unsigned pos = __builtin_amdgcn_mbcnt_hi(
-                        (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, tail));
-                    if (bits != 0u) {
-                        const unsigned p = (unsigned)__builtin_clz(bits);  // 16 t + 4 b + r
-                        bits &= ~(0x80000000u >> p);
-                        wl.ring[pos & 127u] = (unsigned short)(ent + (((p & 16u) | (p & 3u)) << 6) +
-                                                               ((p & 12u) << 2));
-                    }
-                    tail += (unsigned)__popcll(m);
-                }
-                // a full wave; or, with nothing left to queue, the survivors
-                // whose j buffer the next pair takes (at the end: all)
-                const unsigned n = tail - head;
-                if (n < 64u && (m != 0ull || (end ? n == 0u : (int)(mark - head) <= 0))) break;
-                const int take = (int)min(64u, n);
-                __builtin_amdgcn_wave_barrier();
-                CArgs *kd = kernel_args();
-                unsigned long long unsure = 0, unsure_phi = 0;
-                int nb = drain<Prec, EXT>(view_at(kd->views, w.view), kd, wl, stg, head, take,
-                                          mixed, psi, slab_next, slab_lim, direct_n, unsure,
-                                          unsure_phi);
-                if (std::is_same<Prec, float>::value && __builtin_expect(unsure != 0ull, 0)) {
-                    kd = kernel_args();
-                    nb += drain_literal<EXT>(view_at(kd->views, w.view), kd, wl, head, unsure,
-                                             unsure_phi, mixed, psi, direct_n);
-                }
-                if (mixed)
-                    nb_mixed += nb;
-                else
-                    nb_same += nb;
-                head += take;
-            }
-            if (end) break;
-        }
-        __builtin_amdgcn_wave_barrier();
+        walk_item<Prec, EXT, true>(w, vp, psi, pk, wl, stg, tot, [&](int seg) {
+            return HBT_CONST(JWin, vp->mwin)[w.j0 + seg];
+        });
     }
     // per-wave totals of binned pairs
     CArgs *ka = kernel_args();
     if (lane == 0) {
-        if (nb_same) atomic_add_u64(&ka->binned[0], nb_same);
-        if (nb_mixed) atomic_add_u64(&ka->binned[1], nb_mixed);
+        if (tot.same) atomic_add_u64(&ka->binned[0], tot.same);
+        if (tot.mixed) atomic_add_u64(&ka->binned[1], tot.mixed);
     }
     if (slab) {
         // the block's demand per slab, for k_slab_bin (which clamps it to the
         // regions' capacity) and for sizing later launches
-        if (lane == 0 && direct_n) atomic_add_u64(&ka->slab.stats[ka->slab.S], direct_n);
+        if (lane == 0 && tot.direct) atomic_add_u64(&ka->slab.stats[ka->slab.S], tot.direct);
         __syncthreads();
         for (int k = threadIdx.x; k < ka->slab.S; k += blockDim.x)
             ka->slab.sfill[(long long)blockIdx.x * ka->slab.S + k] =

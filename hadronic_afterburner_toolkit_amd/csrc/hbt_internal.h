@@ -152,16 +152,19 @@ inline void pf_record(const Derived &d, double px, double py, double pz, double 
 // dn and C (|dn|, |C| <= 2 S, T <= 4 S), so that of m^2 - X below 100 ulp of
 // max(1, H^2) S^2; the T window allows 64 ulp of 2 S, the q window a margin
 // c of 256 ulp of max(1, H^2) S^2.
-inline void prefilter_margins(const Derived &d, double pmax2, DevParams &P) {
-    const double pm = std::max(1.0, pmax2);
+__host__ __device__ inline void prefilter_margins(double pmax2, DevParams &P) {
+    const double pm = fmax(1.0, pmax2), mid = fabs(P.pf_mid);
     const double eps32 = 5.9604644775390625e-8, eps64 = 1.1102230246251565e-16;
-    const double m = 64.0 * eps32 * (2.0 * pm + std::fabs(d.mid));
-    P.f_half = (float)(d.P.pf_half + m);
+    const double m = 64.0 * eps32 * (2.0 * pm + mid);
+    P.f_half = (float)(P.pf_half + m);
     if (P.qinv) return;  // pf_negc = -inf: the q windows pass every pair
-    const double S = pm + std::fabs(d.mid);
-    const double s2 = std::max(1.0, d.h2) * S * S;
+    const double S = pm + mid;
+    const double s2 = fmax(1.0, P.pf_h2) * S * S;
     P.pf_negc = -256.0 * eps64 * s2;
     P.f_negc = (float)(-256.0 * eps32 * s2);
+}
+inline void prefilter_margins(const Derived &, double pmax2, DevParams &P) {
+    prefilter_margins(pmax2, P);
 }
 
 // Allocator whose construct() without arguments default-initializes: a
@@ -316,6 +319,17 @@ inline bool rapidity_kept(double pz, double E, double cut_min, double cut_max) {
     return ratio > cut_min && ratio < cut_max;
 }
 
+// The fast lists' |pT| range: particles a binnable pair can contain.
+struct PtRange {
+    double lo, hi;
+};
+inline PtRange fast_pt_range(const Derived &d) {
+    const double D = px_window(d);
+    if (!std::isfinite(D)) return PtRange{-INFINITY, INFINITY};
+    return PtRange{(d.P.KT_min - 0.5 * D) * (1.0 - 1e-9),
+                   (std::sqrt(d.P.KT_max_sq) + 0.5 * D) * (1.0 + 1e-9)};
+}
+
 // Rapidity cut of the gathers (HBT_correlation.cpp:255-266, :468-476),
 // psi_ref per group (:181-183, :233-249; over all particles passed in), and
 // the fast lists.  Events keep < 2^18 particles (the fast kernel's
@@ -340,13 +354,10 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
     const double cut_max = tanh(k.HBTrap_max);
     const double cut_min = tanh(k.HBTrap_min);
     auto kept = [&](int64_t i) { return rapidity_kept(soa[2][i], soa[3][i], cut_min, cut_max); };
-    // the fast lists' |pT| range: particles a binnable pair can contain
     const double D = px_window(d);
-    const double r_lo = std::isfinite(D) ? (P.KT_min - 0.5 * D) * (1.0 - 1e-9) : -INFINITY;
-    const double r_hi =
-        std::isfinite(D) ? (std::sqrt(P.KT_max_sq) + 0.5 * D) * (1.0 + 1e-9) : INFINITY;
+    const PtRange r = fast_pt_range(d);
     auto pt_of = [&](int64_t i) { return std::sqrt(soa[0][i] * soa[0][i] + soa[1][i] * soa[1][i]); };
-    auto fast = [&](double pt) { return pt >= r_lo && pt <= r_hi; };
+    auto fast = [&](double pt) { return pt >= r.lo && pt <= r.hi; };
     auto beta_of = [&](int64_t i) { return P.boost ? soa[2][i] / soa[3][i] : soa[2][i]; };
     // pass 1, per event: kept and fast-list counts, and the fast list's
     // momentum and beta scales (FP32 margins)

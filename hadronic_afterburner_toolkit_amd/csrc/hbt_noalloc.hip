@@ -1,12 +1,23 @@
-// hbt_noalloc.hip -- hbt_calculate_noalloc: the plain FP64 pair loops of one
-// buffer (what hbt_upload + hbt_run_same + hbt_run_mixed do with
-// HBT_KERNEL_PLAIN) for callers that cannot allocate device memory: code
-// under HIP graph capture, tight serving loops.  The caller passes the
-// particles, the mixing plan and the histogram in device memory; the
-// rapidity cut's kept particles, their event offsets and the stage
-// counters live in `scratch`, a file-scope device array of fixed size that
-// each GPU holds until the process ends.  No hipMalloc, hipFree or other
-// allocating call is made; every launch goes on the caller's stream.
+// hbt_noalloc.hip -- hbt_calculate_noalloc: the pair loops of one buffer (what
+// hbt_upload + hbt_run_same + hbt_run_mixed do, in FP64) for callers that
+// cannot allocate device memory: code under HIP graph capture, tight serving
+// loops.  The caller passes the particles, the mixing plan and the histogram
+// in device memory; the kept particles and all that is derived from them live
+// in `scratch`, a file-scope device array of fixed size that each GPU holds
+// until the process ends.  No hipMalloc, hipFree or other allocating call is
+// made; every launch goes on the caller's stream.
+//
+// Two steps.  The gather keeps the particles a binned pair can contain
+// (rapidity cut, and |pT| within reach of a K_T bin), in order, as the fast
+// kernel's records and prefilter operands.  The pair kernel walks them in
+// items of 64 i particles like k_fast: every pair takes the matrix-core
+// prefilter, its survivors the literal cascade, 64 at a time.  Nothing is
+// known of the data on the host, so the items are worked out from the kept
+// offsets on the device and there are no momentum windows.
+// One literal cascade per enumerated pair, one thread per i particle (the
+// form before), cost 1420 us for 20 events of 600 particles (1.5e8 pairs) and
+// 335 us for 7 of 90, whose few threads each walked hundreds of pairs one
+// after the other; this form takes 168 (140 of them the pair kernel) and 32.
 //
 // Calls on one GPU share its scratch array: calls that overlap on one GPU
 // (two streams, two host threads) race and must be serialized by the caller.
@@ -18,23 +29,35 @@
 #include "../../include/hbt_hip.h"
 #include "hbt_device.h"
 #include "hbt_internal.h"
-#include "hbt_plain.h"
 
 using namespace hbt;
 
 namespace {
 
-// Scratch layout (bytes): stage counters, kept counts and kept offsets per
-// event, then the kept particles as eight FP64 columns.
 constexpr long long kMaxParticles = HBT_NOALLOC_MAX_PARTICLES;
 constexpr int kMaxEvents = HBT_NOALLOC_MAX_EVENTS;
-constexpr size_t kStageOff = 0;                                   // 16 x u64
-constexpr size_t kCountOff = 256;                                 // kMaxEvents x i64
-constexpr size_t kKoffOff = kCountOff + 8 * (size_t)kMaxEvents;   // (kMaxEvents + 1) x i64
-constexpr size_t kSoaOff = (kKoffOff + 8 * ((size_t)kMaxEvents + 1) + 255) / 256 * 256;
-constexpr size_t kScratchBytes = kSoaOff + 8 * sizeof(double) * (size_t)kMaxParticles;
+constexpr long long kWaves = 4096;     // the pair kernel's resident waves (256 CUs x 16)
+constexpr int kSmallParticles = 8192;  // gathered by one block in one launch
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// What the gather leaves for the pair kernel, beside the lists.
+struct Head {
+    View v;                  // the lists and the grid constants (with margins)
+    PfMake make;
+    double psi;              // 0 (no K_phi bins)
+    int n;                   // kept particles
+    int koff[kMaxEvents + 1];
+};
+
+struct Scratch {
+    Head head;
+    int cnt[kMaxEvents];     // kept per event, largest |pT|^2 and |beta|
+    double pmax2[kMaxEvents], bmax[kMaxEvents];
+    alignas(256) PartRec rec[kMaxParticles + kPfPad];
+    alignas(256) PfOp pf[kMaxParticles + kPfPad];
+    alignas(256) PfBeta bw[kMaxParticles + kPfPad];
+};
+
+static __device__ __align__(256) unsigned char scratch[sizeof(Scratch)];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -64,121 +87,277 @@ int scratch_ptr(int dev, unsigned char **out) {
     return HBT_OK;
 }
 
-__global__ void k_na_zero(unsigned long long *p, int n) {
-    const int i = threadIdx.x;
-    if (i < n) p[i] = 0ull;
+struct GatherArgs {
+    const long long *ev_off;
+    DevSoA in;
+    double cut_min, cut_max;  // tanh of the rapidity bounds
+    PtRange pt;
+    DevParams P;
+    double c_beta;
+    double *bins;
+    const double *plan_cs;
+    int nev;
+};
+
+// A particle of the list: tanh(HBTrap_min) < pz/E < tanh(HBTrap_max)
+// (HBT_correlation.cpp:255-266), and |pT| as a binnable pair needs it.
+struct Kept {
+    bool keep;
+    double p2, beta;
+};
+__device__ __forceinline__ Kept na_kept(const GatherArgs &g, long long i) {
+    const double px = g.in.px[i], py = g.in.py[i], pz = g.in.pz[i], r = pz / g.in.E[i];
+    const double p2 = px * px + py * py, pt = sqrt(p2);
+    return Kept{r > g.cut_min && r < g.cut_max && pt >= g.pt.lo && pt <= g.pt.hi, p2,
+                fabs(g.P.boost ? r : pz)};
 }
 
-// Kept particles per event: tanh(HBTrap_min) < pz/E < tanh(HBTrap_max)
-// (HBT_correlation.cpp:255-266).
-__global__ __launch_bounds__(256) void k_na_count(const long long *ev_off, const double *pz,
-                                                  const double *E, double cut_min,
-                                                  double cut_max, long long *cnt) {
+__device__ __forceinline__ void na_store(const GatherArgs &g, const PfMake &m, Scratch *s,
+                                         long long i, int o) {
+    const PartRec p{g.in.px[i], g.in.py[i], g.in.pz[i], g.in.E[i],
+                    g.in.x[i],  g.in.y[i],  g.in.z[i],  g.in.t[i]};
+    s->rec[o] = p;
+    PfRec32 r;
+    float hi;
+    pf_make(m, p.px, p.py, p.pz, p.E, r, hi);
+    s->pf[o] = PfOp{r.px, r.py, r.nrm, 1.0f};
+    // (the beta window holds for E > 0; other particles take the cascade's word)
+    s->bw[o] = p.E > 0.0 ? PfBeta{r.blo, hi} : PfBeta{-INFINITY, INFINITY};
+}
+
+// The head, once the kept count and the momentum scales are known.
+__device__ __forceinline__ void na_head(const GatherArgs &g, Scratch *s, int n, double pmax2,
+                                        double bmax) {
+    Head &h = s->head;
+    View v{};
+    v.P = g.P;
+    prefilter_margins(pmax2, v.P);
+    v.H.bins = g.bins;
+    v.A = v.B = v.AS = s->rec;
+    v.pfA = v.pfB = v.pfS = s->pf;
+    v.bwA = v.bwB = v.bwS = s->bw;
+    v.plan_cs = g.plan_cs;
+    v.psi = &h.psi;
+    h.v = v;
+    h.make = PfMake{g.P.pf_mid, g.c_beta, bmax, g.P.boost, 0};
+    h.psi = 0.0;
+    h.n = n;
+}
+
+__device__ __forceinline__ double wave_max(double v) {
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off));
+    return v;
+}
+
+// Kept particles per event, and the scales: one block per event.
+__global__ __launch_bounds__(256) void k_na_count(GatherArgs g, Scratch *s) {
     const int e = blockIdx.x;
-    const long long b = ev_off[e], n = ev_off[e + 1] - b;
-    unsigned long long c = 0;
+    const long long b = g.ev_off[e], n = g.ev_off[e + 1] - b;
+    int c = 0;
+    double p2 = 0.0, be = 0.0;
     for (long long i = threadIdx.x; i < n; i += blockDim.x) {
-        const double r = pz[b + i] / E[b + i];
-        c += (r > cut_min && r < cut_max) ? 1ull : 0ull;
+        const Kept k = na_kept(g, b + i);
+        if (!k.keep) continue;
+        c++;
+        p2 = fmax(p2, k.p2);
+        be = fmax(be, k.beta);
     }
     for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off);
-    __shared__ unsigned long long part[4];
-    if (__lane_id() == 0) part[threadIdx.x >> 6] = c;
+    p2 = wave_max(p2);
+    be = wave_max(be);
+    __shared__ int pc[4];
+    __shared__ double pp[4], pb[4];
+    const int w = threadIdx.x >> 6;
+    if (__lane_id() == 0) pc[w] = c, pp[w] = p2, pb[w] = be;
     __syncthreads();
-    if (threadIdx.x == 0) cnt[e] = (long long)(part[0] + part[1] + part[2] + part[3]);
+    if (threadIdx.x == 0) {
+        s->cnt[e] = pc[0] + pc[1] + pc[2] + pc[3];
+        s->pmax2[e] = fmax(fmax(pp[0], pp[1]), fmax(pp[2], pp[3]));
+        s->bmax[e] = fmax(fmax(pb[0], pb[1]), fmax(pb[2], pb[3]));
+    }
 }
 
-// Exclusive scan of the kept counts into event offsets koff[0..nev], one
-// block of 1024 threads, each summing a run of ceil(nev/1024) events.
-__global__ __launch_bounds__(1024) void k_na_scan(const long long *cnt, int nev,
-                                                  long long limit, long long *koff) {
-    __shared__ long long s[1024];
+// Inclusive scan over the 1024 threads of a block.
+__device__ __forceinline__ int block_scan(int v, int *s) {
     const int t = threadIdx.x;
+    s[t] = v;
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1) {  // Hillis-Steele
+        const int x = t >= off ? s[t - off] : 0;
+        __syncthreads();
+        s[t] += x;
+        __syncthreads();
+    }
+    return s[t];
+}
+__device__ __forceinline__ double block_max(double v, double *s) {
+    v = wave_max(v);
+    __syncthreads();
+    if (__lane_id() == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double m = 0.0;
+    for (int k = 0; k < (int)(blockDim.x >> 6); k++) m = fmax(m, s[k]);
+    return m;
+}
+
+// Exclusive scan of the kept counts into event offsets, and the head: one
+// block of 1024 threads, each summing a run of ceil(nev/1024) events.
+// (Offsets are clamped to the list's capacity, so a caller whose n_particles
+// understates its events cannot make a kernel reach past it.)
+__global__ __launch_bounds__(1024) void k_na_scan(GatherArgs g, Scratch *s) {
+    __shared__ int sc[1024];
+    __shared__ double sm[16];
+    const int t = threadIdx.x, nev = g.nev;
     const int per = (nev + 1023) / 1024;
     const int a = min(nev, t * per), b = min(nev, a + per);
     long long sum = 0;
-    for (int e = a; e < b; e++) sum += cnt[e];
-    s[t] = sum;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {  // inclusive Hillis-Steele scan
-        const long long v = t >= off ? s[t - off] : 0;
-        __syncthreads();
-        s[t] += v;
-        __syncthreads();
-    }
-    // offsets are clamped to the kept columns' capacity, so a caller whose
-    // n_particles understates its events cannot make a kernel read past them
-    long long run = t > 0 ? s[t - 1] : 0;
+    double p2 = 0.0, be = 0.0;
     for (int e = a; e < b; e++) {
-        koff[e] = min(run, limit);
-        run += cnt[e];
+        sum = min(sum + s->cnt[e], kMaxParticles);
+        p2 = fmax(p2, s->pmax2[e]);
+        be = fmax(be, s->bmax[e]);
     }
-    if (t == 1023) koff[nev] = min(s[1023], limit);
+    const int cap = (int)kMaxParticles;
+    // (1024 runs of at most 2^18 stay below 2^31)
+    const int incl = block_scan((int)sum, sc);
+    int run = incl - (int)sum;
+    for (int e = a; e < b; e++) {
+        s->head.koff[e] = min(run, cap);
+        run = min(run + s->cnt[e], cap);
+    }
+    p2 = block_max(p2, sm);
+    be = block_max(be, sm);
+    if (t == 1023) {
+        const int n = min(incl, cap);
+        s->head.koff[nev] = n;
+        na_head(g, s, n, p2, be);
+    }
 }
 
 // Order-preserving compaction of each event's kept particles to its kept
 // offset (the reference's gather order: event by event, particle order).
-__global__ __launch_bounds__(256) void k_na_compact(const long long *ev_off, DevSoA in,
-                                                    double cut_min, double cut_max,
-                                                    const long long *koff, double *out,
-                                                    long long stride) {
+__global__ __launch_bounds__(256) void k_na_compact(GatherArgs g, Scratch *s) {
     const int e = blockIdx.x;
-    const long long b = ev_off[e], n = ev_off[e + 1] - b;
+    const long long b = g.ev_off[e], n = g.ev_off[e + 1] - b;
     __shared__ int wsum[4];
-    long long base = koff[e];
+    int base = s->head.koff[e];
+    const PfMake m = s->head.make;
     const int w = threadIdx.x >> 6;
     for (long long c0 = 0; c0 < n; c0 += 256) {
         const long long i = c0 + threadIdx.x;
-        bool keep = false;
-        if (i < n) {
-            const double r = in.pz[b + i] / in.E[b + i];
-            keep = r > cut_min && r < cut_max;
-        }
-        const unsigned long long m = __ballot(keep);
-        const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        if (__lane_id() == 0) wsum[w] = __popcll(m);
+        const bool keep = i < n && na_kept(g, b + i).keep;
+        const unsigned long long mk = __ballot(keep);
+        const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0u));
+        if (__lane_id() == 0) wsum[w] = __popcll(mk);
         __syncthreads();
         int before = 0, total = 0;
         for (int k = 0; k < 4; k++) {
             before += k < w ? wsum[k] : 0;
             total += wsum[k];
         }
-        const long long o = base + before + rank;
-        if (keep && o < stride) {  // stride: the kept columns' capacity
-            const long long s = b + i;
-            out[0 * stride + o] = in.px[s];
-            out[1 * stride + o] = in.py[s];
-            out[2 * stride + o] = in.pz[s];
-            out[3 * stride + o] = in.E[s];
-            out[4 * stride + o] = in.x[s];
-            out[5 * stride + o] = in.y[s];
-            out[6 * stride + o] = in.z[s];
-            out[7 * stride + o] = in.t[s];
-        }
-        base += total;
+        const int o = base + before + rank;
+        if (keep && o < (int)kMaxParticles) na_store(g, m, s, b + i, o);
+        base = min(base + total, (int)kMaxParticles);
         __syncthreads();  // wsum is rewritten by the next chunk
     }
 }
 
-// Same-event tiles over all kept particles of the buffer; the grid is sized
-// from the particles passed in, the kept count comes from koff[nev].
-__global__ __launch_bounds__(TILE) void k_na_same(DevParams P, DevHist H, DevSoA A,
-                                                  const long long *koff, int nev) {
-    const long long n = koff[nev];
-    same_plain_tile(P, H, A, 0, (int)n, 0.0, blockIdx.y, blockIdx.x);
+// The same in one launch for a small buffer: one block, each thread a run of
+// consecutive particles (of a call of 32 us with two launches, a third and a
+// fourth would be a large part).
+__global__ __launch_bounds__(1024) void k_na_gather_small(GatherArgs g, Scratch *s) {
+    __shared__ int sc[1024];
+    __shared__ double sm[16];
+    __shared__ int koff[kSmallParticles + 1];  // kept before each particle
+    const int t = threadIdx.x;
+    const long long b = g.ev_off[0];
+    const int n = (int)min(g.ev_off[g.nev] - b, (long long)kSmallParticles);
+    const int per = (n + 1023) / 1024, i0 = min(n, t * per), i1 = min(n, i0 + per);
+    unsigned keep = 0;  // per <= 8
+    double p2 = 0.0, be = 0.0;
+    for (int i = i0; i < i1; i++) {
+        const Kept k = na_kept(g, b + i);
+        if (!k.keep) continue;
+        keep |= 1u << (i - i0);
+        p2 = fmax(p2, k.p2);
+        be = fmax(be, k.beta);
+    }
+    const int c = __popc(keep), incl = block_scan(c, sc);
+    p2 = block_max(p2, sm);
+    be = block_max(be, sm);
+    int run = incl - c;
+    for (int i = i0; i < i1; i++) {
+        koff[i] = run;
+        run += keep >> (i - i0) & 1u;
+    }
+    if (t == 1023) koff[n] = incl;
+    const PfMake m{g.P.pf_mid, g.c_beta, be, g.P.boost, 0};
+    for (int i = i0, o = incl - c; i < i1; i++)
+        if (keep >> (i - i0) & 1u) na_store(g, m, s, b + i, o++);
+    __syncthreads();
+    for (int e = t; e <= g.nev; e += 1024)
+        s->head.koff[e] = koff[(int)max(0ll, min(g.ev_off[e] - b, (long long)n))];
+    if (t == 1023) na_head(g, s, incl, p2, be);
 }
 
-// Mixed tiles of events [eb, eb + gridDim.z / M); partner ids outside
-// [0, nev) form no pairs.
-__global__ __launch_bounds__(TILE) void k_na_mixed(DevParams P, DevHist H, DevSoA A,
-                                                   const long long *koff, const int *ids,
-                                                   const double *cs, int M, int eb, int nev) {
-    const long long row = (long long)eb * M + blockIdx.z;
-    const int pid = ids[row];
-    if (pid < 0 || pid >= nev) return;
-    mixed_plain_tile(P, H, A, A, koff, koff, ids, cs, M, eb, (long long)eb * M, 0.0,
-                     blockIdx.y, blockIdx.x, blockIdx.z);
+// The pair kernel.  Item k < nsame: i tile k / nchunk against its chunk
+// k % nchunk of the list's j's; then the mixed items: event, i tile of it,
+// and a run of at most `rows` of its M plan rows.
+struct PairArgs {
+    const Head *head;
+    const int *ids;
+    int nev, M;
+    int jchunk, nchunk;  // same-event: j's per item, items per i tile
+    int tiles, rows, runs;  // mixed: i tiles per event, rows per item, items per tile
+    long long nsame, nitems;
+};
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_na_pairs(
+    FastArgs a, PairArgs g) {
+    __shared__ WaveLds wave_lds[4];
+    extern __shared__ __align__(16) char dyn_lds[];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    WaveLds &wl = wave_lds[wv];
+    Stage &stg = ((Stage *)dyn_lds)[wv];
+    WaveTotals tot;
+    tot.slab_next = nullptr;
+    tot.slab_lim = nullptr;
+    CView *vp = HBT_CONST(View, a.views);
+    const int n = HBT_CONST(Head, g.head)->n;
+    const HBT_AS4 int *koff = HBT_CONST(int, g.head->koff);
+    const PfConst<float> pk = pf_const<float>(vp->P);
+    for (long long it = (long long)blockIdx.x * 4 + wv; it < g.nitems;
+         it += (long long)gridDim.x * 4) {
+        WorkItem w{};
+        if (it < g.nsame) {
+            const int i0 = (int)(it / g.nchunk) * 64;
+            const int j0 = i0 + (int)(it % g.nchunk) * g.jchunk;
+            w.ni = min(64, n - i0);
+            w.nj = min(g.jchunk, n - j0);
+            if (w.ni <= 0 || w.nj <= 0) continue;
+            w.i0 = i0;
+            w.j0 = j0;
+            walk_item<double, false, false>(w, vp, 0.0, pk, wl, stg, tot,
+                                            [](int) { return JWin{0, 0, 0, 0}; });
+            continue;
+        }
+        const long long k = it - g.nsame;
+        const int r = (int)(k % g.runs), tile = (int)(k / g.runs % g.tiles);
+        const int e = (int)(k / g.runs / g.tiles);
+        const int ib = koff[e], ie = koff[e + 1];
+        w.kind = 1;
+        w.ni = min(64, ie - ib - tile * 64);
+        w.nj = min(g.rows, g.M - r * g.rows);
+        if (w.ni <= 0 || w.nj <= 0) continue;
+        w.i0 = ib + tile * 64;
+        const long long row0 = (long long)e * g.M + r * g.rows;
+        walk_item<double, false, false>(w, vp, 0.0, pk, wl, stg, tot, [&](int seg) {
+            const int pid = HBT_CONST(int, g.ids)[row0 + seg];
+            const bool ok = pid >= 0 && pid < g.nev;  // other partners form no pairs
+            return JWin{ok ? koff[pid] : 0, ok ? koff[pid + 1] : 0, (int)(row0 + seg), 0};
+        });
+    }
 }
 
 }  // namespace
@@ -229,47 +408,60 @@ int hbt_calculate_noalloc(const hbt_config *cfg, int32_t nev, int64_t n_particle
     unsigned char *scr = nullptr;
     hipStream_t st = (hipStream_t)stream;
     do {
+        if (nev == 0 || n_particles == 0) break;
         rc = scratch_ptr(cfg->device, &scr);
         if (rc) break;
-        unsigned long long *stage = (unsigned long long *)(scr + kStageOff);
-        long long *cnt = (long long *)(scr + kCountOff);
-        long long *koff = (long long *)(scr + kKoffOff);
-        double *kept = (double *)(scr + kSoaOff);
-        const long long stride = kMaxParticles;
-        DevSoA A{kept, kept + stride, kept + 2 * stride, kept + 3 * stride,
-                 kept + 4 * stride, kept + 5 * stride, kept + 6 * stride, kept + 7 * stride};
-        DevSoA in{soa[0], soa[1], soa[2], soa[3], soa[4], soa[5], soa[6], soa[7]};
-        DevHist H{};
-        H.bins = bins;
-        H.stage = stage;
-        const double cut_max = tanh(cfg->HBTrap_max), cut_min = tanh(cfg->HBTrap_min);
-        // the counters start at zero on every call (a fill kernel, not a
-        // memset node, so the call can be captured in a graph)
-        hipLaunchKernelGGL(k_na_zero, dim3(1), dim3(64), 0, st, stage, 16);
-        if (nev > 0) {
-            hipLaunchKernelGGL(k_na_count, dim3(nev), dim3(256), 0, st, (const long long *)ev_off,
-                               soa[2], soa[3], cut_min, cut_max, cnt);
-            hipLaunchKernelGGL(k_na_scan, dim3(1), dim3(1024), 0, st, (const long long *)cnt,
-                               (int)nev, stride, koff);
-            hipLaunchKernelGGL(k_na_compact, dim3(nev), dim3(256), 0, st,
-                               (const long long *)ev_off, in, cut_min, cut_max,
-                               (const long long *)koff, kept, stride);
+        Scratch *s = (Scratch *)scr;
+        GatherArgs g{};
+        g.ev_off = (const long long *)ev_off;
+        g.in = DevSoA{soa[0], soa[1], soa[2], soa[3], soa[4], soa[5], soa[6], soa[7]};
+        g.cut_min = tanh(cfg->HBTrap_min);
+        g.cut_max = tanh(cfg->HBTrap_max);
+        g.pt = fast_pt_range(D);
+        g.P = D.P;
+        g.c_beta = D.c_beta;
+        g.bins = bins;
+        g.plan_cs = cos_sin;
+        g.nev = (int)nev;
+        if (n_particles <= kSmallParticles) {
+            hipLaunchKernelGGL(k_na_gather_small, dim3(1), dim3(1024), 0, st, g, s);
+        } else {
+            hipLaunchKernelGGL(k_na_count, dim3(nev), dim3(256), 0, st, g, s);
+            hipLaunchKernelGGL(k_na_scan, dim3(1), dim3(1024), 0, st, g, s);
+            hipLaunchKernelGGL(k_na_compact, dim3(nev), dim3(256), 0, st, g, s);
         }
-        if (n_particles >= 2) {
-            const int T = (int)((n_particles + TILE - 1) / TILE);
-            hipLaunchKernelGGL(k_na_same, dim3(T, T), dim3(TILE), 0, st, D.P, H, A,
-                               (const long long *)koff, (int)nev);
+        PairArgs p{};
+        p.head = &s->head;
+        p.ids = partner_ids;
+        p.nev = (int)nev;
+        p.M = M;
+        // Items: 64 i's against about 1024 j's (a chunk of the list, or
+        // several plan rows' partners), where an item's own cost, some 750
+        // cycles, is below a tenth of its pairs'; finer, down to 64 j's or one
+        // row, while that leaves waves of the chip idle.
+        const long long tiles = (n_particles + 63) / 64;
+        p.jchunk = 1024;
+        while (p.jchunk > 64 && tiles * ((n_particles + p.jchunk - 1) / p.jchunk) < 2 * kWaves)
+            p.jchunk /= 2;
+        p.nchunk = (int)((n_particles + p.jchunk - 1) / p.jchunk);
+        p.nsame = tiles * p.nchunk;
+        p.tiles = (int)((max_event + 63) / 64);
+        p.rows = 1;
+        if (M > 0 && p.tiles > 0) {
+            const long long ev_tiles = (long long)nev * p.tiles;
+            p.rows = (int)std::max(1ll, std::min<long long>(M, 1024 / std::max<long long>(1, max_event)));
+            while (p.rows > 1 && ev_tiles * ((M + p.rows - 1) / p.rows) < 2 * kWaves) p.rows /= 2;
+            p.runs = (M + p.rows - 1) / p.rows;
+            p.nitems = p.nsame + ev_tiles * p.runs;
+        } else {
+            p.tiles = p.runs = 1;
+            p.nitems = p.nsame;
         }
-        const int Tm = (int)((max_event + TILE - 1) / TILE);
-        if (M > 0 && nev > 0 && Tm > 0) {
-            const int per = std::max(1, 65535 / M);  // gridDim.z below 65536
-            for (int eb = 0; eb < nev; eb += per) {
-                const int ne = std::min(per, (int)nev - eb);
-                hipLaunchKernelGGL(k_na_mixed, dim3(Tm, Tm, ne * M), dim3(TILE), 0, st, D.P, H, A,
-                                   (const long long *)koff, partner_ids, cos_sin, (int)M, eb,
-                                   (int)nev);
-            }
-        }
+        FastArgs a{};
+        a.views = &s->head.v;
+        const long blocks = (long)std::min<long long>((p.nitems + 3) / 4, 2 * kWaves / 4);
+        hipLaunchKernelGGL(k_na_pairs, dim3((unsigned)blocks), dim3(256), 4 * sizeof(Stage), st, a,
+                           p);
         if (hipGetLastError() != hipSuccess) rc = fail(HBT_ERR_HIP, "kernel launch failed");
     } while (false);
     if (cur != cfg->device) hipSetDevice(cur);

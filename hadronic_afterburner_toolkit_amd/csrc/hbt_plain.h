@@ -1,8 +1,7 @@
 // hbt_plain.h -- the plain FP64 kernels' tiles: the literal cascade of
 // HBT_correlation.cpp:291-460 (same-event) and :563-689 (mixed) for one
-// 256 x 256 tile of pairs, with the j tile staged in LDS.  Shared by the
-// context's plain kernels (hbt_engine.hip) and the allocation-free entry
-// point (hbt_noalloc.hip).
+// 256 x 256 tile of pairs, with the j tile staged in LDS, for the context's
+// plain kernels (hbt_engine.hip).
 #pragma once
 #include "hbt_device.h"
 

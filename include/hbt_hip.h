@@ -278,8 +278,8 @@ int hbt_slab_info(hbt_ctx *ctx, int32_t *on, uint64_t *direct, uint64_t *capacit
  * (needed_number_of_pairs >= 1e18), kernel HBT_KERNEL_PLAIN, precision
  * HBT_PREC_FP64; at most HBT_NOALLOC_MAX_PARTICLES particles and
  * HBT_NOALLOC_MAX_EVENTS events (HBT_ERR_CAPACITY beyond).  The kept
- * particles, their offsets and the stage counters live in a fixed device
- * array of about 16 MB per GPU, held until the process ends and shared by
+ * particles, their offsets and prefilter operands live in a fixed device
+ * array of about 24 MB per GPU, held until the process ends and shared by
  * every call on that GPU: calls that overlap on one GPU race.  Returns once
  * the work is queued; the histogram is complete when the stream is.  Errors:
  * hbt_noalloc_last_error(). */
