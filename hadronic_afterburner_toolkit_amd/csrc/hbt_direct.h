@@ -1,0 +1,104 @@
+// hbt_direct.h -- pairs of one buffer without host-built lists: a gather on the
+// device and a pair kernel whose work items follow from the kept offsets.
+// Used by the allocation-free entry point and by the engine's one-buffer path.
+//
+// The gather keeps the particles a binned pair can contain (rapidity cut, and
+// |pT| within reach of a K_T bin), in order, as the fast kernel's records and
+// prefilter operands.  The pair kernel walks them like k_fast, in items of 64
+// i particles: every pair takes the matrix-core prefilter, its survivors the
+// exact cascade, 64 at a time.  There are no momentum windows, so it tests
+// about five times the pairs that k_fast does on sorted lists, at 0.6 ps each;
+// below some 4e9 enumerated pairs the adds' atomics hide that (20 events of
+// 600 particles, 1.5e8 pairs: 140 us against k_fast's 195; of 1500 particles,
+// 9.5e8: 712 against 695; 10 of 4000, 1.8e9: 1225 against 1310), and sorting,
+// windows and items on the host cost several times the kernel.
+#pragma once
+#include "hbt_fast.h"
+#include "hbt_internal.h"
+
+namespace hbt {
+
+// Largest list, and largest number of events, one gather takes.
+constexpr int kGatherSmall = 8192;  // particles gathered by one block in one launch
+
+// The scales of a gathered list and its length.
+struct ListHead {
+    double pmax2, bmax;  // largest |pT|^2 and |beta|
+    int n;
+    int pad;
+};
+
+// A gathered list: event e is [koff[e], koff[e + 1]).  rec, pf and bw have
+// kPfPad entries past cap; cnt, pmax2 and bmax are per event.
+struct List {
+    ListHead *head;
+    int *koff;
+    int *cnt;
+    double *pmax2, *bmax;
+    PartRec *rec;
+    PfOp *pf;
+    PfBeta *bw;
+    int cap;
+};
+
+struct GatherArgs {
+    const long long *ev_off;
+    DevSoA in;
+    double cut_min, cut_max;  // tanh of the rapidity bounds
+    PtRange pt;
+    double mid, c_beta;
+    int boost, qinv;
+    int nev;
+    List out;
+};
+
+// Item k < nsame: i tile k / nchunk against its chunk k % nchunk of the list's
+// j's; then the mixed items: event, i tile of it, and a run of at most `rows`
+// of its M plan rows.
+struct PairArgs {
+    FastArgs f;  // first (kernel_args): the binned counters, no slabs
+    View v;      // the lists A and B, the histograms and the grid constants
+    const ListHead *ha, *hb;
+    const int *koff_a, *koff_b;
+    const int *ids;  // partner of each plan row; outside [0, nev_b): no pairs
+    double psi;
+    int nev_b, M;
+    int jchunk, nchunk;     // same-event: j's per item, items per i tile
+    int tiles, rows, runs;  // mixed: i tiles per event, rows per item, items per tile
+    long long nsame, nitems;
+};
+
+// The grid-dependent part of GatherArgs.
+inline void gather_setup(const Derived &d, const hbt_config &k, GatherArgs &g) {
+    g.cut_min = std::tanh(k.HBTrap_min);
+    g.cut_max = std::tanh(k.HBTrap_max);
+    g.pt = fast_pt_range(d);
+    g.mid = d.P.pf_mid;
+    g.c_beta = d.c_beta;
+    g.boost = d.P.boost;
+    g.qinv = d.P.qinv;
+}
+
+// The lists and histograms of a pair launch.
+inline void pair_lists(PairArgs &p, const List &a, const List &b) {
+    p.v.A = p.v.AS = a.rec;
+    p.v.pfA = p.v.pfS = a.pf;
+    p.v.bwA = p.v.bwS = a.bw;
+    p.v.B = b.rec;
+    p.v.pfB = b.pf;
+    p.v.bwB = b.bw;
+    p.ha = a.head;
+    p.hb = b.head;
+    p.koff_a = a.koff;
+    p.koff_b = b.koff;
+}
+
+// The items of n particles in nev events of at most max_event, M plan rows an
+// event (0: no mixed items).
+void pair_items(PairArgs &p, long long n, long long nev, long long max_event, bool same, int M);
+
+// Kernel launches on st only (they can be captured).  n: particles passed in.
+hipError_t launch_gather(const GatherArgs &g, long long n, hipStream_t st);
+hipError_t launch_pairs(const PairArgs &p, bool f32, bool ext, hipStream_t st);
+
+}  // namespace hbt

@@ -35,6 +35,7 @@
 #include "../../include/hbt_hip.h"
 #include "hbt_device.h"
 #include "hbt_cap.h"
+#include "hbt_direct.h"
 #include "hbt_fast.h"
 #include "hbt_internal.h"
 #include "hbt_plain.h"
@@ -337,6 +338,19 @@ struct Slot {
     std::vector<long long> foff;  // nev+1 fast-list offsets
     hvec<double> f_pt;            // |pT| of the fast list (mixed windows)
     DevRecords ev, srt;
+    bool lists = false;           // the host lists above and their device copies hold this upload
+    // a buffer gathered on the device (hbt_direct.h): its particles as passed
+    // in, in pinned memory (two, in turn: the copy of the last upload may
+    // still run) and on the device, each eight columns, then the offsets
+    bool direct = false;
+    char *h_raw[2] = {};
+    size_t raw_cap[2] = {};
+    hipEvent_t raw_ev[2] = {};    // the copy out of h_raw is done
+    int raw = 0;                  // h_raw of this upload
+    char *d_raw = nullptr;
+    size_t draw_cap = 0;
+    List list{};
+    size_t list_nev = 0;          // events the per-event arrays of list hold
     OrigRank *d_orig = nullptr;   // srt position -> fast-list index, gather rank
     size_t cap = 0, cap_f = 0, cap_ev = 0;
     double pmax2 = 0.0;     // max px^2+py^2 of kept particles
@@ -440,6 +454,14 @@ struct hbt_ctx {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool batch_ready = false;
+    // a batch of one buffer gathered on the device has no items: its pair launch
+    bool batch_direct = false;
+    PairArgs batch_pairs{};
+    // plans on their way to the device (two, in turn, as Slot::h_raw)
+    char *h_plan[2] = {};
+    size_t hplan_cap[2] = {};
+    hipEvent_t plan_ev[2] = {};
+    int plan_k = 0;
     bool batch_capture = true;   // the prepared batch is captured as a graph (launched more than once)
     // histogram privatisation of the fast kernel: slab binning (true) or
     // device-scope atomics; cfg.binning 1 / 0, or hbt_autotune's pick for 2
@@ -513,6 +535,14 @@ void free_slot(Slot &s) {
             if (q) hipFree(q);
     }
     if (s.d_orig) hipFree(s.d_orig);
+    void *lp[] = {s.d_raw,      s.list.head, s.list.koff, s.list.cnt, s.list.pmax2,
+                  s.list.bmax, s.list.rec,  s.list.pf,   s.list.bw};
+    for (void *q : lp)
+        if (q) hipFree(q);
+    for (int k = 0; k < 2; k++) {
+        if (s.h_raw[k]) hipHostFree(s.h_raw[k]);
+        if (s.raw_ev[k]) hipEventDestroy(s.raw_ev[k]);
+    }
     s = Slot();
 }
 
@@ -522,6 +552,7 @@ void drop_graph(hbt_ctx *c) {
     c->graph_exec = nullptr;
     c->graph = nullptr;
     c->batch_ready = false;
+    c->batch_direct = false;
 }
 
 DevHist hist_view(hbt_ctx *c) {
@@ -922,6 +953,10 @@ int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st) {
     return HBT_OK;
 }
 
+// The host's lists of buffers that were gathered on the device, for the paths
+// that walk them.
+int need_lists(hbt_ctx *c);
+
 struct ItemList {
     std::vector<WorkItem> items;
     std::vector<JWin> wins;
@@ -1062,6 +1097,17 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
                   (size_t)maxg * rec * 4 <= kL2BytesPerXcd * 3 ? kMaxQueues : 1);
 }
 
+// The next of two pinned buffers used in turn, of at least `bytes`: free once
+// the copy out of it that ev marks is done.
+int next_pinned(hbt_ctx *c, char **buf, size_t *cap, hipEvent_t *ev, size_t bytes) {
+    if (*ev)
+        HIPCHECK(c, hipEventSynchronize(*ev));
+    else
+        HIPCHECK(c, hipEventCreateWithFlags(ev, hipEventDisableTiming));
+    HIPCHECK(c, ensure_pinned(buf, cap, bytes));
+    return HBT_OK;
+}
+
 // Uploads the plan: ids are relative to the event's own group and are
 // turned into global event indices of the mixed list.
 int upload_plan(hbt_ctx *c, const std::vector<int> &M_per_event, const int32_t *ids,
@@ -1092,16 +1138,27 @@ int upload_plan(hbt_ctx *c, const std::vector<int> &M_per_event, const int32_t *
     }
     const size_t need = (size_t)std::max<long long>(rows, 1);
     if (need > c->plan_cap || !c->d_ids || !c->d_cs) {
-        int rc = dev_alloc(c, &c->d_ids, need);
+        int rc = quiesce(c);
+        if (!rc) rc = dev_alloc(c, &c->d_ids, need);
         if (!rc) rc = dev_alloc(c, &c->d_cs, 2 * need);
         if (rc) return rc;
         c->plan_cap = need;
     }
     int rc = ensure(c, &c->d_rowoff, c->rowoff_cap, (size_t)s.nev + 1);
     if (rc) return rc;
-    HIPCHECK(c, hipMemcpy(c->d_ids, gids.data(), rows * 4, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->d_cs, cs, rows * 16, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->d_rowoff, rowoff.data(), (s.nev + 1) * 8, hipMemcpyHostToDevice));
+    // through pinned memory on the context's stream, in order with the launches
+    // that read the plan before
+    std::vector<StagePiece> pieces;
+    if (rows > 0) {
+        pieces.push_back(StagePiece{c->d_ids, gids.data(), (size_t)rows * 4});
+        pieces.push_back(StagePiece{c->d_cs, cs, (size_t)rows * 16});
+    }
+    pieces.push_back(StagePiece{c->d_rowoff, rowoff.data(), ((size_t)s.nev + 1) * 8});
+    const int k = c->plan_k ^= 1;
+    rc = next_pinned(c, &c->h_plan[k], &c->hplan_cap[k], &c->plan_ev[k], stage_bytes(pieces));
+    if (rc) return rc;
+    HIPCHECK(c, stage_pieces(c->h_plan[k], pieces, c->stream));
+    HIPCHECK(c, hipEventRecord(c->plan_ev[k], c->stream));
     gids.resize((size_t)rows);
     c->plan_gids.swap(gids);
     c->rowoff.swap(rowoff);
@@ -1145,6 +1202,7 @@ int timed_fast(hbt_ctx *c, float *ms) {
 
 // Plain kernels: one launch per group (same) and per group (mixed).
 int run_plain(hbt_ctx *c, bool same, bool mixed) {
+    if (int rc0 = need_lists(c)) return rc0;
     Slot &s = c->slot[0];
     const Slot &m = mixed_slot(c);
     DevHist H = hist_view(c);
@@ -1278,12 +1336,17 @@ int cap_defer_bin(hbt_ctx *c, int nkey3, const CapDefer &dk) {
 
 // d_flag: bin only the keys marked CAP_CROSS there (null: all).
 int run_capped(hbt_ctx *c, bool mixed, const int *d_flag = nullptr) {
+    int rc0 = need_lists(c);
+    if (!rc0) rc0 = quiesce(c);
+    if (!rc0) rc0 = upload_psi(c);
+    if (rc0) return rc0;
     const Slot &s = c->slot[0];
     const Slot &m = mixed_slot(c);
     CapDefer dk;
     // pairs deferred by an uncapped pass queued before this one are binned
     // first, so the records the count pass leaves are this pass's own
-    if (int rc0 = resolve_deferred(c)) return rc0;
+    rc0 = resolve_deferred(c);
+    if (rc0) return rc0;
     const long long nrows = std::max(1ll, s.n);
     const int nkey3 = c->cfg.n_KT * c->P.nphi, nkq = c->cfg.n_KT, nkeys = nkey3 + nkq;
     int rc = ensure(c, &c->d_cnt, c->cnt_cap, (size_t)nkeys * nrows);
@@ -1401,8 +1464,10 @@ int run_capped(hbt_ctx *c, bool mixed, const int *d_flag = nullptr) {
 // every key past the cap before it, 4.0 against 11.2 when every key passes it
 // (of which the position search took 7, one pair after the other).  A copy that
 // cannot be allocated leaves the ordered passes.
-// launch: the call's items; side: the same-event and the mixed side.
-int run_trial(hbt_ctx *c, FastArgs a, const CapSide side[2], bool &done) {
+// launch: queues the call's FP64 launch, its binned counts at the address
+// passed; side: the same-event and the mixed side.
+using TrialLaunch = std::function<hipError_t(unsigned long long *binned)>;
+int run_trial(hbt_ctx *c, const TrialLaunch &launch, const CapSide side[2], bool &done) {
     done = false;
     const int nkey3 = c->cfg.n_KT * c->P.nphi, nkq = c->cfg.n_KT, nkeys = nkey3 + nkq;
     const size_t bins = (size_t)c->nbins * BIN_STRIDE, nq = c->P.qinv ? (size_t)c->nq : 0;
@@ -1431,11 +1496,7 @@ int run_trial(hbt_ctx *c, FastArgs a, const CapSide side[2], bool &done) {
     const void *q[4] = {H.qinv_count, H.qinv_den, H.qinv_sum, H.qinv_num};
     for (int f = 0; f < 4 && nq; f++)
         HIPCHECK(c, hipMemcpyAsync(snap_q + f * nq, q[f], nq * 8, hipMemcpyDeviceToDevice, st));
-    a.slab = SlabArgs{};
-    a.binned = (unsigned long long *)(snap_q + 4 * nq);
-    if (a.nitems > 0)
-        HIPCHECK(c, launch_fast_kernel(a, false, c->P.qinv || c->P.azimuthal,
-                                       fast_blocks(c, a.nitems), st));
+    HIPCHECK(c, launch((unsigned long long *)(snap_q + 4 * nq)));
     rc = resolve_deferred(c);
     if (rc) return rc;
     const uint64_t deferred = c->deferred_total;
@@ -1474,13 +1535,41 @@ int run_trial(hbt_ctx *c, FastArgs a, const CapSide side[2], bool &done) {
     return rc;
 }
 
-// The trial launch of one side, timed.
-int timed_trial(hbt_ctx *c, const CapSide side[2], hipEvent_t *ev, float *ms, bool &done) {
-    FastArgs a;
-    int rc = fast_args(c, a);
-    if (rc) return rc;
+TrialLaunch trial_fast(hbt_ctx *c, FastArgs a) {
+    a.slab = SlabArgs{};
+    return [c, a](unsigned long long *binned) mutable -> hipError_t {
+        a.binned = binned;
+        if (a.nitems <= 0) return hipSuccess;
+        return launch_fast_kernel(a, false, c->P.qinv || c->P.azimuthal, fast_blocks(c, a.nitems),
+                                  c->stream);
+    };
+}
+
+hipError_t launch_direct(hbt_ctx *c, const PairArgs &p, bool f32) {
+    return launch_pairs(p, f32, c->P.qinv || c->P.azimuthal, c->stream);
+}
+
+TrialLaunch trial_direct(hbt_ctx *c, PairArgs p) {
+    return [c, p](unsigned long long *binned) mutable -> hipError_t {
+        p.f.binned = binned;
+        return launch_direct(c, p, false);
+    };
+}
+
+int timed_direct(hbt_ctx *c, const PairArgs &p, hipEvent_t *ev, float *ms) {
     HIPCHECK(c, hipEventRecord(ev[0], c->stream));
-    rc = run_trial(c, a, side, done);
+    HIPCHECK(c, launch_direct(c, p, c->cfg.precision == HBT_PREC_FP32C));
+    HIPCHECK(c, hipEventRecord(ev[1], c->stream));
+    HIPCHECK(c, hipEventSynchronize(ev[1]));
+    HIPCHECK(c, hipEventElapsedTime(ms, ev[0], ev[1]));
+    return HBT_OK;
+}
+
+// The trial launch of one side, timed.
+int timed_trial(hbt_ctx *c, const TrialLaunch &launch, const CapSide side[2], hipEvent_t *ev,
+                float *ms, bool &done) {
+    HIPCHECK(c, hipEventRecord(ev[0], c->stream));
+    int rc = run_trial(c, launch, side, done);
     if (rc || !done) return rc;
     HIPCHECK(c, hipEventRecord(ev[1], c->stream));
     HIPCHECK(c, hipEventSynchronize(ev[1]));
@@ -1490,6 +1579,7 @@ int timed_trial(hbt_ctx *c, const CapSide side[2], hipEvent_t *ev, float *ms, bo
 
 int prepare_and_capture(hbt_ctx *c) {
     drop_graph(c);
+    if (int rc0 = need_lists(c)) return rc0;
     ItemList items;
     build_items(c, true, true, items, c->batch_enum_same);
     c->batch_enum_mixed = c->plan_valid ? c->plan_enum_mixed : 0;
@@ -1535,12 +1625,16 @@ int prepare_and_capture(hbt_ctx *c) {
 // several threads and queues their copies (and the event offsets') on the
 // context's stream.
 int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
-                   const double *const soa[8]) {
+                   const double *const soa[8], bool again) {
     int rc = quiesce(c);
     if (rc) return rc;
-    drop_graph(c);
-    c->plan_valid = false;
-    s.valid = false;  // until every copy has succeeded
+    if (!again) {
+        drop_graph(c);
+        c->plan_valid = false;
+        s.valid = false;  // until every copy has succeeded
+        s.direct = false;
+    }
+    s.lists = false;
     const long long n = h.n, nf = h.nf;
     if ((size_t)n > s.cap || !s.d_soa[0]) {
         for (auto &p : s.d_soa) {
@@ -1584,10 +1678,111 @@ int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
     return HBT_OK;
 }
 
+// One buffer is gathered on the device where the pair kernel without windows
+// is as fast as the windowed one (hbt_direct.h), which spares the host the
+// sorts, windows and items.  Not with slab binning, where the adds are cheap
+// and the windows count.  2^16 particles: 2.1e9 same-event pairs.
+constexpr long long kDirectParticles = 1 << 16;
+constexpr uint64_t kDirectPairs = 4000000000ull;  // same-event and mixed pairs of a call
+
+bool direct_upload(const hbt_ctx *c, int32_t ngroups, int32_t nev, const int64_t *ev_off) {
+    return c->cfg.kernel == HBT_KERNEL_FAST && !c->slab_binning && ngroups == 1 && nev > 0 &&
+           nev <= (1 << 14) && ev_off[nev] - ev_off[0] <= kDirectParticles;
+}
+
+// The upload of one buffer whose lists the device gathers: nothing waits for
+// the device, the copy and the gather queue behind the launches before.
+int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
+                  const int64_t *ev_off, const double *const soa[8]) {
+    Slot &s = c->slot[slot];
+    std::string err;
+    if (int rc = check_buffer(1, grp, nev, ev_off, soa, err)) return fail(c, rc, err);
+    const long long o0 = ev_off[0], n_in = ev_off[nev] - o0;
+    const size_t col = stage_round((size_t)n_in * 8), off_bytes = ((size_t)nev + 1) * 8;
+    const size_t bytes = 8 * col + off_bytes;
+    drop_graph(c);
+    c->plan_valid = false;
+    s.valid = s.direct = s.lists = false;
+    s.raw ^= 1;
+    int rc = next_pinned(c, &s.h_raw[s.raw], &s.raw_cap[s.raw], &s.raw_ev[s.raw], bytes);
+    if (rc) return rc;
+    const bool grow = (size_t)n_in > (size_t)s.list.cap || !s.list.rec;
+    const bool grow_ev = (size_t)nev > s.list_nev || !s.list.koff;
+    if (bytes > s.draw_cap || grow || grow_ev) {
+        rc = quiesce(c);
+        if (!rc && bytes > s.draw_cap) {
+            s.draw_cap = 0;
+            rc = dev_alloc(c, &s.d_raw, bytes);
+            if (!rc) s.draw_cap = bytes;
+        }
+        if (!rc && grow) {
+            s.list.cap = 0;
+            rc = dev_alloc(c, &s.list.rec, (size_t)n_in + kPfPad);
+            if (!rc) rc = dev_alloc(c, &s.list.pf, (size_t)n_in + kPfPad);
+            if (!rc) rc = dev_alloc(c, &s.list.bw, (size_t)n_in + kPfPad);
+            if (!rc) s.list.cap = (int)n_in;
+        }
+        if (!rc && grow_ev) {
+            s.list_nev = 0;
+            rc = dev_alloc(c, &s.list.koff, (size_t)nev + 1);
+            if (!rc) rc = dev_alloc(c, &s.list.cnt, (size_t)nev);
+            if (!rc) rc = dev_alloc(c, &s.list.pmax2, (size_t)nev);
+            if (!rc) rc = dev_alloc(c, &s.list.bmax, (size_t)nev);
+            if (!rc && !s.list.head) rc = dev_alloc(c, &s.list.head, 1);
+            if (!rc) s.list_nev = (size_t)nev;
+        }
+        if (rc) return rc;
+    }
+    // the columns into pinned memory, and the kept particles per event
+    char *raw = s.h_raw[s.raw];
+    int64_t *off = (int64_t *)(raw + 8 * col);
+    for (int e = 0; e <= nev; e++) off[e] = ev_off[e] - o0;
+    const double cut_max = tanh(c->cfg.HBTrap_max), cut_min = tanh(c->cfg.HBTrap_min);
+    s.off.assign((size_t)nev + 1, 0);
+    const long long grain = std::max(1ll, 4096ll * nev / std::max(1ll, n_in));
+    parallel_ranges(nev, grain, [&](long long e0, long long e1) {
+        const int64_t b = ev_off[e0], n = ev_off[e1] - b;
+        for (int a = 0; a < 8; a++)
+            std::memcpy(raw + a * col + (b - o0) * 8, soa[a] + b, (size_t)n * 8);
+        for (long long e = e0; e < e1; e++) {
+            long long kept = 0;
+            for (int64_t i = ev_off[e]; i < ev_off[e + 1]; i++)
+                kept += rapidity_kept(soa[2][i], soa[3][i], cut_min, cut_max);
+            s.off[e + 1] = kept;
+        }
+    });
+    for (int e = 0; e < nev; e++) s.off[e + 1] += s.off[e];
+    HIPCHECK(c, hipMemcpyAsync(s.d_raw, raw, bytes, hipMemcpyHostToDevice, c->stream));
+    HIPCHECK(c, hipEventRecord(s.raw_ev[s.raw], c->stream));
+    GatherArgs g{};
+    g.ev_off = (const long long *)(s.d_raw + 8 * col);
+    double *d[8];
+    for (int a = 0; a < 8; a++) d[a] = (double *)(s.d_raw + a * col);
+    g.in = DevSoA{d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7]};
+    gather_setup(c->D, c->cfg, g);
+    g.nev = nev;
+    g.out = s.list;
+    HIPCHECK(c, launch_gather(g, n_in, c->stream));
+    s.ngroups = 1;
+    s.grp_ev.assign(grp, grp + 2);
+    s.nev = nev;
+    s.n = s.off[nev];
+    s.n_in = n_in;
+    s.psi2.assign(1, 0.0);
+    if (c->P.azimuthal) s.psi2[0] = psi_ref_of(soa[0], soa[1], o0, o0 + n_in, true);
+    if (slot == 0) c->psi = s.psi2;
+    s.valid = s.direct = true;
+    return HBT_OK;
+}
+
+// again: the lists of an upload that the device gathered; its plan, batch and
+// psi_ref stay.
 int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev, int32_t nev,
-                const int64_t *ev_off, const double *const soa[8]) {
+                const int64_t *ev_off, const double *const soa[8], bool again = false) {
     if (slot != 0 && slot != 1) return fail(c, HBT_ERR_ARG, "slot must be 0 or 1");
     if (ngroups < 1 || !grp_ev) return fail(c, HBT_ERR_ARG, "bad buffer");
+    if (!again && ev_off && direct_upload(c, ngroups, nev, ev_off))
+        return upload_direct(c, slot, grp_ev, nev, ev_off, soa);
     HostParticles h;
     std::string err;
     Slot &s = c->slot[slot];
@@ -1597,7 +1792,7 @@ int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev
     // then run while the host sorts the fast lists by px.
     int hook_rc = HBT_OK;
     const std::function<int()> after_keep = [&]() -> int {
-        hook_rc = upload_columns(c, s, nev, h, soa);
+        hook_rc = upload_columns(c, s, nev, h, soa, again);
         return hook_rc;
     };
     int rc = gather_particles(c->D, c->cfg, ngroups, grp_ev, nev, ev_off, soa, h, err, &after_keep);
@@ -1622,16 +1817,80 @@ int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev
     s.f_pt = std::move(h.f_pt);
     s.srt_cell = std::move(h.srt_cell);
     s.srt_py = std::move(h.srt_py);
+    s.pmax2 = h.pmax2;
+    s.lists = true;
+    if (again) return HBT_OK;
     s.ngroups = ngroups;
     s.grp_ev.assign(grp_ev, grp_ev + ngroups + 1);
     s.nev = nev;
     s.n = h.n;
     s.n_in = h.n_in;
     s.off = h.off;
-    s.pmax2 = h.pmax2;
     s.psi2 = h.psi2;
     s.valid = true;
     if (slot == 0) c->psi = h.psi2;
+    return HBT_OK;
+}
+
+int need_lists(hbt_ctx *c) {
+    for (int slot = 0; slot < 2; slot++) {
+        Slot &s = c->slot[slot];
+        if (!s.valid || s.lists) continue;
+        const size_t col = stage_round((size_t)s.n_in * 8);
+        const char *raw = s.h_raw[s.raw];
+        const double *soa[8];
+        for (int a = 0; a < 8; a++) soa[a] = (const double *)(raw + a * col);
+        const std::vector<int64_t> off((const int64_t *)(raw + 8 * col),
+                                       (const int64_t *)(raw + 8 * col) + s.nev + 1);
+        const std::vector<int32_t> grp(s.grp_ev.begin(), s.grp_ev.end());
+        if (int rc = upload_slot(c, slot, 1, grp.data(), s.nev, off.data(), soa, true)) return rc;
+    }
+    return HBT_OK;
+}
+
+// Both lists of the call were gathered on the device, and its pairs are few
+// enough to be walked without windows.
+bool direct_call(const hbt_ctx *c, uint64_t pairs) {
+    return c->slot[0].direct && mixed_slot(c).direct && !c->slab_binning && pairs <= kDirectPairs;
+}
+
+// The pair launch of a direct call: the same-event side, or the mixed side of M
+// plan rows an event, or both.
+PairArgs direct_pairs(hbt_ctx *c, bool same, int M) {
+    const Slot &s = c->slot[0], &m = mixed_slot(c);
+    PairArgs p{};
+    p.v.P = c->P;
+    p.v.H = hist_view(c);
+    p.v.plan_cs = c->d_cs;
+    pair_lists(p, s.list, m.list);
+    p.ids = c->d_ids;
+    p.psi = c->psi.empty() ? 0.0 : c->psi[0];
+    p.nev_b = m.nev;
+    p.f.binned = c->d_binned;
+    long long max_event = 0;
+    for (int e = 0; e < s.nev; e++) max_event = std::max(max_event, s.off[e + 1] - s.off[e]);
+    pair_items(p, s.n, s.nev, max_event, same, M);
+    return p;
+}
+
+uint64_t same_pairs(const Slot &s) {
+    return s.n >= 2 ? (uint64_t)s.n * (uint64_t)(s.n - 1) / 2 : 0;
+}
+
+// The direct batch of one buffer and its plan (M rows an event).
+int prepare_direct(hbt_ctx *c, int M, const int32_t *ids, const double *cs) {
+    const Slot &s = c->slot[0];
+    uint64_t em = 0;
+    int rc = upload_plan(c, std::vector<int>((size_t)s.nev, M), ids, cs, em);
+    if (rc) return rc;
+    c->batch_pairs = direct_pairs(c, true, M);
+    c->batch_enum_same = same_pairs(s);
+    c->batch_enum_mixed = em;
+    c->nitems = (int)std::min<long long>(c->batch_pairs.nitems, INT32_MAX);
+    c->nqueues = 1;
+    c->qoff.assign(2, 0);
+    c->qoff[1] = c->nitems;
+    c->batch_direct = c->batch_ready = true;
     return HBT_OK;
 }
 
@@ -1770,6 +2029,10 @@ int hbt_destroy(hbt_ctx *c) {
     if (c->h_stage) hipHostFree(c->h_stage);
     if (c->h_stage2) hipHostFree(c->h_stage2);
     if (c->h_read) hipHostFree(c->h_read);
+    for (int k = 0; k < 2; k++) {
+        if (c->h_plan[k]) hipHostFree(c->h_plan[k]);
+        if (c->plan_ev[k]) hipEventDestroy(c->plan_ev[k]);
+    }
     for (auto &ev : c->read_ev)
         if (ev) hipEventDestroy(ev);
     delete c;
@@ -1816,8 +2079,12 @@ int hbt_run_same(hbt_ctx *c) {
     if (!rc) rc = quiesce(c);
     if (rc) return rc;
     ItemList items;
-    uint64_t es = 0;
-    build_items(c, true, false, items, es);
+    uint64_t es = same_pairs(c->slot[0]);
+    const bool direct = direct_call(c, es);
+    if (!direct) {
+        if ((rc = need_lists(c))) return rc;
+        build_items(c, true, false, items, es);
+    }
     CapSide side[2];
     rc = check_cap(c, false, es, side[0]);
     if (rc) return rc;
@@ -1826,11 +2093,17 @@ int hbt_run_same(hbt_ctx *c) {
     const bool binds = side[0].binds;
     bool done = false;
     // (a prepared batch keeps its items on the device)
-    if (binds && c->cfg.kernel == HBT_KERNEL_FAST && !c->batch_ready) {
+    if (binds && direct) {
+        rc = timed_trial(c, trial_direct(c, direct_pairs(c, true, 0)), side, c->ev, &c->ms_same,
+                         done);
+        if (rc) return rc;
+    } else if (binds && c->cfg.kernel == HBT_KERNEL_FAST && !c->batch_ready) {
         c->launch_enum_same = es;
         c->launch_enum_mixed = 0;
         rc = upload_items(c, items);
-        if (!rc) rc = timed_trial(c, side, c->ev, &c->ms_same, done);
+        FastArgs a;
+        if (!rc) rc = fast_args(c, a);
+        if (!rc) rc = timed_trial(c, trial_fast(c, a), side, c->ev, &c->ms_same, done);
         if (rc) return rc;
     }
     if (done) {
@@ -1841,6 +2114,10 @@ int hbt_run_same(hbt_ctx *c) {
         HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
         HIPCHECK(c, hipEventSynchronize(c->ev[1]));
         HIPCHECK(c, hipEventElapsedTime(&c->ms_same, c->ev[0], c->ev[1]));
+    } else if (direct) {
+        c->batch_ready = false;
+        rc = timed_direct(c, direct_pairs(c, true, 0), c->ev, &c->ms_same);
+        if (rc) return rc;
     } else {
         c->batch_ready = false;
         c->launch_enum_same = es;
@@ -1876,13 +2153,21 @@ int hbt_run_mixed(hbt_ctx *c, int32_t M, const int32_t *partner_ids, const doubl
     if (rc) return rc;
     const bool binds = side[1].binds;
     bool done = false;
-    if (binds && c->cfg.kernel == HBT_KERNEL_FAST) {
+    const bool direct = direct_call(c, em);
+    if (!direct && (rc = need_lists(c))) return rc;
+    if (binds && direct) {
+        rc = timed_trial(c, trial_direct(c, direct_pairs(c, false, M)), side, c->ev + 2,
+                         &c->ms_mixed, done);
+        if (rc) return rc;
+    } else if (binds && c->cfg.kernel == HBT_KERNEL_FAST) {
         ItemList items;
         build_items(c, false, true, items, es);
         c->launch_enum_same = 0;
         c->launch_enum_mixed = em;
         rc = upload_items(c, items);
-        if (!rc) rc = timed_trial(c, side, c->ev + 2, &c->ms_mixed, done);
+        FastArgs a;
+        if (!rc) rc = fast_args(c, a);
+        if (!rc) rc = timed_trial(c, trial_fast(c, a), side, c->ev + 2, &c->ms_mixed, done);
         if (rc) return rc;
     }
     if (done) {
@@ -1893,6 +2178,9 @@ int hbt_run_mixed(hbt_ctx *c, int32_t M, const int32_t *partner_ids, const doubl
         HIPCHECK(c, hipEventRecord(c->ev[3], c->stream));
         HIPCHECK(c, hipEventSynchronize(c->ev[3]));
         HIPCHECK(c, hipEventElapsedTime(&c->ms_mixed, c->ev[2], c->ev[3]));
+    } else if (direct) {
+        rc = timed_direct(c, direct_pairs(c, false, M), c->ev + 2, &c->ms_mixed);
+        if (rc) return rc;
     } else {
         ItemList items;
         build_items(c, false, true, items, es);
@@ -1944,7 +2232,7 @@ int hbt_prepare_batch(hbt_ctx *c, const int32_t *M_per_group, const int32_t *par
 int hbt_launch_batch(hbt_ctx *c) {
     if (!c) return HBT_ERR_ARG;
     if (!c->batch_ready) return fail(c, HBT_ERR_STATE, "no prepared batch (hbt_prepare_batch)");
-    if (c->slab.resize && c->cfg.kernel == HBT_KERNEL_FAST) {
+    if (c->slab.resize && c->cfg.kernel == HBT_KERNEL_FAST && !c->batch_direct) {
         // the last launch outgrew its slab regions: size them again from its
         // demand (and capture the batch again) before this launch
         int rc0 = quiesce(c);
@@ -1960,7 +2248,8 @@ int hbt_launch_batch(hbt_ctx *c) {
     c->batch_capped = bs || bm;
     bool done = false;
     if ((bs || bm) && c->cfg.kernel == HBT_KERNEL_FAST) {
-        rc = run_trial(c, c->batch_args, side, done);
+        rc = run_trial(c, c->batch_direct ? trial_direct(c, c->batch_pairs)
+                                          : trial_fast(c, c->batch_args), side, done);
         if (rc) return rc;
     }
     if (done) {
@@ -1968,6 +2257,8 @@ int hbt_launch_batch(hbt_ctx *c) {
         rc = bs ? run_capped(c, false) : run_plain(c, true, false);
         if (!rc) rc = bm ? run_capped(c, true) : (c->plan_valid ? run_plain(c, false, true) : 0);
         if (rc) return rc;
+    } else if (c->batch_direct) {
+        HIPCHECK(c, launch_direct(c, c->batch_pairs, c->cfg.precision == HBT_PREC_FP32C));
     } else if (c->cfg.kernel == HBT_KERNEL_FAST) {
         if (c->nitems > 0 && c->graph_exec) {
             HIPCHECK(c, hipGraphLaunch(c->graph_exec, c->stream));
@@ -2062,6 +2353,8 @@ int hbt_autotune(hbt_ctx *c, hbt_tuning *best_out) {
         if (best_out) *best_out = c->tune;
         return HBT_OK;
     }
+    if (c->batch_direct)
+        if (int rc = prepare_and_capture(c)) return rc;
     // histogram privatisation (binning 2): every launch shape is timed with
     // device-scope atomics and with slab binning, and the fastest pair wins.
     // Each is launched twice and the second launch counts: slab regions are
@@ -2318,7 +2611,10 @@ int hbt_calculate_buffer(hbt_ctx *c, hbt_rng *rng) {
     // the previous buffer's launch (already waited for by this buffer's
     // upload): its pairs left to the host are decided before this launch
     // adds its own
-    rc = hbt_sync(c, nullptr);
+    // (a buffer gathered on the device has waited for nothing, and only K_phi
+    // bins leave pairs to the host)
+    const bool direct = direct_call(c, 0);
+    if (!direct || c->P.azimuthal) rc = hbt_sync(c, nullptr);
     if (rc) return rc;
     Slot &s = c->slot[0];
     const Slot &m = mixed_slot(c);
@@ -2339,7 +2635,15 @@ int hbt_calculate_buffer(hbt_ctx *c, hbt_rng *rng) {
         hbt_rng_draw_plan(rng, nev, mixed_nev, c->cfg.number_of_mixed_events, ids.data() + base,
                           cs.data() + 2 * base);
     }
-    rc = prepare_batch(c, Mg.data(), ids.data(), cs.data(), false);
+    uint64_t pairs = same_pairs(s);
+    for (int e = 0; e < s.nev && direct; e++)
+        for (int r = 0; r < Mg[0]; r++) {
+            const int q = ids[(size_t)e * Mg[0] + r];
+            pairs += (uint64_t)(s.off[e + 1] - s.off[e]) * (uint64_t)(m.off[q + 1] - m.off[q]);
+        }
+    rc = direct && direct_call(c, pairs)
+             ? prepare_direct(c, Mg[0], ids.data(), cs.data())
+             : prepare_batch(c, Mg.data(), ids.data(), cs.data(), false);
     // not waited for: the caller's next upload does its host work while the
     // launch runs (hbt_read, hbt_sync and the next upload wait for it)
     if (!rc) rc = hbt_launch_batch(c);

@@ -582,7 +582,8 @@ struct WaveTotals {
 // pair's (the exact cascade has a single call site).
 // RANKED: a same-event pair is oriented by the gather ranks of its particles;
 // otherwise by their places in the list.
-template <typename Prec, bool EXT, bool RANKED, typename Window>
+// Views: the item's view, from the kernel's arguments (Views::at).
+template <typename Prec, bool EXT, bool RANKED, typename Views, typename Window>
 __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double psi,
                                           const PfConst<float> &pk, WaveLds &wl, Stage &stg,
                                           WaveTotals &tot, Window window) {
@@ -756,13 +757,13 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
             __builtin_amdgcn_wave_barrier();
             CArgs *kd = kernel_args();
             unsigned long long unsure = 0, unsure_phi = 0;
-            int nb = drain<Prec, EXT, RANKED>(view_at(kd->views, w.view), kd, wl, stg, head, take,
-                                      mixed, psi, tot.slab_next, tot.slab_lim, tot.direct, unsure,
-                                      unsure_phi);
+            int nb = drain<Prec, EXT, RANKED>(Views::at(kd, w.view), kd, wl, stg, head, take, mixed,
+                                              psi, tot.slab_next, tot.slab_lim, tot.direct, unsure,
+                                              unsure_phi);
             if (std::is_same<Prec, float>::value && __builtin_expect(unsure != 0ull, 0)) {
                 kd = kernel_args();
-                nb += drain_literal<EXT, RANKED>(view_at(kd->views, w.view), kd, wl, head, unsure,
-                                         unsure_phi, mixed, psi, tot.direct);
+                nb += drain_literal<EXT, RANKED>(Views::at(kd, w.view), kd, wl, head, unsure,
+                                                 unsure_phi, mixed, psi, tot.direct);
             }
             if (mixed)
                 tot.mixed += nb;
@@ -786,6 +787,12 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
 // Headline workload (2.5e10 pairs, 4.8e9 evaluated): 5.6 ms in the precision
 // form, of which the prefilter alone 2.6 and the mixed adds' atomic floor 3.3;
 // 8.0 ms with scalar tests and records fetched by scattered loads.
+struct TableViews {
+    static __device__ __forceinline__ CView *at(CArgs *ka, int view) {
+        return view_at(ka->views, view);
+    }
+};
+
 template <typename Prec, bool EXT>
 constexpr int fast_waves_per_eu() {
     return EXT && std::is_same<Prec, double>::value ? 3 : 4;
@@ -837,7 +844,7 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_fast
         const WorkItem w = HBT_CONST(WorkItem, ka->items)[q0 + it];
         CView *vp = view_at(ka->views, w.view);
         const double psi = HBT_CONST(double, vp->psi)[w.grp];
-        walk_item<Prec, EXT, true>(w, vp, psi, pk, wl, stg, tot, [&](int seg) {
+        walk_item<Prec, EXT, true, TableViews>(w, vp, psi, pk, wl, stg, tot, [&](int seg) {
             return HBT_CONST(JWin, vp->mwin)[w.j0 + seg];
         });
     }

@@ -330,14 +330,8 @@ inline PtRange fast_pt_range(const Derived &d) {
                    (std::sqrt(d.P.KT_max_sq) + 0.5 * D) * (1.0 + 1e-9)};
 }
 
-// Rapidity cut of the gathers (HBT_correlation.cpp:255-266, :468-476),
-// psi_ref per group (:181-183, :233-249; over all particles passed in), and
-// the fast lists.  Events keep < 2^18 particles (the fast kernel's
-// survivor encoding).
-inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
-                            const int32_t *grp_ev, int nev, const int64_t *ev_off,
-                            const double *const soa[8], HostParticles &h, std::string &err,
-                            const std::function<int()> *after_keep = nullptr) {
+inline int check_buffer(int ngroups, const int32_t *grp_ev, int nev, const int64_t *ev_off,
+                        const double *const soa[8], std::string &err) {
     if (nev < 0 || ngroups < 0) return err = "negative size", HBT_ERR_ARG;
     if (nev > 0 && (!ev_off || !soa)) return err = "null particle arrays", HBT_ERR_ARG;
     for (int a = 0; a < 8 && nev > 0; a++)
@@ -348,6 +342,48 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
         return err = "group offsets must run from 0 to nev", HBT_ERR_ARG;
     for (int g = 0; g < ngroups; g++)
         if (grp_ev[g + 1] < grp_ev[g]) return err = "group offsets decrease", HBT_ERR_ARG;
+    return HBT_OK;
+}
+
+// psi_ref of the particles [b, e) (HBT_correlation.cpp:233-249): the terms on
+// the host threads (with par), their sums in order.
+inline double psi_ref_of(const double *px, const double *py, int64_t b, int64_t e, bool par) {
+    std::vector<double> cn, sn;
+    auto term = [&](int64_t i, double &c, double &s) {
+        const double phi = atan2(py[i], px[i]);
+        sincos(2 * phi, &s, &c);  // as the reference's build evaluates it
+    };
+    if (par) {
+        cn.resize((size_t)(e - b));
+        sn.resize((size_t)(e - b));
+        parallel_ranges(e - b, 1024, [&](long long k0, long long k1) {
+            for (long long k = k0; k < k1; k++) term(b + k, cn[(size_t)k], sn[(size_t)k]);
+        });
+    }
+    double vr = 0.0, vi = 0.0;
+    for (int64_t i = b; i < e; i++) {
+        double c, s;
+        if (par) {
+            c = cn[(size_t)(i - b)];
+            s = sn[(size_t)(i - b)];
+        } else {
+            term(i, c, s);
+        }
+        vr += c;
+        vi += s;
+    }
+    return atan2(vi, vr) / 2;
+}
+
+// Rapidity cut of the gathers (HBT_correlation.cpp:255-266, :468-476),
+// psi_ref per group (:181-183, :233-249; over all particles passed in), and
+// the fast lists.  Events keep < 2^18 particles (the fast kernel's
+// survivor encoding).
+inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
+                            const int32_t *grp_ev, int nev, const int64_t *ev_off,
+                            const double *const soa[8], HostParticles &h, std::string &err,
+                            const std::function<int()> *after_keep = nullptr) {
+    if (int rc = check_buffer(ngroups, grp_ev, nev, ev_off, soa, err)) return rc;
     const DevParams &P = d.P;
     h.reset();  // every list below is sized and written in full
     h.n_in = nev > 0 ? ev_off[nev] - ev_off[0] : 0;
@@ -435,17 +471,9 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
     h.psi2.assign(ngroups, 0.0);
     if (P.azimuthal) {
         parallel_ranges(ngroups, 1, [&](long long g0, long long g1) {
-            for (long long g = g0; g < g1; g++) {
-                double vr = 0.0, vi = 0.0;
-                for (int64_t i = ev_off[grp_ev[g]]; i < ev_off[grp_ev[g + 1]]; i++) {
-                    const double phi = atan2(soa[1][i], soa[0][i]);
-                    double sn, cn;
-                    sincos(2 * phi, &sn, &cn);  // as the reference's build evaluates it
-                    vr += cn;
-                    vi += sn;
-                }
-                h.psi2[g] = atan2(vi, vr) / 2;
-            }
+            for (long long g = g0; g < g1; g++)
+                h.psi2[g] = psi_ref_of(soa[0], soa[1], ev_off[grp_ev[g]], ev_off[grp_ev[g + 1]],
+                                       false);
         });
     }
     // each group's order by px cell, then py (stable)
