@@ -2444,9 +2444,11 @@ int hbt_last_kernel_ms(hbt_ctx *c, double *same_ms, double *mixed_ms) {
 // Results leave in chunks of bins through kReadSlots pinned slots: while the
 // link fills one, the host pool copies another into the caller's arrays
 // (first touched there, so their page faults are spread over its threads).
-// A chunk is a quarter of the bins, at least 8192 and at most 65536 (3 MB):
-// larger ones only add to the first chunk's latency, smaller ones to the
-// launches.
+// A chunk is a quarter of the bins, at least 8192 and at most 262144 (12.6 MB,
+// 50 MB pinned): larger ones only add to the first chunk's latency, smaller
+// ones to the hand-overs to the host threads, which share the first touch of
+// the caller's pages (318 MB: 14.1 ms with at most 65536 bins, 10.5 with twice
+// and 8.2 with four times that; the copies to pinned memory alone take 6.5).
 int hbt_read(hbt_ctx *c, hbt_result *o) {
     if (!c || !o) return HBT_ERR_ARG;
     if (int rc = resolve_deferred(c)) return rc;
@@ -2458,7 +2460,7 @@ int hbt_read(hbt_ctx *c, hbt_result *o) {
     bool want = false;
     for (void *p : dst) want = want || p;
     const int chunk =
-        (int)std::min(c->nbins, std::min(65536l, std::max(8192l, (c->nbins / 4 + 255) / 256 * 256)));
+        (int)std::min(c->nbins, std::min(262144l, std::max(8192l, (c->nbins / 4 + 255) / 256 * 256)));
     const int nchunks = (int)((c->nbins + chunk - 1) / chunk);
     const size_t slot_bytes = want ? (size_t)chunk * 48 : 0;
     const size_t tail_words = 2 * (size_t)groups + 4 * (size_t)c->nq + 2 * (size_t)nKT;
