@@ -220,6 +220,7 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_pair
     prefilter_margins(fmax(HBT_CONST(ListHead, g.ha)->pmax2, HBT_CONST(ListHead, g.hb)->pmax2), P);
     const PfConst<float> pk = pf_const<float>(P);
     const double psi = g.psi;
+    tot.qlds = qinv_begin<Prec, EXT>(dyn_lds, g.f.qinv_lds);
     for (long long it = (long long)blockIdx.x * 4 + wv; it < g.nitems;
          it += (long long)gridDim.x * 4) {
         WorkItem w{};
@@ -253,6 +254,7 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_pair
         if (tot.same) atomic_add_u64(&g.f.binned[0], tot.same);
         if (tot.mixed) atomic_add_u64(&g.f.binned[1], tot.mixed);
     }
+    qinv_end<Prec, EXT>(vp, tot.qlds, g.f.qinv_lds);
 }
 
 }  // namespace
@@ -295,7 +297,7 @@ hipError_t launch_gather(const GatherArgs &g, long long n, hipStream_t st) {
 hipError_t launch_pairs(const PairArgs &p, bool f32, bool ext, hipStream_t st) {
     if (p.nitems <= 0) return hipSuccess;
     const dim3 blocks((unsigned)std::min<long long>((p.nitems + 3) / 4, 2 * kWaves / 4));
-    const size_t dyn = 4 * sizeof(Stage);
+    const size_t dyn = fast_dynamic_lds(p.f.slab, ext, p.f.qinv_lds);
     // (with the q_inv branch on every pair takes the literal cascade)
     f32 = f32 && !p.v.P.qinv;
     if (f32 && ext) hipLaunchKernelGGL((k_pairs<float, true>), blocks, dim3(256), dyn, st, p);

@@ -901,6 +901,7 @@ int fast_args(hbt_ctx *c, FastArgs &a) {
         a.qoff[q] = q <= c->nqueues ? c->qoff[(size_t)q] : c->nitems;
     a.counter = c->d_counter;
     a.binned = c->d_binned;
+    a.qinv_lds = qinv_lds_bins(c->P);
     a.slab = SlabArgs{};
     int rc = slab_prepare(c, c->nitems);
     if (rc) return rc;
@@ -1867,6 +1868,7 @@ PairArgs direct_pairs(hbt_ctx *c, bool same, int M) {
     p.psi = c->psi.empty() ? 0.0 : c->psi[0];
     p.nev_b = m.nev;
     p.f.binned = c->d_binned;
+    p.f.qinv_lds = qinv_lds_bins(c->P);
     long long max_event = 0;
     for (int e = 0; e < s.nev; e++) max_event = std::max(max_event, s.off[e + 1] - s.off[e]);
     pair_items(p, s.n, s.nev, max_event, same, M);
@@ -1909,7 +1911,7 @@ hipError_t launch_fast_kernel(const FastArgs &a, bool f32, bool ext, long blocks
                               hipStream_t st) {
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, a.counter, a.nqueues);
     if (a.slab.vals && a.slab.S > (ext ? kMaxSlabsKphi : kMaxSlabs)) return hipErrorInvalidValue;
-    const size_t dyn = fast_dynamic_lds(a.slab, ext);
+    const size_t dyn = fast_dynamic_lds(a.slab, ext, a.qinv_lds);
 #define HBT_LAUNCH(T, X) \
     hipLaunchKernelGGL((k_fast<T, X>), dim3(blocks), dim3(256), dyn, st, a)
     // (with the q_inv branch on every pair takes the literal cascade)

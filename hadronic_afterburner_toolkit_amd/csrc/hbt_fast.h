@@ -236,6 +236,7 @@ struct FastArgs {
     int qoff[kMaxQueues + 1];
     int *counter;              // work counters, zeroed before launch
     unsigned long long *binned;  // [2]: binned same, mixed (for stats)
+    int qinv_lds = 0;          // q_inv bins kept in LDS (one view only), or 0
     // slab binning (hbt_slab.h) of the common-case instances; vals == null:
     // every binned pair is added with device-scope atomics
     SlabArgs slab;
@@ -322,20 +323,21 @@ struct Exact;
 template <bool EXT>
 struct Exact<double, EXT> {
     static __device__ __forceinline__ int same(CView *vp, double psi, const char *rec, unsigned a,
-                                               unsigned b, SameRec &out) {
+                                               unsigned b, SameRec &out, const QinvSink &q) {
         const DevParams P = vp->P;
         const DevHist H = vp->H;
         const PartRec p = lds_rec(rec, a), r = lds_rec(rec, b);
         return eval_same_f64<EXT>(P, H, psi, p.px, p.py, p.pz, p.E, p.x, p.y, p.z, p.t, r.px,
-                                  r.py, r.pz, r.E, r.x, r.y, r.z, r.t, out);
+                                  r.py, r.pz, r.E, r.x, r.y, r.z, r.t, out, q);
     }
     static __device__ __forceinline__ int mixed(CView *vp, double psi, const char *rec, unsigned a,
-                                                unsigned b, double2 cs, long &k) {
+                                                unsigned b, double2 cs, long &k,
+                                                const QinvSink &q) {
         const DevParams P = vp->P;
         const DevHist H = vp->H;
         const PartMom p = lds_mom(rec, a), r = lds_mom(rec, b);
         return eval_mixed_f64<EXT>(P, H, psi, p.px, p.py, p.pz, p.E, r.px * cs.x - r.py * cs.y,
-                                   r.px * cs.y + r.py * cs.x, r.pz, r.E, k);
+                                   r.px * cs.y + r.py * cs.x, r.pz, r.E, k, q);
     }
 };
 
@@ -343,13 +345,14 @@ struct Exact<double, EXT> {
 template <bool EXT>
 struct Exact<float, EXT> {
     static __device__ __forceinline__ int same(CView *vp, double psi, const char *rec, unsigned a,
-                                               unsigned b, SameRec &out) {
+                                               unsigned b, SameRec &out, const QinvSink &) {
         const PartRec p = lds_rec(rec, a), r = lds_rec(rec, b);
         out.sure = true;
         return eval_same_fast<EXT>(vp->P, psi, p, r, out);
     }
     static __device__ __forceinline__ int mixed(CView *vp, double psi, const char *rec, unsigned a,
-                                                unsigned b, double2 cs, long &k) {
+                                                unsigned b, double2 cs, long &k,
+                                                const QinvSink &) {
         const PartMom p = lds_mom(rec, a), r = lds_mom(rec, b);
         return eval_mixed_fast<EXT>(vp->P, psi, p.px, p.py, p.pz, p.E, r.px * cs.x - r.py * cs.y,
                                     r.px * cs.y + r.py * cs.x, r.pz, r.E, k);
@@ -422,20 +425,22 @@ struct Stage {
 template <typename Prec, bool EXT, bool RANKED>
 __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, Stage &stg,
                                      unsigned head, int cnt, bool mixed, double psi,
-                                     unsigned *next, const unsigned *lim,
+                                     unsigned *next, const unsigned *lim, double *qlds,
                                      unsigned long long &direct_n, unsigned long long &unsure,
                                      unsigned long long &unsure_phi) {
     const int lane = __lane_id();
     int st = 0;
     SameRec rec;
     long kmix = 0;
+    const QinvSink qs =
+        EXT && std::is_same<Prec, double>::value ? QinvSink{qlds, ka->qinv_lds} : QinvSink();
     if (lane < cnt) {
         const PairAt pr = pair_at<RANKED>(wl, wl.ring[(head + lane) & 127u], mixed);
         const char *base = (const char *)&wl;
         if (mixed)
-            st = Exact<Prec, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], kmix);
+            st = Exact<Prec, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], kmix, qs);
         else
-            st = Exact<Prec, EXT>::same(vp, psi, base, pr.a, pr.b, rec);
+            st = Exact<Prec, EXT>::same(vp, psi, base, pr.a, pr.b, rec, qs);
     }
     if (std::is_same<Prec, float>::value) {
         unsure = __ballot(st < 0);
@@ -508,12 +513,13 @@ __device__ __forceinline__ int drain_literal(CView *vp, CArgs *ka, const WaveLds
         const char *base = (const char *)&wl;
         if (mixed) {
             long k = 0;
-            binned = (Exact<double, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], k) &
-                      ST_BIN) != 0;
+            binned = (Exact<double, EXT>::mixed(vp, psi, base, pr.a, pr.b, wl.rot[pr.buf], k,
+                                                QinvSink()) & ST_BIN) != 0;
             if (binned) add_mixed_direct(vp->H.bins, k);
         } else {
             SameRec rec;
-            binned = (Exact<double, EXT>::same(vp, psi, base, pr.a, pr.b, rec) & ST_BIN) != 0;
+            binned = (Exact<double, EXT>::same(vp, psi, base, pr.a, pr.b, rec, QinvSink()) &
+                      ST_BIN) != 0;
             if (!(cos64 >> lane & 1ull))
                 rec.c = pair_cos_f32(vp->P, lds_rec(base, pr.a), lds_rec(base, pr.b));
             if (binned) add_same_slabwise<float>(vp->H.bins, rec, ka->slab.vals != nullptr);
@@ -564,6 +570,7 @@ struct WaveTotals {
     unsigned long long same = 0, mixed = 0, direct = 0;
     unsigned *slab_next;
     const unsigned *slab_lim;
+    double *qlds = nullptr;  // the block's q_inv histograms (QinvSink)
 };
 
 // ------------------------------------------------------------------ an item
@@ -758,8 +765,8 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
             CArgs *kd = kernel_args();
             unsigned long long unsure = 0, unsure_phi = 0;
             int nb = drain<Prec, EXT, RANKED>(Views::at(kd, w.view), kd, wl, stg, head, take, mixed,
-                                              psi, tot.slab_next, tot.slab_lim, tot.direct, unsure,
-                                              unsure_phi);
+                                              psi, tot.slab_next, tot.slab_lim, tot.qlds, tot.direct,
+                                              unsure, unsure_phi);
             if (std::is_same<Prec, float>::value && __builtin_expect(unsure != 0ull, 0)) {
                 kd = kernel_args();
                 nb += drain_literal<EXT, RANKED>(Views::at(kd, w.view), kd, wl, head, unsure,
@@ -800,8 +807,42 @@ constexpr int fast_waves_per_eu() {
 
 // Dynamic LDS: with slab binning each slab's next record in this block's
 // region and (common case) the regions' ends; without it the waves' Stages.
-inline size_t fast_dynamic_lds(const SlabArgs &s, bool ext) {
-    return s.vals ? (size_t)s.S * sizeof(unsigned) * (ext ? 1 : 2) : 4 * sizeof(Stage);
+// q_inv histograms of up to kMaxQinvLds bins follow the Stages: three blocks
+// with them fill a CU's LDS.
+constexpr int kMaxQinvLds = 560;
+constexpr size_t kQinvBytes = 24;  // two sums and two counts a bin
+inline int qinv_lds_bins(const DevParams &P) {
+    const int nq = P.n_KT * P.qnpts;
+    return P.qinv && nq <= kMaxQinvLds ? nq : 0;
+}
+inline size_t fast_dynamic_lds(const SlabArgs &s, bool ext, int qinv_lds) {
+    return qinv_lds ? 4 * sizeof(Stage) + kQinvBytes * qinv_lds
+           : s.vals ? (size_t)s.S * sizeof(unsigned) * (ext ? 1 : 2) : 4 * sizeof(Stage);
+}
+
+// The block's q_inv histograms: cleared at the kernel's start (null: none), and
+// added to the view's at its end.
+template <typename Prec, bool EXT>
+__device__ __forceinline__ double *qinv_begin(char *dyn_lds, int nq) {
+    if (!EXT || !std::is_same<Prec, double>::value || nq == 0) return nullptr;
+    double *q = (double *)(dyn_lds + 4 * sizeof(Stage));
+    for (int k = threadIdx.x; k < 3 * nq; k += blockDim.x) q[k] = 0.0;
+    __syncthreads();
+    return q;
+}
+template <typename Prec, bool EXT>
+__device__ __forceinline__ void qinv_end(CView *vp, const double *q, int nq) {
+    if (!EXT || !std::is_same<Prec, double>::value || nq == 0) return;
+    __syncthreads();
+    const unsigned *cnt = (const unsigned *)(q + 2 * nq);
+    for (int k = threadIdx.x; k < nq; k += blockDim.x) {
+        if (cnt[k]) {
+            atomic_add_u64(&vp->H.qinv_count[k], cnt[k]);
+            atomic_add_f64(&vp->H.qinv_sum[k], q[k]);
+            atomic_add_f64(&vp->H.qinv_num[k], q[nq + k]);
+        }
+        if (cnt[nq + k]) atomic_add_u64(&vp->H.qinv_den[k], cnt[nq + k]);
+    }
 }
 
 template <typename Prec, bool EXT>
@@ -826,6 +867,7 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_fast
     WaveLds &wl = wave_lds[threadIdx.x >> 6];
     Stage &stg = ((Stage *)dyn_lds)[threadIdx.x >> 6];
     const PfConst<float> pk = pf_const<float>(a.P);
+    tot.qlds = qinv_begin<Prec, EXT>(dyn_lds, a.qinv_lds);
 
     const int nq = a.nqueues;
     int wq = xcc_id() & (nq - 1);  // nq is a power of two
@@ -854,6 +896,7 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_fast
         if (tot.same) atomic_add_u64(&ka->binned[0], tot.same);
         if (tot.mixed) atomic_add_u64(&ka->binned[1], tot.mixed);
     }
+    qinv_end<Prec, EXT>(view_at(ka->views, 0), tot.qlds, ka->qinv_lds);
     if (slab) {
         // the block's demand per slab, for k_slab_bin (which clamps it to the
         // regions' capacity) and for sizing later launches
