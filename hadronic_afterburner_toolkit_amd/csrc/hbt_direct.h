@@ -18,23 +18,29 @@
 
 namespace hbt {
 
-// Largest list, and largest number of events, one gather takes.
-constexpr int kGatherSmall = 8192;  // particles gathered by one block in one launch
+constexpr int kGatherSmall = 2048;  // particles gathered by one block in one launch
 
-// The scales of a gathered list and its length.
-struct ListHead {
-    double pmax2, bmax;  // largest |pT|^2 and |beta|
+// With q_inv bins: the room, relative to H^2, that the prefilter's windows leave
+// for particles off one mass shell (pair_consts in hbt_direct.hip).
+constexpr double kQinvRoom = 1e-3;
+__host__ __device__ inline double qinv_h2(double H) {
+    const double Hm = H * (1.0 + 1e-9) + 1e-12;
+    return Hm * Hm * (1.0 + kQinvRoom) + 1e-12;
+}
+
+// The scales of a gathered list, or of one event of it: largest |pT|^2 and
+// |beta|, smallest and largest E^2 - p^2, and the number of particles.
+struct ListStat {
+    double pmax2, bmax, m2lo, m2hi;
     int n;
-    int pad;
 };
 
 // A gathered list: event e is [koff[e], koff[e + 1]).  rec, pf and bw have
-// kPfPad entries past cap; cnt, pmax2 and bmax are per event.
+// kPfPad entries past cap; stat is per event.
 struct List {
-    ListHead *head;
+    ListStat *head;
     int *koff;
-    int *cnt;
-    double *pmax2, *bmax;
+    ListStat *stat;
     PartRec *rec;
     PfOp *pf;
     PfBeta *bw;
@@ -58,7 +64,7 @@ struct GatherArgs {
 struct PairArgs {
     FastArgs f;  // first (kernel_args): the binned counters, no slabs
     View v;      // the lists A and B, the histograms and the grid constants
-    const ListHead *ha, *hb;
+    const ListStat *ha, *hb;
     const int *koff_a, *koff_b;
     const int *ids;  // partner of each plan row; outside [0, nev_b): no pairs
     double psi;
@@ -74,9 +80,9 @@ inline void gather_setup(const Derived &d, const hbt_config &k, GatherArgs &g) {
     g.cut_max = std::tanh(k.HBTrap_max);
     g.pt = fast_pt_range(d);
     g.mid = d.P.pf_mid;
-    g.c_beta = d.c_beta;
     g.boost = d.P.boost;
     g.qinv = d.P.qinv;
+    g.c_beta = d.P.qinv ? 0.5 * std::sqrt(qinv_h2(d.H)) * (1.0 + 1e-9) : d.c_beta;
 }
 
 // The lists and histograms of a pair launch.

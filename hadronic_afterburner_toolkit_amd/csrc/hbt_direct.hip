@@ -12,17 +12,22 @@ using namespace hbt;
 
 constexpr long long kWaves = 4096;  // the pair kernel's resident waves (256 CUs x 16)
 
+__device__ __forceinline__ ListStat stat_none() {
+    return ListStat{0.0, 0.0, INFINITY, -INFINITY, 0};
+}
+__device__ __forceinline__ ListStat stat_join(const ListStat &a, const ListStat &b) {
+    return ListStat{fmax(a.pmax2, b.pmax2), fmax(a.bmax, b.bmax), fmin(a.m2lo, b.m2lo),
+                    fmax(a.m2hi, b.m2hi), a.n + b.n};
+}
+
 // A particle of the list: tanh(HBTrap_min) < pz/E < tanh(HBTrap_max)
 // (HBT_correlation.cpp:255-266), and |pT| as a binnable pair needs it.
-struct Kept {
-    bool keep;
-    double p2, beta;
-};
-__device__ __forceinline__ Kept list_kept(const GatherArgs &g, long long i) {
-    const double px = g.in.px[i], py = g.in.py[i], pz = g.in.pz[i], r = pz / g.in.E[i];
-    const double p2 = px * px + py * py, pt = sqrt(p2);
-    return Kept{r > g.cut_min && r < g.cut_max && pt >= g.pt.lo && pt <= g.pt.hi, p2,
-                fabs(g.boost ? r : pz)};
+__device__ __forceinline__ bool list_kept(const GatherArgs &g, long long i, ListStat &st) {
+    const double px = g.in.px[i], py = g.in.py[i], pz = g.in.pz[i], E = g.in.E[i], r = pz / E;
+    const double p2 = px * px + py * py, pt = sqrt(p2), m2 = E * E - p2 - pz * pz;
+    const bool keep = r > g.cut_min && r < g.cut_max && pt >= g.pt.lo && pt <= g.pt.hi;
+    if (keep) st = stat_join(st, ListStat{p2, fabs(g.boost ? r : pz), m2, m2, 1});
+    return keep;
 }
 
 __device__ __forceinline__ void list_store(const GatherArgs &g, double bmax, long long i, int o) {
@@ -31,14 +36,28 @@ __device__ __forceinline__ void list_store(const GatherArgs &g, double bmax, lon
     g.out.rec[o] = p;
     PfRec32 r;
     float hi;
-    pf_make(PfMake{g.mid, g.c_beta, bmax, g.boost, g.qinv}, p.px, p.py, p.pz, p.E, r, hi);
+    pf_make(PfMake{g.mid, g.c_beta, bmax, g.boost, 0}, p.px, p.py, p.pz, p.E, r, hi);
     g.out.pf[o] = PfOp{r.px, r.py, r.nrm, 1.0f};
-    // (the beta window holds for E > 0; other particles take the cascade's word)
-    g.out.bw[o] = p.E > 0.0 ? PfBeta{r.blo, hi} : PfBeta{-INFINITY, INFINITY};
+    // (the beta window holds for E > 0; other particles take the cascade's
+    // word, and so do all with q_inv bins and no LCMS boost, whose q_long is
+    // not the LCMS one)
+    g.out.bw[o] = p.E > 0.0 && (!g.qinv || g.boost) ? PfBeta{r.blo, hi}
+                                                    : PfBeta{-INFINITY, INFINITY};
 }
 
-__device__ __forceinline__ double wave_max(double v) {
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off));
+// The block's join of its threads' statistics (in every thread).
+template <int N>
+__device__ __forceinline__ ListStat block_stat(ListStat v) {
+    __shared__ ListStat part[N / 64];
+    for (int off = 32; off > 0; off >>= 1)
+        v = stat_join(v, ListStat{__shfl_down(v.pmax2, off), __shfl_down(v.bmax, off),
+                                  __shfl_down(v.m2lo, off), __shfl_down(v.m2hi, off),
+                                  __shfl_down(v.n, off)});
+    __syncthreads();
+    if (__lane_id() == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = part[0];
+    for (int k = 1; k < N / 64; k++) v = stat_join(v, part[k]);
     return v;
 }
 
@@ -46,28 +65,10 @@ __device__ __forceinline__ double wave_max(double v) {
 __global__ __launch_bounds__(256) void k_gather_count(GatherArgs g) {
     const int e = blockIdx.x;
     const long long b = g.ev_off[e], n = g.ev_off[e + 1] - b;
-    int c = 0;
-    double p2 = 0.0, be = 0.0;
-    for (long long i = threadIdx.x; i < n; i += blockDim.x) {
-        const Kept k = list_kept(g, b + i);
-        if (!k.keep) continue;
-        c++;
-        p2 = fmax(p2, k.p2);
-        be = fmax(be, k.beta);
-    }
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off);
-    p2 = wave_max(p2);
-    be = wave_max(be);
-    __shared__ int pc[4];
-    __shared__ double pp[4], pb[4];
-    const int w = threadIdx.x >> 6;
-    if (__lane_id() == 0) pc[w] = c, pp[w] = p2, pb[w] = be;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        g.out.cnt[e] = pc[0] + pc[1] + pc[2] + pc[3];
-        g.out.pmax2[e] = fmax(fmax(pp[0], pp[1]), fmax(pp[2], pp[3]));
-        g.out.bmax[e] = fmax(fmax(pb[0], pb[1]), fmax(pb[2], pb[3]));
-    }
+    ListStat st = stat_none();
+    for (long long i = threadIdx.x; i < n; i += blockDim.x) list_kept(g, b + i, st);
+    st = block_stat<256>(st);
+    if (threadIdx.x == 0) g.out.stat[e] = st;
 }
 
 // Inclusive scan over the 1024 threads of a block.
@@ -83,15 +84,6 @@ __device__ __forceinline__ int block_scan(int v, int *s) {
     }
     return s[t];
 }
-__device__ __forceinline__ double block_max(double v, double *s) {
-    v = wave_max(v);
-    __syncthreads();
-    if (__lane_id() == 0) s[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double m = 0.0;
-    for (int k = 0; k < (int)(blockDim.x >> 6); k++) m = fmax(m, s[k]);
-    return m;
-}
 
 // Exclusive scan of the kept counts into event offsets, and the head: one
 // block of 1024 threads, each summing a run of ceil(nev/1024) events.
@@ -99,45 +91,71 @@ __device__ __forceinline__ double block_max(double v, double *s) {
 // understates its events cannot make a kernel reach past it.)
 __global__ __launch_bounds__(1024) void k_gather_scan(GatherArgs g) {
     __shared__ int sc[1024];
-    __shared__ double sm[16];
-    const int t = threadIdx.x, nev = g.nev;
+    const int t = threadIdx.x, nev = g.nev, cap = g.out.cap;
     const int per = (nev + 1023) / 1024;
     const int a = min(nev, t * per), b = min(nev, a + per);
-    long long sum = 0;
-    double p2 = 0.0, be = 0.0;
+    ListStat st = stat_none();
     for (int e = a; e < b; e++) {
-        sum = min(sum + g.out.cnt[e], (long long)g.out.cap);
-        p2 = fmax(p2, g.out.pmax2[e]);
-        be = fmax(be, g.out.bmax[e]);
+        ListStat x = g.out.stat[e];
+        x.n = min(x.n, cap - st.n);
+        st = stat_join(st, x);
     }
-    const int cap = g.out.cap;  // (1024 runs of at most 2^20 stay below 2^31)
-    const int incl = block_scan((int)sum, sc);
-    int run = incl - (int)sum;
+    const int incl = block_scan(st.n, sc);  // (1024 runs of at most 2^20 stay below 2^31)
+    int run = incl - st.n;
     for (int e = a; e < b; e++) {
         g.out.koff[e] = min(run, cap);
-        run = min(run + g.out.cnt[e], cap);
+        run = min(run + g.out.stat[e].n, cap);
     }
-    p2 = block_max(p2, sm);
-    be = block_max(be, sm);
+    st = block_stat<1024>(st);
     if (t == 1023) {
-        const int n = min(incl, cap);
-        g.out.koff[nev] = n;
-        *g.out.head = ListHead{p2, be, n, 0};
+        st.n = min(incl, cap);
+        g.out.koff[nev] = st.n;
+        *g.out.head = st;
     }
 }
 
 // Order-preserving compaction of each event's kept particles to its kept
 // offset (the reference's gather order: event by event, particle order).
+// SCAN: each block sums the counts before its event itself, which spares up
+// to kScanEvents events the launch of the scan; the list's length and scales
+// are the last event's block's to write.
+constexpr int kScanEvents = 1024;
+template <bool SCAN>
 __global__ __launch_bounds__(256) void k_gather_compact(GatherArgs g) {
-    const int e = blockIdx.x;
+    const int e = blockIdx.x, cap = g.out.cap;
     const long long b = g.ev_off[e], n = g.ev_off[e + 1] - b;
     __shared__ int wsum[4];
-    int base = g.out.koff[e];
-    const double bmax = g.out.head->bmax;
+    int base;
+    double bmax;
+    if (SCAN) {
+        ListStat st = stat_none(), mine = st;
+        for (int k = threadIdx.x; k < g.nev; k += 256) {
+            ListStat x = g.out.stat[k];
+            x.n = min(x.n, cap);  // (1024 of at most 2^20 stay below 2^31)
+            if (k < e) mine.n += x.n;
+            st = stat_join(st, x);
+        }
+        const int before = block_stat<256>(mine).n;
+        st = block_stat<256>(st);
+        st.n = min(st.n, cap);
+        base = min(before, cap);
+        bmax = st.bmax;
+        if (threadIdx.x == 0) {
+            g.out.koff[e] = base;
+            if (e == g.nev - 1) {
+                g.out.koff[g.nev] = st.n;
+                *g.out.head = st;
+            }
+        }
+    } else {
+        base = g.out.koff[e];
+        bmax = g.out.head->bmax;
+    }
     const int w = threadIdx.x >> 6;
     for (long long c0 = 0; c0 < n; c0 += 256) {
         const long long i = c0 + threadIdx.x;
-        const bool keep = i < n && list_kept(g, b + i).keep;
+        ListStat st = stat_none();
+        const bool keep = i < n && list_kept(g, b + i, st);
         const unsigned long long mk = __ballot(keep);
         const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
                                                    __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0u));
@@ -149,35 +167,28 @@ __global__ __launch_bounds__(256) void k_gather_compact(GatherArgs g) {
             total += wsum[k];
         }
         const int o = base + before + rank;
-        if (keep && o < g.out.cap) list_store(g, bmax, b + i, o);
-        base = min(base + total, g.out.cap);
+        if (keep && o < cap) list_store(g, bmax, b + i, o);
+        base = min(base + total, cap);
         __syncthreads();  // wsum is rewritten by the next chunk
     }
 }
 
 // The same in one launch for a small buffer: one block, each thread a run of
-// consecutive particles (of a call of 32 us with two launches, a third and a
-// fourth would be a large part).
+// consecutive particles (630 particles: a call of 32 us, of which a second
+// launch would be a large part; 4000: 33 us against 18 with a block per event).
 __global__ __launch_bounds__(1024) void k_gather_small(GatherArgs g) {
     __shared__ int sc[1024];
-    __shared__ double sm[16];
     __shared__ int koff[kGatherSmall + 1];  // kept before each particle
     const int t = threadIdx.x;
     const long long b = g.ev_off[0];
     const int n = (int)min(g.ev_off[g.nev] - b, (long long)kGatherSmall);
     const int per = (n + 1023) / 1024, i0 = min(n, t * per), i1 = min(n, i0 + per);
-    unsigned keep = 0;  // per <= 8
-    double p2 = 0.0, be = 0.0;
-    for (int i = i0; i < i1; i++) {
-        const Kept k = list_kept(g, b + i);
-        if (!k.keep) continue;
-        keep |= 1u << (i - i0);
-        p2 = fmax(p2, k.p2);
-        be = fmax(be, k.beta);
-    }
+    unsigned keep = 0;  // per <= 2
+    ListStat st = stat_none();
+    for (int i = i0; i < i1; i++)
+        if (list_kept(g, b + i, st)) keep |= 1u << (i - i0);
     const int c = __popc(keep), incl = block_scan(c, sc);
-    p2 = block_max(p2, sm);
-    be = block_max(be, sm);
+    st = block_stat<1024>(st);
     int run = incl - c;
     for (int i = i0; i < i1; i++) {
         koff[i] = run;
@@ -185,11 +196,11 @@ __global__ __launch_bounds__(1024) void k_gather_small(GatherArgs g) {
     }
     if (t == 1023) koff[n] = incl;
     for (int i = i0, o = incl - c; i < i1; i++)
-        if (keep >> (i - i0) & 1u) list_store(g, be, b + i, o++);
+        if (keep >> (i - i0) & 1u) list_store(g, st.bmax, b + i, o++);
     __syncthreads();
     for (int e = t; e <= g.nev; e += 1024)
         g.out.koff[e] = koff[(int)max(0ll, min(g.ev_off[e] - b, (long long)n))];
-    if (t == 1023) *g.out.head = ListHead{p2, be, incl, 0};
+    if (t == 1023) *g.out.head = st;
 }
 
 // The pair kernel's view: its own argument.
@@ -198,6 +209,37 @@ struct ArgView {
         return (CView *)((const HBT_AS4 char *)ka + offsetof(PairArgs, v));
     }
 };
+
+// The prefilter's constants for two lists' scales.  With q_inv bins a pair
+// that bins in either kind of histogram has |q_side| and |q_long| within
+// sqrt(1 + kQinvRoom) H, but no bound on q_out, so the kernel tests
+// C^2 <= H^2 T alone (dn = 0).  For q_inv: in the LCMS q_E M_t = K_T q_out + d
+// with d = (m1^2 - m2^2) / 2, so q_inv^2 = q_side^2 + q_long^2 +
+// q_out^2 - q_E^2 and the smallest value of the last two, over all q_out, is
+// -d^2 / K^2 with K^2 = (m1^2 + m2^2) / 2 + q_inv^2 / 4 at least the lists'
+// smallest m^2.  Where the lists' m^2 = E^2 - p^2 differ too much for the room,
+// every pair in the K_T window takes the cascade, as all did before: 435 us for
+// 20 events of 200 particles, 105 with the windows.
+__device__ __forceinline__ PfConst<float> pair_consts(DevParams P, const ListStat &st) {
+    if (!P.qinv) {
+        prefilter_margins(st.pmax2, P);
+        return pf_const<float>(P);
+    }
+    const double d = 0.5 * (st.m2hi - st.m2lo), H = fmax(fabs(P.q_lo_cut), fabs(P.q_hi_cut));
+    const bool windows = st.m2lo > 0.0 && d * d <= 0.5 * kQinvRoom * H * H * st.m2lo;
+    if (windows) {
+        P.qinv = 0;
+        P.pf_h2 = qinv_h2(H);
+        prefilter_margins(st.pmax2, P);
+        PfConst<float> k = pf_const<float>(P);
+        k.dn = 0.0f;
+        return k;
+    }
+    prefilter_margins(st.pmax2, P);
+    PfConst<float> k = pf_const<float>(P);
+    k.wide = INFINITY;
+    return k;
+}
 
 // Bound by the adds' atomics (2.35e10 binned same-event and 2.68e10 mixed pairs
 // per second, memory side) where more than a percent of the pairs bins, else
@@ -214,11 +256,10 @@ __attribute__((amdgpu_waves_per_eu(fast_waves_per_eu<Prec, EXT>()))) void k_pair
     tot.slab_next = nullptr;
     tot.slab_lim = nullptr;
     CView *vp = ArgView::at(kernel_args(), 0);
-    const int n = HBT_CONST(ListHead, g.ha)->n;
+    const int n = HBT_CONST(ListStat, g.ha)->n;
     const HBT_AS4 int *ka = HBT_CONST(int, g.koff_a), *kb = HBT_CONST(int, g.koff_b);
-    DevParams P = g.v.P;
-    prefilter_margins(fmax(HBT_CONST(ListHead, g.ha)->pmax2, HBT_CONST(ListHead, g.hb)->pmax2), P);
-    const PfConst<float> pk = pf_const<float>(P);
+    const PfConst<float> pk = pair_consts(
+        g.v.P, stat_join(*(const ListStat *)g.ha, *(const ListStat *)g.hb));
     const double psi = g.psi;
     tot.qlds = qinv_begin<Prec, EXT>(dyn_lds, g.f.qinv_lds);
     for (long long it = (long long)blockIdx.x * 4 + wv; it < g.nitems;
@@ -288,8 +329,12 @@ hipError_t launch_gather(const GatherArgs &g, long long n, hipStream_t st) {
         hipLaunchKernelGGL(k_gather_small, dim3(1), dim3(1024), 0, st, g);
     } else {
         hipLaunchKernelGGL(k_gather_count, dim3(g.nev), dim3(256), 0, st, g);
-        hipLaunchKernelGGL(k_gather_scan, dim3(1), dim3(1024), 0, st, g);
-        hipLaunchKernelGGL(k_gather_compact, dim3(g.nev), dim3(256), 0, st, g);
+        if (g.nev <= kScanEvents) {
+            hipLaunchKernelGGL(k_gather_compact<true>, dim3(g.nev), dim3(256), 0, st, g);
+        } else {
+            hipLaunchKernelGGL(k_gather_scan, dim3(1), dim3(1024), 0, st, g);
+            hipLaunchKernelGGL(k_gather_compact<false>, dim3(g.nev), dim3(256), 0, st, g);
+        }
     }
     return hipGetLastError();
 }

@@ -52,9 +52,12 @@ struct PfRec32 {
 // every pair); sh bounds |X| (the T window's half-width, scaled and rounded
 // up; nsh2 = -sh^2), c0 = H^2 mid + c bounds max(|dn|, |C|)^2 - X, with the q
 // margin c (infinite with the q_inv branch on).
+// dn: 1/2, or 0 where |dn| is left out (q_inv bins: no bound on q_out); wide: 0,
+// or infinity where the beta intervals count for nothing.
 template <typename Prec>
 struct PfConst {
     Prec s, nsh2, c0;
+    Prec dn = (Prec)0.5, wide = 0;
 };
 
 template <typename Prec>
@@ -551,7 +554,7 @@ __device__ __forceinline__ PfBlock pf_block(const PfConst<float> &k, int comp, f
     const float s2 = 2.0f * k.s;
     o.X = comp == 0 ? s2 * x : comp == 1 ? s2 * y : comp == 2 ? k.s : k.s * n;
     const float c = comp == 0 ? -y : comp == 1 ? x : 0.0f;
-    const float d = comp == 2 ? -0.5f : comp == 3 ? 0.5f * n : 0.0f;
+    const float d = comp == 2 ? -k.dn : comp == 3 ? k.dn * n : 0.0f;
     o.P = d + c;
     o.M = d - c;
     return o;
@@ -637,8 +640,8 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
 #pragma unroll
     for (int b = 0; b < 4; b++) {
         const PfBeta r = bwi[min(16 * b + col, w.ni - 1)];
-        ilo[b] = r.lo;
-        ihi[b] = r.hi;
+        ilo[b] = r.lo - pk.wide;
+        ihi[b] = r.hi + pk.wide;
     }
     unsigned cols = 0;  // the bits of the blocks' columns inside the tile
 #pragma unroll

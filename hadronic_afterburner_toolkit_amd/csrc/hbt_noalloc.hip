@@ -31,10 +31,9 @@ constexpr long long kMaxParticles = HBT_NOALLOC_MAX_PARTICLES;
 constexpr int kMaxEvents = HBT_NOALLOC_MAX_EVENTS;
 // The kept particles.
 struct Scratch {
-    ListHead head;
+    ListStat head;
+    ListStat stat[kMaxEvents];
     int koff[kMaxEvents + 1];
-    int cnt[kMaxEvents];
-    double pmax2[kMaxEvents], bmax[kMaxEvents];
     alignas(256) PartRec rec[kMaxParticles + kPfPad];
     alignas(256) PfOp pf[kMaxParticles + kPfPad];
     alignas(256) PfBeta bw[kMaxParticles + kPfPad];
@@ -122,8 +121,7 @@ int hbt_calculate_noalloc(const hbt_config *cfg, int32_t nev, int64_t n_particle
         rc = scratch_ptr(cfg->device, &scr);
         if (rc) break;
         Scratch *s = (Scratch *)scr;
-        const List list{&s->head, s->koff, s->cnt, s->pmax2, s->bmax,
-                        s->rec,   s->pf,   s->bw,  (int)kMaxParticles};
+        const List list{&s->head, s->koff, s->stat, s->rec, s->pf, s->bw, (int)kMaxParticles};
         GatherArgs g{};
         g.ev_off = (const long long *)ev_off;
         g.in = DevSoA{soa[0], soa[1], soa[2], soa[3], soa[4], soa[5], soa[6], soa[7]};

@@ -115,3 +115,36 @@ def test_direct_call_goes_on_as_a_batch():
         g.launch_batch()
     same(a, g.results())
     g.close()
+
+
+@pytest.mark.parametrize("boost", [0, 1])
+@pytest.mark.parametrize("shell", ["on", "rounded", "two masses", "massless"])
+def test_qinv_windows(shell, boost):
+    """q_inv bins: particles on one mass shell, within the room of it (energies
+    rounded to seven digits), of two masses, and massless (the last two leave
+    every pair to the cascade); wide momenta, so that q_out far outside the 3D
+    windows bins in q_inv."""
+    rng = np.random.default_rng(11)
+    buf = events(rng, [150] * 20, 1.2)
+    if shell == "rounded":
+        buf.E[:] = np.array([float("%.6e" % e) for e in buf.E])
+    elif shell == "two masses":
+        p2 = buf.px ** 2 + buf.py ** 2 + buf.pz ** 2
+        buf.E[::3] = np.sqrt(p2[::3] + 0.494 ** 2)
+    elif shell == "massless":
+        buf.E[:] = np.sqrt(buf.px ** 2 + buf.py ** 2 + buf.pz ** 2)
+    params = dict(config(qinv=1), long_comoving_boost=boost, KT_max=1.5)
+    M, ids, cs = hbt.Random(7).draw_plan(buf.nev, buf.nev, 4)
+    g = hbt.HBTCorrelation(params, precision=_lib.HBT_PREC_FP64)
+    g.upload(buf)
+    g.run_same()
+    g.run_mixed(M, ids, cs)
+    a = g.results()
+    g.reset()
+    g.upload(buf)
+    g.prepare_batch([M], ids, cs)
+    g.launch_batch()
+    b = g.results()
+    g.close()
+    assert b.qinv_count.sum() > 5000 and b.qinv_den.sum() > 5000
+    same(a, b)
