@@ -37,12 +37,12 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <unordered_map>
 #include <utility>
 #include <vector>
 
 #include "../../include/hbt_hip.h"
+#include "host_pool.h"
 
 namespace {
 
@@ -364,22 +364,8 @@ struct Picker {
     static constexpr long long kNoBad = 1ll << 40;
 };
 
-template <typename F>
-void par_ranges(long long n, long long min_per_thread, F fn) {
-    const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    const long long nt =
-        std::max(1ll, std::min<long long>(hw, n / std::max(1ll, min_per_thread)));
-    if (nt <= 1) {
-        fn(0ll, n);
-        return;
-    }
-    std::vector<std::thread> th;
-    for (long long t = 0; t < nt; t++) th.emplace_back(fn, n * t / nt, n * (t + 1) / nt);
-    for (auto &x : th) x.join();
-}
-
 // First pass over one buffer: event offsets and sizes of the lists of
-// ids[0..nl), over event ranges on up to 16 threads (the pT cut of
+// ids[0..nl), over event ranges on the host threads (the pT cut of
 // BalanceFunction.cpp:127-129).
 void count_lists(const hbt_bf_config &cfg, int32_t nev, const int64_t *ev_off,
                  const int32_t *monval, const double *const cols[5], const Picker &pk,
@@ -387,7 +373,7 @@ void count_lists(const hbt_bf_config &cfg, int32_t nev, const int64_t *ev_off,
     const int nl = pk.nl;
     const double *px = cols[1], *py = cols[2];
     std::vector<long long> cnt((size_t)nl * std::max(nev, 1), 0);
-    par_ranges(nev, 32, [&](long long e0, long long e1) {
+    hbt::parallel_ranges(nev, 32, [&](long long e0, long long e1) {
         for (long long e = e0; e < e1; e++)
             for (int64_t i = ev_off[e]; i < ev_off[e + 1]; i++) {
                 const unsigned m = pk.mask(monval[i]);
@@ -416,7 +402,7 @@ void fill_lists(const hbt_bf_config &cfg, int32_t nev, const int64_t *ev_off,
     const int nl = pk.nl;
     const double *mass = cols[0], *px = cols[1], *py = cols[2], *pz = cols[3];
     std::mutex mu;
-    par_ranges(nev, 32, [&](long long e0, long long e1) {
+    hbt::parallel_ranges(nev, 32, [&](long long e0, long long e1) {
         double mphi[4] = {0, 0, 0, 0}, my[4] = {0, 0, 0, 0};
         for (long long e = e0; e < e1; e++) {
             long long pos[4] = {0, 0, 0, 0};
