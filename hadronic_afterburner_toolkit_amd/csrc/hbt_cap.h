@@ -255,7 +255,7 @@ __device__ __forceinline__ int nth_hit(bool hit, long long &want) {
 // groups (ngroups+1).  The search ends early, so its time is that of the
 // longest chain of cascades: with one thread per key, thousands of pairs one
 // after the other (a call of 20 events of 600 particles in which six keys
-// pass the cap on either side took 11.2 ms, 4.0 with 64 pairs at a time).
+// pass the cap on either side took 11.2 ms, 3.6 with 64 pairs at a time).
 __global__ __launch_bounds__(64) void k_cap_pos_same(DevParams P, DevSoA A, const long long *gpoff, int ngroups,
                                const double *psi, CapCut *cut, int nkeys, bool qinv_keys,
                                const DeferKey *dk, int ndk) {

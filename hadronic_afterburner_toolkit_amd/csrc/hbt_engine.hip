@@ -243,31 +243,6 @@ __global__ __launch_bounds__(256) void k_zero_hist(DevHist H, long words, long n
     if (t == 0) *H.ndefer = 0;
 }
 
-// Sum of a u64 field over the q bins of each (kt, kphi): the reference's
-// number_of_pairs_*_KTdiff / _KTKphidiff counters.  Element k of group g
-// is h[(g*per + k)*stride].
-// T = double for the count field (integers held exactly below 2^53).
-// Each block sums a run of a group's bins (one block per group, 1024 threads
-// reading a cache line per bin one after the other, took 16.6 us for 6 x 31^3
-// bins; this takes 4.7); out starts at zero.
-template <typename T>
-__global__ __launch_bounds__(1024) void k_sum_groups(const T *h, long per, int stride,
-                                                     unsigned long long *out) {
-    const int g = blockIdx.y;
-    unsigned long long acc = 0;
-    for (long k = (long)blockIdx.x * 1024 + threadIdx.x; k < per; k += (long)gridDim.x * 1024)
-        acc += (unsigned long long)h[((long)g * per + k) * stride];
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off);
-    __shared__ unsigned long long part[16];
-    if (__lane_id() == 0) part[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += part[w];
-        atomic_add_u64(&out[g], t);
-    }
-}
-
 // Histograms on their way to the host.  The host's arrays are one per field
 // while a bin holds its fields side by side: n bins from b0 on leave as six
 // columns of n words (count as an integer, den, and the four sums) straight
@@ -439,6 +414,8 @@ struct hbt_ctx {
     size_t snap_cap = 0;
     int *d_flag = nullptr;      // [2][nkey3 + n_KT] CapKey of each side's keys
     size_t flag_cap = 0;
+    char *h_sums = nullptr;     // pinned: the cap's counters
+    size_t hsums_cap = 0;
     // slab binning of the fast kernel (hbt_slab.h)
     struct {
         bool on = false;            // the next fast launch bins through slabs
@@ -649,37 +626,34 @@ int resolve_deferred(hbt_ctx *c) {
     return HBT_OK;
 }
 
-// Per-(kt,kphi) sums of a u64 histogram field into host memory.
-template <typename T>
-int group_sums(hbt_ctx *c, const T *h, long per, int groups, int stride,
-               std::vector<unsigned long long> &out) {
-    out.assign(groups, 0);
-    if (groups <= 0) return HBT_OK;
-    HIPCHECK(c, launch_zero_words(c->d_sums, (size_t)groups, c->stream));
-    const unsigned blocks = (unsigned)std::min(64l, (per + 1023) / 1024);
-    for (int g = 0; g < groups; g += 65535)
-        hipLaunchKernelGGL(k_sum_groups<T>, dim3(blocks, std::min(65535, groups - g)), dim3(1024),
-                           0, c->stream, h + (long)g * per * stride, per, stride, c->d_sums + g);
-    HIPCHECK(c, hipGetLastError());
-    HIPCHECK(c, hipMemcpyAsync(out.data(), c->d_sums, groups * 8, hipMemcpyDeviceToHost,
-                               c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return HBT_OK;
-}
-
-// One side's cap counters: 3D keys, then q_inv keys (0 without q_inv).
-int cap_counters(hbt_ctx *c, bool mixed, std::vector<unsigned long long> &out) {
-    const int nkey3 = c->cfg.n_KT * c->P.nphi, nkq = c->cfg.n_KT;
+// Both sides' cap counters, out[0] same-event and out[1] mixed: 3D keys, then
+// q_inv keys (0 without q_inv).  One pass over the bins for both, straight into
+// pinned memory: 10 us a call less than a side by itself and through a copy.
+int cap_counters(hbt_ctx *c, std::vector<unsigned long long> out[2]) {
+    const int nkey3 = c->cfg.n_KT * c->P.nphi, nkq = c->cfg.n_KT, nsums = 2 * nkey3;
+    const size_t words = (size_t)nsums + 4 * (size_t)c->nq + 2 * (size_t)nkq;
+    HIPCHECK(c, ensure_pinned(&c->h_sums, &c->hsums_cap, words * 8));
+    HIPCHECK(c, launch_zero_words(c->d_sums, (size_t)nsums, c->stream));
     const long per = (long)c->P.qnpts * c->P.qnpts * c->P.qnpts;
-    std::vector<unsigned long long> cq(nkq, 0);
-    int rc = mixed ? group_sums(c, (const unsigned long long *)(c->d_bins + BIN_DEN), per, nkey3,
-                                BIN_STRIDE, out)
-                   : group_sums(c, (const double *)(c->d_bins + BIN_COUNT), per, nkey3,
-                                BIN_STRIDE, out);
-    if (!rc && c->P.qinv)
-        rc = group_sums(c, mixed ? c->d_qinv_den : c->d_qinv_count, c->P.qnpts, nkq, 1, cq);
-    out.insert(out.end(), cq.begin(), cq.end());
-    return rc;
+    for (long b0 = 0; b0 < c->nbins; b0 += 1l << 28) {
+        const int n = (int)std::min(1l << 28, c->nbins - b0);
+        hipLaunchKernelGGL(k_read_bins, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_bins,
+                           b0, n, per, nullptr, c->d_sums, c->d_sums + nkey3);
+    }
+    unsigned long long *h = (unsigned long long *)c->h_sums;
+    hipLaunchKernelGGL(k_read_tail, dim3(1), dim3(256), 0, c->stream, c->d_sums, nsums,
+                       hist_view(c), (int)c->nq, nkq, c->P.qnpts, h);
+    HIPCHECK(c, hipGetLastError());
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    const unsigned long long *q = h + nsums + 4 * c->nq;
+    for (int m = 0; m < 2; m++) {
+        out[m].assign(h + m * nkey3, h + (m + 1) * nkey3);
+        if (c->P.qinv)
+            out[m].insert(out[m].end(), q + m * nkq, q + (m + 1) * nkq);
+        else
+            out[m].resize((size_t)nkey3 + nkq, 0);
+    }
+    return HBT_OK;
 }
 
 // The pair cap (HBT_correlation.cpp:402-406, :651-655, q_inv :340-341,
@@ -693,19 +667,28 @@ struct CapSide {
     bool binds = false;
     std::vector<unsigned long long> count;
 };
-int check_cap(hbt_ctx *c, bool mixed, uint64_t enum_call, CapSide &side) {
-    bool &binds = side.binds;
-    binds = false;
-    const uint64_t total = (mixed ? c->enum_mixed_total : c->enum_same_total) + enum_call;
+int check_cap(hbt_ctx *c, const uint64_t enum_call[2], CapSide side[2]) {
     const bool qinv = c->cfg.invariant_radius_flag == 1;
-    if (total <= c->needed + 1 && (!qinv || total <= c->needed_qinv)) return HBT_OK;
-    const int groups = c->cfg.n_KT * c->P.nphi;
-    std::vector<unsigned long long> &cnt = side.count;
-    if (int rc = cap_counters(c, mixed, cnt)) return rc;
-    for (int k = 0; k < groups; k++)
-        if (cnt[k] + enum_call > c->needed + 1) binds = true;
-    for (int k = groups; k < groups + c->cfg.n_KT && qinv; k++)
-        if (cnt[k] + enum_call > c->needed_qinv) binds = true;
+    bool look = false;
+    for (int m = 0; m < 2; m++) {
+        const uint64_t total = (m ? c->enum_mixed_total : c->enum_same_total) + enum_call[m];
+        side[m].binds = enum_call[m] > 0 &&
+                        (total > c->needed + 1 || (qinv && total > c->needed_qinv));
+        look = look || side[m].binds;
+    }
+    if (!look) return HBT_OK;
+    std::vector<unsigned long long> cnt[2];
+    if (int rc = cap_counters(c, cnt)) return rc;
+    const size_t nkey3 = (size_t)c->cfg.n_KT * c->P.nphi;
+    for (int m = 0; m < 2; m++) {
+        bool binds = false;
+        for (size_t k = 0; k < cnt[m].size(); k++)
+            if (k < nkey3 || qinv)
+                binds = binds || cnt[m][k] + enum_call[m] >
+                                     (k < nkey3 ? c->needed + 1 : c->needed_qinv);
+        side[m].binds = side[m].binds && binds;
+        side[m].count.swap(cnt[m]);
+    }
     return HBT_OK;
 }
 
@@ -1369,10 +1352,10 @@ int run_capped(hbt_ctx *c, bool mixed, const int *d_flag = nullptr) {
     if (rc) return rc;
     HIPCHECK(c, hipMemsetAsync(c->d_cnt, 0, (size_t)nkeys * nrows * 4, c->stream));
     // remaining capacity per key from the counters so far (sums of the bins)
-    std::vector<unsigned long long> c3;
-    rc = cap_counters(c, mixed, c3);
+    std::vector<unsigned long long> cnt[2];
+    rc = cap_counters(c, cnt);
     if (rc) return rc;
-    const std::vector<unsigned long long> lim = cap_room(c, c3);
+    const std::vector<unsigned long long> lim = cap_room(c, cnt[mixed]);
     std::vector<long long> gpoff(s.ngroups + 1);
     for (int g = 0; g <= s.ngroups; g++) gpoff[g] = s.off[s.grp_ev[g]];
     HIPCHECK(c, hipMemcpy(c->d_lim, lim.data(), nkeys * 8, hipMemcpyHostToDevice));
@@ -1473,8 +1456,8 @@ int run_capped(hbt_ctx *c, bool mixed, const int *d_flag = nullptr) {
 // the cap before the call, or passed it, get their bins back from a copy taken
 // before the launch; only for keys that passed it the ordered passes then run.
 // A buffer of 20 events of 600 particles (1.5e8 pairs), host work included:
-// 1.1 ms against 3.75 with the ordered passes alone, 1.15 against 3.6 with
-// every key past the cap before it, 4.0 against 11.2 when every key passes it
+// 0.40 ms against 3.75 with the ordered passes alone, 0.43 against 3.6 with
+// every key past the cap before it, 3.6 against 11.2 when every key passes it
 // (of which the position search took 7, one pair after the other).  A copy that
 // cannot be allocated leaves the ordered passes.
 // launch: queues the call's FP64 launch, its binned counts at the address
@@ -1515,14 +1498,14 @@ int run_trial(hbt_ctx *c, const TrialLaunch &launch, const CapSide side[2], bool
     const uint64_t deferred = c->deferred_total;
     std::vector<int> flag((size_t)2 * nkeys, CAP_OK);
     bool restore = false, cross[2] = {false, false};
+    std::vector<unsigned long long> now[2];
+    rc = cap_counters(c, now);
+    if (rc) return rc;
     for (int m = 0; m < 2; m++) {
         if (!side[m].binds) continue;
-        CapSide now;
-        rc = cap_counters(c, m == 1, now.count);
-        if (rc) return rc;
         const auto room = cap_room(c, side[m].count);
         for (int k = 0; k < nkeys; k++) {
-            const unsigned long long n = now.count[k] - side[m].count[k];
+            const unsigned long long n = now[m][k] - side[m].count[k];
             if (n <= room[k]) continue;
             flag[(size_t)m * nkeys + k] = room[k] ? CAP_CROSS : CAP_FULL;
             restore = true;
@@ -2041,6 +2024,7 @@ int hbt_destroy(hbt_ctx *c) {
     if (c->h_stage) hipHostFree(c->h_stage);
     if (c->h_stage2) hipHostFree(c->h_stage2);
     if (c->h_read) hipHostFree(c->h_read);
+    if (c->h_sums) hipHostFree(c->h_sums);
     for (int k = 0; k < 2; k++) {
         if (c->h_plan[k]) hipHostFree(c->h_plan[k]);
         if (c->plan_ev[k]) hipEventDestroy(c->plan_ev[k]);
@@ -2098,7 +2082,8 @@ int hbt_run_same(hbt_ctx *c) {
         build_items(c, true, false, items, es);
     }
     CapSide side[2];
-    rc = check_cap(c, false, es, side[0]);
+    const uint64_t call[2] = {es, 0};
+    rc = check_cap(c, call, side);
     if (rc) return rc;
     rc = upload_psi(c);
     if (rc) return rc;
@@ -2159,7 +2144,8 @@ int hbt_run_mixed(hbt_ctx *c, int32_t M, const int32_t *partner_ids, const doubl
     rc = upload_plan(c, Me, partner_ids, cos_sin, em);
     if (rc) return rc;
     CapSide side[2];
-    rc = check_cap(c, true, em, side[1]);
+    const uint64_t call[2] = {0, em};
+    rc = check_cap(c, call, side);
     if (rc) return rc;
     rc = upload_psi(c);
     if (rc) return rc;
@@ -2252,8 +2238,8 @@ int hbt_launch_batch(hbt_ctx *c) {
         if (rc0) return rc0;
     }
     CapSide side[2];
-    int rc = check_cap(c, false, c->batch_enum_same, side[0]);
-    if (!rc) rc = check_cap(c, true, c->batch_enum_mixed, side[1]);
+    const uint64_t call[2] = {c->batch_enum_same, c->batch_enum_mixed};
+    int rc = check_cap(c, call, side);
     if (rc) return rc;
     const bool bs = side[0].binds, bm = side[1].binds;
     HIPCHECK(c, hipEventRecord(c->ev[0], c->stream));
