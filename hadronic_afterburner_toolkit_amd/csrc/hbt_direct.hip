@@ -38,11 +38,8 @@ __device__ __forceinline__ void list_store(const GatherArgs &g, double bmax, lon
     float hi;
     pf_make(PfMake{g.mid, g.c_beta, bmax, g.boost, 0}, p.px, p.py, p.pz, p.E, r, hi);
     g.out.pf[o] = PfOp{r.px, r.py, r.nrm, 1.0f};
-    // (the beta window holds for E > 0; other particles take the cascade's
-    // word, and so do all with q_inv bins and no LCMS boost, whose q_long is
-    // not the LCMS one)
-    g.out.bw[o] = p.E > 0.0 && (!g.qinv || g.boost) ? PfBeta{r.blo, hi}
-                                                    : PfBeta{-INFINITY, INFINITY};
+    // (with q_inv bins and no LCMS boost q_long is not the LCMS one: no window)
+    g.out.bw[o] = !g.qinv || g.boost ? PfBeta{r.blo, hi} : PfBeta{-INFINITY, INFINITY};
 }
 
 // The block's join of its threads' statistics (in every thread).

@@ -7,7 +7,7 @@
 // idle while any lane continues, so a direct port pays the whole cascade
 // (sqrt, three to five divisions, cos) for almost every pair.  Here the
 // work items' windows leave out most pairs unevaluated, every evaluated pair
-// costs three matrix-core products and 7 VALU operations, and only its
+// costs its share of three matrix-core products and 9 VALU operations, and only its
 // survivors (~1.4% of the enumerated pairs on the bench workload) reach the
 // exact cascade, 64 at a time with all lanes busy.
 //
@@ -18,13 +18,16 @@
 //        / |p1T + p2T| = dn / sqrt(T), dn = n1 - n2, n = |pT|^2)
 //   q_side^2 = C^2 / T <= H^2                (q_side = (p1T - p2T)x(p1T + p2T)
 //        / |p1T + p2T|, whose numerator is C = 2 (p1x p2y - p1y p2x))
-//   |beta1 - beta2| <= (H/2) (1/E1 + 1/E2)   (from |q_long| <= H, M_t <= K_E,
-//        q_long M_t = E2 pz1 - E1 pz2; beta = pz/E)
+//   |y1 - y2| <= (H/2) (1/m_T1 + 1/m_T2)     (y the rapidity, E = m_T cosh y, pz =
+//        m_T sinh y: q_long M_t = E2 pz1 - E1 pz2 = m_T1 m_T2 sinh(y1 - y2) and
+//        M_t <= (m_T1 + m_T2) / 2 cosh((y1 - y2) / 2), so |q_long| <= H needs
+//        2 sinh(|y1 - y2| / 2) <= (H/2) (1/m_T1 + 1/m_T2); the test passes 1 % more
+//        pairs than |q_long| <= H itself, 6 % fewer than the same in beta and E)
 // with H = max(|q_lo_cut|, |q_hi_cut|).  The two q windows are one test,
 // max(|dn|, |C|)^2 <= H^2 T.  T, dn and C are bilinear in the two particles'
 // (px, py, n, 1), so the matrix cores form them.
 // For mixed pairs the i particle is rotated by -theta instead of rotating
-// every j by +theta (T, dn, C and beta are rotation invariant); the exact
+// every j by +theta (T, dn, C and y are rotation invariant); the exact
 // cascade then uses the reference's rotated j (HBT_correlation.cpp:522-523).
 #pragma once
 #include "hbt_device.h"
@@ -36,7 +39,7 @@ namespace hbt {
 
 // Per-particle prefilter record: nrm = px^2+py^2 - mid/2 (so that
 // n1 + n2 + 2 p1.p2 = T - mid), and blo, the lower end of the particle's
-// beta interval [beta - cw, beta + cw] (beta = pz/E, or pz without the LCMS
+// longitudinal interval [y - cw, y + cw] (y the rapidity, or pz without the LCMS
 // boost); the upper end bhi is kept beside the records.  The kernel reads the
 // FP32 records, which pass every pair the exact cascade of either precision
 // accepts; the FP64 ones state the same tests without FP32's rounding.
@@ -53,7 +56,7 @@ struct PfRec32 {
 // up; nsh2 = -sh^2), c0 = H^2 mid + c bounds max(|dn|, |C|)^2 - X, with the q
 // margin c (infinite with the q_inv branch on).
 // dn: 1/2, or 0 where |dn| is left out (q_inv bins: no bound on q_out); wide: 0,
-// or infinity where the beta intervals count for nothing.
+// or infinity where the longitudinal intervals count for nothing.
 template <typename Prec>
 struct PfConst {
     Prec s, nsh2, c0;
@@ -75,8 +78,8 @@ __host__ __device__ __forceinline__ PfConst<Prec> pf_const(const DevParams &P) {
 
 // The prefilter's tests of one pair (for a mixed pair, i rotated by
 // -theta): it passes where all four values are negative.  K_T window: X^2 -
-// (s half)^2; q_out and q_side: max(|dn|, |C|)^2 - X - (H^2 mid + c); beta:
-// |beta_i - beta_j| <= cw_i + cw_j as the overlap of the two beta intervals,
+// (s half)^2; q_out and q_side: max(|dn|, |C|)^2 - X - (H^2 mid + c); q_long:
+// |y_i - y_j| <= cw_i + cw_j as the overlap of the two longitudinal intervals,
 // blo_i - bhi_j and blo_j - bhi_i.  The margins leave every pair the exact
 // cascade accepts strictly inside.  The host's check of the margins evaluates
 // this function; the kernel forms X, dn and C on the matrix cores, whose order
@@ -113,8 +116,8 @@ __host__ __device__ __forceinline__ bool pf_pass(const PfTerms<Prec> &t) {
 }
 
 // What a particle's prefilter record needs beside its momentum: the window
-// centre, the beta half-width's numerator H/2, the largest |beta| of the list
-// (FP32 margins), and the analysis' boost and q_inv switches.
+// centre, the longitudinal half-width's numerator H/2, the largest |beta| of the
+// list (|pz| without the LCMS boost; margins), and the analysis' boost and q_inv switches.
 struct PfMake {
     double mid, c_beta, bm;
     int boost, qinv;
@@ -128,22 +131,35 @@ __host__ __device__ __forceinline__ float next_float(float x, bool up) {
     return __builtin_bit_cast(float, b + ((x > 0.0f) == up ? 1 : -1));
 }
 
-// FP32 record of one particle: cw also covers the rounding of beta (|beta|
-// <= bm over the list) and of cw itself; the interval's ends are rounded to
-// nearest, then one FP32 ulp outward.
-__host__ __device__ __forceinline__ void pf_make(const PfMake &m, double px, double py, double pz,
-                                                 double E, PfRec32 &r, float &bhi) {
-    const double eps32 = 5.9604644775390625e-8;
-    const double beta = m.boost ? pz / E : pz;
-    const double cw = m.qinv ? INFINITY
-                             : (m.boost ? m.c_beta / E : m.c_beta) * (1.0 + 8 * eps32) +
-                                   4 * eps32 * fmax(1.0, m.bm);
-    r = PfRec32{(float)px, (float)py, (float)(px * px + py * py - 0.5 * m.mid),
-                next_float((float)(beta - cw), false)};
-    bhi = next_float((float)(beta + cw), true);
+// Where a particle's longitudinal interval [y - cw, y + cw] lies: y its rapidity
+// and cw = (H/2) / m_T (or pz and H/2 without the LCMS boost; no window with the
+// q_inv branch on, or for E <= 0).  eps: the rounding unit of the interval's
+// ends.  cw also covers the rounding of y and of cw: with |beta| <= bm over the
+// list, cosh^2 y <= 1 / (1 - bm^2) scales beta's own rounding.
+struct LongWindow {
+    double y, cw;
+};
+__host__ __device__ __forceinline__ LongWindow long_window(const PfMake &m, double pz, double E,
+                                                           double eps) {
+    if (m.qinv || !(E > 0.0)) return LongWindow{0.0, INFINITY};
+    if (!m.boost) return LongWindow{pz, m.c_beta * (1.0 + 8 * eps) + 4 * eps * fmax(1.0, m.bm)};
+    const double g = 8.9e-16 / (1.0 - m.bm * m.bm);
+    if (!(g >= 0.0 && g < 1.0)) return LongWindow{0.0, INFINITY};
+    return LongWindow{atanh(pz / E), m.c_beta / sqrt((E - pz) * (E + pz)) * (1.0 + 8 * eps + g) +
+                                         4 * eps * fmax(1.0, atanh(m.bm)) + g};
 }
 
-// A particle as the kernel's matrix-core operand, and its beta interval.
+// FP32 record of one particle; the interval's ends are rounded to nearest, then
+// one FP32 ulp outward.
+__host__ __device__ __forceinline__ void pf_make(const PfMake &m, double px, double py, double pz,
+                                                 double E, PfRec32 &r, float &bhi) {
+    const LongWindow w = long_window(m, pz, E, 5.9604644775390625e-8);
+    r = PfRec32{(float)px, (float)py, (float)(px * px + py * py - 0.5 * m.mid),
+                next_float((float)(w.y - w.cw), false)};
+    bhi = next_float((float)(w.y + w.cw), true);
+}
+
+// A particle as the kernel's matrix-core operand, and its longitudinal interval.
 struct __align__(16) PfOp {
     float px, py, nrm, one;
 };
@@ -174,7 +190,7 @@ struct View {
     const PfOp *pfA;     // prefilter operands of A, of B,
     const PfOp *pfB;
     const PfOp *pfS;     // and of the same-event fast list sorted by (px cell, py) per group
-    const PfBeta *bwA;   // their beta intervals
+    const PfBeta *bwA;   // their longitudinal intervals
     const PfBeta *bwB;
     const PfBeta *bwS;
     const OrigRank *origS;     // cell-sorted position -> fast-list index and gather rank
@@ -190,8 +206,8 @@ struct View {
 };
 
 // The fast lists on the device, from the uploaded records A (per event,
-// |pT|-sorted) and the cell-sorted order: the prefilter operands and beta
-// intervals of both orders, and the cell-sorted copy of the records, AS[q] =
+// |pT|-sorted) and the cell-sorted order: the prefilter operands and
+// longitudinal intervals of both orders, and the cell-sorted copy of the records, AS[q] =
 // A[orr[q].idx].
 static __global__ __launch_bounds__(256) void k_build_lists(PfMake m, const PartRec *__restrict__ A,
                                                             const OrigRank *__restrict__ orr,
@@ -794,9 +810,10 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
 // (128 VGPRs, no spills in the hot path); the K_phi / q_inv instance of the
 // FP64 form, whose main path is the literal cascade with atan2 and the
 // host-defer path, runs at three.
-// Headline workload (2.5e10 pairs, 4.8e9 evaluated): 5.6 ms in the precision
+// Headline workload (2.5e10 pairs, 4.8e9 evaluated): 5.4 ms in the precision
 // form, of which the prefilter alone 2.6 and the mixed adds' atomic floor 3.3;
-// 8.0 ms with scalar tests and records fetched by scattered loads.
+// 8.0 ms with scalar tests and records fetched by scattered loads.  Bound by
+// vector instructions: 9 a tested pair, some 230 a batch of 64 survivors.
 struct TableViews {
     static __device__ __forceinline__ CView *at(CArgs *ka, int view) {
         return view_at(ka->views, view);

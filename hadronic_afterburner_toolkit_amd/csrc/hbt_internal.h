@@ -125,19 +125,16 @@ inline PfMake pf_maker(const Derived &d, double bm) {
 }
 
 // Prefilter record of one particle: px, py, nrm = |pT|^2 - mid/2, and its
-// beta interval [blo, bhi] = beta -/+ cw with cw = (H/2) / E (or H/2
-// without the LCMS boost; infinite with the q_inv branch on): the beta test
-// |beta1 - beta2| <= cw1 + cw2 holds exactly when blo1 <= bhi2 and
-// blo2 <= bhi1.  The ends are rounded outward (blo down, bhi up), so the
-// two comparisons pass every pair the real-valued test passes.  The kernel
-// uses the FP32 records (pf_make, on the device).
+// longitudinal interval [blo, bhi] (long_window): the test |y1 - y2| <= cw1 +
+// cw2 holds exactly when blo1 <= bhi2 and blo2 <= bhi1.  The ends are rounded
+// outward (blo down, bhi up), so the two comparisons pass every pair the
+// real-valued test passes.  The kernel uses the FP32 records (pf_make, on the
+// device).
 inline void pf_record(const Derived &d, double px, double py, double pz, double E, double bm,
                       PfRec64 &r, double &bhi) {
-    const DevParams &P = d.P;
-    const double beta = P.boost ? pz / E : pz;
-    const double cw = P.qinv ? INFINITY : (P.boost ? d.c_beta / E : d.c_beta);
-    r = PfRec64{px, py, px * px + py * py - 0.5 * d.mid, std::nextafter(beta - cw, -INFINITY)};
-    bhi = std::nextafter(beta + cw, INFINITY);
+    const LongWindow w = long_window(pf_maker(d, bm), pz, E, 1.1102230246251565e-16);
+    r = PfRec64{px, py, px * px + py * py - 0.5 * d.mid, std::nextafter(w.y - w.cw, -INFINITY)};
+    bhi = std::nextafter(w.y + w.cw, INFINITY);
 }
 
 inline void pf_record(const Derived &d, double px, double py, double pz, double E, double bm,
