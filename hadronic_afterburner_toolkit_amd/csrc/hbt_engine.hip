@@ -541,7 +541,10 @@ void free_slot(Slot &s) {
 }
 
 void drop_graph(hbt_ctx *c) {
-    if (c->graph_exec) hipGraphExecDestroy(c->graph_exec);
+    if (c->graph_exec) {
+        hipStreamSynchronize(c->stream);  // a launch of it may still run
+        hipGraphExecDestroy(c->graph_exec);
+    }
     if (c->graph) hipGraphDestroy(c->graph);
     c->graph_exec = nullptr;
     c->graph = nullptr;
@@ -961,7 +964,7 @@ struct ItemList {
 };
 
 // Work items: same-event tiles of every group, then mixed tiles of every
-// event.  Same: i tile of 64R particles x j chunk of its px window.
+// event.  Same: i tile of 64 particles x j chunk of its px window.
 // Mixed: i tile x up to kchunk partner windows of the event's plan rows.
 // enum_same receives the reference's same-event pair count; the mixed
 // count is known from the plan (upload_plan).

@@ -4,8 +4,8 @@
 // Every binned pair is one read-modify-write of a random 64-byte bin.  Done
 // as a device-scope atomic, each such access is executed at the memory side
 // of this part at about 2.35e10 per second for the whole chip, whatever the
-// histogram's size or placement: that rate, not arithmetic, bounds the fast
-// kernel.  The histogram (qnpts^3 bins per K_T bin, tens of MB) cannot live
+// histogram's size or placement: without slabs that rate, not arithmetic, bounds
+// the fast kernel.  The histogram (qnpts^3 bins per K_T bin, tens of MB) cannot live
 // in LDS, and a block's binned pairs land in random bins, so there is
 // nothing to combine inside one block.  Instead, for same-event pairs:
 //
@@ -28,8 +28,9 @@
 //     histogram, plain read-modify-write: each bin has one owner.
 //
 // Mixed pairs add one u32 to the denominator directly: their atomic is the
-// cheaper pattern, and a 2-byte record store per pair measured costlier than
-// it.
+// cheaper pattern and hidden under the kernel's arithmetic.  As 2-byte records
+// counted in LDS by a kernel of their own they took 2 % off the headline
+// batch's precision form and nothing off its FP64 form.
 //
 // In slab mode the precision form's per-pair values are FP32 (records and
 // the direct path alike), accumulated in FP64; without slab binning they

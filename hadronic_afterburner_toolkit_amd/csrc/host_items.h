@@ -27,7 +27,7 @@ struct JWin {
 struct WorkItem {
     long long i0;   // first i particle (same-event: cell-sorted list, mixed: fast list)
     long long j0;   // same-event: first j particle; mixed: first window (View::mwin)
-    int ni;         // number of i particles (<= 64*R)
+    int ni;         // number of i particles (<= 64)
     int nj;         // same-event: number of j particles; mixed: number of windows
     int kind;       // 0 same-event, 1 mixed
     int grp;        // group (buffer) of the pair, selects psi_ref
@@ -36,7 +36,7 @@ struct WorkItem {
 
 // Launch shape of the fast kernel's work items.
 struct ItemShape {
-    int TI;  // i particles per item (64 R)
+    int TI;  // i particles per item (64)
     int JC;  // same-event j chunk
     int KC;  // mixed partner windows per item
 };

@@ -220,8 +220,9 @@ int hbt_prepare_batch(hbt_ctx *ctx, const int32_t *M_per_group, const int32_t *p
 /* Enqueues the prepared batch on the context's stream (asynchronous).
  * Launches may be queued back to back.  An upload, hbt_prepare_batch,
  * hbt_run_same/mixed, hbt_set_psi_ref or a tuning change issued before
- * hbt_sync first waits for the queued launches, which therefore see the
- * data they were launched on. */
+ * hbt_sync waits for the queued launches, or (an upload of one small buffer)
+ * queues its device work behind them: they see the data they were launched
+ * on.  An upload has copied the caller's arrays when it returns. */
 int hbt_launch_batch(hbt_ctx *ctx);
 
 /* Waits for the context's stream; *batch_ms (may be NULL) receives the
@@ -229,7 +230,9 @@ int hbt_launch_batch(hbt_ctx *ctx);
 int hbt_sync(hbt_ctx *ctx, double *batch_ms);
 
 /* Pairs enumerated by one launch of the prepared batch (same-event
- * sum N_g(N_g-1)/2, mixed sum N_e * sum N_partner) and its work items. */
+ * sum N_g(N_g-1)/2, mixed sum N_e * sum N_partner) and its work items (an
+ * upper bound where hbt_calculate_buffer ran one buffer on lists gathered on
+ * the device). */
 int hbt_batch_info(hbt_ctx *ctx, uint64_t *enum_same, uint64_t *enum_mixed, int32_t *nitems);
 
 /* How hbt_launch_batch issues the prepared batch: *graph = 1 when it
@@ -291,8 +294,8 @@ int hbt_calculate_noalloc(const hbt_config *cfg, int32_t nev, int64_t n_particle
                           double *bins, void *stream);
 const char *hbt_noalloc_last_error(void);
 
-/* Launch shape of the fast kernel: R i-particles per lane (1, 2, 4), j
- * chunk of same-event tiles, partner windows per mixed work item (one per
+/* Launch shape of the fast kernel: R (1, 2, 4; accepted and kept, every tile
+ * holds 64 i particles), j chunk of same-event tiles, partner windows per mixed work item (one per
  * plan row whose partner has particles in the tile's |pT| window),
  * persistent blocks per CU; ms is the measured batch time when set by
  * hbt_autotune. */
