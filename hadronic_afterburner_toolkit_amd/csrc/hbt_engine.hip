@@ -753,9 +753,18 @@ View make_view(hbt_ctx *c) {
 
 // Kernel arguments of the context's own launches: one view (index 0),
 // copied to the device before the launch (and before a graph capture).
+
+// A CU holds four blocks (LDS and registers), three of the FP64 K_phi / q_inv
+// instance.  A launch of more (blocks_per_cu above that) starts the others when
+// the queue is empty: they bin nothing, but each has its share of the slab
+// regions, so the working blocks' regions were half as large under the same
+// budget and more pairs went past them.  Headline batch at eight blocks per CU
+// (results included): 6.76 ms, its first launch 13.4, and half of it in FP64
+// 7.51 and 10.1; now 6.62, 7.9, 5.51 and 6.2.
 long fast_blocks(const hbt_ctx *c, int nitems) {
-    return std::max(1l, std::min<long>((long)c->cu_count * c->tune.blocks_per_cu,
-                                       ((long)nitems + 3) / 4));
+    const bool ext64 = c->P.qinv || (c->P.azimuthal && c->cfg.precision != HBT_PREC_FP32C);
+    const long per_cu = std::min(c->tune.blocks_per_cu, ext64 ? 3 : 4);
+    return std::max(1l, std::min<long>((long)c->cu_count * per_cu, ((long)nitems + 3) / 4));
 }
 
 // Reads the demand the last slab-binned launch measured (after the stream
