@@ -9,8 +9,8 @@
 // exact cascade, 64 at a time.  There are no momentum windows, so it tests
 // about five times the pairs that k_fast does on sorted lists, at 0.6 ps each;
 // below some 4e9 enumerated pairs the adds' atomics hide that (20 events of
-// 600 particles, 1.5e8 pairs: 140 us against k_fast's 195; of 1500 particles,
-// 9.5e8: 712 against 695; 10 of 4000, 1.8e9: 1225 against 1310), and sorting,
+// 600 particles, 1.5e8 pairs: 151 us against k_fast's 190; of 1500 particles,
+// 9.5e8: 718 against 670; 10 of 4000, 1.8e9: 1245 against 1200), and sorting,
 // windows and items on the host cost several times the kernel.
 #pragma once
 #include "hbt_fast.h"

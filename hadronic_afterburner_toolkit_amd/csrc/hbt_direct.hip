@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void k_gather_compact(GatherArgs g) {
 }
 
 // The same in one launch for a small buffer: one block, each thread a run of
-// consecutive particles (630 particles: a call of 32 us, of which a second
+// consecutive particles (630 particles: a call of 35 us, of which a second
 // launch would be a large part; 4000: 33 us against 18 with a block per event).
 __global__ __launch_bounds__(1024) void k_gather_small(GatherArgs g) {
     __shared__ int sc[1024];

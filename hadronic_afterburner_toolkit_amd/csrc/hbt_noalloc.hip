@@ -11,7 +11,7 @@
 // One literal cascade per enumerated pair, one thread per i particle (the
 // form before), cost 1420 us for 20 events of 600 particles (1.5e8 pairs) and
 // 335 us for 7 of 90, whose few threads each walked hundreds of pairs one
-// after the other; this form takes 168 (140 of them the pair kernel) and 32.
+// after the other; this form takes 175 (151 of them the pair kernel) and 35.
 //
 // Calls on one GPU share its scratch array: calls that overlap on one GPU
 // (two streams, two host threads) race and must be serialized by the caller.
