@@ -339,7 +339,7 @@ hipError_t launch_gather(const GatherArgs &g, long long n, hipStream_t st) {
 hipError_t launch_pairs(const PairArgs &p, bool f32, bool ext, hipStream_t st) {
     if (p.nitems <= 0) return hipSuccess;
     const dim3 blocks((unsigned)std::min<long long>((p.nitems + 3) / 4, 2 * kWaves / 4));
-    const size_t dyn = fast_dynamic_lds(p.f.slab, ext, p.f.qinv_lds);
+    const size_t dyn = fast_dynamic_lds(0, ext, p.f.qinv_lds);
     // (with the q_inv branch on every pair takes the literal cascade)
     f32 = f32 && !p.v.P.qinv;
     if (f32 && ext) hipLaunchKernelGGL((k_pairs<float, true>), blocks, dim3(256), dyn, st, p);

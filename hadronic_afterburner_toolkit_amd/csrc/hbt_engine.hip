@@ -751,20 +751,26 @@ View make_view(hbt_ctx *c) {
     return v;
 }
 
-// Kernel arguments of the context's own launches: one view (index 0),
-// copied to the device before the launch (and before a graph capture).
-
-// A CU holds four blocks (LDS and registers), three of the FP64 K_phi / q_inv
-// instance.  A launch of more (blocks_per_cu above that) starts the others when
-// the queue is empty: they bin nothing, but each has its share of the slab
-// regions, so the working blocks' regions were half as large under the same
-// budget and more pairs went past them.  Headline batch at eight blocks per CU
-// (results included): 6.76 ms, its first launch 13.4, and half of it in FP64
-// 7.51 and 10.1; now 6.62, 7.9, 5.51 and 6.2.
-long fast_blocks(const hbt_ctx *c, int nitems) {
-    const bool ext64 = c->P.qinv || (c->P.azimuthal && c->cfg.precision != HBT_PREC_FP32C);
-    const long per_cu = std::min(c->tune.blocks_per_cu, ext64 ? 3 : 4);
-    return std::max(1l, std::min<long>((long)c->cu_count * per_cu, ((long)nitems + 3) / 4));
+// Blocks per CU of a launch of the fast kernel: blocks_per_cu, and no more than
+// a CU holds (the instance's registers and its LDS: four, three of the FP64
+// K_phi / q_inv instance and of a slab-binned K_phi launch of more than 1248
+// slabs).  A launch of more starts the others when the queue is empty: they bin
+// nothing, but each has its share of the slab regions, so the working blocks'
+// regions were smaller under the same budget and more pairs went past them.
+// Headline batch at eight blocks per CU (results included): 6.76 ms, its first
+// launch 13.4, and half of it in FP64 7.51 and 10.1; now 6.62, 7.9, 5.51 and
+// 6.2.  A quarter of it in 16 K_phi bins (3936 slabs), the kernels: 5.73 ms at
+// four blocks a CU, 3.15 at the three that fit.
+int blocks_per_cu(const hbt_ctx *c, bool f32, bool slab) {
+    const bool ext = c->P.qinv || c->P.azimuthal;
+    f32 = f32 && !c->P.qinv;
+    const int slabs = slab ? c->cfg.n_KT * c->P.nphi * c->P.qnpts : 0;
+    return std::min(c->tune.blocks_per_cu,
+                    fast_resident_blocks(f32, ext, fast_dynamic_lds(slabs, ext, qinv_lds_bins(c->P))));
+}
+long fast_blocks(const hbt_ctx *c, int nitems, bool f32, bool slab) {
+    return std::max(1l, std::min<long>((long)c->cu_count * blocks_per_cu(c, f32, slab),
+                                       ((long)nitems + 3) / 4));
 }
 
 // Reads the demand the last slab-binned launch measured (after the stream
@@ -843,8 +849,8 @@ int slab_prepare(hbt_ctx *c, int nitems) {
     const int S = c->cfg.n_KT * c->P.nphi * q, SB = q * q;
     sl.on = c->slab_binning && slab_applies(c) && nitems > 0;
     if (!sl.on) return HBT_OK;
-    const int nblk = (int)fast_blocks(c, nitems);
     const bool f32 = c->cfg.precision == HBT_PREC_FP32C;
+    const int nblk = (int)fast_blocks(c, nitems, f32, true);
     const size_t vsz = f32 ? 16 : 32;
     if (sl.S != S) sl.have_hist = false;
     sl.S = S;
@@ -895,6 +901,8 @@ int slab_prepare(hbt_ctx *c, int nitems) {
     return HBT_OK;
 }
 
+// Kernel arguments of the context's own launches: one view (index 0),
+// copied to the device before the launch (and before a graph capture).
 int fast_args(hbt_ctx *c, FastArgs &a) {
     set_prefilter_margins(c);
     const View v = make_view(c);
@@ -933,9 +941,9 @@ int fast_args(hbt_ctx *c, FastArgs &a) {
 // The fast kernel, and with slab binning its two binning kernels, queued on
 // st (kernel launches only: this runs inside a graph capture).
 int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st) {
-    const long blocks = fast_blocks(c, a.nitems);
     const bool f32 = c->cfg.precision == HBT_PREC_FP32C;
     const bool slab = a.slab.vals != nullptr;
+    const long blocks = fast_blocks(c, a.nitems, f32, slab);
     if (slab) {
         if (blocks != c->slab.nblk)
             return fail(c, HBT_ERR_STATE, "slab regions sized for another launch shape");
@@ -1548,8 +1556,8 @@ TrialLaunch trial_fast(hbt_ctx *c, FastArgs a) {
     return [c, a](unsigned long long *binned) mutable -> hipError_t {
         a.binned = binned;
         if (a.nitems <= 0) return hipSuccess;
-        return launch_fast_kernel(a, false, c->P.qinv || c->P.azimuthal, fast_blocks(c, a.nitems),
-                                  c->stream);
+        return launch_fast_kernel(a, false, c->P.qinv || c->P.azimuthal,
+                                  fast_blocks(c, a.nitems, false, false), c->stream);
     };
 }
 
@@ -1916,7 +1924,7 @@ hipError_t launch_fast_kernel(const FastArgs &a, bool f32, bool ext, long blocks
                               hipStream_t st) {
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, a.counter, a.nqueues);
     if (a.slab.vals && a.slab.S > (ext ? kMaxSlabsKphi : kMaxSlabs)) return hipErrorInvalidValue;
-    const size_t dyn = fast_dynamic_lds(a.slab, ext, a.qinv_lds);
+    const size_t dyn = fast_dynamic_lds(a.slab.vals ? a.slab.S : 0, ext, a.qinv_lds);
 #define HBT_LAUNCH(T, X) \
     hipLaunchKernelGGL((k_fast<T, X>), dim3(blocks), dim3(256), dyn, st, a)
     // (with the q_inv branch on every pair takes the literal cascade)

@@ -30,6 +30,8 @@
 // every j by +theta (T, dn, C and y are rotation invariant); the exact
 // cascade then uses the reference's rotated j (HBT_correlation.cpp:522-523).
 #pragma once
+#include <algorithm>
+
 #include "hbt_device.h"
 #include "hbt_f32.h"
 #include "hbt_slab.h"
@@ -835,9 +837,20 @@ inline int qinv_lds_bins(const DevParams &P) {
     const int nq = P.n_KT * P.qnpts;
     return P.qinv && nq <= kMaxQinvLds ? nq : 0;
 }
-inline size_t fast_dynamic_lds(const SlabArgs &s, bool ext, int qinv_lds) {
+// slabs: of a slab-binned launch, else 0.
+inline size_t fast_dynamic_lds(int slabs, bool ext, int qinv_lds) {
     return qinv_lds ? 4 * sizeof(Stage) + kQinvBytes * qinv_lds
-           : s.vals ? (size_t)s.S * sizeof(unsigned) * (ext ? 1 : 2) : 4 * sizeof(Stage);
+           : slabs  ? (size_t)slabs * sizeof(unsigned) * (ext ? 1 : 2) : 4 * sizeof(Stage);
+}
+// Blocks of an instance that a CU holds at once: as many as its registers
+// leave room for (a block has one wave on each of the four SIMDs), and its LDS,
+// which is handed out in steps of 1280 bytes.
+constexpr size_t kCuLds = 160 * 1024, kLdsStep = 1280;
+inline int fast_resident_blocks(bool f32, bool ext, size_t dynamic_lds) {
+    const size_t steps = (4 * sizeof(WaveLds) + dynamic_lds + kLdsStep - 1) / kLdsStep;
+    const int waves = f32 ? fast_waves_per_eu<float, true>()
+                      : ext ? fast_waves_per_eu<double, true>() : fast_waves_per_eu<double, false>();
+    return std::min(waves, (int)(kCuLds / kLdsStep / steps));
 }
 
 // The block's q_inv histograms: cleared at the kernel's start (null: none), and
