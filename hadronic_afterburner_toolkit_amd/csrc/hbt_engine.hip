@@ -1027,13 +1027,11 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
     const Slot &s = c->slot[0];
     ItemShape sh = item_shape(c->tune);
     const double D = px_window(c->D);
-    // a launch with fewer items than kItemsPerWave per resident wave (one
-    // buffer of the per-buffer path, a small request) leaves most waves idle
-    // and ends on its largest item: its j chunks and partner windows per item
-    // shrink (to 64 j's and one window at most) until it has enough
-    const size_t waves = (size_t)std::max(1, c->cu_count) * (size_t)c->tune.blocks_per_cu * 4;
+    const bool f32 = c->cfg.precision == HBT_PREC_FP32C;
+    const size_t waves = (size_t)std::max(1, c->cu_count) * 4 *
+                         (size_t)blocks_per_cu(c, f32, c->slab_binning && slab_applies(c));
     std::vector<uint64_t> pairs;
-    for (;;) {
+    auto build = [&]() {
         L.items.clear();
         L.wins.clear();
         pairs.clear();
@@ -1046,14 +1044,28 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
             items_mixed(sh, s.foff, s.grp_ev, c->rowoff, c->plan_gids, m.foff, s.f_pt.data(),
                         m.f_pt.data(), pt_window(c->D), 0, L.items, L.wins, &pairs);
         }
-        const size_t want = kItemsPerWave * waves;
-        if (L.items.size() >= want || (sh.JC <= 64 && sh.KC <= 1)) break;
-        // items grow about inversely with the chunk sizes: one rebuild with
-        // both cut by the missing factor (rounded up to a power of two)
-        int f = 2;
-        while ((size_t)f * L.items.size() < want && f < 64) f *= 2;
-        sh.JC = std::max(64, sh.JC / f);
-        sh.KC = std::max(1, sh.KC / f);
+    };
+    build();
+    // a launch with fewer items than kItemsPerWave per resident wave (one
+    // buffer of the per-buffer path, a small request) leaves most waves idle
+    // and ends on its largest item: its j chunks and partner windows per item
+    // are halved (to 64 j's and one window at most) until the items' own sizes
+    // say that there are enough, and the items built once more (a build of
+    // three groups of 50 events of 600 particles takes 0.4 ms of host time, the
+    // batch 0.4 to 1.8 on the device)
+    const size_t want = kItemsPerWave * waves;
+    if (L.items.size() < want && (sh.JC > 64 || sh.KC > 1)) {
+        size_t n = 0;
+        while (n < want && (sh.JC > 64 || sh.KC > 1)) {
+            sh.JC = std::max(64, sh.JC / 2);
+            sh.KC = std::max(1, sh.KC / 2);
+            n = 0;
+            for (const WorkItem &w : L.items) {
+                const int per = w.kind == 0 ? sh.JC : sh.KC;
+                n += (size_t)((w.nj + per - 1) / per);
+            }
+        }
+        build();
     }
     // larger items first, by factor-4 size classes (stable inside a class,
     // which keeps a group's items together): the persistent waves pull items
@@ -2383,7 +2395,9 @@ int hbt_autotune(hbt_ctx *c, hbt_tuning *best_out) {
     // enough items to fill the chip; large ones amortize the per-item setup
     const int JCs[] = {256, 1024, 4096};
     const int KCs[] = {1, 4, 16};
-    const int BPCs[] = {4, 8, 16};
+    // blocks per CU: as many as it holds (more do not start together, fewer leave
+    // it idle)
+    constexpr int kBlocks = 4;
     // One timed launch per candidate is noisy (a few %), so the fastest few
     // candidates of the sweep are timed again, kRetime launches each, and
     // the lowest median wins.
@@ -2403,22 +2417,21 @@ int hbt_autotune(hbt_ctx *c, hbt_tuning *best_out) {
         return upload_items(c, items);
     };
     for (int jc : JCs)
-        for (int kc : KCs)
-            for (int bpc : BPCs) {
-                const hbt_tuning t{1, jc, kc, bpc, 0.0};
-                int rc = use(t, c->slab_binning);
+        for (int kc : KCs) {
+            const hbt_tuning t{1, jc, kc, kBlocks, 0.0};
+            int rc = use(t, c->slab_binning);
+            if (rc) return rc;
+            for (int m = 0; m < (both ? 2 : 1); m++) {
+                if (both) c->slab_binning = m == 1;
+                float ms = 0.f;
+                rc = timed_fast(c, &ms);
+                if (!rc) rc = timed_fast(c, &ms);
                 if (rc) return rc;
-                for (int m = 0; m < (both ? 2 : 1); m++) {
-                    if (both) c->slab_binning = m == 1;
-                    float ms = 0.f;
-                    rc = timed_fast(c, &ms);
-                    if (!rc) rc = timed_fast(c, &ms);
-                    if (rc) return rc;
-                    hbt_tuning tm = t;
-                    tm.ms = ms;
-                    cands.push_back(Cand{tm, c->slab_binning});
-                }
+                hbt_tuning tm = t;
+                tm.ms = ms;
+                cands.push_back(Cand{tm, c->slab_binning});
             }
+        }
     std::sort(cands.begin(), cands.end(),
               [](const Cand &x, const Cand &y) { return x.t.ms < y.t.ms; });
     constexpr int kFinalists = 4, kRetime = 5;
@@ -2445,6 +2458,9 @@ int hbt_autotune(hbt_ctx *c, hbt_tuning *best_out) {
     }
     c->tune = best;
     c->slab_binning = best_slab;
+    c->tune.blocks_per_cu =
+        blocks_per_cu(c, c->cfg.precision == HBT_PREC_FP32C, best_slab);  // as launched
+    best = c->tune;
     int rc = prepare_and_capture(c);
     if (!rc) rc = zero_hist(c);
     if (rc) return rc;

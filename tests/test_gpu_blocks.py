@@ -49,3 +49,29 @@ def test_no_more_blocks_than_a_cu_holds(prec, nphi, blocks):
         same, items, cap = measured(per_cu)
         assert items >= 4 * 4 * cus  # items for every block
         assert cap == capacity(cus * min(per_cu, blocks)), per_cu
+
+
+@pytest.mark.parametrize("prec,nphi,blocks", [(_lib.HBT_PREC_FP32C, 0, 4),
+                                              (_lib.HBT_PREC_FP64, 3, 3)])
+def test_items_and_autotuner_follow_the_blocks_that_run(prec, nphi, blocks):
+    """A small batch is cut into items for the waves that run, and hbt_autotune
+    reports a number of blocks that it launched."""
+    params = dict(qnpts=21, q_min=-0.15, q_max=0.15, n_KT=4, KT_min=0.2, KT_max=0.7,
+                  HBTrap_min=-1.0, HBTrap_max=1.0, needed_number_of_pairs=1e18,
+                  azimuthal_flag=int(nphi > 0), n_Kphi=max(1, nphi))
+    buf = samples.generate(9, 60, 300.0)
+    bufs = [buf.events(e, 20) for e in (0, 20, 40)]
+    plans = [hbt.Random(k).draw_plan(20, 20, 60) for k in range(3)]
+    items = {}
+    for per_cu in (blocks, 8, 16):
+        g = hbt.HBTCorrelation(params, precision=prec)
+        g.set_tuning(1, 1024, 8, per_cu)
+        g.upload_groups(bufs)
+        g.prepare_batch(np.array([p[0] for p in plans], np.int32),
+                        np.concatenate([p[1] for p in plans]),
+                        np.concatenate([p[2] for p in plans]))
+        items[per_cu] = g.batch_info()[2]
+        if per_cu == 16:
+            assert g.autotune()["blocks_per_cu"] == blocks
+        g.close()
+    assert items[blocks] == items[8] == items[16]
