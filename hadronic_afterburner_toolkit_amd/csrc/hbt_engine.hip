@@ -1491,7 +1491,8 @@ int run_capped(hbt_ctx *c, bool mixed, const int *d_flag = nullptr) {
 // 0.40 ms against 3.75 with the ordered passes alone, 0.43 against 3.6 with
 // every key past the cap before it, 3.6 against 11.2 when every key passes it
 // (of which the position search took 7, one pair after the other).  A copy that
-// cannot be allocated leaves the ordered passes.
+// cannot be allocated leaves the ordered passes, and so do more K_phi edge pairs
+// than the deferral buffer holds.
 // launch: queues the call's FP64 launch, its binned counts at the address
 // passed; side: the same-event and the mixed side.
 using TrialLaunch = std::function<hipError_t(unsigned long long *binned)>;
@@ -1525,6 +1526,23 @@ int run_trial(hbt_ctx *c, const TrialLaunch &launch, const CapSide side[2], bool
     for (int f = 0; f < 4 && nq; f++)
         HIPCHECK(c, hipMemcpyAsync(snap_q + f * nq, q[f], nq * 8, hipMemcpyDeviceToDevice, st));
     HIPCHECK(c, launch((unsigned long long *)(snap_q + 4 * nq)));
+    if (c->P.azimuthal) {
+        // both sides at once may leave the host more K_phi edge pairs than the
+        // buffer holds, where each side by itself does not: then the trial is
+        // undone
+        unsigned n = 0;
+        HIPCHECK(c, hipMemcpyAsync(&n, c->d_ndefer, sizeof(n), hipMemcpyDeviceToHost, st));
+        HIPCHECK(c, hipStreamSynchronize(st));
+        if (n > kDeferCap) {
+            HIPCHECK(c, hipMemcpyAsync(c->d_bins, c->d_snap, bins * 8, hipMemcpyDeviceToDevice, st));
+            for (int f = 0; f < 4 && nq; f++)
+                HIPCHECK(c, hipMemcpyAsync((void *)q[f], snap_q + f * nq, nq * 8,
+                                           hipMemcpyDeviceToDevice, st));
+            HIPCHECK(c, hipMemsetAsync(c->d_ndefer, 0, sizeof(unsigned), st));
+            done = false;
+            return HBT_OK;
+        }
+    }
     rc = resolve_deferred(c);
     if (rc) return rc;
     const uint64_t deferred = c->deferred_total;
