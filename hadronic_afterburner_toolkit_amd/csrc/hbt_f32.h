@@ -12,7 +12,8 @@
 // near an edge, one whether all are in range.
 //
 // Bit-identical counts: every bin coordinate (K_T index, bin indices) is
-// within 1e-9 bins of the reference's; a pair with a coordinate within
+// within 1e-9 bins of the reference's, q_long within 1e-9 GeV besides
+// (kBoostMax); a pair boosted further, or with a coordinate within
 // the guard (DevParams::guard, which also covers the 1e-8 GeV between the
 // windows' cuts and the outer bin edges and the FP32 rounding of a record's
 // values) of an edge is re-run through the literal FP64 cascade
@@ -56,6 +57,13 @@ __device__ __forceinline__ double pair_cos_f32(const Params &P, const PartRec &p
     return cos_reduced_f32(P, P.hbarC_inv * (q_E * (p1.t - p2.t) - q_x * (p1.x - p2.x) -
                                              q_y * (p1.y - p2.y) - q_z * (p1.z - p2.z)));
 }
+
+// Largest (gamma beta)^2 of a pair's longitudinal boost whose q_long is taken
+// from here.  Its rounding, and that of the literal form, grow as gamma^2 2^-53
+// (the cancellations of M_t^2 = E^2 - p_z^2 and of q_z - beta q_E): below 1e-9
+// GeV up to gamma = 1000 (a rapidity of 7.6), 1e-5 at a rapidity of 13, where
+// 1e-4 of the pairs would fall into the next bin.
+constexpr double kBoostMax = 1e6;
 
 constexpr double GUARD_PHI = 4e-6;   // radians, around K_phi bin edges
 
@@ -104,8 +112,9 @@ __device__ __forceinline__ int cascade_fast(const Params &P, double p1x, double 
     b.q_side = fma(b.q_y, sx, -(b.q_x * sy)) * rK;
     b.q_long = b.q_z;
     if (P.boost) {  // gamma (q_z - beta q_E) = (K_E q_z - K_z q_E) / M_t
-        const double rM = rsqrt_refined(fma(sE, sE, -(sz * sz)));
-        b.q_long = fma(sE, b.q_z, -(sz * b.q_E)) * rM;
+        const double z2 = sz * sz, M2 = fma(sE, sE, -z2);
+        b.q_long = fma(sE, b.q_z, -(sz * b.q_E)) * rsqrt_refined(M2);
+        if (z2 > kBoostMax * M2) near = 0.0;
     }
     b.io = bin_coord(fma(b.q_out, P.inv_dq, P.q_off), near);
     b.is = bin_coord(fma(b.q_side, P.inv_dq, P.q_off), near);
