@@ -65,6 +65,7 @@ __device__ __forceinline__ double pair_cos_f32(const Params &P, const PartRec &p
 // 1e-4 of the pairs would fall into the next bin.
 constexpr double kBoostMax = 1e6;
 
+constexpr double kEdge = 1e-9;       // bins
 constexpr double GUARD_PHI = 4e-6;   // radians, around K_phi bin edges
 
 // A bin coordinate raised by one: its integer part, and its distance to the
@@ -92,8 +93,9 @@ __device__ __forceinline__ int kphi_index_fast(const Params &P, double K_x, doub
 }
 
 // The K/q cascade of the precision form.  Returns ST_BIN with the bins in b,
-// 0, or -1 or -2 when a decision is ambiguous (-2: only the K_phi bin is).  Works on 2K (the reference's K
-// times a power of two: its products round alike).
+// 0, or -1 or -2 when a decision is ambiguous (-2: the pair lies on an edge or a
+// cut to within kEdge bins, or misses only its K_phi bin: its cos is FP64's too).
+// Works on 2K (the reference's K times a power of two: its products round alike).
 template <bool EXT = false, typename Params>
 __device__ __forceinline__ int cascade_fast(const Params &P, double p1x, double p1y,
                                             double p1z, double p1E, double p2x, double p2y,
@@ -119,7 +121,8 @@ __device__ __forceinline__ int cascade_fast(const Params &P, double p1x, double 
     b.io = bin_coord(fma(b.q_out, P.inv_dq, P.q_off), near);
     b.is = bin_coord(fma(b.q_side, P.inv_dq, P.q_off), near);
     b.il = bin_coord(fma(b.q_long, P.inv_dq, P.q_off), near);
-    if (near < P.guard) return -1;
+    if (near < P.guard)
+        return near < kEdge || fabs(near - 1e-8 * P.inv_dq) < kEdge ? -2 : -1;
     const unsigned q = max(max((unsigned)b.io, (unsigned)b.is), (unsigned)b.il);
     // (the last K_T index, n_KT - 1, holds only K_perp = KT_max: near an edge)
     if (q >= (unsigned)P.qnpts || (unsigned)b.kt >= (unsigned)(P.n_KT - 1)) return 0;

@@ -441,14 +441,14 @@ struct Stage {
 // about 2.4e10 per second whatever the histogram's size or placement, so
 // the count is an FP64 add in the same instruction as the sums: one access
 // per binned pair.
-// unsure: the lanes whose pair the precision form could not decide, unsure_phi
-// those of them that miss only their K_phi bin.
+// unsure: the lanes whose pair the precision form could not decide, cos64 those
+// of them whose cos is taken from the literal form too.
 template <typename Prec, bool EXT, bool RANKED>
 __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, Stage &stg,
                                      unsigned head, int cnt, bool mixed, double psi,
                                      unsigned *next, const unsigned *lim, double *qlds,
                                      unsigned long long &direct_n, unsigned long long &unsure,
-                                     unsigned long long &unsure_phi) {
+                                     unsigned long long &cos64) {
     const int lane = __lane_id();
     int st = 0;
     SameRec rec;
@@ -465,7 +465,7 @@ __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, St
     }
     if (std::is_same<Prec, float>::value) {
         unsure = __ballot(st < 0);
-        if (EXT) unsure_phi = __ballot(st == -2);
+        if (__builtin_expect(unsure != 0ull, 0)) cos64 = __ballot(st == -2);
     }
     const bool binned = st > 0 && (st & ST_BIN) != 0;
     const int nbinned = __popcll(__ballot(binned));
@@ -784,14 +784,14 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
             const int take = (int)min(64u, n);
             __builtin_amdgcn_wave_barrier();
             CArgs *kd = kernel_args();
-            unsigned long long unsure = 0, unsure_phi = 0;
+            unsigned long long unsure = 0, cos64 = 0;
             int nb = drain<Prec, EXT, RANKED>(Views::at(kd, w.view), kd, wl, stg, head, take, mixed,
                                               psi, tot.slab_next, tot.slab_lim, tot.qlds, tot.direct,
-                                              unsure, unsure_phi);
+                                              unsure, cos64);
             if (std::is_same<Prec, float>::value && __builtin_expect(unsure != 0ull, 0)) {
                 kd = kernel_args();
                 nb += drain_literal<EXT, RANKED>(Views::at(kd, w.view), kd, wl, head, unsure,
-                                                 unsure_phi, mixed, psi, tot.direct);
+                                                 cos64, mixed, psi, tot.direct);
             }
             if (mixed)
                 tot.mixed += nb;
