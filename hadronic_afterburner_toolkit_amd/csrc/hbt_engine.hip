@@ -322,7 +322,7 @@ struct Slot {
     std::vector<int> grp_ev;       // ngroups+1
     std::vector<long long> off;    // nev+1, kept-particle offsets
     std::vector<double> psi2;      // psi_ref (n=2) per group, over all particles passed in
-    double *d_soa[8] = {};   // plain kernels (structure of arrays)
+    double *d_soa[8] = {};   // plain and ordered cap kernels (structure of arrays)
     long long *d_off = nullptr;
     // fast kernel: the fast list (particles whose |pT| can reach a K_T bin,
     // |pT|-sorted per event) and its (px cell, py)-sorted copy per group
@@ -331,6 +331,8 @@ struct Slot {
     hvec<double> f_pt;            // |pT| of the fast list (mixed windows)
     DevRecords ev, srt;
     bool lists = false;           // the host lists above and their device copies hold this upload
+    bool columns = false;         // and so do d_soa and d_off
+    bool gathered = false;        // and (a direct upload) list: its gather is queued
     // a buffer gathered on the device (hbt_direct.h): its particles as passed
     // in, in pinned memory (two, in turn: the copy of the last upload may
     // still run) and on the device, each eight columns, then the offsets
@@ -969,9 +971,10 @@ int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st) {
     return HBT_OK;
 }
 
-// The host's lists of buffers that were gathered on the device, for the paths
-// that walk them.
+// What an upload that the device gathers leaves undone until a path asks for
+// it: the host's lists, the columns in gather order.
 int need_lists(hbt_ctx *c);
+int need_columns(hbt_ctx *c);
 
 struct ItemList {
     std::vector<WorkItem> items;
@@ -1230,7 +1233,7 @@ int timed_fast(hbt_ctx *c, float *ms) {
 
 // Plain kernels: one launch per group (same) and per group (mixed).
 int run_plain(hbt_ctx *c, bool same, bool mixed) {
-    if (int rc0 = need_lists(c)) return rc0;
+    if (int rc0 = need_columns(c)) return rc0;
     Slot &s = c->slot[0];
     const Slot &m = mixed_slot(c);
     DevHist H = hist_view(c);
@@ -1364,7 +1367,7 @@ int cap_defer_bin(hbt_ctx *c, int nkey3, const CapDefer &dk) {
 
 // d_flag: bin only the keys marked CAP_CROSS there (null: all).
 int run_capped(hbt_ctx *c, bool mixed, const int *d_flag = nullptr) {
-    int rc0 = need_lists(c);
+    int rc0 = need_columns(c);
     if (!rc0) rc0 = quiesce(c);
     if (!rc0) rc0 = upload_psi(c);
     if (rc0) return rc0;
@@ -1665,39 +1668,21 @@ int prepare_and_capture(hbt_ctx *c) {
     return HBT_OK;
 }
 
-// First half of an upload, called from the gather once the kept particles
-// are known: waits for queued work, invalidates the slot, sizes its device
-// buffers, gathers the kept columns into the pinned staging buffer on
-// several threads and queues their copies (and the event offsets') on the
-// context's stream.
-int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
-                   const double *const soa[8], bool again) {
-    int rc = quiesce(c);
-    if (rc) return rc;
-    if (!again) {
-        drop_graph(c);
-        c->plan_valid = false;
-        s.valid = false;  // until every copy has succeeded
-        s.direct = false;
-    }
-    s.lists = false;
-    const long long n = h.n, nf = h.nf;
+// The kept columns in gather order, and the event offsets off, for the plain and
+// the ordered cap kernels: fill(column a's place in the pinned staging buffer)
+// writes them on several threads, then their copies are queued on the context's
+// stream.  The stream is idle on entry.
+int send_columns(hbt_ctx *c, Slot &s, long long n, int32_t nev, const std::vector<long long> &off,
+                 const std::function<void(double *const dst[8])> &fill) {
+    int rc = HBT_OK;
+    s.columns = false;
     if ((size_t)n > s.cap || !s.d_soa[0]) {
+        s.cap = 0;
         for (auto &p : s.d_soa) {
             rc = dev_alloc(c, &p, (size_t)n);
             if (rc) return rc;
         }
         s.cap = (size_t)n;
-    }
-    if ((size_t)nf > s.cap_f || !s.d_orig) {
-        for (DevRecords *r : {&s.ev, &s.srt}) {
-            if (!rc) rc = dev_alloc(c, &r->rec, (size_t)nf + kPfPad);
-            if (!rc) rc = dev_alloc(c, &r->pf, (size_t)nf + kPfPad);
-            if (!rc) rc = dev_alloc(c, &r->bw, (size_t)nf + kPfPad);
-        }
-        if (!rc) rc = dev_alloc(c, &s.d_orig, (size_t)nf + kPfPad);
-        if (rc) return rc;
-        s.cap_f = (size_t)nf;
     }
     if ((size_t)nev + 1 > s.cap_ev || !s.d_off) {
         rc = dev_alloc(c, &s.d_off, (size_t)nev + 1);
@@ -1708,20 +1693,53 @@ int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
     const size_t off_bytes = ((size_t)nev + 1) * 8;
     HIPCHECK(c, ensure_pinned(&c->h_stage, &c->stage_cap, 8 * col_bytes + stage_round(off_bytes)));
     char *stage = c->h_stage;
-    parallel_ranges(n, 1 << 15, [&](long long k0, long long k1) {
-        for (int a = 0; a < 8; a++) {
-            double *dst = reinterpret_cast<double *>(stage + a * col_bytes);
-            const double *src = soa[a];
-            for (long long k = k0; k < k1; k++) dst[k] = src[h.keep[k]];
-        }
-    });
+    double *dst[8];
+    for (int a = 0; a < 8; a++) dst[a] = reinterpret_cast<double *>(stage + a * col_bytes);
+    fill(dst);
     for (int a = 0; a < 8 && n > 0; a++)
-        HIPCHECK(c, hipMemcpyAsync(s.d_soa[a], stage + a * col_bytes, (size_t)n * 8,
-                                   hipMemcpyHostToDevice, c->stream));
-    std::memcpy(stage + 8 * col_bytes, h.off.data(), off_bytes);
+        HIPCHECK(c, hipMemcpyAsync(s.d_soa[a], dst[a], (size_t)n * 8, hipMemcpyHostToDevice,
+                                   c->stream));
+    std::memcpy(stage + 8 * col_bytes, off.data(), off_bytes);
     HIPCHECK(c, hipMemcpyAsync(s.d_off, stage + 8 * col_bytes, off_bytes, hipMemcpyHostToDevice,
                                c->stream));
+    s.columns = true;
     return HBT_OK;
+}
+
+// First half of an upload, called from the gather once the kept particles
+// are known: waits for queued work that may read the slot, sizes the lists'
+// device buffers and sends the columns.  again: the lists of an upload that the
+// device gathers; the columns wait for a path that reads them.
+int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
+                   const double *const soa[8], bool again) {
+    int rc = quiesce(c);
+    if (rc) return rc;
+    if (!again) {
+        drop_graph(c);
+        c->plan_valid = false;
+        s.valid = false;  // until every copy has succeeded
+        s.direct = s.gathered = s.columns = false;
+    }
+    s.lists = false;
+    const long long nf = h.nf;
+    if ((size_t)nf > s.cap_f || !s.d_orig) {
+        s.cap_f = 0;
+        for (DevRecords *r : {&s.ev, &s.srt}) {
+            if (!rc) rc = dev_alloc(c, &r->rec, (size_t)nf + kPfPad);
+            if (!rc) rc = dev_alloc(c, &r->pf, (size_t)nf + kPfPad);
+            if (!rc) rc = dev_alloc(c, &r->bw, (size_t)nf + kPfPad);
+        }
+        if (!rc) rc = dev_alloc(c, &s.d_orig, (size_t)nf + kPfPad);
+        if (rc) return rc;
+        s.cap_f = (size_t)nf;
+    }
+    if (again) return HBT_OK;
+    return send_columns(c, s, h.n, nev, h.off, [&](double *const dst[8]) {
+        parallel_ranges(h.n, 1 << 15, [&](long long k0, long long k1) {
+            for (int a = 0; a < 8; a++)
+                for (long long k = k0; k < k1; k++) dst[a][k] = soa[a][h.keep[k]];
+        });
+    });
 }
 
 // One buffer is gathered on the device where the pair kernel without windows
@@ -1736,48 +1754,23 @@ bool direct_upload(const hbt_ctx *c, int32_t ngroups, int32_t nev, const int64_t
            nev <= (1 << 14) && ev_off[nev] - ev_off[0] <= kDirectParticles;
 }
 
-// The upload of one buffer whose lists the device gathers: nothing waits for
-// the device, the copy and the gather queue behind the launches before.
+// The upload of one buffer whose lists the device gathers: its columns into
+// pinned memory, and the kept particles per event.  Nothing waits for the
+// device, and nothing is sent to it: which lists the call needs is not known yet.
 int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
                   const int64_t *ev_off, const double *const soa[8]) {
     Slot &s = c->slot[slot];
     std::string err;
     if (int rc = check_buffer(1, grp, nev, ev_off, soa, err)) return fail(c, rc, err);
     const long long o0 = ev_off[0], n_in = ev_off[nev] - o0;
-    const size_t col = stage_round((size_t)n_in * 8), off_bytes = ((size_t)nev + 1) * 8;
-    const size_t bytes = 8 * col + off_bytes;
+    const size_t col = stage_round((size_t)n_in * 8);
     drop_graph(c);
     c->plan_valid = false;
-    s.valid = s.direct = s.lists = false;
+    s.valid = s.direct = s.gathered = s.columns = s.lists = false;
     s.raw ^= 1;
-    int rc = next_pinned(c, &s.h_raw[s.raw], &s.raw_cap[s.raw], &s.raw_ev[s.raw], bytes);
+    int rc = next_pinned(c, &s.h_raw[s.raw], &s.raw_cap[s.raw], &s.raw_ev[s.raw],
+                         8 * col + ((size_t)nev + 1) * 8);
     if (rc) return rc;
-    const bool grow = (size_t)n_in > (size_t)s.list.cap || !s.list.rec;
-    const bool grow_ev = (size_t)nev > s.list_nev || !s.list.koff;
-    if (bytes > s.draw_cap || grow || grow_ev) {
-        rc = quiesce(c);
-        if (!rc && bytes > s.draw_cap) {
-            s.draw_cap = 0;
-            rc = dev_alloc(c, &s.d_raw, bytes);
-            if (!rc) s.draw_cap = bytes;
-        }
-        if (!rc && grow) {
-            s.list.cap = 0;
-            rc = dev_alloc(c, &s.list.rec, (size_t)n_in + kPfPad);
-            if (!rc) rc = dev_alloc(c, &s.list.pf, (size_t)n_in + kPfPad);
-            if (!rc) rc = dev_alloc(c, &s.list.bw, (size_t)n_in + kPfPad);
-            if (!rc) s.list.cap = (int)n_in;
-        }
-        if (!rc && grow_ev) {
-            s.list_nev = 0;
-            rc = dev_alloc(c, &s.list.koff, (size_t)nev + 1);
-            if (!rc) rc = dev_alloc(c, &s.list.stat, (size_t)nev);
-            if (!rc && !s.list.head) rc = dev_alloc(c, &s.list.head, 1);
-            if (!rc) s.list_nev = (size_t)nev;
-        }
-        if (rc) return rc;
-    }
-    // the columns into pinned memory, and the kept particles per event
     char *raw = s.h_raw[s.raw];
     int64_t *off = (int64_t *)(raw + 8 * col);
     for (int e = 0; e <= nev; e++) off[e] = ev_off[e] - o0;
@@ -1796,17 +1789,6 @@ int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
         }
     });
     for (int e = 0; e < nev; e++) s.off[e + 1] += s.off[e];
-    HIPCHECK(c, hipMemcpyAsync(s.d_raw, raw, bytes, hipMemcpyHostToDevice, c->stream));
-    HIPCHECK(c, hipEventRecord(s.raw_ev[s.raw], c->stream));
-    GatherArgs g{};
-    g.ev_off = (const long long *)(s.d_raw + 8 * col);
-    double *d[8];
-    for (int a = 0; a < 8; a++) d[a] = (double *)(s.d_raw + a * col);
-    g.in = DevSoA{d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7]};
-    gather_setup(c->D, c->cfg, g);
-    g.nev = nev;
-    g.out = s.list;
-    HIPCHECK(c, launch_gather(g, n_in, c->stream));
     s.ngroups = 1;
     s.grp_ev.assign(grp, grp + 2);
     s.nev = nev;
@@ -1819,7 +1801,60 @@ int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
     return HBT_OK;
 }
 
-// again: the lists of an upload that the device gathered; its plan, batch and
+// The device's lists of such an upload: the copy and the gather queue behind the
+// launches before.
+int gather_direct(hbt_ctx *c, Slot &s) {
+    if (s.gathered) return HBT_OK;
+    const long long n_in = s.n_in;
+    const size_t col = stage_round((size_t)n_in * 8);
+    const size_t bytes = 8 * col + ((size_t)s.nev + 1) * 8;
+    const bool grow = (size_t)n_in > (size_t)s.list.cap || !s.list.rec;
+    const bool grow_ev = (size_t)s.nev > s.list_nev || !s.list.koff;
+    if (bytes > s.draw_cap || grow || grow_ev) {
+        int rc = quiesce(c);
+        if (!rc && bytes > s.draw_cap) {
+            s.draw_cap = 0;
+            rc = dev_alloc(c, &s.d_raw, bytes);
+            if (!rc) s.draw_cap = bytes;
+        }
+        if (!rc && grow) {
+            s.list.cap = 0;
+            rc = dev_alloc(c, &s.list.rec, (size_t)n_in + kPfPad);
+            if (!rc) rc = dev_alloc(c, &s.list.pf, (size_t)n_in + kPfPad);
+            if (!rc) rc = dev_alloc(c, &s.list.bw, (size_t)n_in + kPfPad);
+            if (!rc) s.list.cap = (int)n_in;
+        }
+        if (!rc && grow_ev) {
+            s.list_nev = 0;
+            rc = dev_alloc(c, &s.list.koff, (size_t)s.nev + 1);
+            if (!rc) rc = dev_alloc(c, &s.list.stat, (size_t)s.nev);
+            if (!rc && !s.list.head) rc = dev_alloc(c, &s.list.head, 1);
+            if (!rc) s.list_nev = (size_t)s.nev;
+        }
+        if (rc) return rc;
+    }
+    HIPCHECK(c, hipMemcpyAsync(s.d_raw, s.h_raw[s.raw], bytes, hipMemcpyHostToDevice, c->stream));
+    HIPCHECK(c, hipEventRecord(s.raw_ev[s.raw], c->stream));
+    GatherArgs g{};
+    g.ev_off = (const long long *)(s.d_raw + 8 * col);
+    double *d[8];
+    for (int a = 0; a < 8; a++) d[a] = (double *)(s.d_raw + a * col);
+    g.in = DevSoA{d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7]};
+    gather_setup(c->D, c->cfg, g);
+    g.nev = s.nev;
+    g.out = s.list;
+    HIPCHECK(c, launch_gather(g, n_in, c->stream));
+    s.gathered = true;
+    return HBT_OK;
+}
+
+int gather_slots(hbt_ctx *c) {
+    int rc = gather_direct(c, c->slot[0]);
+    if (!rc && c->slot[1].valid) rc = gather_direct(c, c->slot[1]);
+    return rc;
+}
+
+// again: the lists of an upload that the device gathers; its plan, batch and
 // psi_ref stay.
 int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev, int32_t nev,
                 const int64_t *ev_off, const double *const soa[8], bool again = false) {
@@ -1876,30 +1911,59 @@ int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev
     return HBT_OK;
 }
 
+// The columns of a direct upload in pinned memory, as passed in.
+void raw_columns(const Slot &s, const double *soa[8], const int64_t **off) {
+    const size_t col = stage_round((size_t)s.n_in * 8);
+    const char *raw = s.h_raw[s.raw];
+    for (int a = 0; a < 8; a++) soa[a] = (const double *)(raw + a * col);
+    *off = (const int64_t *)(raw + 8 * col);
+}
+
 int need_lists(hbt_ctx *c) {
     for (int slot = 0; slot < 2; slot++) {
         Slot &s = c->slot[slot];
         if (!s.valid || s.lists) continue;
-        const size_t col = stage_round((size_t)s.n_in * 8);
-        const char *raw = s.h_raw[s.raw];
         const double *soa[8];
-        for (int a = 0; a < 8; a++) soa[a] = (const double *)(raw + a * col);
-        const std::vector<int64_t> off((const int64_t *)(raw + 8 * col),
-                                       (const int64_t *)(raw + 8 * col) + s.nev + 1);
+        const int64_t *off;
+        raw_columns(s, soa, &off);
         const std::vector<int32_t> grp(s.grp_ev.begin(), s.grp_ev.end());
-        if (int rc = upload_slot(c, slot, 1, grp.data(), s.nev, off.data(), soa, true)) return rc;
+        if (int rc = upload_slot(c, slot, 1, grp.data(), s.nev, off, soa, true)) return rc;
     }
     return HBT_OK;
 }
 
-// Both lists of the call were gathered on the device, and its pairs are few
+int need_columns(hbt_ctx *c) {
+    for (Slot &s : c->slot) {
+        if (!s.valid || s.columns) continue;
+        if (int rc = quiesce(c)) return rc;
+        const double *soa[8];
+        const int64_t *off;
+        raw_columns(s, soa, &off);
+        const double cut_max = tanh(c->cfg.HBTrap_max), cut_min = tanh(c->cfg.HBTrap_min);
+        const int rc = send_columns(c, s, s.n, s.nev, s.off, [&](double *const dst[8]) {
+            parallel_ranges(s.nev, std::max(1ll, 4096ll * s.nev / std::max(1ll, s.n_in)),
+                            [&](long long e0, long long e1) {
+                long long k = s.off[e0];
+                for (int64_t i = off[e0]; i < off[e1]; i++) {
+                    if (!rapidity_kept(soa[2][i], soa[3][i], cut_min, cut_max)) continue;
+                    for (int a = 0; a < 8; a++) dst[a][k] = soa[a][i];
+                    k++;
+                }
+            });
+        });
+        if (rc) return rc;
+    }
+    return HBT_OK;
+}
+
+// Both lists of the call can be gathered on the device, and its pairs are few
 // enough to be walked without windows.
 bool direct_call(const hbt_ctx *c, uint64_t pairs) {
     return c->slot[0].direct && mixed_slot(c).direct && !c->slab_binning && pairs <= kDirectPairs;
 }
 
-// The pair launch of a direct call: the same-event side, or the mixed side of M
-// plan rows an event, or both.
+// The pair launch of a direct call (its slots are gathered): the same-event side,
+// or the mixed side of M plan rows an event, or both.
 PairArgs direct_pairs(hbt_ctx *c, bool same, int M) {
     const Slot &s = c->slot[0], &m = mixed_slot(c);
     PairArgs p{};
@@ -1926,7 +1990,8 @@ uint64_t same_pairs(const Slot &s) {
 int prepare_direct(hbt_ctx *c, int M, const int32_t *ids, const double *cs) {
     const Slot &s = c->slot[0];
     uint64_t em = 0;
-    int rc = upload_plan(c, std::vector<int>((size_t)s.nev, M), ids, cs, em);
+    int rc = gather_slots(c);
+    if (!rc) rc = upload_plan(c, std::vector<int>((size_t)s.nev, M), ids, cs, em);
     if (rc) return rc;
     c->batch_pairs = direct_pairs(c, true, M);
     c->batch_enum_same = same_pairs(s);
@@ -2127,7 +2192,9 @@ int hbt_run_same(hbt_ctx *c) {
     ItemList items;
     uint64_t es = same_pairs(c->slot[0]);
     const bool direct = direct_call(c, es);
-    if (!direct) {
+    if (direct) {
+        if ((rc = gather_slots(c))) return rc;
+    } else {
         if ((rc = need_lists(c))) return rc;
         build_items(c, true, false, items, es);
     }
@@ -2202,7 +2269,7 @@ int hbt_run_mixed(hbt_ctx *c, int32_t M, const int32_t *partner_ids, const doubl
     const bool binds = side[1].binds;
     bool done = false;
     const bool direct = direct_call(c, em);
-    if (!direct && (rc = need_lists(c))) return rc;
+    if ((rc = direct ? gather_slots(c) : need_lists(c))) return rc;
     if (binds && direct) {
         rc = timed_trial(c, trial_direct(c, direct_pairs(c, false, M)), side, c->ev + 2,
                          &c->ms_mixed, done);
@@ -2672,6 +2739,17 @@ int hbt_calculate_buffer(hbt_ctx *c, hbt_rng *rng) {
     if (rc) return rc;
     Slot &s = c->slot[0];
     const Slot &m = mixed_slot(c);
+    // (the device gathers the lists while the host draws the plan, where they
+    // are needed whatever it draws)
+    if (direct) {
+        long long most = 0;
+        for (int e = 0; e < m.nev; e++) most = std::max(most, m.off[e + 1] - m.off[e]);
+        const int M = c->cfg.number_of_mixed_events > 0 ? c->cfg.number_of_mixed_events
+                                                        : m.nev / 2 + 1;
+        if (direct_call(c, same_pairs(s) + (uint64_t)s.n * (uint64_t)M * (uint64_t)most))
+            rc = gather_slots(c);
+        if (rc) return rc;
+    }
     std::vector<int32_t> Mg(s.ngroups, 0);
     std::vector<int32_t> ids;
     std::vector<double> cs;
