@@ -771,8 +771,7 @@ int blocks_per_cu(const hbt_ctx *c, bool f32, bool slab) {
                     fast_resident_blocks(f32, ext, fast_dynamic_lds(slabs, ext, qinv_lds_bins(c->P))));
 }
 long fast_blocks(const hbt_ctx *c, int nitems, bool f32, bool slab) {
-    return std::max(1l, std::min<long>((long)c->cu_count * blocks_per_cu(c, f32, slab),
-                                       ((long)nitems + 3) / 4));
+    return item_blocks(nitems, (long)c->cu_count * blocks_per_cu(c, f32, slab));
 }
 
 // Reads the demand the last slab-binned launch measured (after the stream
@@ -1051,15 +1050,21 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
     build();
     // a launch with fewer items than kItemsPerWave per resident wave (one
     // buffer of the per-buffer path, a small request) leaves most waves idle
-    // and ends on its largest item: its j chunks and partner windows per item
-    // are halved (to 64 j's and one window at most) until the items' own sizes
-    // say that there are enough, and the items built once more (a build of
-    // three groups of 50 events of 600 particles takes 0.4 ms of host time, the
-    // batch 0.4 to 1.8 on the device)
+    // and ends on its largest item, as does one of twice that of large items
+    // (8 groups of 50 events of 600 particles, 8e4 pairs an item: 4.5 ms, 4.2
+    // with half of that).  The j chunks and partner windows per item are halved
+    // (to 64 j's and one window at most) until the items' own sizes say that
+    // there are enough, and the items built once more (a build of three such
+    // groups takes 0.4 ms of host time).
     const size_t want = kItemsPerWave * waves;
-    if (L.items.size() < want && (sh.JC > 64 || sh.KC > 1)) {
-        size_t n = 0;
-        while (n < want && (sh.JC > 64 || sh.KC > 1)) {
+    uint64_t total = 0;
+    for (uint64_t v : pairs) total += v;
+    auto enough = [&](size_t n) {
+        return n >= 2 * want || (n >= want && total <= kLargeItem * (uint64_t)n) ||
+               (sh.JC <= 64 && sh.KC <= 1);
+    };
+    if (size_t n = L.items.size(); !enough(n)) {
+        while (!enough(n)) {
             sh.JC = std::max(64, sh.JC / 2);
             sh.KC = std::max(1, sh.KC / 2);
             n = 0;

@@ -514,8 +514,22 @@ inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
 
 // Work items per resident wave below which a launch's items are made smaller.
 constexpr size_t kItemsPerWave = 4;
+// Pairs of an item, on average over the launch, above which twice as many are made.
+constexpr uint64_t kLargeItem = 1 << 15;
 // L2 of one XCD (MI355X: 4 MB).
 constexpr size_t kL2BytesPerXcd = (size_t)4 << 20;
+
+// Blocks of a launch of `items` work items on at most `resident` of them: a wave
+// for every two items, or, up to 512 waves, for each.  A small launch is bound by
+// the queues' counters (a wave polls each queue once more before it ends, and
+// one counter takes some 1e8 adds a second): 8 groups of 8 events of 100
+// particles (3500 items) take 100 us with a wave for each item, 74 with one for
+// two, 20 events of 600 132 and 113, 4 groups of 10 of 60 54 and 46; 10 events of
+// 60 29 and 36.
+inline long item_blocks(long items, long resident) {
+    return std::max(1l, std::min(resident, std::max((items + 7) / 8,
+                                                    std::min((items + 3) / 4, 128l))));
+}
 
 // A tile is the 64 particles of a wave's four matrix blocks, whatever
 // t.R (its range of 1, 2 and 4 stays accepted): larger tiles would widen

@@ -511,9 +511,11 @@ void launcher_loop(hbt_server *s) {
             for (int q = 0; q <= kMaxQueues; q++) a.qoff[q] = q == 0 ? 0 : a.nitems;
             a.counter = s->d_counter;
             a.binned = s->d_misc + 16;
-            const long blocks = std::max(
-                1l, std::min<long>((long)s->cu_count * s->sc.tune.blocks_per_cu,
-                                   ((long)items.size() + 3) / 4));
+            const int per_cu =
+                std::min(s->sc.tune.blocks_per_cu,
+                         fast_resident_blocks(s->f32 && !s->D.P.qinv, s->ext,
+                                              fast_dynamic_lds(0, s->ext, 0)));
+            const long blocks = item_blocks((long)items.size(), (long)s->cu_count * per_cu);
             if (e == hipSuccess)
                 e = launch_fast_kernel(a, s->f32, s->ext, blocks, s->s_compute);
             if (e == hipSuccess) e = hipEventRecord(s->step_t1[buf], s->s_compute);

@@ -75,3 +75,23 @@ def test_items_and_autotuner_follow_the_blocks_that_run(prec, nphi, blocks):
             assert g.autotune()["blocks_per_cu"] == blocks
         g.close()
     assert items[blocks] == items[8] == items[16]
+
+
+@pytest.mark.parametrize("nev,mult,M", [(2, 30.0, 2), (10, 60.0, 5), (20, 100.0, 12), (40, 150.0, 12)])
+def test_a_small_launch_has_a_wave_for_two_items(nev, mult, M):
+    """Beyond 512 waves; up to them, a wave for each."""
+    params = dict(qnpts=21, q_min=-0.15, q_max=0.15, n_KT=4, KT_min=0.2, KT_max=0.7,
+                  HBTrap_min=-1.0, HBTrap_max=1.0, needed_number_of_pairs=1e18, hbt_binning=1)
+    bufs = [samples.generate(s, nev, mult) for s in range(3)]
+    plans = [hbt.Random(k).draw_plan(nev, nev, M) for k in range(3)]
+    g = hbt.HBTCorrelation(params)
+    g.upload_groups(bufs)
+    g.prepare_batch(np.array([M] * 3, np.int32), np.concatenate([p[1] for p in plans]),
+                    np.concatenate([p[2] for p in plans]))
+    same, _, items = g.batch_info()
+    capacity = g.slab_info()["capacity"]
+    g.close()
+    slabs = 4 * 21
+    blocks = max((items + 7) // 8, min((items + 3) // 4, 128))
+    assert blocks < 1024
+    assert capacity == (int(np.ceil(1.25 * (3.0 * 0.03 * same / slabs / blocks))) + 32) * slabs * blocks
