@@ -12,11 +12,11 @@
 // near an edge, one whether all are in range.
 //
 // Bit-identical counts: every bin coordinate (K_T index, bin indices) is
-// within 1e-9 bins of the reference's, q_long within 1e-9 GeV besides
-// (kBoostMax); a pair boosted further, or with a coordinate within
-// the guard (DevParams::guard, which also covers the 1e-8 GeV between the
-// windows' cuts and the outer bin edges and the FP32 rounding of a record's
-// values) of an edge is re-run through the literal FP64 cascade
+// within 1e-9 bins of the reference's, q_long within 1e-8 GeV besides; a pair
+// with a coordinate within the guard (DevParams::guard, which also covers the
+// 1e-8 GeV between the windows' cuts and the outer bin edges and the FP32
+// rounding of a record's values) of an edge, or of lists with particles of
+// larger boosts (boost_guard), is re-run through the literal FP64 cascade
 // (eval_*_f64), so bins and counts equal the reference's exactly.  The
 // accumulated q values carry ~1e-13 relative error, cos ~1e-7 absolute (FP32
 // in slab records); sums are accumulated in FP64 (atomics) or exact fixed
@@ -58,15 +58,21 @@ __device__ __forceinline__ double pair_cos_f32(const Params &P, const PartRec &p
                                              q_y * (p1.y - p2.y) - q_z * (p1.z - p2.z)));
 }
 
-// Largest (gamma beta)^2 of a pair's longitudinal boost whose q_long is taken
-// from here.  Its rounding, and that of the literal form, grow as gamma^2 2^-53
-// (the cancellations of M_t^2 = E^2 - p_z^2 and of q_z - beta q_E): below 1e-9
-// GeV up to gamma = 1000 (a rapidity of 7.6), 1e-5 at a rapidity of 13, where
-// 1e-4 of the pairs would fall into the next bin.
-constexpr double kBoostMax = 1e6;
-
-constexpr double kEdge = 1e-9;       // bins
 constexpr double GUARD_PHI = 4e-6;   // radians, around K_phi bin edges
+
+// Whether a pair's coordinates (literal, of a binned pair; T = 4 K_perp^2) lie on
+// a bin edge or a window's cut to within 1e-9 bins: its cos is then FP64's.
+template <typename Params>
+__device__ __forceinline__ bool on_edge(const Params &P, double T, const SameRec &r) {
+    const double w[4] = {fma(sqrt(T), P.kt_scale, P.kt_off), fma(r.qo, P.inv_dq, P.q_off),
+                         fma(r.qs, P.inv_dq, P.q_off), fma(r.ql, P.inv_dq, P.q_off)};
+    bool on = false;
+    for (int k = 0; k < 4; k++) {
+        const double d = fabs(w[k] - rint(w[k]));
+        on = on || d < 1e-9 || (k > 0 && fabs(d - 1e-8 * P.inv_dq) < 1e-9);
+    }
+    return on;
+}
 
 // A bin coordinate raised by one: its integer part, and its distance to the
 // nearest integer folded into the smallest so far.
@@ -93,8 +99,7 @@ __device__ __forceinline__ int kphi_index_fast(const Params &P, double K_x, doub
 }
 
 // The K/q cascade of the precision form.  Returns ST_BIN with the bins in b,
-// 0, or -1 or -2 when a decision is ambiguous (-2: the pair lies on an edge or a
-// cut to within kEdge bins, or misses only its K_phi bin: its cos is FP64's too).
+// 0, or -1 or -2 when a decision is ambiguous (-2: only the K_phi bin is).
 // Works on 2K (the reference's K times a power of two: its products round alike).
 template <bool EXT = false, typename Params>
 __device__ __forceinline__ int cascade_fast(const Params &P, double p1x, double p1y,
@@ -114,15 +119,13 @@ __device__ __forceinline__ int cascade_fast(const Params &P, double p1x, double 
     b.q_side = fma(b.q_y, sx, -(b.q_x * sy)) * rK;
     b.q_long = b.q_z;
     if (P.boost) {  // gamma (q_z - beta q_E) = (K_E q_z - K_z q_E) / M_t
-        const double z2 = sz * sz, M2 = fma(sE, sE, -z2);
-        b.q_long = fma(sE, b.q_z, -(sz * b.q_E)) * rsqrt_refined(M2);
-        if (z2 > kBoostMax * M2) near = 0.0;
+        const double rM = rsqrt_refined(fma(sE, sE, -(sz * sz)));
+        b.q_long = fma(sE, b.q_z, -(sz * b.q_E)) * rM;
     }
     b.io = bin_coord(fma(b.q_out, P.inv_dq, P.q_off), near);
     b.is = bin_coord(fma(b.q_side, P.inv_dq, P.q_off), near);
     b.il = bin_coord(fma(b.q_long, P.inv_dq, P.q_off), near);
-    if (near < P.guard)
-        return near < kEdge || fabs(near - 1e-8 * P.inv_dq) < kEdge ? -2 : -1;
+    if (near < P.guard) return -1;
     const unsigned q = max(max((unsigned)b.io, (unsigned)b.is), (unsigned)b.il);
     // (the last K_T index, n_KT - 1, holds only K_perp = KT_max: near an edge)
     if (q >= (unsigned)P.qnpts || (unsigned)b.kt >= (unsigned)(P.n_KT - 1)) return 0;

@@ -442,7 +442,7 @@ struct Stage {
 // the count is an FP64 add in the same instruction as the sums: one access
 // per binned pair.
 // unsure: the lanes whose pair the precision form could not decide, cos64 those
-// of them whose cos is taken from the literal form too.
+// of them that miss only their K_phi bin.
 template <typename Prec, bool EXT, bool RANKED>
 __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, Stage &stg,
                                      unsigned head, int cnt, bool mixed, double psi,
@@ -465,7 +465,7 @@ __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, St
     }
     if (std::is_same<Prec, float>::value) {
         unsure = __ballot(st < 0);
-        if (__builtin_expect(unsure != 0ull, 0)) cos64 = __ballot(st == -2);
+        if (EXT) cos64 = __ballot(st == -2);
     }
     const bool binned = st > 0 && (st & ST_BIN) != 0;
     const int nbinned = __popcll(__ballot(binned));
@@ -521,7 +521,8 @@ __device__ __forceinline__ int drain(CView *vp, CArgs *ka, const WaveLds &wl, St
 // the FP64 form, each added directly.  After the exact stage of its batch
 // rather than inside it: the literal cascade's registers then do not add to
 // the exact stage's.  cos stays the form's own (FP32), except for the lanes
-// cos64.
+// cos64 and for pairs on an edge (on_edge, asked here and not in the exact stage:
+// there it cost 2 % of the headline batch's kernel).
 template <bool EXT, bool RANKED>
 __device__ __forceinline__ int drain_literal(CView *vp, CArgs *ka, const WaveLds &wl, unsigned head,
                                              unsigned long long lanes, unsigned long long cos64,
@@ -541,8 +542,11 @@ __device__ __forceinline__ int drain_literal(CView *vp, CArgs *ka, const WaveLds
             SameRec rec;
             binned = (Exact<double, EXT>::same(vp, psi, base, pr.a, pr.b, rec, QinvSink()) &
                       ST_BIN) != 0;
-            if (!(cos64 >> lane & 1ull))
-                rec.c = pair_cos_f32(vp->P, lds_rec(base, pr.a), lds_rec(base, pr.b));
+            if (binned && !(cos64 >> lane & 1ull)) {
+                const PartRec p = lds_rec(base, pr.a), r = lds_rec(base, pr.b);
+                const double sx = p.px + r.px, sy = p.py + r.py;
+                if (!on_edge(vp->P, sx * sx + sy * sy, rec)) rec.c = pair_cos_f32(vp->P, p, r);
+            }
             if (binned) add_same_slabwise<float>(vp->H.bins, rec, ka->slab.vals != nullptr);
         }
     }
