@@ -1082,13 +1082,13 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
     // which keeps a group's items together): the persistent waves pull items
     // in queue order, so the launch ends on small items instead of one wave
     // finishing a large one (uneven multiplicities make items differ by 10x
-    // and more).  Inside a class the same-event items come first, or, with slab
-    // binning, same-event and mixed items take turns in proportion to their
-    // numbers: the mixed items' denominator adds are bound by the memory-side
-    // atomic rate, the same-event items by arithmetic, and side by side they
-    // overlap.  (Without slabs both add with atomics, and turns only cost: three
-    // groups of 20 events of 60 particles take 72 us so, 57 without, 8 of 50 of
-    // 600 4.19 ms and 4.08.)
+    // and more).  Inside a class same-event and mixed items take turns in
+    // proportion to their numbers: the mixed items' denominator adds are bound
+    // by the memory-side atomic rate, the same-event items by arithmetic, and
+    // side by side they overlap.  Without slab binning both add with atomics,
+    // and in a launch of few items a wave the turns only cost (three groups of 20
+    // events of 60 particles: 72 us, 57 with the same-event items first; the
+    // headline batch: 13.5 ms and 13.9).
     // (a counting sort over the 33 classes of a 64-bit count, then a merge of
     // the two kinds of each class)
     auto size_class = [&](size_t k) {
@@ -1112,13 +1112,14 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
         spairs[at] = pairs[k];
     }
     // (start[c] is now the end of class c's run: same-event items, then mixed)
+    const bool turns = slab || n >= 2 * want;
     for (size_t c = 0, b = 0; c < 33; b = start[c++]) {
         const size_t e = start[c];
         size_t i = b, m = b;
         while (m < e && sorted[m].kind == 0) m++;
         const size_t ns = m - b, nm = e - m;
         for (size_t at = b, j = m; at < e; at++) {
-            const bool take_same = j == e || (i < m && (!slab || (i - b) * nm <= (j - m) * ns));
+            const bool take_same = j == e || (i < m && (!turns || (i - b) * nm <= (j - m) * ns));
             const size_t k = take_same ? i++ : j++;
             L.items[at] = sorted[k];
             pairs[at] = spairs[k];
