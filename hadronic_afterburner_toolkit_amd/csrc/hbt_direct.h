@@ -7,11 +7,11 @@
 // prefilter operands.  The pair kernel walks them like k_fast, in items of 64
 // i particles: every pair takes the matrix-core prefilter, its survivors the
 // exact cascade, 64 at a time.  There are no momentum windows, so it tests
-// about five times the pairs that k_fast does on sorted lists, at 0.6 ps each;
-// below some 4e9 enumerated pairs the adds' atomics hide that (20 events of
-// 600 particles, 1.5e8 pairs: 151 us against k_fast's 190; of 1500 particles,
-// 9.5e8: 718 against 670; 10 of 4000, 1.8e9: 1245 against 1200), and sorting,
-// windows and items on the host cost several times the kernel.
+// about five times the pairs that k_fast does on sorted lists, at 0.3 ps each:
+// the kernel by itself is the slower one at a narrow q window or from some 3e8
+// pairs on (20 events of 600 particles, 1.5e8 pairs, q_max 0.15: 160 us against
+// k_fast's 167; 50 of 600, 9e8: 732 against 696, and 464 against 233 at 0.05),
+// but sorting, windows and items on the host cost several times the kernel.
 #pragma once
 #include "hbt_fast.h"
 #include "hbt_internal.h"

@@ -333,6 +333,7 @@ struct Slot {
     bool lists = false;           // the host lists above and their device copies hold this upload
     bool columns = false;         // and so do d_soa and d_off
     bool gathered = false;        // and (a direct upload) list: its gather is queued
+    bool ran[2] = {};             // its same-event, its mixed side has been run
     // a buffer gathered on the device (hbt_direct.h): its particles as passed
     // in, in pinned memory (two, in turn: the copy of the last upload may
     // still run) and on the device, each eight columns, then the offsets
@@ -453,6 +454,7 @@ struct hbt_ctx {
     bool batch_ready = false;
     // a batch of one buffer gathered on the device has no items: its pair launch
     bool batch_direct = false;
+    bool batch_launched = false;  // since it was prepared
     PairArgs batch_pairs{};
     // plans on their way to the device (two, in turn, as Slot::h_raw)
     char *h_plan[2] = {};
@@ -552,7 +554,7 @@ void drop_graph(hbt_ctx *c) {
     c->graph_exec = nullptr;
     c->graph = nullptr;
     c->batch_ready = false;
-    c->batch_direct = false;
+    c->batch_direct = c->batch_launched = false;
 }
 
 DevHist hist_view(hbt_ctx *c) {
@@ -1730,7 +1732,7 @@ int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
         drop_graph(c);
         c->plan_valid = false;
         s.valid = false;  // until every copy has succeeded
-        s.direct = s.gathered = s.columns = false;
+        s.direct = s.gathered = s.columns = s.ran[0] = s.ran[1] = false;
     }
     s.lists = false;
     const long long nf = h.nf;
@@ -1754,12 +1756,32 @@ int upload_columns(hbt_ctx *c, Slot &s, int32_t nev, const HostParticles &h,
     });
 }
 
-// One buffer is gathered on the device where the pair kernel without windows
-// is as fast as the windowed one (hbt_direct.h), which spares the host the
-// sorts, windows and items.  Not with slab binning, where the adds are cheap
-// and the windows count.  2^16 particles: 2.1e9 same-event pairs.
+// One buffer is gathered on the device and its pairs are walked without windows
+// (hbt_direct.h), which spares the host the sorts, windows and items: of a call
+// on a new upload those cost more than the windows save, up to the 4e9 pairs
+// measured and for any q window.  50 events of 1200 particles (3.7e9 pairs), upload
+// included: 1.33 ms at a q_max of 0.01, 2.00 at 0.08 and 5.13 at 0.2 against 2.46,
+// 3.20 and 7.83; of 600 (9e8) 0.52, 0.73 and 1.51 against 1.93, 1.82 and 3.10.
+// Not with slab binning, where the adds are cheap and the windows count.  2^16
+// particles: 2.1e9 same-event pairs.
 constexpr long long kDirectParticles = 1 << 16;
 constexpr uint64_t kDirectPairs = 4000000000ull;  // same-event and mixed pairs of a call
+
+// Where the same upload is run again, the lists are built once and the kernels
+// count alone.  A batch: 50 x 1200 at a q_max of 0.05 1.54 ms without windows and
+// 0.39 with, at 0.15 2.70 and 2.16; 50 x 600 0.46 and 0.23 at 0.05, 0.73 and 0.70
+// at 0.15; 20 x 600 (1.5e8 pairs) 0.10 and 0.07.  One side, its items built on the
+// host each time: same-event pairs of 50 x 1200 0.75 and 0.35 ms at 0.03, 1.57 and
+// 1.97 at 0.15, of 50 x 890 (1e9) 0.55 and 0.56 at 0.08; mixed pairs only where
+// the rows are long: 8 events of 8000 0.42 and 0.34 at 0.01, 0.65 and 0.70 at 0.08,
+// 50 x 1200 0.53 and 0.98.
+bool windows_pay_batch(const hbt_ctx *c, uint64_t pairs) {
+    return pairs >= 1000000000ull || (pairs >= 250000000ull && c->D.H <= 0.12);
+}
+bool windows_pay_side(const hbt_ctx *c, uint64_t pairs, long long rows) {
+    return pairs >= 1000000000ull &&
+           (rows == 0 ? c->D.H <= 0.09 : c->D.H <= 0.05 && pairs / (uint64_t)rows >= 50000000ull);
+}
 
 bool direct_upload(const hbt_ctx *c, int32_t ngroups, int32_t nev, const int64_t *ev_off) {
     return c->cfg.kernel == HBT_KERNEL_FAST && !c->slab_binning && ngroups == 1 && nev > 0 &&
@@ -1778,7 +1800,7 @@ int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
     const size_t col = stage_round((size_t)n_in * 8);
     drop_graph(c);
     c->plan_valid = false;
-    s.valid = s.direct = s.gathered = s.columns = s.lists = false;
+    s.valid = s.direct = s.gathered = s.columns = s.lists = s.ran[0] = s.ran[1] = false;
     s.raw ^= 1;
     int rc = next_pinned(c, &s.h_raw[s.raw], &s.raw_cap[s.raw], &s.raw_ev[s.raw],
                          8 * col + ((size_t)nev + 1) * 8);
@@ -1983,6 +2005,16 @@ int need_columns(hbt_ctx *c) {
 // enough to be walked without windows.
 bool direct_call(const hbt_ctx *c, uint64_t pairs) {
     return c->slot[0].direct && mixed_slot(c).direct && !c->slab_binning && pairs <= kDirectPairs;
+}
+
+// The same for one side run by itself (rows: plan rows, 0 for the same-event
+// side): not where it has run on this upload before, or the host's lists are
+// there, and the windows pay.
+bool direct_side(hbt_ctx *c, uint64_t pairs, long long rows) {
+    Slot &s = c->slot[0];
+    const bool lists = s.ran[rows > 0] || (s.lists && mixed_slot(c).lists);
+    s.ran[rows > 0] = true;
+    return direct_call(c, pairs) && !(lists && windows_pay_side(c, pairs, rows));
 }
 
 // The pair launch of a direct call (its slots are gathered): the same-event side,
@@ -2215,7 +2247,7 @@ int hbt_run_same(hbt_ctx *c) {
     if (rc) return rc;
     ItemList items;
     uint64_t es = same_pairs(c->slot[0]);
-    const bool direct = direct_call(c, es);
+    const bool direct = direct_side(c, es, 0);
     if (direct) {
         if ((rc = gather_slots(c))) return rc;
     } else {
@@ -2292,7 +2324,7 @@ int hbt_run_mixed(hbt_ctx *c, int32_t M, const int32_t *partner_ids, const doubl
     if (rc) return rc;
     const bool binds = side[1].binds;
     bool done = false;
-    const bool direct = direct_call(c, em);
+    const bool direct = direct_side(c, em, (long long)s.nev * M);
     if ((rc = direct ? gather_slots(c) : need_lists(c))) return rc;
     if (binds && direct) {
         rc = timed_trial(c, trial_direct(c, direct_pairs(c, false, M)), side, c->ev + 2,
@@ -2371,6 +2403,13 @@ int hbt_prepare_batch(hbt_ctx *c, const int32_t *M_per_group, const int32_t *par
 int hbt_launch_batch(hbt_ctx *c) {
     if (!c) return HBT_ERR_ARG;
     if (!c->batch_ready) return fail(c, HBT_ERR_STATE, "no prepared batch (hbt_prepare_batch)");
+    if (c->batch_direct && c->batch_launched &&
+        windows_pay_batch(c, c->batch_enum_same + c->batch_enum_mixed)) {
+        int rc0 = quiesce(c);
+        c->batch_capture = true;  // launched more than once
+        if (!rc0) rc0 = prepare_and_capture(c);
+        if (rc0) return rc0;
+    }
     if (c->slab.resize && c->cfg.kernel == HBT_KERNEL_FAST && !c->batch_direct) {
         // the last launch outgrew its slab regions: size them again from its
         // demand (and capture the batch again) before this launch
@@ -2410,6 +2449,7 @@ int hbt_launch_batch(hbt_ctx *c) {
         if (rc) return rc;
     }
     HIPCHECK(c, hipEventRecord(c->ev[1], c->stream));
+    c->batch_launched = true;
     c->enum_same_total += c->batch_enum_same;
     c->enum_mixed_total += c->batch_enum_mixed;
     return HBT_OK;

@@ -88,3 +88,49 @@ def test_paths_of_one_upload(own_mixed, cap):
         ref = getattr(y, key)
         err = np.abs(getattr(x, key) - ref) / np.maximum(np.abs(ref), n * scale)
         assert float(err.max()) <= 1e-12, key
+
+
+def times(a, b, k):
+    """a's histograms are k times b's (counts exactly)."""
+    assert np.array_equal(a.num_count, b.num_count * np.uint64(k))
+    assert np.array_equal(a.den, b.den * np.uint64(k))
+    n = np.maximum(b.num_count.astype(np.float64), 1.0)
+    for key, scale in (("q_out_sum", .0525), ("q_side_sum", .0525), ("q_long_sum", .0525),
+                       ("num", 1.0)):
+        ref = getattr(b, key)
+        err = np.abs(getattr(a, key) / k - ref) / np.maximum(np.abs(ref), n * scale)
+        assert float(err.max()) <= 1e-12, key
+
+
+@pytest.mark.parametrize("mult,lists", [(100.0, False), (900.0, True)])
+def test_a_large_narrow_batch_launched_again_takes_the_lists(mult, lists):
+    """hbt_batch_graph tells the form: the walk without windows is no graph."""
+    params = dict(config(), q_min=-0.05, q_max=0.05, number_of_mixed_events=0)
+    buf = samples.generate(5, 20, mult)
+    g = hbt.HBTCorrelation(params)
+    g.calculate_HBT_correlation_function(buf, hbt.Random(1))
+    assert (sum(g.batch_info()[:2]) > 250000000) == lists
+    one = g.results()
+    assert not g.batch_graph()
+    for _ in range(2):
+        g.launch_batch()
+    assert g.batch_graph() == lists
+    times(g.results(), one, 3)
+    g.close()
+
+
+@pytest.mark.parametrize("nev,mult", [(20, 100.0), (6, 8000.0)])
+def test_a_side_run_again(nev, mult):
+    params = dict(config(), q_min=-0.03, q_max=0.03)
+    buf = samples.generate(6, nev, mult)
+    plan = hbt.Random(1).draw_plan(nev, nev, 3)
+    g = hbt.HBTCorrelation(params)
+    g.upload(buf)
+    g.run_same()
+    g.run_mixed(*plan)
+    one = g.results()
+    for _ in range(2):
+        g.run_same()
+        g.run_mixed(*plan)
+    times(g.results(), one, 3)
+    g.close()
