@@ -259,19 +259,36 @@ struct SameRec {
     bool sure;      // every coordinate at least DevParams::guard from a bin edge
 };
 
+// One more in a 32-bit count whose wraps go to the 64-bit total it will be added
+// to: inc(lo) adds one and returns the count before, add(total, v) adds v.
+template <typename Inc, typename Add>
+__host__ __device__ __forceinline__ void count_carry(unsigned *lo, unsigned long long *total,
+                                                     Inc inc, Add add) {
+    if (inc(lo) == 0xffffffffu) add(total, 1ull << 32);
+}
+
 // Where a q_inv pair goes (bin k of [K_T][q]): the histograms in memory, or,
 // with lds set, the block's own sum[nq], num[nq], count[nq] and den[nq] in
-// LDS, which the kernel adds to the histograms at its end.  A q_inv histogram
+// LDS, which the kernel adds to the histograms at its end (the 32-bit counts
+// carry into them).  A q_inv histogram
 // has a few hundred bins, so every pair of the launch meets in the same few
 // cache lines: a buffer of 20 events of 200 particles (1.7e7 pairs, 1.6 % of
 // them in the q_inv window) took 806 us with adds to memory, 435 with LDS.
 struct QinvSink {
     double *lds = nullptr;
     int nq = 0;
+    static __device__ __forceinline__ void count(unsigned *lo, unsigned long long *total) {
+        count_carry(
+            lo, total,
+            [](unsigned *p) {
+                return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+            },
+            [](unsigned long long *p, unsigned long long v) { atomic_add_u64(p, v); });
+    }
     __device__ __forceinline__ void same(const DevHist &H, long k, double q, double c) const {
         if (lds) {
-            __hip_atomic_fetch_add((unsigned *)(lds + 2 * nq) + k, 1u, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+            count((unsigned *)(lds + 2 * nq) + k, &H.qinv_count[k]);
             __hip_atomic_fetch_add(lds + k, q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             __hip_atomic_fetch_add(lds + nq + k, c, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -283,8 +300,7 @@ struct QinvSink {
     }
     __device__ __forceinline__ void mixed(const DevHist &H, long k) const {
         if (lds)
-            __hip_atomic_fetch_add((unsigned *)(lds + 2 * nq) + nq + k, 1u, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+            count((unsigned *)(lds + 2 * nq) + nq + k, &H.qinv_den[k]);
         else
             atomic_add_u64(&H.qinv_den[k], 1ull);
     }

@@ -873,11 +873,10 @@ __device__ __forceinline__ void qinv_end(CView *vp, const double *q, int nq) {
     __syncthreads();
     const unsigned *cnt = (const unsigned *)(q + 2 * nq);
     for (int k = threadIdx.x; k < nq; k += blockDim.x) {
-        if (cnt[k]) {
-            atomic_add_u64(&vp->H.qinv_count[k], cnt[k]);
-            atomic_add_f64(&vp->H.qinv_sum[k], q[k]);
-            atomic_add_f64(&vp->H.qinv_num[k], q[nq + k]);
-        }
+        if (cnt[k]) atomic_add_u64(&vp->H.qinv_count[k], cnt[k]);
+        // (not by the count: one that has wrapped may be 0)
+        if (q[k] != 0.0) atomic_add_f64(&vp->H.qinv_sum[k], q[k]);
+        if (q[nq + k] != 0.0) atomic_add_f64(&vp->H.qinv_num[k], q[nq + k]);
         if (cnt[nq + k]) atomic_add_u64(&vp->H.qinv_den[k], cnt[nq + k]);
     }
 }
