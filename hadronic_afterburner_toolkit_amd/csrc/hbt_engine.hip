@@ -1064,6 +1064,8 @@ void build_items(hbt_ctx *c, bool same, bool mixed, ItemList &L, uint64_t &enum_
     const size_t want = kItemsPerWave * waves;
     uint64_t total = 0;
     for (uint64_t v : pairs) total += v;
+    // (with q_inv bins every pair of the K_T window takes the literal cascade)
+    if (c->P.qinv) total *= 4;
     auto enough = [&](size_t n) {
         return n >= 2 * want || (n >= want && total <= kLargeItem * (uint64_t)n) ||
                (sh.JC <= 64 && sh.KC <= 1);
