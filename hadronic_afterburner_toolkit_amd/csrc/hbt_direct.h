@@ -21,7 +21,7 @@ namespace hbt {
 constexpr int kGatherSmall = 2048;  // particles gathered by one block in one launch
 
 // With q_inv bins: the room, relative to H^2, that the prefilter's windows leave
-// for particles off one mass shell (pair_consts in hbt_direct.hip).
+// for particles off one mass shell (pair_consts).
 constexpr double kQinvRoom = 1e-3;
 __host__ __device__ inline double qinv_h2(double H) {
     const double Hm = H * (1.0 + 1e-9) + 1e-12;
@@ -34,6 +34,45 @@ struct ListStat {
     double pmax2, bmax, m2lo, m2hi;
     int n;
 };
+
+__host__ __device__ __forceinline__ ListStat stat_none() {
+    return ListStat{0.0, 0.0, INFINITY, -INFINITY, 0};
+}
+__host__ __device__ __forceinline__ ListStat stat_join(const ListStat &a, const ListStat &b) {
+    return ListStat{fmax(a.pmax2, b.pmax2), fmax(a.bmax, b.bmax), fmin(a.m2lo, b.m2lo),
+                    fmax(a.m2hi, b.m2hi), a.n + b.n};
+}
+
+// The prefilter's constants for two lists' scales.  With q_inv bins a pair
+// that bins in either kind of histogram has |q_side| and |q_long| within
+// sqrt(1 + kQinvRoom) H, but no bound on q_out, so the kernel tests
+// C^2 <= H^2 T alone (dn = 0).  For q_inv: in the LCMS q_E M_t = K_T q_out + d
+// with d = (m1^2 - m2^2) / 2, so q_inv^2 = q_side^2 + q_long^2 +
+// q_out^2 - q_E^2 and the smallest value of the last two, over all q_out, is
+// -d^2 / K^2 with K^2 = (m1^2 + m2^2) / 2 + q_inv^2 / 4 at least the lists'
+// smallest m^2.  Where the lists' m^2 = E^2 - p^2 differ too much for the room,
+// every pair in the K_T window takes the cascade, as all did before: 435 us for
+// 20 events of 200 particles, 105 with the windows.
+__host__ __device__ __forceinline__ PfConst<float> pair_consts(DevParams P, const ListStat &st) {
+    if (!P.qinv) {
+        prefilter_margins(st.pmax2, P);
+        return pf_const<float>(P);
+    }
+    const double d = 0.5 * (st.m2hi - st.m2lo), H = fmax(fabs(P.q_lo_cut), fabs(P.q_hi_cut));
+    const bool windows = st.m2lo > 0.0 && d * d <= 0.5 * kQinvRoom * H * H * st.m2lo;
+    if (windows) {
+        P.qinv = 0;
+        P.pf_h2 = qinv_h2(H);
+        prefilter_margins(st.pmax2, P);
+        PfConst<float> k = pf_const<float>(P);
+        k.dn = 0.0f;
+        return k;
+    }
+    prefilter_margins(st.pmax2, P);
+    PfConst<float> k = pf_const<float>(P);
+    k.wide = INFINITY;
+    return k;
+}
 
 // A gathered list: event e is [koff[e], koff[e + 1]).  rec, pf and bw have
 // kPfPad entries past cap; stat is per event.

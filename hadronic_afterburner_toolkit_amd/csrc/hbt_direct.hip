@@ -12,14 +12,6 @@ using namespace hbt;
 
 constexpr long long kWaves = 4096;  // the pair kernel's resident waves (256 CUs x 16)
 
-__device__ __forceinline__ ListStat stat_none() {
-    return ListStat{0.0, 0.0, INFINITY, -INFINITY, 0};
-}
-__device__ __forceinline__ ListStat stat_join(const ListStat &a, const ListStat &b) {
-    return ListStat{fmax(a.pmax2, b.pmax2), fmax(a.bmax, b.bmax), fmin(a.m2lo, b.m2lo),
-                    fmax(a.m2hi, b.m2hi), a.n + b.n};
-}
-
 // A particle of the list: tanh(HBTrap_min) < pz/E < tanh(HBTrap_max)
 // (HBT_correlation.cpp:255-266), and |pT| as a binnable pair needs it.
 __device__ __forceinline__ bool list_kept(const GatherArgs &g, long long i, ListStat &st) {
@@ -206,37 +198,6 @@ struct ArgView {
         return (CView *)((const HBT_AS4 char *)ka + offsetof(PairArgs, v));
     }
 };
-
-// The prefilter's constants for two lists' scales.  With q_inv bins a pair
-// that bins in either kind of histogram has |q_side| and |q_long| within
-// sqrt(1 + kQinvRoom) H, but no bound on q_out, so the kernel tests
-// C^2 <= H^2 T alone (dn = 0).  For q_inv: in the LCMS q_E M_t = K_T q_out + d
-// with d = (m1^2 - m2^2) / 2, so q_inv^2 = q_side^2 + q_long^2 +
-// q_out^2 - q_E^2 and the smallest value of the last two, over all q_out, is
-// -d^2 / K^2 with K^2 = (m1^2 + m2^2) / 2 + q_inv^2 / 4 at least the lists'
-// smallest m^2.  Where the lists' m^2 = E^2 - p^2 differ too much for the room,
-// every pair in the K_T window takes the cascade, as all did before: 435 us for
-// 20 events of 200 particles, 105 with the windows.
-__device__ __forceinline__ PfConst<float> pair_consts(DevParams P, const ListStat &st) {
-    if (!P.qinv) {
-        prefilter_margins(st.pmax2, P);
-        return pf_const<float>(P);
-    }
-    const double d = 0.5 * (st.m2hi - st.m2lo), H = fmax(fabs(P.q_lo_cut), fabs(P.q_hi_cut));
-    const bool windows = st.m2lo > 0.0 && d * d <= 0.5 * kQinvRoom * H * H * st.m2lo;
-    if (windows) {
-        P.qinv = 0;
-        P.pf_h2 = qinv_h2(H);
-        prefilter_margins(st.pmax2, P);
-        PfConst<float> k = pf_const<float>(P);
-        k.dn = 0.0f;
-        return k;
-    }
-    prefilter_margins(st.pmax2, P);
-    PfConst<float> k = pf_const<float>(P);
-    k.wide = INFINITY;
-    return k;
-}
 
 // Bound by the adds' atomics (2.35e10 binned same-event and 2.68e10 mixed pairs
 // per second, memory side) where more than a percent of the pairs bins, else

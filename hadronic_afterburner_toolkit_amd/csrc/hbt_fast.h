@@ -79,13 +79,11 @@ __host__ __device__ __forceinline__ PfConst<Prec> pf_const(const DevParams &P) {
 }
 
 // The prefilter's tests of one pair (for a mixed pair, i rotated by
-// -theta): it passes where all four values are negative.  K_T window: X^2 -
-// (s half)^2; q_out and q_side: max(|dn|, |C|)^2 - X - (H^2 mid + c); q_long:
-// |y_i - y_j| <= cw_i + cw_j as the overlap of the two longitudinal intervals,
-// blo_i - bhi_j and blo_j - bhi_i.  The margins leave every pair the exact
-// cascade accepts strictly inside.  The host's check of the margins evaluates
-// this function; the kernel forms X, dn and C on the matrix cores, whose order
-// of the four products the margins cover too.
+// -theta): it passes where all four values are negative, that is, where the
+// largest is.  K_T window: X^2 - (s half)^2; q_out and q_side: max(|dn|, |C|)^2 -
+// X - (H^2 mid + c); q_long: |y_i - y_j| <= cw_i + cw_j as the overlap of the two
+// longitudinal intervals, blo_i - bhi_j and blo_j - bhi_i.  The margins leave
+// every pair the exact cascade accepts strictly inside.
 __host__ __device__ __forceinline__ float pf_fma(float a, float b, float c) {
     return __builtin_fmaf(a, b, c);
 }
@@ -94,27 +92,68 @@ __host__ __device__ __forceinline__ double pf_fma(double a, double b, double c) 
 }
 __host__ __device__ __forceinline__ float pf_abs(float a) { return __builtin_fabsf(a); }
 __host__ __device__ __forceinline__ double pf_abs(double a) { return __builtin_fabs(a); }
+__host__ __device__ __forceinline__ float pf_max(float a, float b) { return __builtin_fmaxf(a, b); }
+__host__ __device__ __forceinline__ double pf_max(double a, double b) {
+    return __builtin_fmax(a, b);
+}
 
+// Operands of one i particle, component 0..3, against a j particle's (px, py, n,
+// 1): X = s (T - mid), and P = (dn + C) / 2, M = (dn - C) / 2 with dn = in - jn
+// and C = 2 (ix jy - iy jx), so that max(|dn|, |C|) = |P| + |M| is one addition (a
+// maximum would first quiet both operands).
+template <typename Prec>
+struct PfBlock {
+    Prec X, P, M;
+};
+template <typename Prec>
+__host__ __device__ __forceinline__ PfBlock<Prec> pf_block(const PfConst<Prec> &k, int comp, Prec x,
+                                                           Prec y, Prec n) {
+    PfBlock<Prec> o;
+    const Prec s2 = (Prec)2 * k.s;
+    o.X = comp == 0 ? s2 * x : comp == 1 ? s2 * y : comp == 2 ? k.s : k.s * n;
+    const Prec c = comp == 0 ? -y : comp == 1 ? x : (Prec)0;
+    const Prec d = comp == 2 ? -k.dn : comp == 3 ? k.dn * n : (Prec)0;
+    o.P = d + c;
+    o.M = d - c;
+    return o;
+}
+
+// The largest of a pair's tests, from the products X, P and M and the two
+// longitudinal intervals (i's widened by k.wide).
+template <typename Prec>
+__host__ __device__ __forceinline__ Prec pf_test(Prec X, Prec P, Prec M, Prec ilo, Prec ihi,
+                                                 Prec jlo, Prec jhi, const PfConst<Prec> &k) {
+    const Prec e = pf_abs(P) + pf_abs(M);
+    return pf_max(pf_max(pf_fma(e, e, -X) - k.c0, pf_fma(X, X, k.nsh2)),
+                  pf_max(ilo - jhi, jlo - ihi));
+}
+
+// A pair's test on the host, for the check of the margins: the kernel's operands
+// and test, the four products added in order (the matrix cores' order is not
+// known; the margins cover any).
 template <typename Prec>
 struct PfTerms {
-    Prec v[4];
+    Prec m;
 };
-
 template <typename Prec>
 __host__ __device__ __forceinline__ PfTerms<Prec> pf_terms(Prec ix, Prec iy, Prec in, Prec ilo,
                                                            Prec ihi, Prec jx, Prec jy, Prec jn,
                                                            Prec jlo, Prec jhi,
                                                            const PfConst<Prec> &k) {
-    const Prec s2 = (Prec)2 * k.s;
-    const Prec X = pf_fma(jx, s2 * ix, pf_fma(jy, s2 * iy, pf_fma(jn, k.s, k.s * in)));
-    const Prec dn = pf_fma(jn, (Prec)-0.5, (Prec)0.5 * in);
-    const Prec m = pf_abs(pf_fma(jx, -iy, pf_fma(jy, ix, dn))) + pf_abs(pf_fma(jx, iy, pf_fma(jy, -ix, dn)));
-    return PfTerms<Prec>{{pf_fma(X, X, k.nsh2), pf_fma(m, m, -X) - k.c0, ilo - jhi, jlo - ihi}};
+    const Prec j[4] = {jx, jy, jn, (Prec)1};
+    Prec X = 0, P = 0, M = 0;
+    for (int c = 0; c < 4; c++) {
+        const PfBlock<Prec> b = pf_block(k, c, ix, iy, in);
+        X = pf_fma(j[c], b.X, X);
+        P = pf_fma(j[c], b.P, P);
+        M = pf_fma(j[c], b.M, M);
+    }
+    return PfTerms<Prec>{pf_test(X, P, M, ilo - k.wide, ihi + k.wide, jlo, jhi, k)};
 }
 
 template <typename Prec>
 __host__ __device__ __forceinline__ bool pf_pass(const PfTerms<Prec> &t) {
-    return t.v[0] < 0 && t.v[1] < 0 && t.v[2] < 0 && t.v[3] < 0;
+    return t.m < 0;
 }
 
 // What a particle's prefilter record needs beside its momentum: the window
@@ -562,26 +601,6 @@ __device__ __forceinline__ int xcc_id() {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// Matrix-core operands of the 16 i particles of a block, one value per lane:
-// lane l holds component l / 16 of particle l % 16.  Against a j tile's rows
-// (px, py, n, 1): X = s (T - mid), and P = (dn + C) / 2, M = (dn - C) / 2
-// with dn = in - jn and C = 2 (ix jy - iy jx), so that max(|dn|, |C|) =
-// |P| + |M| is one addition (a maximum would first quiet both operands).
-struct PfBlock {
-    float X, P, M;
-};
-__device__ __forceinline__ PfBlock pf_block(const PfConst<float> &k, int comp, float x, float y,
-                                            float n) {
-    PfBlock o;
-    const float s2 = 2.0f * k.s;
-    o.X = comp == 0 ? s2 * x : comp == 1 ? s2 * y : comp == 2 ? k.s : k.s * n;
-    const float c = comp == 0 ? -y : comp == 1 ? x : 0.0f;
-    const float d = comp == 2 ? -k.dn : comp == 3 ? k.dn * n : 0.0f;
-    o.P = d + c;
-    o.M = d - c;
-    return o;
-}
-
 // Bits (from the top: block b, row r at bit 15 - (4 b + r)) of the rows of a
 // tile that are in range: the first n of this lane's four rows.
 __device__ __forceinline__ unsigned rows_first(int n) {
@@ -644,9 +663,10 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
         if (RANKED && !mixed) wl.irank[lane] = vp->origS[w.i0 + min(lane, last)].rank;
     }
     float ilo[4], ihi[4];
-    PfBlock blk[4];
-    // The i blocks, rotated by -theta for a mixed segment (columns past the
-    // tile's end repeat its last particle; `cols` masks them).
+    PfBlock<float> blk[4];
+    // The i blocks, rotated by -theta for a mixed segment, one value per lane: lane
+    // l holds component l / 16 of particle l % 16 (columns past the tile's end
+    // repeat its last particle; `cols` masks them).
     auto load_blocks = [&](double c, double s) {
 #pragma unroll
         for (int b = 0; b < 4; b++) {
@@ -730,10 +750,8 @@ __device__ __forceinline__ void walk_item(const WorkItem &w, CView *vp, double p
                         __builtin_amdgcn_mfma_f32_16x16x4f32(A[t], blk[b].M, o, 0, 0, 0);
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
-                        const float e = fabsf(U[r]) + fabsf(V[r]);
-                        const float m = fmaxf(
-                            fmaxf(fmaf(e, e, -X[r]) - pk.c0, fmaf(X[r], X[r], pk.nsh2)),
-                            fmaxf(ilo[b] - jw[t][r].hi, jw[t][r].lo - ihi[b]));
+                        const float m = pf_test(X[r], U[r], V[r], ilo[b], ihi[b], jw[t][r].lo,
+                                                jw[t][r].hi, pk);
                         // bits << 1 | sign of m
                         bits = __builtin_amdgcn_alignbit(bits, __builtin_bit_cast(unsigned, m),
                                                          31);
