@@ -433,6 +433,7 @@ struct hbt_ctx {
         double hist_enum_s = 0;
         int hist_nblk = 0;
         bool have_hist = false, pending = false, resize = false;
+        bool captured = false;      // a captured launch whose demand the first replay measures
         uint64_t direct = 0;        // binned same-event pairs of the last launch added directly
         char *d_vals = nullptr;
         long long *d_sbase = nullptr;
@@ -555,6 +556,7 @@ void drop_graph(hbt_ctx *c) {
     c->graph = nullptr;
     c->batch_ready = false;
     c->batch_direct = c->batch_launched = false;
+    c->slab.captured = false;
 }
 
 DevHist hist_view(hbt_ctx *c) {
@@ -945,7 +947,7 @@ int fast_args(hbt_ctx *c, FastArgs &a) {
 
 // The fast kernel, and with slab binning its two binning kernels, queued on
 // st (kernel launches only: this runs inside a graph capture).
-int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st) {
+int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st, bool capture = false) {
     const bool f32 = c->cfg.precision == HBT_PREC_FP32C;
     const bool slab = a.slab.vals != nullptr;
     const long blocks = fast_blocks(c, a.nitems, f32, slab);
@@ -969,7 +971,7 @@ int launch_fast(hbt_ctx *c, FastArgs &a, hipStream_t st) {
                            (const SlabPart *)c->slab.d_parts, a.slab.uoff, a.slab.S, a.slab.SB,
                            c->d_bins);
         HIPCHECK(c, hipGetLastError());
-        c->slab.pending = true;
+        (capture ? c->slab.captured : c->slab.pending) = true;
     }
     return HBT_OK;
 }
@@ -1671,7 +1673,7 @@ int prepare_and_capture(hbt_ctx *c) {
     bool captured = c->batch_capture &&
                     hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
     if (captured) {
-        rc = launch_fast(c, a, c->stream);
+        rc = launch_fast(c, a, c->stream, true);
         captured = hipStreamEndCapture(c->stream, &g) == hipSuccess && !rc && g;
     }
     if (captured) captured = hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0) == hipSuccess;
@@ -2442,6 +2444,8 @@ int hbt_launch_batch(hbt_ctx *c) {
     } else if (c->cfg.kernel == HBT_KERNEL_FAST) {
         if (c->nitems > 0 && c->graph_exec) {
             HIPCHECK(c, hipGraphLaunch(c->graph_exec, c->stream));
+            c->slab.pending = c->slab.pending || c->slab.captured;
+            c->slab.captured = false;
         } else if (c->nitems > 0) {
             rc = launch_fast(c, c->batch_args, c->stream);
             if (rc) return rc;

@@ -95,3 +95,28 @@ def test_a_small_launch_has_a_wave_for_two_items(nev, mult, M):
     blocks = max((items + 7) // 8, min((items + 3) // 4, 128))
     assert blocks < 1024
     assert capacity == (int(np.ceil(1.25 * (3.0 * 0.03 * same / slabs / blocks))) + 32) * slabs * blocks
+
+
+def test_regions_are_sized_from_launches_only():
+    """The demand of a batch that is prepared but not launched is not known: asking
+    for it, or preparing again, leaves the first launch's regions as they are."""
+    params = dict(qnpts=21, q_min=-0.15, q_max=0.15, n_KT=4, KT_min=0.2, KT_max=0.7,
+                  HBTrap_min=-1.0, HBTrap_max=1.0, needed_number_of_pairs=1e18, hbt_binning=1)
+    bufs = [samples.generate(s, 20, 200.0) for s in range(3)]
+    plans = [hbt.Random(k).draw_plan(20, 20, 5) for k in range(3)]
+    g = hbt.HBTCorrelation(params)
+    g.upload_groups(bufs)
+    for _ in range(3):
+        g.prepare_batch(np.array([5] * 3, np.int32), np.concatenate([p[1] for p in plans]),
+                        np.concatenate([p[2] for p in plans]))
+        same, _, items = g.batch_info()
+        blocks = max((items + 7) // 8, min((items + 3) // 4, 128))
+        slabs = 4 * 21
+        first = (int(np.ceil(1.25 * (3.0 * 0.03 * same / slabs / blocks))) + 32) * slabs * blocks
+        assert g.slab_info()["capacity"] == first
+        g.sync()
+    g.launch_batch()
+    g.sync()
+    g.set_tuning(1, 512, 4, 4)  # prepared again, from the launch's demand
+    assert 0 < g.slab_info()["capacity"] != first
+    g.close()
