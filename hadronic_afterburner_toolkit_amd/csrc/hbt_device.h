@@ -20,17 +20,15 @@ struct DevParams {
     double KT_min_sq, KT_max_sq, hbarC_inv, two_pi;
     // Conservative prefilter thresholds (a pair the exact cascade accepts
     // always passes).  Per particle the record holds nrm = |pT|^2 - mid/2,
-    // so for a pair u = T - mid and v = Q - mid come from one dot product
-    // (T = |p1T+p2T|^2 = 4 K_perp^2, Q = |p1T-p2T|^2) and dn = |p1T|^2 -
-    // |p2T|^2 from the two records.  As q_out = dn / sqrt(T) and q_side^2 =
-    // Q - q_out^2, the windows |q_out|, |q_side| <= H read dn^2 <= H^2 T and
-    // (Q - H^2) T <= dn^2; each side carries the rounding margin c.
+    // so for a pair T - mid (T = |p1T+p2T|^2 = 4 K_perp^2), dn = |p1T|^2 -
+    // |p2T|^2 and C = 2 (p1x p2y - p1y p2x) are dot products of the two records.
+    // As q_out = dn / sqrt(T) and q_side = C / sqrt(T), the windows |q_out|,
+    // |q_side| <= H read max(|dn|, |C|)^2 <= H^2 T, with the rounding margin c.
     double pf_half;   // |T - mid| <= pf_half
     double pf_h2;     // H^2 with margin (0 with the q_inv branch on)
-    double pf_midh2;  // mid - pf_h2
     double pf_negc;   // -c (-inf with the q_inv branch on: the q tests pass every pair)
     double pf_mid;
-    float f_half, f_h2, f_midh2, f_negc, f_mid, f_pad;
+    float f_half, f_negc;
     // precision-form exact-stage constants
     // (bin coordinates raised by one: kt_scale * 2 K_perp + kt_off, inv_dq * q
     // + q_off; a pair with one within `guard` of an integer takes the literal

@@ -2061,6 +2061,7 @@ int prepare_direct(hbt_ctx *c, int M, const int32_t *ids, const double *cs) {
     c->qoff.assign(2, 0);
     c->qoff[1] = c->nitems;
     c->batch_direct = c->batch_ready = true;
+    c->batch_launched = false;
     return HBT_OK;
 }
 

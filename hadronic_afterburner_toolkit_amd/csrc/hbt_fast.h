@@ -338,10 +338,7 @@ __device__ __forceinline__ CArgs *kernel_args() {
 #endif
 }
 
-// ------------------------------------------------------- wave helpers
-
-// ---------------------------------------------------------------- drain
-// Each lane takes one queued survivor (lane < cnt), runs the exact cascade.
+// ------------------------------------------------------------ exact stage
 // A wave's LDS.  The exact stage takes 64 scattered survivors at a time; read
 // from memory, each of their 128-byte pairs of records would cost the vector
 // cache eight accesses per lane (measured: its address and data units 88 and

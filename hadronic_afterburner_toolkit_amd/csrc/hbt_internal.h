@@ -104,13 +104,9 @@ inline int derive(const hbt_config &k, Derived &d, std::string &err) {
     const double Hm = d.H * (1.0 + 1e-9) + 1e-12;
     d.h2 = Hm * Hm * (1.0 + 1e-9) + 1e-12;
     P.pf_h2 = P.qinv ? 0.0 : d.h2;
-    P.pf_midh2 = d.mid - P.pf_h2;
     P.pf_negc = P.qinv ? -INFINITY : 0.0;
     d.c_beta = 0.5 * Hm;
-    P.f_mid = (float)d.mid;
     P.f_half = (float)P.pf_half;
-    P.f_h2 = (float)P.pf_h2;
-    P.f_midh2 = (float)P.pf_midh2;
     P.f_negc = (float)P.pf_negc;
     d.needed = (uint64_t)(unsigned long long)k.needed_number_of_pairs;
     d.needed_qinv = (uint64_t)50 * d.needed;
@@ -128,8 +124,8 @@ inline PfMake pf_maker(const Derived &d, double bm) {
 // longitudinal interval [blo, bhi] (long_window): the test |y1 - y2| <= cw1 +
 // cw2 holds exactly when blo1 <= bhi2 and blo2 <= bhi1.  The ends are rounded
 // outward (blo down, bhi up), so the two comparisons pass every pair the
-// real-valued test passes.  The kernel uses the FP32 records (pf_make, on the
-// device).
+// real-valued test passes.  For the host's check of the margins; the lists get
+// their FP32 records on the device (pf_make).
 inline void pf_record(const Derived &d, double px, double py, double pz, double E, double bm,
                       PfRec64 &r, double &bhi) {
     const LongWindow w = long_window(pf_maker(d, bm), pz, E, 1.1102230246251565e-16);
@@ -390,8 +386,7 @@ inline double psi_ref_of(const double *px, const double *py, int64_t b, int64_t 
 
 // Rapidity cut of the gathers (HBT_correlation.cpp:255-266, :468-476),
 // psi_ref per group (:181-183, :233-249; over all particles passed in), and
-// the fast lists.  Events keep < 2^18 particles (the fast kernel's
-// survivor encoding).
+// the fast lists.  Events keep < 2^18 particles (a limit of the entry points).
 inline int gather_particles(const Derived &d, const hbt_config &k, int ngroups,
                             const int32_t *grp_ev, int nev, const int64_t *ev_off,
                             const double *const soa[8], HostParticles &h, std::string &err,
