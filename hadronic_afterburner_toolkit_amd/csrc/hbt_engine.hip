@@ -601,8 +601,8 @@ int zero_hist(hbt_ctx *c) {
 // Pairs the device left to the host (K_phi within kphi_guard of a bin edge):
 // the host runs the same FP64 cascade with glibc's atan2 (kphi_index's host
 // build), as the reference does, and adds each pair it bins to the device
-// histogram.  Called after the stream is idle, before results are read.  A
-// capped run cannot place such a pair in the cap's order and fails instead.
+// histogram.  Called after the stream is idle, before results are read.  (The
+// ordered passes of a capped run collect such pairs themselves: CapDefer.)
 int resolve_deferred(hbt_ctx *c) {
     if (!c->P.azimuthal) return HBT_OK;  // only K_phi bins defer pairs
     HIPCHECK(c, hipStreamSynchronize(c->stream));

@@ -112,9 +112,19 @@ int hbt_reset(hbt_ctx *ctx);
  * kept particles resident in HBM.  slot 0 = same-event list, slot 1 = the
  * mixed-event list when read_in_real_mixed_events=1 (otherwise slot 1
  * aliases slot 0, particleSamples.cpp:528-531).  soa = {px,py,pz,E,x,y,z,t}.
- * The copies go through pinned host buffers that the context keeps (sized
- * to its largest upload) until hbt_destroy; the call returns once they are
- * done, so the caller may reuse its arrays at once. */
+ * The copies go through pinned host buffers that the context keeps until
+ * hbt_destroy, each sized to its largest use (two for uploads of groups, two
+ * per slot for one buffer, two for plans, one for results); the call returns
+ * once the caller's arrays have been read, so they may be reused at once.  One
+ * buffer of up to 65536 particles is sent to the device by the first call that
+ * needs it, so HBT_ERR_NOMEM may come from that call instead.
+ *
+ * Device memory kept until hbt_destroy beside the uploads: the histograms; on
+ * the fast kernel, once a call comes whose enumerated pairs might bind the pair
+ * cap (needed_number_of_pairs), a copy of them (64 bytes a bin: 26 MB for
+ * 41^3 x 6 bins, 2.1 GB for 61^3 x 9 x 16; a copy that cannot be allocated is
+ * done without, at the speed of the ordered passes); with slab binning the
+ * record regions. */
 int hbt_upload(hbt_ctx *ctx, int32_t slot, int32_t nev, const int64_t *ev_off,
                const double *const soa[8]);
 
@@ -259,9 +269,10 @@ int hbt_slab_info(hbt_ctx *ctx, int32_t *on, uint64_t *direct, uint64_t *capacit
 /* ---- allocation-free entry point ------------------------------------------
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops): the same-event
- * and mixed-event pairs of one buffer with the plain FP64 kernel -- what
- * hbt_upload + hbt_run_same + hbt_run_mixed do for a context created with
- * HBT_KERNEL_PLAIN, HBT_PREC_FP64 -- with every array in device memory owned
+ * and mixed-event pairs of one buffer in FP64 -- what hbt_upload +
+ * hbt_run_same + hbt_run_mixed do for a context created with
+ * HBT_KERNEL_PLAIN, HBT_PREC_FP64 (a prefilter in FP32 only discards pairs
+ * that its margins prove outside the bins) -- with every array in device memory owned
  * by the caller, launched on the caller's stream, and no allocation:
  *   ev_off[nev+1] (int64, device): event offsets into the soa columns;
  *   soa[8] (host array of device pointers): px py pz E x y z t of the
@@ -297,8 +308,10 @@ const char *hbt_noalloc_last_error(void);
 /* Launch shape of the fast kernel: R (1, 2, 4; accepted and kept, every tile
  * holds 64 i particles), j chunk of same-event tiles, partner windows per mixed work item (one per
  * plan row whose partner has particles in the tile's |pT| window),
- * persistent blocks per CU; ms is the measured batch time when set by
- * hbt_autotune. */
+ * persistent blocks per CU (a launch takes at most what a CU holds: four, or
+ * three of the FP64 K_phi / q_inv form and of slab-binned K_phi launches of
+ * many slabs; hbt_autotune reports the blocks launched); ms is the measured
+ * batch time when set by hbt_autotune. */
 typedef struct {
     int32_t R;
     int32_t jchunk;
