@@ -349,7 +349,7 @@ struct Slot {
     OrigRank *d_orig = nullptr;   // srt position -> fast-list index, gather rank
     size_t cap = 0, cap_f = 0, cap_ev = 0;
     double pmax2 = 0.0;     // max px^2+py^2 of kept particles
-    double bg = 0.0;        // max guard_beta of them
+    bool boosted = false;   // one of them is boosted
     hvec<int> srt_cell;           // px cell and py of the sorted copy (work-item windows)
     hvec<double> srt_py;
     bool valid = false;
@@ -724,7 +724,7 @@ int ensure(hbt_ctx *c, T **p, size_t &cap, size_t n) {
 
 void set_prefilter_margins(hbt_ctx *c) {
     prefilter_margins(c->D, std::max(c->slot[0].pmax2, mixed_slot(c).pmax2), c->P);
-    boost_guard(c->D, std::max(c->slot[0].bg, mixed_slot(c).bg), c->P);
+    boost_guard(c->D, c->slot[0].boosted || mixed_slot(c).boosted, c->P);
 }
 
 int upload_psi(hbt_ctx *c) {
@@ -1814,7 +1814,7 @@ int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
     for (int e = 0; e <= nev; e++) off[e] = ev_off[e] - o0;
     const double cut_max = tanh(c->cfg.HBTrap_max), cut_min = tanh(c->cfg.HBTrap_min);
     s.off.assign((size_t)nev + 1, 0);
-    std::vector<double> bg((size_t)nev, 0.0);
+    std::vector<char> far((size_t)nev, 0);
     const long long grain = std::max(1ll, 4096ll * nev / std::max(1ll, n_in));
     parallel_ranges(nev, grain, [&](long long e0, long long e1) {
         const int64_t b = ev_off[e0], n = ev_off[e1] - b;
@@ -1822,20 +1822,20 @@ int upload_direct(hbt_ctx *c, int32_t slot, const int32_t *grp, int32_t nev,
             std::memcpy(raw + a * col + (b - o0) * 8, soa[a] + b, (size_t)n * 8);
         for (long long e = e0; e < e1; e++) {
             long long kept = 0;
-            double b = 0.0;
+            bool b = false;
             for (int64_t i = ev_off[e]; i < ev_off[e + 1]; i++) {
-                if (!rapidity_kept(soa[2][i], soa[3][i], cut_min, cut_max)) continue;
-                kept++;
-                b = std::max(b, guard_beta(soa[2][i], soa[3][i]));
+                const bool k = rapidity_kept(soa[2][i], soa[3][i], cut_min, cut_max);
+                kept += k;
+                b |= k & boosted(soa[2][i], soa[3][i]);
             }
             s.off[e + 1] = kept;
-            bg[(size_t)e] = b;
+            far[(size_t)e] = b;
         }
     });
-    s.bg = 0.0;
+    s.boosted = false;
     for (int e = 0; e < nev; e++) {
         s.off[e + 1] += s.off[e];
-        s.bg = std::max(s.bg, bg[(size_t)e]);
+        s.boosted |= far[(size_t)e] != 0;
     }
     s.ngroups = 1;
     s.grp_ev.assign(grp, grp + 2);
@@ -1947,7 +1947,7 @@ int upload_slot(hbt_ctx *c, int32_t slot, int32_t ngroups, const int32_t *grp_ev
     s.pmax2 = h.pmax2;
     s.lists = true;
     if (again) return HBT_OK;
-    s.bg = h.bg;
+    s.boosted = h.boosted;
     s.ngroups = ngroups;
     s.grp_ev.assign(grp_ev, grp_ev + ngroups + 1);
     s.nev = nev;
@@ -2027,7 +2027,7 @@ PairArgs direct_pairs(hbt_ctx *c, bool same, int M) {
     const Slot &s = c->slot[0], &m = mixed_slot(c);
     PairArgs p{};
     p.v.P = c->P;
-    boost_guard(c->D, std::max(s.bg, m.bg), p.v.P);
+    boost_guard(c->D, s.boosted || m.boosted, p.v.P);
     p.v.H = hist_view(c);
     p.v.plan_cs = c->d_cs;
     pair_lists(p, s.list, m.list);

@@ -125,7 +125,8 @@ struct Part {
     std::vector<uint64_t> item_pairs;
     size_t next = 0;           // next item to launch
     uint64_t pairs_left = 0;   // enumerated pairs not yet launched
-    double pmax2 = 0.0, bg = 0.0;
+    double pmax2 = 0.0;
+    bool boosted = false;
     // device residency
     size_t foot = 0, arena_off = 0;
     size_t o_rec = 0, o_srec = 0, o_pf = 0, o_bw = 0, o_spf = 0, o_sbw = 0, o_orig = 0, o_win = 0,
@@ -286,7 +287,7 @@ void make_part_view(hbt_server *s, Part &p) {
     v.plan_cs = (const double *)(b + p.o_cs);
     v.psi = (const double *)(b + p.o_psi);
     v.P = s->D.P;
-    boost_guard(s->D, p.bg, v.P);
+    boost_guard(s->D, p.boosted, v.P);
 }
 
 // Uploads a part into its arena block on the upload stream (clearing the
@@ -956,7 +957,7 @@ int hbt_server_submit(hbt_server *s, int32_t nev, const int64_t *ev_off,
                                   ev_off + p.e0, soa, p.hp, err);
         if (rc == HBT_OK) {
             p.pmax2 = p.hp.pmax2;
-            p.bg = p.hp.bg;
+            p.boosted = p.hp.boosted;
             const long long r0 = rowoff[(size_t)p.e0];
             p.rowoff.resize((size_t)p.nev + 1);
             for (int e = 0; e <= p.nev; e++) p.rowoff[(size_t)e] = rowoff[(size_t)(p.e0 + e)] - r0;
